@@ -125,6 +125,34 @@ def test_gemm_generic_gives_few_rows_the_same_bits_as_many(shape):
     assert rel_err(few, plain_linear(x[:m].double().cpu(), w.double().cpu(), b.double().cpu())) < 5e-6
 
 
+@pytest.mark.parametrize("n,k", [(33, 5), (96, 513), (2046, 1026), (2064, 1028), (4200, 512), (500, 7000)])
+def test_gemm_generic_at_the_edges_of_its_kernels_and_gated(n, k):
+    """Rows around 8 (two blocks of K at once), 16, 32, 64 (tiles begin) and the tiles' sizes, matrices around 8 and 16 rows a
+    compute unit, ragged blocks of K and rows that no 16-byte load fits: the same bits whatever kernel runs, right against float64
+    (5e-6 of the largest value, as above), and with the gate applied
+    in the kernel what the activation kernel makes of the plain product."""
+    from tlie_amd import ops
+    torch.manual_seed(n + k)
+    x = torch.randn(300, k, device=DEV)
+    w = torch.randn(n, k, device=DEV) / math.sqrt(k)
+    b = torch.randn(n, device=DEV)
+    many = ops.gemm_generic(x, w, b, torch.float32).dense()
+    assert rel_err(many, plain_linear(x.double().cpu(), w.double().cpu(), b.double().cpu())) < 5e-6
+    for m in (1, 8, 9, 16, 17, 32, 33, 64, 65, 97, 128, 129):
+        rows = x[:m].contiguous()
+        few = ops.gemm_generic(rows, w, b, torch.float32)
+        assert torch.equal(few.dense(), many[:m]), m
+        if n % 2 == 0:
+            for gate in (None, ("clamped_swish", 1.7, 0.8)):
+                name, alpha, limit = gate or ("silu", 1.0, 0.0)
+                want = ops.silu_mul(few, torch.float32, interleaved=True, gate=name, alpha=alpha, limit=limit)
+                got = ops.gemm_generic(rows, w, b, torch.float32, gated=True, gate=gate)
+                assert got.shape == want.shape and rel_err(got, want) < 1e-6, (m, gate)
+    if n % 2:
+        with pytest.raises(Exception):
+            ops.gemm_generic(x, w, b, torch.float32, gated=True)
+
+
 @pytest.mark.parametrize("shape", [(65, 96, 64), (200, 2560, 2048), (333, 177, 200), (70, 129, 333), (1024, 2048, 5632)])
 def test_library_product_of_many_rows(shape):
     """The vendor library's product, called directly where it offers an algorithm (and through

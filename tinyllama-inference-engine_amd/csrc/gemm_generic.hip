@@ -1,208 +1,365 @@
-// y[M, N] = x[M, K] . W[N, K]^T (+ bias[N]) with every product and sum in true 32-bit: plain
-// v_fma_f32 on values widened to float, no matrix instruction, no reduced-precision mode.
+// y[M, N] = x[M, K] . W[N, K]^T (+ bias[N]) with every product and sum in true 32-bit, on the matrix
+// cores' 32-bit instruction (v_mfma_f32_16x16x4_f32): values widened to float, no reduced-precision mode.  Optionally the gated feed-forward's activation in the same kernel.
 //
 // reference: the only product of the reference's device path is a library call with 16-bit
 // inputs and 32-bit accumulation (GemmFp16RowMajor, src/cuda/kernels.cu:342-368); its 32-bit
-// model multiplies row by vector in a plain loop (src/model.cpp:65-72).  This kernel is that
-// plain loop, tiled through LDS: a 64x64 tile of y per 256-thread block, 16 columns of K per
-// step, each thread a 4x4 patch.
+// model multiplies row by vector in a plain loop (src/model.cpp:65-72).
+//
+// What a 32-bit matrix instruction computes was measured on an MI355X, on 250 thousand results each of
+// ordinary values, of exponents spread over 40 powers of two and of denormals: bit for bit the chain of fused
+// multiply-adds fma(a[k], b[k], .) in the order of k, starting from C.  So the kernels here give the bits that a
+// plain loop of v_fma_f32 over k gives, at twice its rate (packed 32-bit instructions are not used in this
+// library): 143 TFLOP/s over the chip in chains of such instructions.
 //
 // The order of the sum of one output is fixed by K alone: K is cut into blocks of 512 from index 0;
 // within a block the products are added one by one in index order (a chain of fused multiply-adds
 // that starts at zero), and the blocks' sums are added to a total, which starts at zero, in index
 // order.  Whatever M and N are, and whichever of the kernels below runs, an output gets the same
 // bits: a token's result does not depend on what else is in the batch.  (Blocks, and not one chain
-// over all of K, so that a product of few rows can give the blocks to different waves: a chain of
-// 5632 dependent multiply-adds alone takes longer than reading the whole matrix.)
+// over all of K, so that a product of few rows can give the blocks to different waves.)
 #include "common.h"
 
-#include <type_traits>
+#include <cmath>
 
 namespace tlie {
 
-constexpr int kTileM = 64, kTileN = 64, kTileK = 16;
-constexpr int kBlockK = 512;          // the blocks of K whose sums are formed apart (a multiple of every tile's width)
+typedef float floatx4 __attribute__((ext_vector_type(4)));
 
-template <typename X, typename W, typename O>
-__global__ void __launch_bounds__(256)
-gemm_generic_kernel(const X* __restrict__ x, const W* __restrict__ w, const W* __restrict__ bias,
-                    O* __restrict__ y, int M, int N, int K) {
-  __shared__ float xs[kTileK][kTileM + 4];
-  __shared__ float ws[kTileK][kTileN + 4];
-  const int m0 = blockIdx.y * kTileM, n0 = blockIdx.x * kTileN;
-  const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;   // patch: rows ty*4.., cols tx*4..
-  float acc[4][4] = {}, total[4][4] = {};
-  for (int k0 = 0; k0 < K; k0 += kTileK) {
-    // 64 rows x 16 k of each operand: 1024 values, 4 per thread
-    for (int i = threadIdx.x; i < kTileM * kTileK; i += 256) {
-      const int r = i / kTileK, c = i % kTileK;
-      const int m = m0 + r, n = n0 + r, k = k0 + c;
-      xs[c][r] = (m < M && k < K) ? to_float(x[static_cast<size_t>(m) * K + k]) : 0.f;
-      ws[c][r] = (n < N && k < K) ? to_float(w[static_cast<size_t>(n) * K + k]) : 0.f;
-    }
-    __syncthreads();
+constexpr int kBlockK = 512;          // the blocks of K whose sums are formed apart (a multiple of every tile's width)
+constexpr int kNoGate = -1;           // else a gate of common.h: W's rows alternate gate and up, y is [M, N / 2]
+
+// Four consecutive values of a row as floats; the row is `K` long and the four may reach past its end: what lies
+// there is read from inside the row and must be dropped by the caller.  WIDE: K and k are multiples of 4 and the
+// rows are aligned for four values, so the four lie all inside or all past the end.
+template <bool WIDE, typename T>
+__device__ __forceinline__ float4 fetch4(const T* __restrict__ row, int k, int K) {
+  if (WIDE) return load4(row + min(k, K - 4));
+  return make_float4(to_float(row[min(k, K - 1)]), to_float(row[min(k + 1, K - 1)]), to_float(row[min(k + 2, K - 1)]),
+                     to_float(row[min(k + 3, K - 1)]));
+}
+
+__device__ __forceinline__ float4 inside(float4 v, int k, int K) {
+  return make_float4(k < K ? v.x : 0.f, k + 1 < K ? v.y : 0.f, k + 2 < K ? v.z : 0.f, k + 3 < K ? v.w : 0.f);
+}
+
+__device__ __forceinline__ void swap32(float& a, float& b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  a = __uint_as_float(r[0]), b = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ void swap16(float& a, float& b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  a = __uint_as_float(r[0]), b = __uint_as_float(r[1]);
+}
+// A lane of the quarter g (lanes 16 g ..) holds the values 4 g .. 4 g + 3 of sixteen; afterwards it holds g, 4 + g, 8 + g,
+// 12 + g: what it gives to four matrix instructions of four k each, so that these take the k in their order.
+__device__ __forceinline__ void to_quarters(float4& v) {
+  swap32(v.x, v.z);
+  swap32(v.y, v.w);
+  swap16(v.x, v.y);
+  swap16(v.z, v.w);
+}
+
+// ---- few rows of x (decoding, short portions) ------------------------------------------------------------
+// Bound by reading W.  A workgroup owns R rows of W (columns of y) and all M <= 16 MT rows of x; its waves take the blocks
+// of K in turn, each block one chain of matrix instructions whose operands go straight from memory into registers: a
+// lane asks for 16 bytes of a row (a wave for 16 rows by 64 bytes) and four swaps between lanes put 16 k in the order of
+// the chain.  RING such loads of W are on their way per wave, and x (which comes from the caches) some ahead; no barrier
+// until the blocks' sums meet in LDS, where the first waves add them in index order and apply bias and gate.
+// PAIR (at most 8 rows of x, R = 8): of the instruction's 16 x 16 results two quarters of 8 x 8 are used, one for each of
+// two blocks of K: lanes 0 .. 7 of a sixteen bring both operands' rows from the one block, lanes 8 .. 15 from the other.
+// Twice the workgroups of R = 16, and no lane brings what another one has.
+template <typename X, typename W, typename O, int MT, int R, bool PAIR, int RING, int WAVES, bool WIDE>
+__global__ void __launch_bounds__(64 * WAVES)
+gemm_generic_few_kernel(const X* __restrict__ x, const W* __restrict__ w, const W* __restrict__ bias,
+                        O* __restrict__ y, int M, int N, int K, int gate, float alpha, float limit) {
+  static_assert(!PAIR || (MT == 1 && R == 8), "two blocks at once: 8 rows of W, 8 of x");
+  constexpr int SC = 8 / MT < RING / 2 ? 8 / MT : RING / 2;      // loads of x asked for together
+  constexpr int kJobK = PAIR ? 2 * kBlockK : kBlockK, kPartK = 16 * RING;
+  extern __shared__ __attribute__((aligned(16))) float sums[];   // [block][rows of x][R rows of W]
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+  const int r = lane & 15, g = lane >> 4;
+  const int n0 = blockIdx.x * R;
+  const W* w_row = w + static_cast<size_t>(min(n0 + r % R, N - 1)) * K;
+  const X* x_row[MT];
 #pragma unroll
-    for (int c = 0; c < kTileK; ++c) {
-      float a[4], b[4];
+  for (int i = 0; i < MT; ++i) x_row[i] = x + static_cast<size_t>(min(16 * i + (PAIR ? r & 7 : r), M - 1)) * K;
+  const int jobs = (K + kJobK - 1) / kJobK;                // of one block of K, or of two
+  const int first = (PAIR ? (r >> 3) * kBlockK : 0) + 4 * g;     // this lane's k within a job's first 16
+  float4 ring[RING], xs[2][SC][MT];
+  int k0 = wave * kJobK;
+  if (k0 < K) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = xs[c][ty * 4 + i];
+    for (int c = 0; c < SC; ++c)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) b[j] = ws[c][tx * 4 + j];
+      for (int i = 0; i < MT; ++i) xs[0][c][i] = fetch4<WIDE>(x_row[i], k0 + first + 16 * c, K);
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
-    }
-    if ((k0 + kTileK) % kBlockK == 0 || k0 + kTileK >= K) {     // a block of K ends: its sums join the totals
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) total[i][j] += acc[i][j], acc[i][j] = 0.f;
-    }
-    __syncthreads();
+    for (int c = 0; c < RING; ++c) ring[c] = fetch4<WIDE>(w_row, k0 + first + 16 * c, K);
   }
+  for (int job = wave; job < jobs; job += waves) {
+    const int end = min(job * kJobK + kBlockK, K);
+    floatx4 acc[MT];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int m = m0 + ty * 4 + i;
-    if (m >= M) continue;
+    for (int i = 0; i < MT; ++i) acc[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+    while (k0 < end) {                                     // (all of these the same for the whole wave)
+      const int next = k0 + kPartK < end ? k0 + kPartK : (job + waves) * kJobK;
+      const bool more = next < K, edge = k0 + kPartK + (PAIR ? kBlockK : 0) > K;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int n = n0 + tx * 4 + j;
-      if (n >= N) continue;
-      float v = total[i][j];
-      if (bias) v += to_float(bias[n]);
-      y[static_cast<size_t>(m) * N + n] = from_float<O>(v);
+      for (int c = 0; c < RING; ++c) {
+        if (c % SC == 0) {                                 // the next few pieces of x
+          const int to = (c / SC + 1) & 1;
+          const int from = (c + SC < RING ? k0 + 16 * (c + SC) : next) + first;
+          if (c + SC < RING || more) {
+#pragma unroll
+            for (int e = 0; e < SC; ++e)
+#pragma unroll
+              for (int i = 0; i < MT; ++i) xs[to][e][i] = fetch4<WIDE>(x_row[i], from + 16 * e, K);
+          }
+        }
+        float4 a = ring[c], b[MT];
+#pragma unroll
+        for (int i = 0; i < MT; ++i) b[i] = xs[(c / SC) & 1][c % SC][i];
+        if (edge) {                                        // past the end of K: zeros
+          a = inside(a, k0 + first + 16 * c, K);
+#pragma unroll
+          for (int i = 0; i < MT; ++i) b[i] = inside(b[i], k0 + first + 16 * c, K);
+        }
+        if (more) ring[c] = fetch4<WIDE>(w_row, next + first + 16 * c, K);
+        to_quarters(a);
+#pragma unroll
+        for (int i = 0; i < MT; ++i) to_quarters(b[i]);
+        // (last, behind every branch: see the kernel of many rows)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int i = 0; i < MT; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32((&a.x)[e], (&b[i].x)[e], acc[i], 0, 0, 0);
+      }
+      k0 = next;
+    }
+    // lane (r, g) holds what the instruction's rows 4 g .. 4 g + 3 (of W) have for its column r (of x)
+    if (PAIR) {
+      if ((r >> 3) == (g >> 1))
+        *reinterpret_cast<float4*>(sums + (2 * job + (r >> 3)) * 64 + (r & 7) * 8 + 4 * (g & 1)) = make_float4(acc[0][0], acc[0][1], acc[0][2], acc[0][3]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+        *reinterpret_cast<float4*>(sums + (job * MT + i) * 256 + r * 16 + 4 * g) = make_float4(acc[i][0], acc[i][1], acc[i][2], acc[i][3]);
+    }
+  }
+  __syncthreads();
+  const int blocks = (K + kBlockK - 1) / kBlockK;
+  constexpr int kQuads = R / 4, kRows = PAIR ? 8 : 16 * MT;
+  for (int t = threadIdx.x; t < kQuads * kRows; t += blockDim.x) {
+    const int m = t / kQuads, j = t % kQuads * 4, n = n0 + j;       // four neighbouring columns of y
+    if (m >= M || n >= N) continue;
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int b = 0; b < blocks; ++b) {                     // in index order
+      const float4 s = *reinterpret_cast<const float4*>(sums + (b * kRows + m) * R + j);
+      v.x += s.x, v.y += s.y, v.z += s.z, v.w += s.w;
+    }
+    const float out[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int e = 0; e < 4; e += 2) {
+      float p = out[e], u = out[e + 1];
+      if (n + e >= N) break;
+      if (bias) {
+        p += to_float(bias[n + e]);
+        if (n + e + 1 < N) u += to_float(bias[n + e + 1]);
+      }
+      if (gate != kNoGate) {
+        y[static_cast<size_t>(m) * (N / 2) + (n + e) / 2] = from_float<O>(gated_value(p, u, gate, alpha, limit));
+      } else {
+        y[static_cast<size_t>(m) * N + n + e] = from_float<O>(p);
+        if (n + e + 1 < N) y[static_cast<size_t>(m) * N + n + e + 1] = from_float<O>(u);
+      }
     }
   }
 }
 
-// The same sums for few rows of x (decoding, short portions): with M below 64 the tiles above leave
-// most of their threads idle and give the chip N / 64 workgroups, each walking K in steps of 16
-// between barriers.  Here a workgroup owns 16 columns of y and all M <= 16 * MT rows: a team of 256
-// threads, thread (n, m) adding up y[m + 16 i][n] for i < MT with the chain of the kernel above
-// (same blocks, same order: the same bits, so a step may take either).  TEAMS teams of a workgroup
-// take the blocks of K in turn (team t the blocks t, t + TEAMS, ...), leave their blocks' sums in
-// LDS, and the first team adds them up in index order.  W and x come through LDS in tiles of KT k,
-// kAhead tiles of W asked for ahead (the weights come from memory and nothing else occupies the
-// workgroup meanwhile), x, which comes from the caches, one tile ahead.
-constexpr int kFewN = 16;
-constexpr int kFewMaxBlocks = 16;      // blocks of K whose sums the teams can park in LDS (K up to 8192)
+// ---- many rows of x (prompts) ------------------------------------------------------------------------------
+// Bound by the matrix cores.  A workgroup of four waves makes TN columns by TM rows of y, a wave a quarter of that in
+// tiles of 16 by 16 (of 32 by 32, whose instruction is 5% faster alone, a wave would have one chain where it has four:
+// 11264 x 2048 at 1000 rows 475 us against 424); 32 k of both operands lie in LDS, twice, one barrier a turn; D turns'
+// loads are on their way in registers (a turn of a 64 x 64 tile is 0.4 us of products, a load from memory takes one to
+// two).  Within 16 k a row lies as 0 4 8 12 1 5 ..: one 16-byte read then gives a lane what four matrix instructions take
+// from it, in the order of k.  Rows are 36 floats apart, so that eight rows' reads cover the banks once.
+// Measured beside the plain multiply-adds before (64 x 64 tiles, loads a turn of 16 k ahead): 1000 rows by 11264 x 2048
+// 424 us against 805 (109 TFLOP/s), by 2048 x 5632 222 against 880, 2048 rows by 11264 x 2048 835 against 1489.
+constexpr int kStepK = 32, kStride = kStepK + 4;
 
-template <typename X, typename W, typename O, int MT, int TEAMS, int KT>
-__global__ void __launch_bounds__(256 * TEAMS)
-gemm_generic_few_kernel(const X* __restrict__ x, const W* __restrict__ w, const W* __restrict__ bias,
-                        O* __restrict__ y, int M, int N, int K) {
-  constexpr int kPer = KT / 16;                          // values of a tile's row a thread brings (8 or 4)
-  constexpr int kAhead = 4;
-  __shared__ __attribute__((aligned(16))) float ws[TEAMS][kFewN][KT + 4];
-  __shared__ __attribute__((aligned(16))) float xs[TEAMS][16 * MT][KT + 4];
-  __shared__ float sums[TEAMS > 1 ? kFewMaxBlocks : 1][256];
-  const int n0 = blockIdx.x * kFewN;
-  const int team = threadIdx.x >> 8, t = threadIdx.x & 255;
-  const int tn = t % 16, tm = t / 16;
-  const int load_row = t / 16, load_col = (t % 16) * kPer;
-  const int blocks = (K + kBlockK - 1) / kBlockK;
-  constexpr int kTilesPerBlock = kBlockK / KT;
-  const int rounds = (blocks + TEAMS - 1) / TEAMS;       // every team walks so many blocks (the last may be beyond K: zeros)
-  const int tiles = rounds * kTilesPerBlock;
-  // tile q of this team: block (q / tiles per block) * TEAMS + team, k from block * 512 + (q % tiles per block) * KT
-  auto tile_k = [&](int q) { return ((q / kTilesPerBlock) * TEAMS + team) * kBlockK + (q % kTilesPerBlock) * KT; };
-  float w_ring[kAhead][kPer], x_next[MT][kPer];
-  // (whole 16-byte loads where the rows allow them: both operands float, K a multiple of 4, bases aligned)
-  const bool wide = std::is_same<X, float>::value && std::is_same<W, float>::value && (K & 3) == 0 &&
-                    ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) & 15) == 0;
-  auto fetch_row = [&](float (&out)[kPer], const auto* base, bool live, int k) {
-    using Source = std::remove_cv_t<std::remove_pointer_t<decltype(base)>>;
-    if (std::is_same<Source, float>::value && wide && k + kPer <= K) {
+template <typename X, typename W, typename O, int TN, int TM, int D, bool WIDE>
+__global__ void __launch_bounds__(256)
+gemm_generic_kernel(const X* __restrict__ x, const W* __restrict__ w, const W* __restrict__ bias,
+                    O* __restrict__ y, int M, int N, int K, int gate, float alpha, float limit) {
+  constexpr int A = TN / 32, B = TM / 32;            // a wave's tiles
+  extern __shared__ __attribute__((aligned(16))) float lds[];
+  float* ws = lds;                                         // [2][TN][kStride]
+  float* xs = lds + 2 * TN * kStride;                      // [2][TM][kStride]
+  // workgroups go to the chip's eight dies in turn: each die gets a stretch of neighbouring tiles, rows of y first, so
+  // that its cache holds their rows of W
+  const int m_tiles = (M + TM - 1) / TM, tiles = m_tiles * ((N + TN - 1) / TN);
+  const int each = tiles / 8, over = tiles % 8, die = blockIdx.x % 8;
+  const int tile = die * each + min(die, over) + blockIdx.x / 8;
+  const int n0 = tile / m_tiles * TN, m0 = tile % m_tiles * TM;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int row = threadIdx.x >> 3, piece = threadIdx.x & 7;           // 32 rows a pass, eight 16-byte pieces a row
+  const W* w_row[TN / 32];
+  const X* x_row[TM / 32];
 #pragma unroll
-      for (int j = 0; j < kPer; j += 4) {
-        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (live) v = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(base) + k + j);
-        out[j] = v.x, out[j + 1] = v.y, out[j + 2] = v.z, out[j + 3] = v.w;
-      }
-      return;
+  for (int p = 0; p < TN / 32; ++p) w_row[p] = w + static_cast<size_t>(min(n0 + row + 32 * p, N - 1)) * K;
+#pragma unroll
+  for (int p = 0; p < TM / 32; ++p) x_row[p] = x + static_cast<size_t>(min(m0 + row + 32 * p, M - 1)) * K;
+  float4 w_next[D][TN / 32], x_next[D][TM / 32];
+  auto ask = [&](int slot, int step) {
+    const int k = step * kStepK + 4 * piece;
+#pragma unroll
+    for (int p = 0; p < TN / 32; ++p) w_next[slot][p] = fetch4<WIDE>(w_row[p], k, K);
+#pragma unroll
+    for (int p = 0; p < TM / 32; ++p) x_next[slot][p] = fetch4<WIDE>(x_row[p], k, K);
+  };
+  auto put_row = [&](float* at, const float4& v) {
+    at += (piece >> 2) * 16 + (piece & 3);
+    at[0] = v.x, at[4] = v.y, at[8] = v.z, at[12] = v.w;
+  };
+  auto put = [&](int slot, int step) {
+    const int k = step * kStepK + 4 * piece, buffer = step & 1;
+    if (step * kStepK + kStepK > K) {                      // (the last: what lies past K is zero)
+#pragma unroll
+      for (int p = 0; p < TN / 32; ++p) w_next[slot][p] = inside(w_next[slot][p], k, K);
+#pragma unroll
+      for (int p = 0; p < TM / 32; ++p) x_next[slot][p] = inside(x_next[slot][p], k, K);
     }
 #pragma unroll
-    for (int j = 0; j < kPer; ++j) out[j] = (live && k + j < K) ? to_float(base[k + j]) : 0.f;
+    for (int p = 0; p < TN / 32; ++p) put_row(ws + (buffer * TN + row + 32 * p) * kStride, w_next[slot][p]);
+#pragma unroll
+    for (int p = 0; p < TM / 32; ++p) put_row(xs + (buffer * TM + row + 32 * p) * kStride, x_next[slot][p]);
   };
-  auto fetch_w = [&](float (&out)[kPer], int q) {
-    const int n = n0 + load_row;
-    fetch_row(out, w + static_cast<size_t>(min(n, N - 1)) * K, n < N, tile_k(q) + load_col);
-  };
-  auto fetch_x = [&](int q) {
+  floatx4 acc[A][B] = {}, total[A][B] = {};
+  const int steps = (K + kStepK - 1) / kStepK;
+  const float* my_w = ws + ((wave & 1) * (TN / 2) + (lane & 15)) * kStride + (lane >> 4) * 4;
+  const float* my_x = xs + ((wave >> 1) * (TM / 2) + (lane & 15)) * kStride + (lane >> 4) * 4;
+  // (the matrix instructions stand last in a turn, behind every branch: this compiler has been seen to read their results
+  // too early, without the wait they need, where a branch lay between)
 #pragma unroll
-    for (int i = 0; i < MT; ++i) {
-      const int m = load_row + 16 * i;
-      fetch_row(x_next[i], x + static_cast<size_t>(min(m, M - 1)) * K, m < M, tile_k(q) + load_col);
-    }
-  };
-  float acc[MT], total[MT];
+  for (int j = 0; j < D; ++j)
+    if (j < steps) ask(j, j);
+  put(0, 0);
+  if (D < steps) ask(0, D);
+  for (int base = 0; base < steps; base += D) {
 #pragma unroll
-  for (int i = 0; i < MT; ++i) acc[i] = 0.f, total[i] = 0.f;
+    for (int j = 0; j < D; ++j) {
+      const int s = base + j;
+      if (s >= steps) break;                               // (the same for the whole workgroup)
+      lds_barrier();                                       // this turn's tiles are whole, the last turn's have been read
+      if (s > 0 && s % (kBlockK / kStepK) == 0) {          // a block of K has ended: its sums join the totals
 #pragma unroll
-  for (int j = 0; j < kAhead; ++j)
-    if (j < tiles) fetch_w(w_ring[j], j);
-  fetch_x(0);
-  for (int base = 0; base < tiles; base += kAhead) {
+        for (int i = 0; i < A; ++i)
 #pragma unroll
-    for (int j = 0; j < kAhead; ++j) {
-      const int q = base + j;
-      if (q >= tiles) break;                               // (the same for the whole workgroup)
-      __syncthreads();                                     // the last tile has been used
-#pragma unroll
-      for (int e = 0; e < kPer; e += 4)
-        *reinterpret_cast<float4*>(&ws[team][load_row][load_col + e]) = make_float4(w_ring[j][e], w_ring[j][e + 1], w_ring[j][e + 2], w_ring[j][e + 3]);
-#pragma unroll
-      for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int e = 0; e < kPer; e += 4)
-          *reinterpret_cast<float4*>(&xs[team][load_row + 16 * i][load_col + e]) = make_float4(x_next[i][e], x_next[i][e + 1], x_next[i][e + 2], x_next[i][e + 3]);
-      __syncthreads();
-      if (q + kAhead < tiles) fetch_w(w_ring[j], q + kAhead);
-      if (q + 1 < tiles) fetch_x(q + 1);
-      // (beyond K a tile holds zeros, as the tiles of the kernel above do: adding them changes nothing;
-      // eight steps unrolled: the reads from LDS of several steps are asked for together, ahead of the
-      // chain of multiply-adds that waits for them)
-#pragma unroll 8
-      for (int c = 0; c < KT; c += 4) {
-        const float4 b = *reinterpret_cast<const float4*>(&ws[team][tn][c]);
-#pragma unroll
-        for (int i = 0; i < MT; ++i) {
-          const float4 a = *reinterpret_cast<const float4*>(&xs[team][tm + 16 * i][c]);
-          acc[i] = fmaf(a.x, b.x, acc[i]);
-          acc[i] = fmaf(a.y, b.y, acc[i]);
-          acc[i] = fmaf(a.z, b.z, acc[i]);
-          acc[i] = fmaf(a.w, b.w, acc[i]);
-        }
+          for (int u = 0; u < B; ++u) total[i][u] += acc[i][u], acc[i][u] = floatx4{};
       }
-      if (q % kTilesPerBlock == kTilesPerBlock - 1) {     // the team's block ends
-        const int block = (q / kTilesPerBlock) * TEAMS + team;
-        if (TEAMS == 1) {
+      if (s + 1 < steps) put((j + 1) % D, s + 1);
+      if (s + 1 + D < steps) ask((j + 1) % D, s + 1 + D);
+      const float* wt = my_w + (s & 1) * TN * kStride;
+      const float* xt = my_x + (s & 1) * TM * kStride;
 #pragma unroll
-          for (int i = 0; i < MT; ++i) total[i] += acc[i];
-        } else if (block < blocks) {
-          sums[block][t] = acc[0];
-        }
+      for (int e = 0; e < kStepK; e += 16) {
+        float4 a[A], b[B];
 #pragma unroll
-        for (int i = 0; i < MT; ++i) acc[i] = 0.f;
+        for (int i = 0; i < A; ++i) a[i] = *reinterpret_cast<const float4*>(wt + 16 * i * kStride + e);
+#pragma unroll
+        for (int i = 0; i < B; ++i) b[i] = *reinterpret_cast<const float4*>(xt + 16 * i * kStride + e);
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+          for (int i = 0; i < A; ++i)
+#pragma unroll
+            for (int u = 0; u < B; ++u) acc[i][u] = __builtin_amdgcn_mfma_f32_16x16x4f32((&a[i].x)[c], (&b[u].x)[c], acc[i][u], 0, 0, 0);
       }
     }
   }
-  if (TEAMS > 1) {
-    __syncthreads();
-    if (team != 0) return;
-    for (int b = 0; b < blocks; ++b) total[0] += sums[b][t];   // in index order
-  }
-  const int n = n0 + tn;
-  if (n >= N) return;
 #pragma unroll
-  for (int i = 0; i < MT; ++i) {
-    const int m = tm + 16 * i;
-    if (m >= M) continue;
-    float v = total[i];
-    if (bias) v += to_float(bias[n]);
-    y[static_cast<size_t>(m) * N + n] = from_float<O>(v);
+  for (int i = 0; i < A; ++i)
+#pragma unroll
+    for (int u = 0; u < B; ++u) total[i][u] += acc[i][u];
+  // a lane holds four neighbouring columns of one row of each tile
+  const bool whole = (N & 3) == 0;
+#pragma unroll
+  for (int i = 0; i < A; ++i)
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+      const int m = m0 + (wave >> 1) * (TM / 2) + 16 * u + (lane & 15);
+      const int n = n0 + (wave & 1) * (TN / 2) + 16 * i + 4 * (lane >> 4);
+      if (m >= M || n >= N) continue;
+      float v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        v[e] = total[i][u][e];
+        if (bias && n + e < N) v[e] += to_float(bias[n + e]);
+      }
+      if (gate != kNoGate) {
+        O* at = y + static_cast<size_t>(m) * (N / 2) + n / 2;
+        at[0] = from_float<O>(gated_value(v[0], v[1], gate, alpha, limit));
+        if (n + 2 < N) at[1] = from_float<O>(gated_value(v[2], v[3], gate, alpha, limit));
+      } else if (whole) {
+        store4(y + static_cast<size_t>(m) * N + n, v[0], v[1], v[2], v[3]);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (n + e < N) y[static_cast<size_t>(m) * N + n + e] = from_float<O>(v[e]);
+      }
+    }
+}
+
+template <typename X, typename W, typename O, int MT, int R, bool PAIR, int RING, int WAVES, bool WIDE>
+int launch_few(const X* x, const W* w, const W* bias, O* y, int M, int N, int K, int gate, float alpha, float limit, hipStream_t s) {
+  const int job_k = PAIR ? 2 * kBlockK : kBlockK, jobs = (K + job_k - 1) / job_k, turns = (jobs + WAVES - 1) / WAVES;
+  const int waves = (jobs + turns - 1) / turns;            // as many for each turn
+  const int bytes = jobs * (PAIR ? 2 * 64 : 16 * MT * R) * static_cast<int>(sizeof(float));
+  hipLaunchKernelGGL((gemm_generic_few_kernel<X, W, O, MT, R, PAIR, RING, WAVES, WIDE>), dim3((N + R - 1) / R), dim3(64 * waves), bytes, s,
+                     x, w, bias, y, M, N, K, gate, alpha, limit);
+  return launch_status();
+}
+
+template <typename X, typename W, typename O, int TN, int TM, int D, bool WIDE>
+int launch_tiles(const X* x, const W* w, const W* bias, O* y, int M, int N, int K, int gate, float alpha, float limit, hipStream_t s) {
+  const long long tiles = static_cast<long long>((M + TM - 1) / TM) * ((N + TN - 1) / TN);
+  if (tiles > 0x7fffffff) return kBadArgument;
+  constexpr int kBytes = 2 * (TN + TM) * kStride * static_cast<int>(sizeof(float));
+  static_assert(kBytes <= 64 * 1024, "within what a launch may ask for without an attribute");
+  hipLaunchKernelGGL((gemm_generic_kernel<X, W, O, TN, TM, D, WIDE>), dim3(static_cast<unsigned>(tiles)), dim3(256), kBytes, s, x, w, bias,
+                     y, M, N, K, gate, alpha, limit);
+  return launch_status();
+}
+
+template <typename X, typename W, typename O, bool WIDE>
+int launch_product(const X* x, const W* w, const W* bias, O* y, int M, int N, int K, int gate, float alpha, float limit,
+                   int compute_units, hipStream_t s) {
+  const long long blocks = (K + kBlockK - 1) / kBlockK;
+  // Few rows of x: the kernel that reads W straight into registers, while the sums of the blocks fit LDS.  A matrix of at
+  // most 8 rows a compute unit takes two blocks at once (2048 x 2048, 8 rows of x: 10.1 us against 12.0; 2560 x 2048, where
+  // some units would get two workgroups: 14.8 against 12.3).  More than 16 rows of x go there only while W has at most 16 rows
+  // a unit: every workgroup reads all of x (64 rows, 2048 x 2048: 24.7 us against 34.4 in tiles; 11264 x 2048: 70.1 against 46.1).
+  // One block of K or less gives a workgroup one wave: such products go in tiles (96 x 96, 16 rows: 3.3 us against 4.0).
+  const int mt = M <= 16 ? 1 : (M <= 32 ? 2 : 4);
+  if (M <= 64 && blocks > 1 && blocks * mt * 1024 <= 64 * 1024 && (mt == 1 || (N + 15) / 16 <= compute_units)) {
+    constexpr int kRing = WIDE ? 16 : 8;
+    if (mt == 4) return launch_few<X, W, O, 4, 16, false, 8, 8, WIDE>(x, w, bias, y, M, N, K, gate, alpha, limit, s);
+    if (mt == 2) return launch_few<X, W, O, 2, 16, false, 8, WIDE ? 12 : 8, WIDE>(x, w, bias, y, M, N, K, gate, alpha, limit, s);
+    if (M <= 8 && (N + 7) / 8 <= compute_units) return launch_few<X, W, O, 1, 8, true, kRing, 12, WIDE>(x, w, bias, y, M, N, K, gate, alpha, limit, s);
+    return launch_few<X, W, O, 1, 16, false, kRing, 12, WIDE>(x, w, bias, y, M, N, K, gate, alpha, limit, s);
   }
+  // Tiles of 64 x 64, 64 x 32 or 32 x 32: alone on its compute unit a tile takes 50, 40 or 35 us for K = 2048 (the way of its
+  // loads), of which its products are 28.6, 14.3 and 7.2; several tiles to a unit reach 0.75, 0.69 and 0.62 of the matrix
+  // cores' rate (measured at 11264 x 2048 and 1000 rows: 424, 459 and 510 us).  The least of the three estimates:
+  const double rows[3] = {64, 64, 32}, cols[3] = {64, 32, 32}, alone[3] = {50, 40, 35}, busy[3] = {28.6 / 0.75, 14.3 / 0.69, 7.2 / 0.62};
+  int best = 0;
+  double least = 0;
+  for (int i = 0; i < 3; ++i) {
+    const double tiles = ceil(N / rows[i]) * ceil(M / cols[i]), time = fmax(alone[i], busy[i] * ceil(tiles / compute_units));
+    if (i == 0 || time < least) best = i, least = time;
+  }
+  if (best == 0) return launch_tiles<X, W, O, 64, 64, 2, WIDE>(x, w, bias, y, M, N, K, gate, alpha, limit, s);
+  if (best == 1) return launch_tiles<X, W, O, 64, 32, 4, WIDE>(x, w, bias, y, M, N, K, gate, alpha, limit, s);
+  return launch_tiles<X, W, O, 32, 32, 4, WIDE>(x, w, bias, y, M, N, K, gate, alpha, limit, s);
 }
 
 }  // namespace tlie
@@ -210,27 +367,18 @@ gemm_generic_few_kernel(const X* __restrict__ x, const W* __restrict__ w, const 
 using namespace tlie;
 
 extern "C" int tlie_gemm_generic(const void* x, int x_dtype, const void* w, int w_dtype, const void* bias,
-                                 void* y, int y_dtype, int M, int N, int K, void* stream) {
-  if (M <= 0 || N <= 0 || K <= 0) return kBadArgument;
-  const dim3 grid((N + kTileN - 1) / kTileN, (M + kTileM - 1) / kTileM);
-  if (grid.y > 65535) return kBadArgument;
+                                 void* y, int y_dtype, int M, int N, int K, int gate, float alpha, float limit, int compute_units,
+                                 void* stream) {
+  if (M <= 0 || N <= 0 || K <= 0 || compute_units <= 0) return kBadArgument;
+  if (gate < kNoGate || gate > kGateClampedSwish || (gate != kNoGate && N % 2 != 0)) return kBadArgument;
   hipStream_t s = (hipStream_t)stream;
-  const dim3 few((N + kFewN - 1) / kFewN);
 #define TLIE_CASE(XC, X, WC, W, OC, O)                                                                       \
   if (x_dtype == XC && w_dtype == WC && y_dtype == OC) {                                                     \
-    if (M <= 16 && K >= 2 * kBlockK && K <= kFewMaxBlocks * kBlockK)                                         \
-      hipLaunchKernelGGL((gemm_generic_few_kernel<X, W, O, 1, 4, 64>), few, dim3(1024), 0, s, (const X*)x,    \
-                         (const W*)w, (const W*)bias, (O*)y, M, N, K);                                       \
-    else if (M <= 16)                                                                                        \
-      hipLaunchKernelGGL((gemm_generic_few_kernel<X, W, O, 1, 1, 128>), few, dim3(256), 0, s, (const X*)x,    \
-                         (const W*)w, (const W*)bias, (O*)y, M, N, K);                                       \
-    else if (M <= 64)                                                                                        \
-      hipLaunchKernelGGL((gemm_generic_few_kernel<X, W, O, 4, 1, 128>), few, dim3(256), 0, s, (const X*)x,    \
-                         (const W*)w, (const W*)bias, (O*)y, M, N, K);                                       \
-    else                                                                                                     \
-      hipLaunchKernelGGL((gemm_generic_kernel<X, W, O>), grid, dim3(256), 0, s, (const X*)x, (const W*)w,     \
-                         (const W*)bias, (O*)y, M, N, K);                                                    \
-    return launch_status();                                                                                  \
+    /* four values of a row in one load where every row of both operands is aligned for it */               \
+    const bool wide = (K & 3) == 0 && reinterpret_cast<uintptr_t>(x) % (4 * sizeof(X)) == 0 &&               \
+                      reinterpret_cast<uintptr_t>(w) % (4 * sizeof(W)) == 0;                                 \
+    return wide ? launch_product<X, W, O, true>((const X*)x, (const W*)w, (const W*)bias, (O*)y, M, N, K, gate, alpha, limit, compute_units, s)   \
+                : launch_product<X, W, O, false>((const X*)x, (const W*)w, (const W*)bias, (O*)y, M, N, K, gate, alpha, limit, compute_units, s); \
   }
   TLIE_CASE(kF32, float, kF32, float, kF32, float)
   TLIE_CASE(kBF16, bf16, kBF16, bf16, kBF16, bf16)

@@ -1605,8 +1605,11 @@ def pass_input(residual: torch.Tensor, tokens: torch.Tensor, table: torch.Tensor
     return out
 
 
-def gemm_generic(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, out_dtype: torch.dtype) -> Product:
-    """y = x . W^T (+ bias), every product and sum in true 32-bit.  W is [out, in]."""
+def gemm_generic(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, out_dtype: torch.dtype, gated: bool = False,
+                 gate=None):
+    """y = x . W^T (+ bias), every product and sum in true 32-bit.  W is [out, in].  gated: W's rows alternate gate and up,
+    and the kernel stores silu(gate) * up [rows, out / 2], which is returned as a tensor; gate: (name, alpha, limit) of
+    another gate than SiLU (see `silu_mul`)."""
     _device_tensor(x, "x", (torch.float32, torch.bfloat16))
     _device_tensor(weight, "weight", (torch.float32, torch.bfloat16))
     if x.dim() != 2 or weight.dim() != 2 or x.shape[1] != weight.shape[1]:
@@ -1615,13 +1618,15 @@ def gemm_generic(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | Non
         _device_tensor(bias, "bias", weight.dtype)
         if bias.shape != (weight.shape[0],):
             raise invalid_shape("gemm: bias needs one entry per output")
-    out = torch.empty((x.shape[0], weight.shape[0]), dtype=out_dtype, device=x.device)
-    if x.shape[0] == 0:
-        return Product(out, 1)
-    _check(library().tlie_gemm_generic(_ptr(x), dtype_code(x.dtype), _ptr(weight), dtype_code(weight.dtype), _ptr(bias),
-                                       _ptr(out), dtype_code(out_dtype), x.shape[0], weight.shape[0], x.shape[1],
-                                       _stream()), "gemm_generic")
-    return Product(out, 1)
+    if gated and weight.shape[0] % 2 != 0:
+        raise invalid_shape("gemm: the gated product needs an even number of rows of W")
+    kind, alpha, limit = _gate_args(gate)
+    out = torch.empty((x.shape[0], weight.shape[0] // 2 if gated else weight.shape[0]), dtype=out_dtype, device=x.device)
+    if x.shape[0] > 0:
+        _check(library().tlie_gemm_generic(_ptr(x), dtype_code(x.dtype), _ptr(weight), dtype_code(weight.dtype), _ptr(bias),
+                                           _ptr(out), dtype_code(out_dtype), x.shape[0], weight.shape[0], x.shape[1],
+                                           kind if gated else -1, alpha, limit, _compute_units(x.device), _stream()), "gemm_generic")
+    return out if gated else Product(out, 1)
 
 
 # state: None (not tried), True, False (not there); fallbacks: products that took this library's plain kernel instead

@@ -2,7 +2,8 @@
 (src/model.cpp:65-72; src/cuda/kernels.cu:359-363).
 
 Which kernel runs is decided here and nowhere else:
-  float32 activations            the true 32-bit kernel (plain FMAs, no matrix instruction)
+  float32 activations            the true 32-bit kernel (32-bit matrix instructions: the bits of plain FMAs), which also
+                                 applies the gated feed-forward's gate itself
   bfloat16, weight kept float32  the same kernel on widened values
   bfloat16, at most 16 rows      the rows kernel when the caller folds something in: the norm before the
                                  product, the SiLU gate or the add into the residual after it
@@ -83,4 +84,4 @@ class Linear:
                 # once: in the library's own kernel, or where it offers none for that in a kernel of this library
                 return Product(ops.library_mm(x, self.weight, out_dtype, bias=self.bias), 1)
             return Product(ops.library_mm(x, self.weight, out_dtype), 1)   # (float32: the output head's logits for many rows)
-        return ops.gemm_generic(x, self.weight, self.bias, out_dtype)
+        return ops.gemm_generic(x, self.weight, self.bias, out_dtype, gated=gated and self.out_features % 2 == 0, gate=gate)
