@@ -257,6 +257,42 @@ def test_attention_generic(dtype, case):
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("case", [
+    dict(nq=32, nkv=4, d=64, page=16), dict(nq=32, nkv=4, d=64, page=32, window=90), dict(nq=24, nkv=8, d=32, page=16, chunk=100, sink=True),
+    dict(nq=64, nkv=2, d=16, page=16), dict(nq=20, nkv=4, d=48, page=16), dict(nq=32, nkv=8, d=64, page=8, softcap=4.0, sink=True),
+])
+def test_the_three_forms_of_the_plain_attention_kernel_give_the_same_bits(dtype, case):
+    """Head sizes up to 64: a workgroup a token and head (few tokens), a token and key head (many tokens of one each), or 64
+    columns (several tokens a sequence).  Sizes known to the kernel beforehand and others; the last position's value of one key
+    head is infinite, which no earlier token may notice."""
+    from tlie_amd import ops
+    nq, nkv, d, page = case["nq"], case["nkv"], case["d"], case["page"]
+    window, chunk, softcap = case.get("window"), case.get("chunk"), case.get("softcap")
+    tokens = 333
+    torch.manual_seed(nq + d)
+    q, k, v = torch.randn(tokens, nq, d), torch.randn(tokens, nkv, d), torch.randn(tokens, nkv, d)
+    v[-1, 0, 3] = math.inf
+    cache, pages = build_cache(k, v, page, DT[dtype], shuffle_seed=d)
+    table = torch.tensor([pages], dtype=torch.int32, device=DEV)
+    sink = torch.randn(nq, device=DEV) if case.get("sink") else None
+
+    def run(rows, tiled):
+        return ops.attention_generic(q[rows].to(DT[dtype]).reshape(len(rows), nq * d).to(DEV).contiguous(), cache.to(DEV), table,
+                                     torch.zeros(len(rows), dtype=torch.int32, device=DEV), torch.tensor(rows, dtype=torch.int32, device=DEV),
+                                     nq, nkv, d, window, 1.0 / math.sqrt(d), tiled=tiled, chunk=chunk, sink=sink, softcap=softcap)
+    every = list(range(tokens))
+    shared, grouped = run(every, True), run(every, False)
+    assert len(every) * nq >= 4 * 256 and nq > nkv                                     # (what sends them to the second form)
+    assert torch.isfinite(shared[:-1].float()).all() and not torch.isfinite(shared[-1].float()).all()
+    assert torch.equal(shared[:-1], grouped[:-1]) and torch.equal(shared[-1].nan_to_num(1e9), grouped[-1].nan_to_num(1e9))
+    some = [0, 1, page - 1, page, 63, 64, 200, 255, 256, 331]
+    assert torch.equal(run(some, False), shared[some])                                 # (a workgroup a token and head)
+    if sink is None and chunk is None and softcap is None:
+        want = plain_attention(rounded(q, DT[dtype]), rounded(k, DT[dtype]), rounded(v, DT[dtype]), window=window)
+        assert rel_err(shared.view(tokens, nq, d)[:-1], want[:-1]) < TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("case", [
     dict(nq=8, nkv=2, d=64, page=16, window=None), dict(nq=6, nkv=3, d=48, page=16, window=70),
     dict(nq=5, nkv=5, d=7, page=8, window=None), dict(nq=40, nkv=1, d=16, page=16, window=300),   # 40 heads a group: two blocks of heads
 ])

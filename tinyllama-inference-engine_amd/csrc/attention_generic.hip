@@ -33,7 +33,7 @@ namespace tlie {
 // in the order of their index; at the end the groups' results are put together in the order of
 // the groups.  Which keys meet in which sum, and in which order, depends on the positions alone.
 // seq_start (or null) with min_tokens: the step's cumulative token counts per sequence; tokens of
-// sequences that bring min_tokens tokens or more are then left to the tiled kernel below, which
+// sequences that bring min_tokens tokens or more are then left to the kernel of many tokens below, which
 // is launched beside this one for the same step and leaves the others to this one.
 // The attended values go out in the activation type, or, when the caller works on with them in 32-bit (two
 // maps of attention whose difference is normed), as floats: `out` then points to floats whatever T is.
@@ -187,223 +187,541 @@ attention_generic_kernel(const T* __restrict__ q, const T* __restrict__ cache, c
   }
 }
 
-// The same attention for steps that bring several tokens of a sequence (prompt portions): a
-// workgroup serves up to 32 columns, a column being a (token, query head) pair, of up to 32 / heads
-// consecutive tokens of the step and the heads of one kv head (or 32 of them), and brings every
-// chunk of 64 keys and values through LDS once for all of them, where the kernel above reads
-// each key and value again for every column (a prompt of 2048 tokens: 34 GB of cache traffic a layer).
-//
-// The arithmetic of a column is the kernel's above, operation for operation: chunk c of the context
-// belongs to running state c % 4 (there: to thread group c % 4), a chunk's scores are 64 dot products
-// summed in the order of the dims, its maximum and sum are the same reductions over a wave, the
-// values are added in the order of the keys, and the four states meet in the same order at the end.
-// A column therefore gets the same bits from either kernel, and a step may take whichever is faster.
-// Head sizes (of keys and of values) up to 64.  Tokens of a workgroup that belong to different sequences are served one
-// run of equal sequences after the other.
-constexpr int kTiledCols = 32, kTiledWaves = 8, kTiledSlots = kTiledCols / kTiledWaves;     // columns a workgroup, its waves, columns a wave
+// ---- head sizes up to 64, on the matrix cores' 32-bit instruction ------------------------------------------
+// v_mfma_f32_16x16x4_f32 gives, bit for bit, the chain of fused multiply-adds over k in their order, starting from C
+// (measured; see the 32-bit products).  Scores are therefore instructions over a head's dims, and values instructions over
+// a chunk's keys that continue a state's sums: the sums of the kernel above, operation for operation.  A column, a (token,
+// query head) pair, is one of an instruction's sixteen; chunk c of 64 keys belongs to the column's running state c % 4; the
+// maximum and the sum of a chunk's probabilities are taken over the key's bits in the order wave_sum takes them; the four
+// states meet in the same order at the end.  Both kernels below and the one above give a column the same bits, and a step may
+// take whichever is faster.
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ void swap32(float& a, float& b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  a = __uint_as_float(r[0]), b = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ void swap16(float& a, float& b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  a = __uint_as_float(r[0]), b = __uint_as_float(r[1]);
+}
+// A lane of the quarter g (lanes 16 g ..) holds the values 4 g .. 4 g + 3 of sixteen; afterwards it holds g, 4 + g, 8 + g,
+// 12 + g: what it gives to four instructions of four k each, so that these take the k in their order.
+__device__ __forceinline__ void to_quarters(float (&v)[4]) {
+  swap32(v[0], v[2]);
+  swap32(v[1], v[3]);
+  swap16(v[0], v[1]);
+  swap16(v[2], v[3]);
+}
+// The sum and the maximum with the lane 32 (then 16) away: for keys, with the key whose bit 3 (then bit 2) differs.
+__device__ __forceinline__ float sum_quarters(float v) {
+  float a = v, b = v;
+  swap32(a, b);
+  v = a + b, a = v, b = v;
+  swap16(a, b);
+  return a + b;
+}
+__device__ __forceinline__ float max_quarters(float v) {
+  float a = v, b = v;
+  swap32(a, b);
+  v = fmaxf(a, b), a = v, b = v;
+  swap16(a, b);
+  return fmaxf(a, b);
+}
+
+// Four values of a row from i on, of which `count` exist (the others are zero and not read).  `wide`: four that exist lie
+// aligned for one load.
 template <typename T>
+__device__ __forceinline__ void row4(float (&v)[4], const T* __restrict__ row, int i, int count, bool wide) {
+  if (wide && i + 4 <= count) {
+    const float4 f = load4(row + i);
+    v[0] = f.x, v[1] = f.y, v[2] = f.z, v[3] = f.w;
+    return;
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = i + e < count ? to_float(row[i + e]) : 0.f;
+}
+
+// One running state of a column: lane (column l & 15, quarter g) keeps the dims 16 t + 4 g .. + 3 of its sum of values.
+struct ColumnState {
+  float top = -INFINITY, sum = 0.f;
+  floatx4 acc[4] = {};
+};
+
+// A chunk's scores (dot[t]: keys 16 t + 4 g .. + 3, from `start`) become probabilities, in place, and the state takes in their
+// maximum and sum; its values are scaled and wait for the chunk's.
+template <bool CAP>
+__device__ __forceinline__ void take_scores(floatx4 (&dot)[4], ColumnState& state, int start, int lo, int pos, int g, float scale, float softcap) {
+  float top = -INFINITY;
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int j = start + 16 * t + 4 * g + i;
+      const float score = CAP && softcap > 0.f ? softcap * tanhf(dot[t][i] * scale / softcap) : dot[t][i] * scale;
+      dot[t][i] = j >= lo && j <= pos ? score : -INFINITY;
+      top = fmaxf(top, dot[t][i]);
+    }
+  const float new_max = fmaxf(state.top, max_quarters(top));
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int j = start + 16 * t + 4 * g + i;
+      const float weight = expf(dot[t][i] - new_max);
+      dot[t][i] = j >= lo && j <= pos ? weight : 0.f;
+    }
+  // over the key's bits 5, 4, 3, 2, 1, 0, as wave_sum over one key a lane
+  float part[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) part[i] = sum_quarters((dot[0][i] + dot[2][i]) + (dot[1][i] + dot[3][i]));
+  const float chunk_sum = (part[0] + part[2]) + (part[1] + part[3]);
+  const float alpha = new_max == -INFINITY ? 1.f : expf(state.top - new_max);
+  state.sum = state.sum * alpha + chunk_sum;
+  state.top = new_max;
+#pragma unroll
+  for (int t = 0; t < 4; ++t) state.acc[t] *= alpha;
+}
+
+// ---- many tokens a sequence ----
+// A workgroup of four waves serves up to 64 columns, of up to 64 / heads consecutive tokens of the step and the heads of
+// one kv head (or 64 of them), a wave 16 of them, and brings every chunk of 64 keys and values through LDS once for all (the
+// kernel above reads each key and value again for every column: a prompt of 2048 tokens would be 34 GB of cache traffic a
+// layer).  Bound by the matrix cores: a chunk is 128 instructions of 32 clocks a wave.  The chunk after the next is asked for, and the
+// next stored behind a barrier, before a chunk's products.  Rows lie in LDS 16 dims (keys) at a time as 0 4 8 12 1 5 ..: one
+// 16-byte read gives a lane what four instructions take from it; 68 floats apart, sixteen rows' reads cover the banks once.
+// Later tokens see more keys: workgroups are taken from the step's end, in rounds of one for each compute unit, every second
+// round backwards, so that the two that share a unit add up to the same length (in an earlier form of this kernel 103 us against 146
+// for a prompt of 1000 tokens).
+// 32 heads of 64 on 4, beside the form of plain multiply-adds before: a prompt of 1000 tokens 75 us against 493, of 2048 237 (73
+// TFLOP/s) against 1756; without groups 84 against 942.
+// Tokens of a workgroup that belong to different sequences are served one run of equal sequences after the other.
+// C > 0: both head sizes are 16 C, a page holds a power of two of rows, 16 at least, cache and queries are aligned for loads of
+// four, and scores have no cap: a chunk's sixteen rows a piece then lie on one page.  C = 0: everything else.
+constexpr int kTiledCols = 64, kTiledWaves = 4, kRowStride = 68;
+template <typename T, int C>
 __global__ void __launch_bounds__(64 * kTiledWaves)
 attention_generic_tiled_kernel(const T* __restrict__ q, const T* __restrict__ cache, const int* __restrict__ block_table,
                                int max_blocks, const int* __restrict__ token_seq, const int* __restrict__ positions,
                                T* __restrict__ out, int tokens, int nq, int nkv, int d, int dv, int page_size, int window,
                                int chunk, const float* __restrict__ sink, float scale, float softcap, int tokens_per_block, int heads_per_block, const int* __restrict__ seq_start, int min_tokens,
-                               int vshare, int out_f32) {
-  extern __shared__ __attribute__((aligned(16))) float lds[];
-  // rows of a multiple of 4 floats, so that four values are one LDS read, plus 4: a wave's lanes, each
-  // on a row of its own, then spread over the banks
-  const int k_stride = (d + 3) / 4 * 4 + 4, q_stride = (d + 3) / 4 * 4;
-  constexpr int kValueStride = 68;
-  float* k_tile = lds;                             // [64 keys][k_stride]
-  float* v_tile = k_tile + 64 * k_stride;          // [dv][68]
-  float* q_tile = v_tile + dv * kValueStride;       // [32 columns][q_stride]
-  float* prob = q_tile + kTiledCols * q_stride;    // [waves][4 columns][64 keys]
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int G = nq / nkv, kv_head = blockIdx.y;
-  const int tok0 = blockIdx.x * tokens_per_block, head0 = blockIdx.z * heads_per_block;
+                               int vshare, int out_f32, int units) {
+  __shared__ __attribute__((aligned(16))) float k_tile[2][64 * kRowStride];      // [key][dims]
+  __shared__ __attribute__((aligned(16))) float v_tile[2][64 * kRowStride];      // [dim][keys]
+  __shared__ int infinite[2];                      // the last chunk in this half of v_tile that held a value that is not finite
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
+  const int G = nq / nkv;
+  const int round = blockIdx.x / units, in_round = blockIdx.x - round * units;
+  const int place = round % 2 == 0 ? blockIdx.x : round * units + min(units, static_cast<int>(gridDim.x) - round * units) - 1 - in_round;
+  const int kv_head = place % nkv, tok0 = ((static_cast<int>(gridDim.x) - 1 - place) / nkv) * tokens_per_block, head0 = blockIdx.z * heads_per_block;
   const int ntok = min(tokens_per_block, tokens - tok0), nheads = min(heads_per_block, G - head0);
   const int ncols = ntok * nheads;                 // column c = (token c / nheads, head c % nheads)
   // (vshare key heads in a row read one value head: a page then holds nkv planes of keys and nkv / vshare of values)
   const size_t page_stride = static_cast<size_t>(page_size) * (static_cast<size_t>(nkv) * d + static_cast<size_t>(nkv / vshare) * dv);
-  const size_t head_offset = static_cast<size_t>(kv_head) * page_size * d;
-  const size_t v_offset = static_cast<size_t>(nkv) * page_size * d + static_cast<size_t>(kv_head / vshare) * page_size * dv;
+  const T* keys = cache + static_cast<size_t>(kv_head) * page_size * d;
+  const T* values = cache + static_cast<size_t>(nkv) * page_size * d + static_cast<size_t>(kv_head / vshare) * page_size * dv;
+  constexpr int kDims = C > 0 ? C : 4;             // sixteens of dims
+  const int page_bits = 31 - __builtin_clz(page_size), in_page = page_size - 1;        // (where pages hold a power of two)
+  // whole loads of four where rows allow them
+  const bool aligned = C > 0 || ((reinterpret_cast<uintptr_t>(cache) % (4 * sizeof(T))) == 0 && (page_size & 3) == 0);
+  const bool wide_k = aligned && (d & 3) == 0, wide_q = C > 0 || ((d & 3) == 0 && (reinterpret_cast<uintptr_t>(q) % (4 * sizeof(T))) == 0);
+  if (threadIdx.x < 2) infinite[threadIdx.x] = -1;
 
-  for (int e = threadIdx.x; e < ncols * d; e += 64 * kTiledWaves) {
-    const int c = e / d, i = e - c * d;
-    q_tile[c * q_stride + i] = to_float(q[(static_cast<size_t>(tok0 + c / nheads) * nq + kv_head * G + head0 + c % nheads) * d + i]);
+  // this wave's columns
+  const int column = wave * 16 + r;
+  const int col_tok = column < ncols ? column / nheads : -1, col_head = kv_head * G + head0 + max(column, 0) % nheads;
+  const int col_pos = col_tok >= 0 ? positions[tok0 + col_tok] : -1;
+  int col_lo = window > 0 ? max(0, col_pos - window + 1) : 0;
+  if (chunk > 0 && col_pos >= 0) col_lo = max(col_lo, col_pos - col_pos % chunk);
+  float query[kDims][4];                           // dims 16 c + 4 j + g
+#pragma unroll
+  for (int c = 0; c < kDims; ++c) {
+    row4(query[c], q + (static_cast<size_t>(tok0 + max(col_tok, 0)) * nq + col_head) * d, 16 * c + 4 * g, C > 0 ? 16 * C : (col_tok >= 0 ? d : 0), wide_q);
+    to_quarters(query[c]);
   }
-  // this wave's columns: slot s is column wave + kTiledWaves * s
-  int col_pos[kTiledSlots], col_lo[kTiledSlots], col_tok[kTiledSlots];     // col_tok: the column's token among the workgroup's, or -1
-#pragma unroll
-  for (int s = 0; s < kTiledSlots; ++s) {
-    const int c = wave + kTiledWaves * s;
-    bool live = c < ncols;
-    if (live && seq_start != nullptr) {            // a token of a sequence that brings few tokens is the other kernel's
-      const int seq = token_seq[tok0 + c / nheads];
-      live = seq_start[seq + 1] - seq_start[seq] >= min_tokens;
-    }
-    col_tok[s] = live ? c / nheads : -1;
-    col_pos[s] = live ? positions[tok0 + col_tok[s]] : -1;
-    col_lo[s] = live && window > 0 ? max(0, col_pos[s] - window + 1) : 0;
-    if (live && chunk > 0) col_lo[s] = max(col_lo[s], col_pos[s] - col_pos[s] % chunk);
-  }
-  float run_max[4][kTiledSlots], run_sum[4][kTiledSlots], acc[4][kTiledSlots];
-#pragma unroll
-  for (int g = 0; g < 4; ++g)
-#pragma unroll
-    for (int s = 0; s < kTiledSlots; ++s) run_max[g][s] = -INFINITY, run_sum[g][s] = 0.f, acc[g][s] = 0.f;
+  ColumnState kept0, kept1, kept2, kept3;          // (not an array: the compiler would keep it in memory)
 
-  // runs of tokens of one sequence, in the order of the tokens (a column belongs to the run its token
-  // lies in: a sequence may come twice among a workgroup's tokens, when a recorded step pads its
-  // tokens with tokens of its first sequence)
+  int stamp = 0;                                   // chunks so far
   int run_first = 0;
   while (run_first < ntok) {                       // (the same for every thread: the barriers below are the workgroup's)
     const int seq = token_seq[tok0 + run_first];
     int run_end = run_first + 1;
     while (run_end < ntok && token_seq[tok0 + run_end] == seq) ++run_end;
-    if (seq_start != nullptr && seq_start[seq + 1] - seq_start[seq] < min_tokens) {   // (the same for every thread)
+    if (seq_start != nullptr && seq_start[seq + 1] - seq_start[seq] < min_tokens) {   // left to the kernel of few tokens (the same for every thread)
       run_first = run_end;
       continue;
     }
-    // the keys the run's columns see: from the least lower bound to the last token's position
-    int hi = -1, lo = 1 << 30;
+    // the keys the run's columns see: from the least lower bound to the last position; those that all of them see: from the
+    // greatest lower bound to the first position
+    int hi = -1, lo = 1 << 30, all_hi = 1 << 30, all_lo = 0;
     for (int t = run_first; t < run_end; ++t) {
       const int pos = positions[tok0 + t];
-      hi = max(hi, pos);
       int bound = window > 0 ? max(0, pos - window + 1) : 0;
       if (chunk > 0) bound = max(bound, pos - pos % chunk);
-      lo = min(lo, bound);
+      hi = max(hi, pos), lo = min(lo, bound), all_hi = min(all_hi, pos), all_lo = max(all_lo, bound);
     }
+    if (run_end - run_first < ntok) all_hi = -1;   // (columns of another run are in the same instructions)
+    const bool mine = col_tok >= run_first && col_tok < run_end;
+    const int my_pos = mine ? col_pos : -1;
     const int* pages = block_table + static_cast<size_t>(seq) * max_blocks;
-    for (int base = (lo / 256) * 256; base <= hi; base += 256) {
+    const int first = lo / 256 * 256, chunks = (hi - first) / 64 + 1;      // (chunk n of the walk belongs to state n % 4)
+
+    float k_next[4][4], v_next[4][4];
+    int page_of[4];                                // (C > 0) the pages of the sixteens of the chunk that is asked for next
+    auto look_up = [&](int n) {
+      if (C > 0) {
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int start = base + g * 64;
-        if (start > hi) break;                     // (uniform)
-        __syncthreads();                           // the tiles of the chunk before have been read
-        for (int e = threadIdx.x; e < 64 * d; e += 64 * kTiledWaves) {
-          const int r = e / d, i = e - r * d, j = start + r;
-          if (j <= hi && j >= lo)
-            k_tile[r * k_stride + i] = to_float(cache[static_cast<size_t>(pages[j / page_size]) * page_stride + head_offset +
-                                                      static_cast<size_t>(j % page_size) * d + i]);
+        for (int p = 0; p < 4; ++p) page_of[p] = pages[min(max(first + 64 * n + 16 * p, lo), hi) >> page_bits];
+      }
+    };
+    auto ask = [&](int n) {                        // a thread brings four pieces of four of either
+      const int start = first + 64 * n, piece = threadIdx.x & 15;
+      if (C > 0) {
+        // keys: rows tid / 16 of the four sixteens; values: the four keys of this thread's piece, of dims tid / 16 + 16 p.
+        // What lies outside lo .. hi is read from within the same pages, and masked (keys) or set to zero (values).
+        const int row = threadIdx.x >> 4;
+        const int mine = piece >> 2, v_page = mine == 0 ? page_of[0] : (mine == 1 ? page_of[1] : (mine == 2 ? page_of[2] : page_of[3]));
+        const int jv = start + 4 * piece;
+        const T* v_at = values + static_cast<size_t>(v_page) * page_stride + (jv & in_page);
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+          const int j = start + 16 * p + row;
+          if (4 * piece < 16 * C) {
+            const float4 f = load4(keys + static_cast<size_t>(page_of[p]) * page_stride + static_cast<size_t>(j & in_page) * (16 * C) + 4 * piece);
+            k_next[p][0] = f.x, k_next[p][1] = f.y, k_next[p][2] = f.z, k_next[p][3] = f.w;
+          }
+          if (p < C) {
+            const float4 f = load4(v_at + static_cast<size_t>(row + 16 * p) * page_size);
+            v_next[p][0] = f.x, v_next[p][1] = f.y, v_next[p][2] = f.z, v_next[p][3] = f.w;
+          }
         }
-        for (int e = threadIdx.x; e < 64 * dv; e += 64 * kTiledWaves) {
-          const int dim = e >> 6, r = e & 63, j = start + r;
-          if (j <= hi && j >= lo)
-            v_tile[dim * kValueStride + r] = to_float(cache[static_cast<size_t>(pages[j / page_size]) * page_stride + v_offset +
-                                                  static_cast<size_t>(dim) * page_size + j % page_size]);
-        }
-        __syncthreads();
-        // four columns at a time: their dot products share each read of a key, and the chains of
-        // additions of one column wait for each other less
+        return;
+      }
 #pragma unroll
-        for (int b = 0; b < kTiledSlots / 4; ++b) {
-          bool any = false;
+      for (int p = 0; p < 4; ++p) {
+        const int row = (threadIdx.x >> 4) + 16 * p;
+        const int j = min(max(start + row, lo), hi);                       // (a key outside is masked: any that was written will do)
+        row4(k_next[p], keys + static_cast<size_t>(pages[j / page_size]) * page_stride + static_cast<size_t>(j % page_size) * d, 4 * piece, d, wide_k);
+        const int jv = start + 4 * piece;          // keys jv .. jv + 3 of dim `row`
+        if (aligned && jv >= lo && jv + 3 <= hi) {
+          row4(v_next[p], values + static_cast<size_t>(pages[jv / page_size]) * page_stride + static_cast<size_t>(row) * page_size + jv % page_size, 0, row < dv ? 4 : 0, true);
+        } else {
 #pragma unroll
-          for (int u = 0; u < 4; ++u)
-            any |= col_tok[b * 4 + u] >= run_first && col_tok[b * 4 + u] < run_end && col_pos[b * 4 + u] >= start && col_lo[b * 4 + u] < start + 64;
-          if (!any) continue;                      // (uniform over the wave: the columns are the wave's)
-          const int j = start + lane;
-          float dot[4] = {0.f, 0.f, 0.f, 0.f};
-          const float* key = k_tile + lane * k_stride;
-          const float* query[4];
-#pragma unroll
-          for (int u = 0; u < 4; ++u) query[u] = q_tile + min(wave + kTiledWaves * (b * 4 + u), kTiledCols - 1) * q_stride;
-          // (four dims a read; the additions of a column stay in the order of the dims)
-          int i = 0;
-#pragma unroll 4
-          for (; i + 4 <= d; i += 4) {
-            const float4 kv = *reinterpret_cast<const float4*>(key + i);
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-              const float4 qv = *reinterpret_cast<const float4*>(query[u] + i);
-              dot[u] += qv.x * kv.x;
-              dot[u] += qv.y * kv.y;
-              dot[u] += qv.z * kv.z;
-              dot[u] += qv.w * kv.w;
-            }
-          }
-          for (; i < d; ++i) {
-            const float kv = key[i];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) dot[u] += query[u][i] * kv;
-          }
-          float* my_prob = prob + (wave * 4) * 64;
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            const int s = b * 4 + u;
-            const bool column = col_tok[s] >= run_first && col_tok[s] < run_end && col_pos[s] >= start && col_lo[s] < start + 64;   // a chunk without keys changes nothing
-            if (!column) continue;                 // (uniform over the wave)
-            const bool valid = j >= col_lo[s] && j <= col_pos[s];
-            const float score = valid ? (softcap > 0.f ? softcap * tanhf(dot[u] * scale / softcap) : dot[u] * scale) : -INFINITY;
-            const float new_max = fmaxf(run_max[g][s], wave_max(score));
-            const float p = valid ? expf(score - new_max) : 0.f;
-            my_prob[u * 64 + lane] = p;
-            const float chunk_sum = wave_sum(p);
-            const float alpha = new_max == -INFINITY ? 1.f : expf(run_max[g][s] - new_max);
-            run_sum[g][s] = run_sum[g][s] * alpha + chunk_sum;
-            run_max[g][s] = new_max;
-            acc[g][s] *= alpha;
-          }
-          // what one lane wrote to prob above, another lane of the wave reads below: the writes are
-          // ordered before the reads for the compiler and the memory model (no instruction on this hardware,
-          // where a wave's LDS operations complete in order)
-          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-          __builtin_amdgcn_wave_barrier();
-          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-          if (lane < dv) {
-            const float* value = v_tile + lane * kValueStride;
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-              const int s = b * 4 + u;
-              const bool column = col_tok[s] >= run_first && col_tok[s] < run_end && col_pos[s] >= start && col_lo[s] < start + 64;
-              if (!column) continue;
-              const int first = max(0, col_lo[s] - start), last = min(64, col_pos[s] - start + 1);
-              float sum = acc[g][s];
-              const float* weight = my_prob + u * 64;
-              int jj = first;
-              for (; jj < last && (jj & 3) != 0; ++jj) sum += weight[jj] * value[jj];
-#pragma unroll 4
-              for (; jj + 4 <= last; jj += 4) {           // (four keys a read; the additions stay in the order of the keys)
-                const float4 pv = *reinterpret_cast<const float4*>(weight + jj), vv = *reinterpret_cast<const float4*>(value + jj);
-                sum += pv.x * vv.x;
-                sum += pv.y * vv.y;
-                sum += pv.z * vv.z;
-                sum += pv.w * vv.w;
-              }
-              for (; jj < last; ++jj) sum += weight[jj] * value[jj];
-              acc[g][s] = sum;
-            }
+          for (int e = 0; e < 4; ++e) {
+            const int je = jv + e;
+            v_next[p][e] = row < dv && je >= lo && je <= hi
+                ? to_float(values[static_cast<size_t>(pages[je / page_size]) * page_stride + static_cast<size_t>(row) * page_size + je % page_size]) : 0.f;
           }
         }
       }
+    };
+    auto put = [&](int n, int half) {
+      const int start = first + 64 * n, piece = threadIdx.x & 15;
+      const bool outside = start < lo || start + 63 > hi, partial = start < all_lo || start + 63 > all_hi;     // (uniform)
+      bool odd = false;
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        const int at = ((threadIdx.x >> 4) + 16 * p) * kRowStride + (piece >> 2) * 16 + (piece & 3);
+        if (4 * piece < 16 * kDims) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) k_tile[half][at + 4 * e] = k_next[p][e];
+        }
+        if (p < kDims) {
+          if (C > 0 && outside) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v_next[p][e] = start + 4 * piece + e >= lo && start + 4 * piece + e <= hi ? v_next[p][e] : 0.f;
+          }
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v_tile[half][at + 4 * e] = v_next[p][e];
+          if (partial) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) odd |= !(fabsf(v_next[p][e]) < INFINITY);
+          }
+        }
+      }
+      if (odd) infinite[half] = stamp + n;
+    };
+    __syncthreads();                               // (the run before is done with LDS; `infinite` is set)
+    // state by state, the chunks of each in their order: n, n + 4, .., then the next state's (one copy of the code, and one
+    // state in the works; the others wait in `kept`)
+    auto after = [&](int n) { return n + 4 < chunks ? n + 4 : (n & 3) + 1 + ((n & 3) == 3 ? chunks : 0); };
+    int n = 0, n1 = after(0), half = 0;            // this chunk, the next (chunks or more: none)
+    look_up(0);
+    ask(0);
+    look_up(n1);
+    put(0, 0);
+    if (n1 < chunks) ask(n1);
+    ColumnState own = kept0;
+    while (n < chunks) {                           // (uniform)
+      const int n2 = n1 < chunks ? after(n1) : n1;
+      lds_barrier();                               // chunk n is whole, the one before has been read
+      if (n1 < chunks) put(n1, half ^ 1);
+      look_up(n2);
+      if (n2 < chunks) ask(n2);
+      const int start = first + 64 * n;
+      if (!__all(my_pos < start || col_lo > start + 63)) {                 // (else no column of the wave sees it)
+        floatx4 dot[4] = {};
+        const float* key = k_tile[half] + r * kRowStride + 4 * g;
+#pragma unroll
+        for (int c = 0; c < kDims; ++c) {
+          if (16 * c >= d) break;                  // (dims past d are zeros)
+          float4 a[4];
+#pragma unroll
+          for (int t = 0; t < 4; ++t) a[t] = *reinterpret_cast<const float4*>(key + 16 * t * kRowStride + 16 * c);
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) dot[t] = __builtin_amdgcn_mfma_f32_16x16x4f32((&a[t].x)[e], query[c][e], dot[t], 0, 0, 0);
+        }
+        take_scores<C == 0>(dot, own, start, col_lo, my_pos, g, scale, softcap);
+        if (infinite[half] != stamp + n) {
+          const float* value = v_tile[half] + r * kRowStride + 4 * g;
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {
+            float weight[4] = {dot[t][0], dot[t][1], dot[t][2], dot[t][3]};
+            to_quarters(weight);
+            float4 a[kDims];
+#pragma unroll
+            for (int u = 0; u < kDims; ++u) a[u] = *reinterpret_cast<const float4*>(value + 16 * u * kRowStride + 16 * t);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+              for (int u = 0; u < kDims; ++u) own.acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32((&a[u].x)[e], weight[e], own.acc[u], 0, 0, 0);
+          }
+        } else {
+          // a value that is not finite, among keys that some column must not see: zero times it would be no zero there, so every
+          // column adds its own keys and no others, in the same order
+#pragma unroll
+          for (int t = 0; t < 4; ++t)
+            for (int from = 0; from < 4; ++from)
+#pragma unroll
+              for (int i = 0; i < 4; ++i) {
+                const int at = 16 * t + 4 * from + i, j = start + at;
+                const float weight = __shfl(dot[t][i], 16 * from + r, 64);
+                if (j < col_lo || j > my_pos) continue;
+#pragma unroll
+                for (int u = 0; u < kDims; ++u)
+#pragma unroll
+                  for (int e = 0; e < 4; ++e)
+                    own.acc[u][e] = fmaf(weight, v_tile[half][(16 * u + 4 * g + e) * kRowStride + 16 * t + 4 * i + from], own.acc[u][e]);
+              }
+        }
+      }
+      if (n1 >= chunks || (n1 & 3) != (n & 3)) {   // the state's last chunk
+        if ((n & 3) == 0) kept0 = own, own = kept1;
+        else if ((n & 3) == 1) kept1 = own, own = kept2;
+        else if ((n & 3) == 2) kept2 = own, own = kept3;
+        else kept3 = own;
+      }
+      n = n1, n1 = n2, half ^= 1;
     }
+    stamp += chunks;
     run_first = run_end;
   }
+  if (col_tok < 0) return;
+  if (seq_start != nullptr) {                      // a token of a sequence that brings few tokens is the other kernel's
+    const int seq = token_seq[tok0 + col_tok];
+    if (seq_start[seq + 1] - seq_start[seq] < min_tokens) return;
+  }
   // the four states of a column into one, in their order
-  if (lane < dv) {
+  float top = fmaxf(fmaxf(kept0.top, kept1.top), fmaxf(kept2.top, kept3.top)), total = 0.f;
+  floatx4 result[kDims] = {};
+  if (sink != nullptr) {
+    top = fmaxf(top, sink[col_head]);
+    total = expf(sink[col_head] - top);
+  }
+  auto join = [&](const ColumnState& one) {
+    if (one.top == -INFINITY) return;
+    const float w = expf(one.top - top);
+    total += w * one.sum;
 #pragma unroll
-    for (int s = 0; s < kTiledSlots; ++s) {
-      const int c = wave + kTiledWaves * s;
-      if (c >= ncols || col_tok[s] < 0) continue;
-      float top = -INFINITY;
+    for (int u = 0; u < kDims; ++u)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) top = fmaxf(top, run_max[g][s]);
-      float total = 0.f, result = 0.f;
-      if (sink != nullptr) {
-        const float own = sink[kv_head * G + head0 + c % nheads];
-        top = fmaxf(top, own);
-        total = expf(own - top);
-      }
+      for (int e = 0; e < 4; ++e) result[u][e] += w * one.acc[u][e];
+  };
+  join(kept0);
+  join(kept1);
+  join(kept2);
+  join(kept3);
+  const size_t row = (static_cast<size_t>(tok0 + col_tok) * nq + col_head) * dv;
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const float m = run_max[g][s];
-        if (m == -INFINITY) continue;
-        const float w = expf(m - top);
-        total += w * run_sum[g][s];
-        result += w * acc[g][s];
-      }
-      store_result(out, (static_cast<size_t>(tok0 + c / nheads) * nq + kv_head * G + head0 + c % nheads) * dv + lane, result / total, out_f32);
+  for (int u = 0; u < kDims; ++u)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int dim = 16 * u + 4 * g + e;
+      if (dim < dv) store_result(out, row + dim, result[u][e] / total, out_f32);
     }
+}
+
+// ---- few tokens a sequence (decoding) ----
+// A workgroup of four waves serves one token and up to 16 heads of one kv head; wave w takes the chunks of state w, with keys
+// and values straight from the cache into registers (a lane asks for 16 bytes of a key or of a dim's row of values), the next
+// chunk's asked for while this one's products run.  The kernel of one head a workgroup reads a key once for each of the heads that
+// share it; what a chunk takes here (some 4 us) does not fall with the number of heads, so that kernel stays for steps of little
+// work (the line is drawn where it is launched).
+template <typename T, int C>
+__global__ void __launch_bounds__(256)
+attention_generic_few_kernel(const T* __restrict__ q, const T* __restrict__ cache, const int* __restrict__ block_table,
+                             int max_blocks, const int* __restrict__ token_seq, const int* __restrict__ positions,
+                             T* __restrict__ out, int nq, int nkv, int d, int dv, int page_size, int window, int chunk,
+                             const float* __restrict__ sink, float scale, float softcap,
+                             const int* __restrict__ seq_start, int min_tokens, int vshare, int out_f32) {
+  __shared__ __attribute__((aligned(16))) float states[4][16][68];        // [state][column][64 dims, maximum, sum]
+  const int t0 = blockIdx.x, seq = token_seq[t0];
+  if (seq_start != nullptr && seq_start[seq + 1] - seq_start[seq] >= min_tokens) return;      // (the same for the whole workgroup)
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
+  const int G = nq / nkv, kv_head = blockIdx.y, head0 = blockIdx.z * 16, nheads = min(16, G - head0);
+  const int pos = positions[t0];
+  int lo = window > 0 ? max(0, pos - window + 1) : 0;
+  if (chunk > 0) lo = max(lo, pos - pos % chunk);
+  const int* pages = block_table + static_cast<size_t>(seq) * max_blocks;
+  const size_t page_stride = static_cast<size_t>(page_size) * (static_cast<size_t>(nkv) * d + static_cast<size_t>(nkv / vshare) * dv);
+  const T* keys = cache + static_cast<size_t>(kv_head) * page_size * d;
+  const T* values = cache + static_cast<size_t>(nkv) * page_size * d + static_cast<size_t>(kv_head / vshare) * page_size * dv;
+  constexpr int kDims = C > 0 ? C : 4;
+  const int page_bits = 31 - __builtin_clz(page_size), in_page = page_size - 1;
+  const bool aligned = C > 0 || ((reinterpret_cast<uintptr_t>(cache) % (4 * sizeof(T))) == 0 && (page_size & 3) == 0);
+  const bool wide_k = aligned && (d & 3) == 0, wide_q = C > 0 || ((d & 3) == 0 && (reinterpret_cast<uintptr_t>(q) % (4 * sizeof(T))) == 0);
+  const int kc = C > 0 ? C : (d + 15) / 16, vc = C > 0 ? C : (dv + 15) / 16;
+  float query[kDims][4];
+#pragma unroll
+  for (int c = 0; c < kDims; ++c) {
+    row4(query[c], q + (static_cast<size_t>(t0) * nq + kv_head * G + head0 + min(r, nheads - 1)) * d, 16 * c + 4 * g, C > 0 ? 16 * C : d, wide_q);
+    to_quarters(query[c]);
+  }
+  const int first = lo / 256 * 256 + 64 * wave;
+  float k_next[4][kDims][4], v_next[4][kDims][4];
+  int page_of[4];                                  // (C > 0) the pages of the four sixteens of the chunk that is asked for next
+  auto look_up = [&](int start) {
+    if (C > 0) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) page_of[t] = pages[min(max(start + 16 * t, lo), pos) >> page_bits];
+    }
+  };
+  auto ask_keys = [&](int start) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const T* row;
+      if (C > 0) {
+        row = keys + static_cast<size_t>(page_of[t]) * page_stride + static_cast<size_t>((start + 16 * t + r) & in_page) * (16 * C);
+      } else {
+        const int j = min(max(start + 16 * t + r, lo), pos);
+        row = keys + static_cast<size_t>(pages[j / page_size]) * page_stride + static_cast<size_t>(j % page_size) * d;
+      }
+#pragma unroll
+      for (int c = 0; c < kDims; ++c) {
+        if (C > 0) {
+          const float4 f = load4(row + 16 * c + 4 * g);
+          k_next[t][c][0] = f.x, k_next[t][c][1] = f.y, k_next[t][c][2] = f.z, k_next[t][c][3] = f.w;
+        } else if (c < kc) {
+          row4(k_next[t][c], row, 16 * c + 4 * g, d, wide_k);
+        }
+      }
+    }
+  };
+  // (a value outside lo .. pos counts as zero; C > 0: `hide` sets it to zero before it is used)
+  auto ask_values = [&](int start) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int jv = start + 16 * t + 4 * g;
+      if (C > 0) {
+        const T* at = values + static_cast<size_t>(page_of[t]) * page_stride + static_cast<size_t>(r) * page_size + (jv & in_page);
+#pragma unroll
+        for (int u = 0; u < kDims; ++u) {
+          const float4 f = load4(at + static_cast<size_t>(16 * u) * page_size);
+          v_next[t][u][0] = f.x, v_next[t][u][1] = f.y, v_next[t][u][2] = f.z, v_next[t][u][3] = f.w;
+        }
+      } else {
+#pragma unroll
+        for (int u = 0; u < kDims; ++u)
+          if (u < vc)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const int je = jv + e;
+              v_next[t][u][e] = je >= lo && je <= pos
+                  ? to_float(values[static_cast<size_t>(pages[je / page_size]) * page_stride + static_cast<size_t>(min(16 * u + r, dv - 1)) * page_size + je % page_size]) : 0.f;
+            }
+      }
+    }
+  };
+  auto hide = [&](int start) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int u = 0; u < kDims; ++u)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int j = start + 16 * t + 4 * g + e;
+          v_next[t][u][e] = j >= lo && j <= pos ? v_next[t][u][e] : 0.f;
+        }
+  };
+  ColumnState state;
+  if (first <= pos) {
+    look_up(first);
+    ask_keys(first);
+    ask_values(first);
+    look_up(first + 256);
+  }
+  for (int start = first; start <= pos; start += 256) {
+    const bool more = start + 256 <= pos, partial = start < lo || start + 63 > pos;      // (uniform)
+    floatx4 dot[4] = {};
+#pragma unroll
+    for (int c = 0; c < kDims; ++c) {
+      if (c >= kc) break;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) to_quarters(k_next[t][c]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) dot[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(k_next[t][c][e], query[c][e], dot[t], 0, 0, 0);
+    }
+    if (more) ask_keys(start + 256);
+    take_scores<C == 0>(dot, state, start, lo, pos, g, scale, softcap);
+    if (C > 0 && partial) hide(start);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      float weight[4] = {dot[t][0], dot[t][1], dot[t][2], dot[t][3]};
+      to_quarters(weight);
+#pragma unroll
+      for (int u = 0; u < kDims; ++u)
+        if (u < vc) to_quarters(v_next[t][u]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int u = 0; u < kDims; ++u)
+          if (u < vc) state.acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(v_next[t][u][e], weight[e], state.acc[u], 0, 0, 0);
+    }
+    if (more) {
+      ask_values(start + 256);
+      look_up(start + 512);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+    *reinterpret_cast<float4*>(&states[wave][r][16 * u + 4 * g]) = make_float4(state.acc[u][0], state.acc[u][1], state.acc[u][2], state.acc[u][3]);
+  if (g == 0) states[wave][r][64] = state.top, states[wave][r][65] = state.sum;
+  __syncthreads();
+  // the four states into one, in their order: a wave a column, a lane a dim
+  for (int column = wave; column < nheads; column += 4) {
+    const int head = kv_head * G + head0 + column;
+    float top = -INFINITY;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) top = fmaxf(top, states[s][column][64]);
+    float total = 0.f, result = 0.f;
+    if (sink != nullptr) {                         // the sink counts once: exp(sink) in the denominator, nothing in the sum of values
+      top = fmaxf(top, sink[head]);
+      total = expf(sink[head] - top);
+    }
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const float m = states[s][column][64];
+      if (m == -INFINITY) continue;                // a state that saw no key
+      const float w = expf(m - top);
+      total += w * states[s][column][65];
+      result += w * states[s][column][lane];
+    }
+    if (lane < dv) store_result(out, (static_cast<size_t>(t0) * nq + head) * dv + lane, result / total, out_f32);
   }
 }
 
@@ -415,37 +733,65 @@ extern "C" int tlie_attention_generic(const void* q, const void* cache, int dtyp
                                       int max_blocks, const int* token_seq, const int* positions, void* out,
                                       int tokens, int nq, int nkv, int d, int dv, int page_size, int window, int chunk,
                                       const float* sink, float scale, int tiled, const int* seq_start, int min_tokens,
-                                      int vshare, int out_f32, float softcap, void* stream) {
+                                      int vshare, int out_f32, float softcap, int compute_units, void* stream) {
   // tiled 0: the kernel of one (token, head) a workgroup; 1: the kernel that shares keys among a
   // sequence's tokens (head sizes up to 64); 2: both, each token served by one of them: the second
   // takes the sequences that bring min_tokens tokens or more (seq_start: int32 [sequences + 1], the
   // step's cumulative token counts), the first the others.  A token gets the same bits from either.
   // (d only bounds the length of a dot product; dv is served by one thread a dim of a group of at most 256)
   if (tokens <= 0 || nq <= 0 || nkv <= 0 || nq % nkv != 0 || d <= 0 || d > 4096 || dv <= 0 || dv > 256 || page_size <= 0 ||
-      max_blocks <= 0 || chunk < 0 || vshare <= 0 || nkv % vshare != 0 || softcap < 0.f)
+      max_blocks <= 0 || chunk < 0 || compute_units <= 0 || vshare <= 0 || nkv % vshare != 0 || softcap < 0.f)
     return kBadArgument;
   if (tiled < 0 || tiled > 2 || (tiled == 2 && (seq_start == nullptr || min_tokens < 1))) return kBadArgument;
   if (dtype != kF32 && dtype != kBF16) return kBadArgument;
   if (d > 64 || dv > 64) tiled = 0;
   const int* select = tiled == 2 ? seq_start : nullptr;
+  // sixteens of dims where the kernels for head sizes up to 64 know the sizes beforehand (see there), else 0
+  const bool known = d == dv && d % 16 == 0 && d <= 64 && page_size >= 16 && (page_size & (page_size - 1)) == 0 &&
+                     (reinterpret_cast<uintptr_t>(cache) | reinterpret_cast<uintptr_t>(q)) % (dtype == kF32 ? 16 : 8) == 0 && softcap == 0.f;
+  const int sixteens = known && d != 48 ? d / 16 : 0;
+#define TLIE_BY_SIZE(LAUNCH)                                                                                  \
+  if (dtype == kF32) {                                                                                        \
+    if (sixteens == 1) LAUNCH(float, 1);                                                                      \
+    else if (sixteens == 2) LAUNCH(float, 2);                                                                 \
+    else if (sixteens == 4) LAUNCH(float, 4);                                                                 \
+    else LAUNCH(float, 0);                                                                                    \
+  } else {                                                                                                    \
+    if (sixteens == 1) LAUNCH(bf16, 1);                                                                       \
+    else if (sixteens == 2) LAUNCH(bf16, 2);                                                                  \
+    else if (sixteens == 4) LAUNCH(bf16, 4);                                                                  \
+    else LAUNCH(bf16, 0);                                                                                     \
+  }
   if (tiled) {
     // (the same bits as the kernel below, for steps whose sequences bring several tokens each)
     const int G = nq / nkv;
     const int heads_per_block = G < kTiledCols ? G : kTiledCols;
     const int tokens_per_block = kTiledCols / heads_per_block;
-    const dim3 grid((tokens + tokens_per_block - 1) / tokens_per_block, nkv, (G + heads_per_block - 1) / heads_per_block);
-    const size_t rounded = (static_cast<size_t>(d) + 3) / 4 * 4;
-    const size_t bytes = (64 * (rounded + 4) + static_cast<size_t>(dv) * 68 + kTiledCols * rounded + kTiledWaves * 4 * 64) * sizeof(float);
-    if (dtype == kF32)
-      hipLaunchKernelGGL((attention_generic_tiled_kernel<float>), grid, dim3(64 * kTiledWaves), bytes, (hipStream_t)stream, (const float*)q,
-                         (const float*)cache, block_table, max_blocks, token_seq, positions, (float*)out, tokens, nq, nkv, d, dv,
-                         page_size, window, chunk, sink, scale, softcap, tokens_per_block, heads_per_block, select, min_tokens, vshare, out_f32);
-    else
-      hipLaunchKernelGGL((attention_generic_tiled_kernel<bf16>), grid, dim3(64 * kTiledWaves), bytes, (hipStream_t)stream, (const bf16*)q,
-                         (const bf16*)cache, block_table, max_blocks, token_seq, positions, (bf16*)out, tokens, nq, nkv, d, dv,
-                         page_size, window, chunk, sink, scale, softcap, tokens_per_block, heads_per_block, select, min_tokens, vshare, out_f32);
+    const long long blocks = static_cast<long long>((tokens + tokens_per_block - 1) / tokens_per_block) * nkv;
+    if (blocks > 0x7fffffff) return kBadArgument;
+    const dim3 grid(static_cast<unsigned>(blocks), 1, (G + heads_per_block - 1) / heads_per_block);
+#define TLIE_TILED(T, C)                                                                                                       \
+  hipLaunchKernelGGL((attention_generic_tiled_kernel<T, C>), grid, dim3(64 * kTiledWaves), 0, (hipStream_t)stream, (const T*)q,      \
+                     (const T*)cache, block_table, max_blocks, token_seq, positions, (T*)out, tokens, nq, nkv, d, dv, page_size,      \
+                     window, chunk, sink, scale, softcap, tokens_per_block, heads_per_block, select, min_tokens, vshare, out_f32, compute_units)
+    TLIE_BY_SIZE(TLIE_TILED)
+#undef TLIE_TILED
     const int status = launch_status();
     if (status != kOk || tiled == 1) return status;
+  }
+  // Head sizes up to 64: the kernel that serves a kv head's query heads together, where they are several and the step has
+  // work for four workgroups a compute unit in the kernel of one head each (64 tokens of 500 keys, 32 heads on 4: 17.4 us against
+  // 54; 8 tokens of 100 keys 9.0 against 6.7; 64 tokens of 500 keys, 32 heads on 32: 144 against 116).
+  if (d <= 64 && dv <= 64 && nq / nkv >= 2 && static_cast<long long>(tokens) * nq >= 4LL * compute_units) {
+    const dim3 grid(tokens, nkv, (nq / nkv + 15) / 16);
+    if (grid.y > 65535 || grid.z > 65535) return kBadArgument;
+#define TLIE_FEW(T, C)                                                                                                         \
+  hipLaunchKernelGGL((attention_generic_few_kernel<T, C>), grid, dim3(256), 0, (hipStream_t)stream, (const T*)q, (const T*)cache,    \
+                     block_table, max_blocks, token_seq, positions, (T*)out, nq, nkv, d, dv, page_size, window, chunk, sink, scale,  \
+                     softcap, select, min_tokens, vshare, out_f32)
+    TLIE_BY_SIZE(TLIE_FEW)
+#undef TLIE_FEW
+    return launch_status();
   }
   // keys a group of threads takes in one turn: the least of 64, 128, 256 that holds both head sizes (beyond 256 dims of
   // a key: 256)
@@ -467,5 +813,6 @@ extern "C" int tlie_attention_generic(const void* q, const void* cache, int dtyp
   else
     return kBadArgument;
 #undef TLIE_LAUNCH
+#undef TLIE_BY_SIZE
   return launch_status();
 }

@@ -18,7 +18,6 @@ from .errors import EngineError, ErrorCode, invalid_argument, invalid_shape
 F32, BF16 = 0, 1
 ROWS_MAX = 16          # the most rows the products take that fold in the layer's neighbouring arithmetic
 ATTENTION_MAX_HEAD_DIM = 256   # the largest head size that both attention kernels take
-GENERIC_TILED_MIN_TOKENS = 4   # a sequence's tokens in a step from which the plain attention shares its reads of the keys
 _CODES = {torch.float32: F32, torch.bfloat16: BF16}
 
 
@@ -276,7 +275,7 @@ def rope_cache(qkv: Product, positions: torch.Tensor, slot_map: torch.Tensor, in
 def attention_generic(q: torch.Tensor, cache: torch.Tensor, block_table: torch.Tensor, token_seq: torch.Tensor,
                       positions: torch.Tensor, num_heads: int, num_kv_heads: int, head_dim: int,
                       window: int | None, scale: float, tiled: bool | int = False, seq_start: torch.Tensor | None = None,
-                      min_tokens: int = GENERIC_TILED_MIN_TOKENS, value_dim: int | None = None, chunk: int | None = None,
+                      min_tokens: int | None = None, value_dim: int | None = None, chunk: int | None = None,
                       sink: torch.Tensor | None = None, value_heads: int | None = None, float_out: bool = False,
                       softcap: float | None = None) -> torch.Tensor:
     """Causal attention of every token over its sequence's cached keys; any number of tokens per
@@ -319,6 +318,7 @@ def attention_generic(q: torch.Tensor, cache: torch.Tensor, block_table: torch.T
     if num_heads % num_kv_heads != 0:
         raise invalid_shape("attention: the number of heads must be a multiple of the number of kv heads")
     tiled = int(tiled)
+    min_tokens = generic_tiled_min_tokens(num_heads, num_kv_heads) if min_tokens is None else int(min_tokens)
     if tiled == 2:
         _device_tensor(seq_start, "seq_start", torch.int32)
         if seq_start.dim() != 1 or seq_start.shape[0] != block_table.shape[0] + 1 or min_tokens < 1:
@@ -331,27 +331,39 @@ def attention_generic(q: torch.Tensor, cache: torch.Tensor, block_table: torch.T
                                             num_heads, num_kv_heads, head_dim, value_dim, page_size,
                                             int(window) if window else 0, int(chunk) if chunk else 0, _ptr(sink),
                                             ctypes.c_float(scale), tiled,
-                                            _ptr(seq_start if tiled == 2 else None), int(min_tokens),
+                                            _ptr(seq_start if tiled == 2 else None), min_tokens,
                                             num_kv_heads // value_heads, 1 if float_out else 0,
-                                            ctypes.c_float(float(softcap) if softcap else 0.0), _stream()),
+                                            ctypes.c_float(float(softcap) if softcap else 0.0), _compute_units(q.device), _stream()),
            "attention_generic")
     return out
 
 
-def attention_generic_plan(ctx, head_dim: int, value_dim: int | None = None) -> int:
-    """Which form of the plain attention kernel a step takes (the `tiled` of `attention_generic`): the
-    one that shares each read of the keys among a sequence's tokens pays from a few tokens a
-    sequence on, and costs dearly where a workgroup's 32 columns belong to many sequences of one
-    token (it walks each one's context in turn).  A launched step is decided from its host arrays;
-    a recorded step of portions, whose cut changes from replay to replay, launches both and lets
-    each sequence's token count on the device decide."""
-    if max(head_dim, value_dim or head_dim) > 64 or ctx.max_new < GENERIC_TILED_MIN_TOKENS:
+def generic_tiled_min_tokens(heads: int, kv_heads: int) -> int:
+    """A sequence's tokens in a step from which the plain attention may share its reads of the keys among them: half the
+    tokens that a workgroup of 64 columns holds, 8 at least (a workgroup serves the sequences in it one after the other:
+    64 sequences of 4 tokens, 32 heads on 4, 500 keys: 75 us against 47)."""
+    return max(8, 32 // (heads // kv_heads))
+
+
+def attention_generic_plan(ctx, heads: int, kv_heads: int, head_dim: int, value_dim: int | None = None) -> int:
+    """Which form of the plain attention kernel a step takes (the `tiled` of `attention_generic`): the one that shares each
+    read of the keys among a sequence's tokens pays where its workgroups fill the chip.  A chunk of keys takes a
+    workgroup of it some 4 us however few they are; the form of a workgroup a token and key head (a token and query head,
+    without groups) takes as long as it has work.  Measured on an MI355X, the two meet at some 256 tokens of 4 key heads of
+    64 (4 x 64 tokens behind 1500: 114 us against 110, 1 x 400 199 against 130, 16 x 8 68 against 107), at more than 1600 of one
+    key head of 32, some 2500 of two of 16, and, without groups, at some 64 of 32 heads of 64 (4 x 64: 40 against 21).
+    A launched step is decided from its host arrays; a recorded step of portions, whose cut changes from replay to replay,
+    launches both and lets each sequence's token count on the device decide."""
+    widest = max(head_dim, value_dim or head_dim)
+    least = generic_tiled_min_tokens(heads, kv_heads)
+    work = ctx.num_tokens * (kv_heads if heads > kv_heads else (heads + 1) // 2) * widest
+    if widest > 64 or ctx.max_new < least or work < 1 << 16:
         return 0
     if ctx.tile_owner is not None:
         return 2
     starts = ctx.host["seq_start"]
     counts = starts[1:] - starts[:-1]
-    many = int((counts >= GENERIC_TILED_MIN_TOKENS).sum())
+    many = int((counts >= least).sum())
     return 1 if many == len(counts) else (2 if many else 0)
 
 

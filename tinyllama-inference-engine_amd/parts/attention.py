@@ -262,7 +262,7 @@ class Attention(Mixer):
                                           chunk=self.chunk, sink=self.sink, softcap=self.softcap)
         else:
             attended = ops.attention_generic(q, binding.cache, pages.block_table, ctx.token_seq, ctx.positions, self.nq, self.nkv,
-                                             self.d, self.window, self.scale, tiled=ops.attention_generic_plan(ctx, self.d, self.dv),
+                                             self.d, self.window, self.scale, tiled=ops.attention_generic_plan(ctx, self.nq, self.nkv, self.d, self.dv),
                                              seq_start=ctx.seq_start, value_dim=self.dv, chunk=self.chunk, sink=self.sink,
                                              softcap=self.softcap)
         if self.head_gate:
@@ -299,7 +299,7 @@ class Attention(Mixer):
         else:
             attended = ops.attention_generic(q, binding.cache, pages.block_table, ctx.token_seq, ctx.positions, self.nq,
                                              self.nkv, self.d, self.window, self.scale,
-                                             tiled=ops.attention_generic_plan(ctx, self.d), seq_start=ctx.seq_start)
+                                             tiled=ops.attention_generic_plan(ctx, self.nq, self.nkv, self.d), seq_start=ctx.seq_start)
         if self.head_gate:
             attended = ops.head_gate(attended, gates, gates.cols - self.gate_cols, self.nq)
         return self.o(attended, into=into)
