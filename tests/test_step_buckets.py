@@ -1,6 +1,7 @@
 """Which steps a recording serves, and at which padded sizes: decided on the host, tested without a GPU."""
 from types import SimpleNamespace
 
+import pytest
 import torch
 
 from tlie_amd.engine.step import DecodeGraph, ModelRunner, PortionGraph, StepEntry
@@ -117,3 +118,30 @@ def test_the_attention_work_list_equals_a_tile_by_tile_walk():
             made = ops.attention_tiles(start, per_kv, col_tiles, seq_len)
             assert made.dtype == np.int32 and made.flags["C_CONTIGUOUS"]
             assert np.array_equal(made, walk(start, per_kv, col_tiles, seq_len))
+
+
+@pytest.mark.parametrize("heads, kv_heads, dim, tokens, before, want", [
+    # (columns a wave / 16, parts of the keys, through LDS)
+    (32, 8, 128, 2048, 0, (2, 1, True)), (32, 8, 128, 2048, 6000, (2, 1, True)), (32, 8, 128, 1536, 0, (1, 1, True)),
+    (32, 8, 128, 1024, 2000, (1, 1, True)), (32, 8, 128, 1024, 5000, (2, 2, True)),
+    (32, 8, 128, 512, 500, (1, 1, True)), (32, 8, 128, 512, 1500, (2, 4, True)),
+    (32, 8, 128, 256, 500, (2, 1, False)), (32, 8, 128, 256, 1500, (1, 4, True)), (32, 8, 128, 256, 4000, (2, 8, True)),
+    (32, 8, 128, 128, 700, (1, 4, True)),
+    (32, 4, 64, 2048, 0, (1, 1, True)), (32, 4, 64, 512, 1500, (2, 1, False)), (32, 4, 64, 8192, 0, (2, 1, True)),
+    (4, 2, 16, 1700, 0, (1, 1, True)),
+])
+def test_how_the_prompt_attention_is_cut(heads, kv_heads, dim, tokens, before, want):
+    """The launch of the tiled attention kernel for one portion of `tokens` behind `before` positions on 256 compute units: parts
+    cover the whole sequence in multiples of 32, and a window is never cut."""
+    from types import SimpleNamespace
+    import numpy as np
+    import torch
+    from tlie_amd import ops
+    ctx = SimpleNamespace(max_new=tokens, num_seqs=1, num_tokens=tokens, max_context=before + tokens, scratch={}, tile_owner=None,
+                          compute_units=256, tokens=torch.zeros(1), host={"seq_start": np.array([0, tokens]), "seq_len": np.array([before + tokens])})
+    tiles, col_tiles, nsplit, split_len, waves, shared = ops.attention_plan(ctx, heads // kv_heads, kv_heads, dim)
+    assert (col_tiles, nsplit, shared) == want
+    assert tiles.shape[0] == -(-tokens * (heads // kv_heads) // (16 * col_tiles * (4 if shared else 1))) and (waves == 4 or not shared)
+    if nsplit > 1:
+        assert split_len % 32 == 0 and nsplit * split_len >= before + tokens > (nsplit - 1) * split_len
+        assert ops.attention_plan(ctx, heads // kv_heads, kv_heads, dim, reach=1024)[2] == 1 or not shared

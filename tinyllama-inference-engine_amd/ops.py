@@ -2132,11 +2132,7 @@ def attention_plan(ctx, groups_per_kv: int, num_kv_heads: int, head_dim: int, re
         col_tiles = attention_col_tiles(head_dim)
         # sequences of some length with portions of many columns: 4 waves take columns of their own
         # of one tile and every block of keys is brought once for all of them, through LDS (a
-        # prompt of 1536 tokens: 34 us against 42; of 8192: 450 against 780; of 512: 15 against
-        # 13).  Each wave takes 32 columns, or 16 while that leaves no more tiles than two and a
-        # half for every compute unit: the smaller ones then fill the chip better, four
-        # workgroups a compute unit (2048 tokens: 51 us against 63; 2560: 74 against 81; 3072:
-        # 100 against 98; 4096: 162 against 150)
+        # prompt of 1536 tokens: 34 us against 42; of 8192: 450 against 780; of 512: 15 against 13)
         shared = (col_tiles == 2 and head_dim <= 128 and ctx.max_context >= 768
                   and ctx.num_tokens * groups_per_kv >= 64 * ctx.num_seqs)
 
@@ -2152,10 +2148,51 @@ def attention_plan(ctx, groups_per_kv: int, num_kv_heads: int, head_dim: int, re
                 else:
                     ctx.scratch[key] = torch.from_numpy(make(ctx.host)).to(ctx.tokens.device)
             return ctx.scratch[key]
+        parts = 1
+        if shared:
+            # How many columns a wave takes (32, or 16) and into how many parts the keys are cut, by the workgroups that 32
+            # columns a wave make.  A recorded step counts by its tokens (its list also holds empty tiles), and by an eighth
+            # of its sequences.
+            columns = ctx.num_tokens * groups_per_kv
+            if ctx.tile_owner is None:
+                starts = ctx.host["seq_start"]
+                tiles_wide = int(((starts[1:] - starts[:-1]) * groups_per_kv + 127 >> 7).sum())
+            else:
+                tiles_wide = (columns + 127) // 128 + ctx.num_seqs // 8
+            blocks, units = tiles_wide * num_kv_heads, ctx.compute_units
+            if head_dim <= 64:
+                # bound by vector arithmetic: 16 columns a wave, four workgroups a unit, while that is at most five for two
+                # units (2048 tokens, 32 heads on 4: 47 us against 60; 3072: 100 against 98; 4096: 162 against 150).  At
+                # 5 for 8 units or fewer, waves that share a tile's keys without LDS (512 tokens behind 500: 20.5 us
+                # against 25.2, behind 1500: 32.1 against 41.1; 1024 tokens: 25.3 against 24.8; smaller heads not measured)
+                if 8 * blocks <= 5 * units and head_dim > 32:
+                    shared = False
+                elif 2 * blocks <= 5 * units:
+                    col_tiles = 1
+            elif 2 * blocks < 3 * units or (2 * blocks <= 5 * units and ctx.max_context < 2048):
+                # heads of more dims are bound by the LDS: a wave of 32 columns reads a block of keys once where two of 16 read it
+                # twice.  Above five workgroups for two units, and from three on where keys are many, 32 columns it is (32 heads of
+                # 128 on 8, 2048 tokens behind 0: 83 us against 89, behind 2000: 152 against 214, behind 6000: 323 against 460;
+                # 1536 behind 0: 64 against 55, behind 2000: 135 against 168).
+                # Fewer are filled up to two a unit by cutting the keys, where these are many: 1024 tokens behind 5000 171 us in
+                # two parts against 189 with 16 columns (behind 2000 103 against 95); 512 behind 1000 46 in four parts against
+                # 48, behind 1500 51 against 60, behind 7000 115 against 199; 128 behind 4000 39 in eight parts against 46
+                # without LDS.  Up to a quarter of a unit each, 16 columns in four parts up to 3072 positions (128 behind 700
+                # 21 us against 24 without LDS, behind 1500 26 against 29; 256 behind 1500 36 against 36, behind 500 28
+                # against 22).  A window's parts would mostly be empty.
+                whole, context_least = reach is not None, 4096 if 2 * blocks > units else 1536
+                if 4 * blocks > units or whole:
+                    if ctx.max_context >= context_least and not whole:
+                        parts = min(4, (2 * units + blocks - 1) // blocks)
+                    else:
+                        col_tiles = 1
+                elif ctx.max_context >= 3072:
+                    parts = min(8, (2 * units + blocks - 1) // blocks)
+                elif ctx.max_context >= 1536 or 8 * blocks <= units:
+                    col_tiles, parts = 1, 4
+                else:
+                    shared = False
         tiles = tiles_of(col_tiles * (4 if shared else 1))
-        if shared and 2 * tiles.shape[0] * num_kv_heads <= 5 * ctx.compute_units:
-            col_tiles = 1
-            tiles = tiles_of(4)
         count = tiles.shape[0] * (4 if shared else 1)
     tiles_all = count * num_kv_heads
     if not decode:
@@ -2166,7 +2203,8 @@ def attention_plan(ctx, groups_per_kv: int, num_kv_heads: int, head_dim: int, re
         # Up to 4 waves share a tile's keys, each with 128 or more: a tile that sees the whole of
         # a long sequence then takes a quarter of the time, and it is the longest tiles that
         # the step waits for (a prompt of 2048 tokens: 70 us against 87 with one wave a tile)
-        nsplit = max(1, min((512 + tiles_all - 1) // tiles_all, 16, ctx.max_context // 256))
+        # From 256 tiles on four waves each do (256 tokens, 32 heads of 128 on 8, behind 500: 22 us against 30 in two parts)
+        nsplit = parts if shared else max(1, min((512 + tiles_all - 1) // tiles_all if tiles_all < 256 else 1, 16, ctx.max_context // 256))
         waves = 4 if shared else 1
         while (not shared and waves < 4 and waves * 2 <= attention_max_waves(head_dim, col_tiles)
                and ctx.max_context >= nsplit * waves * 2 * 128):
@@ -2176,8 +2214,9 @@ def attention_plan(ctx, groups_per_kv: int, num_kv_heads: int, head_dim: int, re
         # meet in the merge kernel); then the waves of a workgroup share them, which costs no
         # launch, while a wave keeps 128 keys or more and the step has 2048 waves at most
         # (measured inside whole steps at 2048 positions: batch 1 16 parts x 1 wave, batch 8
-        # 8 x 2, batch 64 1 x 8)
-        nsplit = max(1, min((256 + tiles_all - 1) // tiles_all, 16, (context + 63) // 64))
+        # 8 x 2, batch 64 1 x 8).  More than 16 parts only of 256 keys or more (8000 positions, 8 key heads of 128, batch 1,
+        # with the merge: 17.4 us in 32 parts against 19.4 in 16)
+        nsplit = max(1, min((256 + tiles_all - 1) // tiles_all, max(16, min(32, context // 256)), (context + 63) // 64))
         waves = 1
         while (waves * 2 <= attention_max_waves(head_dim) and tiles_all * nsplit * waves * 2 <= 2048
                and context >= nsplit * waves * 2 * 128):
