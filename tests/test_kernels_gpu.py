@@ -125,6 +125,38 @@ def test_gemm_generic_gives_few_rows_the_same_bits_as_many(shape):
     assert rel_err(few, plain_linear(x[:m].double().cpu(), w.double().cpu(), b.double().cpu())) < 5e-6
 
 
+@pytest.mark.parametrize("rows", [1, 17, 33, 48, 64])
+@pytest.mark.parametrize("n, k", [(1000, 840), (18, 8), (131, 64), (250, 2056), (66, 520)])
+def test_gemm_ring_at_the_edges_of_its_strips_and_turns(rows, n, k):
+    """Every number of strips, with ragged last strips, halves and splits, turns fewer and more than the ring is deep, a half
+    without columns; W holds an infinity and a NaN in rows of their own, which must stay there.  Tolerance: the float32 sums of
+    K exact products in any order, K * 2^-24 of the sum of their magnitudes; the gate's one rounding to bfloat16 more."""
+    from tlie_amd import ops
+    torch.manual_seed(rows * n + k)
+    x = torch.randn(rows, k).bfloat16().to(DEV)
+    w = (torch.randn(n, k) / math.sqrt(k)).bfloat16().to(DEV)
+    b = torch.randn(n).bfloat16().to(DEV)
+    xd, wd, bd = x.double(), w.double(), b.double()
+    want = xd @ wd.T + bd
+    bound = (k + 8) * 2.0 ** -24 * (xd.abs() @ wd.abs().T + bd.abs())
+    for strips in range(1, 9):
+        for split_len in {64, 320, (k + 63) // 64 * 64}:
+            y = ops.gemm_ring(x, w, b, split_len=split_len, strips=strips)
+            assert y.nsplit == -(-k // split_len)
+            assert ((y.data.double().sum(0) - want).abs() <= bound).all(), (strips, split_len)
+        if n % 2 == 0:
+            got = ops.gemm_ring(x, w, b, gated=True, split_len=(k + 63) // 64 * 64, strips=strips)
+            assert rel_err(got, plain_silu_mul(want[:, 0::2], want[:, 1::2])) < 6e-3, strips
+    for whole in (False, True):
+        y = ops.gemm_ring(x, w, b, whole=whole)
+        assert ((y.data.double().sum(0) - want).abs() <= bound).all() and (y.nsplit == 1 or not whole)
+    w[n // 2, k - 1], w[n - 1, 0] = math.inf, math.nan
+    y = ops.gemm_ring(x, w, b).data.sum(0)
+    others = [i for i in range(n) if i not in (n // 2, n - 1)]
+    assert ((y[:, others].double() - want[:, others]).abs() <= bound[:, others]).all()
+    assert not y[:, n // 2].isfinite().any() and y[:, n - 1].isnan().all()
+
+
 @pytest.mark.parametrize("n,k", [(33, 5), (96, 513), (2046, 1026), (2064, 1028), (4200, 512), (500, 7000)])
 def test_gemm_generic_at_the_edges_of_its_kernels_and_gated(n, k):
     """Rows around 8 (two blocks of K at once), 16, 32, 64 (tiles begin) and the tiles' sizes, matrices around 8 and 16 rows a

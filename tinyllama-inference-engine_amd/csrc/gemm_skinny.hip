@@ -174,6 +174,147 @@ gemm_skinny_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ 
   }
 }
 
+// The same product with W in a ring of registers: the path of gated products of 17 to 64 rows and of large matrices.
+//
+// The kernel above keeps one chunk of W and x ahead, between two barriers for all waves, and reads the same columns of x in
+// every workgroup at once.  Three things held it at half of memory's rate: the chunk's loads have to come back before the next
+// are asked for; rows of x and W lie a multiple of 4 KiB apart, so that workgroups in step ask the same few of an L2's 16
+// channels; and x comes from the L2 once per compute unit, beside W.  Here
+//   * a workgroup has S strips of 16 rows of W and two waves a strip, which take a half of the split's columns each;
+//   * a wave asks for W and its share of x kDepth turns of 64 columns ahead and waits only for the oldest of them (the last
+//     turns, which ask for nothing, are code of their own: with a condition around the loads the compiler would wait for all);
+//   * workgroup b begins at turn (b / 8) % turns and goes round, so that the workgroups of a die ask for different columns;
+//   * x goes through LDS in two buffers, one barrier a turn that waits for LDS alone.
+// Measured with cold weights (us, the kernel above -> this): gated 11264 x 2048 at 64 rows 20.3 -> 15.0, at 32 16.0 -> 13.6;
+// gated 22016 x 4096 at 24 rows 48.5 -> 36.3; gated 28672 x 4096 at 64 rows 63.8 -> 49.6; 32000 x 2048 at 64 rows 38.1 -> 31.5;
+// 4096 x 11008 at 24 rows 25.7 in 11 parts -> 20.2 in 2.  Without the loads of x the first takes 12.7: W's 46 MB at 6 TB/s and
+// the launch.  Four waves a strip are slower (17.8), as is a ring of 8 (17.0) or 2 (17.3 with four waves).
+constexpr int kDepth = 4, kHalves = 2;
+
+template <int NT, int S, bool GATED>
+__global__ void __launch_bounds__(64 * S * kHalves)
+gemm_skinny_ring_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, const uint16_t* __restrict__ bias,
+                        float* __restrict__ y, uint16_t* __restrict__ act, int M, int N, int K, int split_len, int half_len,
+                        int gate_kind, float gate_alpha, float gate_limit) {
+  constexpr int kStride = 64 + kSkinnyPad, kTile = NT * 16 * kStride;          // a half's x of one turn
+  constexpr int kRing = 2 * kHalves * kTile * 2, kSums = S * kHalves * NT * 1024;
+  constexpr int kPieces = (2 * NT + S - 1) / S;                                // 1 KiB pieces of x that a wave stages a turn
+  __shared__ __attribute__((aligned(16))) char lds[kRing > kSums ? kRing : kSums];
+  uint16_t* const xs = reinterpret_cast<uint16_t*>(lds);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int strip = wave % S, half = wave / S;
+  const int col = lane & 15, grp = lane >> 4;
+  const int k_begin = blockIdx.y * split_len + half * half_len;
+  const int k_end = min(min(K, (static_cast<int>(blockIdx.y) + 1) * split_len), k_begin + half_len);
+  const int k_last = max(k_end, 8) - 8;              // columns from k_end on are loaded from here and become zeros
+  const int turns = half_len >> 6, rotation = (blockIdx.x >> 3) % turns;
+  const int n_base = min((static_cast<int>(blockIdx.x) * S + strip) * 16, N - 1);     // (rows beyond N: the last row, never stored)
+  const uint16_t* const w_base = w + static_cast<size_t>(n_base) * K;
+  const int w_row = min(col, N - 1 - n_base) * K;
+  int x_row[kPieces], x_slot[kPieces], x_k[kPieces];
+#pragma unroll
+  for (int i = 0; i < kPieces; ++i) {
+    const int piece = min(strip + i * S, 2 * NT - 1) * 64 + lane;              // (a piece staged twice is the same bytes)
+    x_row[i] = min(piece >> 3, M - 1) * K;
+    x_k[i] = (piece & 7) * 8;
+    x_slot[i] = half * kTile + (piece >> 3) * kStride + x_k[i];
+  }
+  // the columns of turn n (n < turns + kDepth), going round
+  auto column = [&](int n) {
+    n += rotation;
+    n = n >= turns ? n - turns : n;
+    return k_begin + min(n >= turns ? n - turns : n, turns - 1) * 64;
+  };
+  Pack16 a[kDepth][2];
+  uint4 staged[kDepth][kPieces];
+  auto load = [&](int n, int slot) {
+    const int k = column(n);
+#pragma unroll
+    for (int i = 0; i < kPieces; ++i) staged[slot][i] = *reinterpret_cast<const uint4*>(x + x_row[i] + min(k + x_k[i], k_last));
+#pragma unroll
+    for (int h = 0; h < 2; ++h) a[slot][h].u = *reinterpret_cast<const uint4*>(w_base + w_row + min(k + grp * 16 + h * 8, k_last));
+  };
+  auto store_x = [&](int n, int slot, int buffer) {
+    const int k = column(n);
+#pragma unroll
+    for (int i = 0; i < kPieces; ++i) {
+      uint4 v = staged[slot][i];
+      if (k + x_k[i] >= k_end) v = make_uint4(0, 0, 0, 0);
+      *reinterpret_cast<uint4*>(xs + buffer * kHalves * kTile + x_slot[i]) = v;
+    }
+  };
+  floatx4 acc[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+  auto turn = [&](int n, int slot, bool next, bool more) {
+    if (next) store_x(n + 1, (slot + 1) % kDepth, (slot + 1) & 1);
+    const int k = column(n) + grp * 16;
+    Pack16 w0 = a[slot][0], w1 = a[slot][1];
+    if (k >= k_end) w0.u = make_uint4(0, 0, 0, 0);
+    if (k + 8 >= k_end) w1.u = make_uint4(0, 0, 0, 0);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const uint16_t* from = xs + ((slot & 1) * kHalves + half) * kTile + (t * 16 + col) * kStride + grp * 16;
+      Pack16 b0, b1;
+      b0.u = *reinterpret_cast<const uint4*>(from);
+      b1.u = *reinterpret_cast<const uint4*>(from + 8);
+      acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w0.v, b0.v, acc[t], 0, 0, 0);
+      acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w1.v, b1.v, acc[t], 0, 0, 0);
+    }
+    if (more) load(n + kDepth, slot);
+    lds_barrier();                                   // this turn's x has been read, the next one's is whole
+  };
+#pragma unroll
+  for (int d = 0; d < kDepth; ++d) load(d, d);
+  store_x(0, 0, 0);
+  lds_barrier();
+  int n = 0;
+  for (; n + 2 * kDepth - 1 < turns; n += kDepth) {
+#pragma unroll
+    for (int u = 0; u < kDepth; ++u) turn(n + u, u, true, true);
+  }
+#pragma unroll
+  for (int u = 0; u < 2 * kDepth - 1; ++u)
+    if (n + u < turns) turn(n + u, u % kDepth, n + u + 1 < turns, n + u + kDepth < turns);
+
+  // acc[t][j] = this half's y[token t*16 + (lane & 15)][n_base + grp*4 + j]; the halves meet in LDS, in a fixed order
+  float4* const sums = reinterpret_cast<float4*>(lds);
+#pragma unroll
+  for (int t = 0; t < NT; ++t) sums[(wave * NT + t) * 64 + lane] = make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]);
+  lds_barrier();
+  for (int pair = wave; pair < S * NT; pair += S * kHalves) {
+    const int st = pair % S, t = pair / S;
+    const float4 low = sums[(st * NT + t) * 64 + lane], high = sums[((S + st) * NT + t) * 64 + lane];
+    float v[4] = {low.x + high.x, low.y + high.y, low.z + high.z, low.w + high.w};
+    const int row = (blockIdx.x * S + st) * 16 + grp * 4, token = t * 16 + col;
+    if (token >= M || row >= N) continue;
+    if (bias != nullptr && blockIdx.y == 0) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (row + j < N) v[j] += bf16_bits_to_float(bias[row + j]);
+    }
+    if (GATED) {
+      // (N is even and row a multiple of 4: a gate and its up are neighbours in this lane)
+      uint16_t* gated = act + static_cast<size_t>(token) * (N / 2) + (row >> 1);
+      const float first = gated_value(v[0], v[1], gate_kind, gate_alpha, gate_limit);
+      if ((N & 3) == 0) *reinterpret_cast<uint32_t*>(gated) = pack_bf16(first, gated_value(v[2], v[3], gate_kind, gate_alpha, gate_limit));
+      else {
+        gated[0] = __bfloat16_as_ushort(__float2bfloat16(first));
+        if (row + 3 < N) gated[1] = __bfloat16_as_ushort(__float2bfloat16(gated_value(v[2], v[3], gate_kind, gate_alpha, gate_limit)));
+      }
+      continue;
+    }
+    float* out = y + (static_cast<size_t>(blockIdx.y) * M + token) * N + row;
+    if ((N & 3) == 0) {
+      *reinterpret_cast<float4*>(out) = make_float4(v[0], v[1], v[2], v[3]);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (row + j < N) out[j] = v[j];
+    }
+  }
+}
+
 }  // namespace tlie
 
 using namespace tlie;
@@ -212,7 +353,41 @@ int dispatch_skinny(dim3 grid, int waves, int strips, int tiles, hipStream_t s, 
   return launch_skinny<4, 2, GATED>(grid, waves, s, x, w, bias, y, act, M, N, K, split_len, gate_kind, gate_alpha, gate_limit);
 }
 
+template <int NT, int S>
+int launch_ring(dim3 grid, hipStream_t s, const uint16_t* x, const uint16_t* w, const uint16_t* bias, float* y, uint16_t* act,
+                int M, int N, int K, int split_len, int gate_kind, float gate_alpha, float gate_limit) {
+  const int half_len = (split_len + 64 * kHalves - 1) / (64 * kHalves) * 64;
+  const dim3 block(64 * S * kHalves);
+  if (act != nullptr)
+    hipLaunchKernelGGL((gemm_skinny_ring_kernel<NT, S, true>), grid, block, 0, s, x, w, bias, y, act, M, N, K, split_len, half_len, gate_kind, gate_alpha, gate_limit);
+  else
+    hipLaunchKernelGGL((gemm_skinny_ring_kernel<NT, S, false>), grid, block, 0, s, x, w, bias, y, act, M, N, K, split_len, half_len, gate_kind, gate_alpha, gate_limit);
+  return launch_status();
+}
+
 }  // namespace
+
+// The same product by gemm_skinny_ring_kernel: strips (1 to 8) of 16 rows of W a workgroup; split_len, nsplit, y, act and the
+// gate as below.
+extern "C" int tlie_gemm_skinny_ring(const void* x, const void* w, const void* bias, float* y, void* act, int M, int N, int K,
+                                     int split_len, int strips, int gate_kind, float gate_alpha, float gate_limit, void* stream) {
+  if (gate_kind != kGateSilu && gate_kind != kGateClampedSwish) return kBadArgument;
+  if (M <= 0 || M > 64 || N <= 0 || K <= 0 || (K & 7) != 0 || K > (1 << 24) || split_len <= 0 || (split_len & 63) != 0) return kBadArgument;
+  const int nsplit = (K - 1) / split_len + 1;
+  if (act != nullptr ? (nsplit != 1 || (N & 1) != 0) : y == nullptr) return kBadArgument;
+  if (strips < 1 || strips > 8 || nsplit > 65535) return kBadArgument;
+  const dim3 grid((N - 1) / (16 * strips) + 1, nsplit);
+  const int tiles = (M + 15) / 16;
+#define TLIE_RING(NT, S)                                                                                                      \
+  if (tiles == NT && strips == S)                                                                                             \
+    return launch_ring<NT, S>(grid, (hipStream_t)stream, (const uint16_t*)x, (const uint16_t*)w, (const uint16_t*)bias, y,    \
+                              (uint16_t*)act, M, N, K, split_len, gate_kind, gate_alpha, gate_limit);
+#define TLIE_RINGS(NT) TLIE_RING(NT, 1) TLIE_RING(NT, 2) TLIE_RING(NT, 3) TLIE_RING(NT, 4) TLIE_RING(NT, 5) TLIE_RING(NT, 6) TLIE_RING(NT, 7) TLIE_RING(NT, 8)
+  TLIE_RINGS(1) TLIE_RINGS(2) TLIE_RINGS(3) TLIE_RINGS(4)
+#undef TLIE_RINGS
+#undef TLIE_RING
+  return kBadArgument;
+}
 
 // x [M, K], w [N, K], bias [N] or null: bfloat16.  y: float [nsplit, M, N] with
 // nsplit = ceil(K / split_len).  M <= 64, K % 8 == 0, split_len % 64 == 0.

@@ -122,7 +122,9 @@ def bench_kernels(cfg: dict, batch: int = 8, context: int = 2048, prompt: int = 
             count = _copies(n * k * 2)
             weights = [rand(n, k) for _ in range(count)]
             x = rand(batch, k, scale=1.0)
-            if batch <= ops.SKINNY_MAX_ROWS and name == "gate_up":
+            if ops.gemm_ring_takes(x, weights[0], name == "gate_up"):
+                launch, kind = (lambda i: ops.gemm_ring(x, weights[i], None, gated=name == "gate_up", whole=name == "head")), "gemm_ring"
+            elif batch <= ops.SKINNY_MAX_ROWS and name == "gate_up":
                 launch, kind = (lambda i: ops.gemm_skinny(x, weights[i], None, gated=True)), "gemm_skinny (gated)"
             elif batch <= ops.SKINNY_MAX_ROWS:
                 launch, kind = (lambda i: ops.gemm_skinny(x, weights[i], None)), "gemm_skinny"

@@ -2005,6 +2005,33 @@ def skinny_gated_plan(rows: int, out_features: int, in_features: int, compute_un
     return best[1], best[2]
 
 
+_RING_PLANS: dict = {}
+
+
+def ring_plan(rows: int, out_features: int, in_features: int, compute_units: int = 256, split: bool = True) -> tuple[int, int]:
+    """(k values per split, strips a workgroup) of `gemm_ring`: the workgroups that end
+    first by what a compute unit reads, its rows of W at 22 GB/s, x at 90 GB/s (both measured to within a tenth from 2048 x 2048
+    to 32000 x 4096 at 24 to 64 rows), and by the partial sums, which few compute units read again in the next kernel (3 TB/s);
+    of equals the one with more strips, for which x is read fewer times."""
+    key = (rows, out_features, in_features, compute_units, split)
+    if key not in _RING_PLANS:
+        best = None
+        for strips in range(1, 9):
+            blocks = -(-out_features // (16 * strips))
+            for nsplit in range(1, 17 if split else 2):
+                split_len = (-(-in_features // nsplit) + 63) // 64 * 64
+                if -(-in_features // split_len) != nsplit:
+                    continue
+                rounds = -(-blocks * nsplit // compute_units)
+                # microseconds; half a one for a round's first and last turns
+                cost = (rounds * (split_len * 2 * (16 * strips / 22e3 + rows / 90e3) + 0.5)
+                        + nsplit * rows * out_features * 8 / 3e6 * (nsplit > 1))
+                if best is None or cost < best[0] or (cost == best[0] and strips > best[2]):
+                    best = (cost, split_len, strips)
+        _RING_PLANS[key] = best[1:]
+    return _RING_PLANS[key]
+
+
 def _gate_args(gate) -> tuple:
     """(kind, alpha, limit) as the kernels take them, from None (the SiLU gate) or (name, alpha, limit)."""
     if gate is None:
@@ -2059,6 +2086,45 @@ def gemm_skinny(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None
     _check(library().tlie_gemm_skinny(_ptr(x), _ptr(weight), _ptr(bias), _ptr(out), _ptr(None), rows, out_features, in_features,
                                       split_len, waves, strips, *_gate_args(None), _stream()), "gemm_skinny")
     return Product(out, nsplit)
+
+
+def gemm_ring_takes(x: torch.Tensor, weight: torch.Tensor, gated: bool = False) -> bool:
+    """Matrices of 32 MB or more for more than 16 rows (us, skinny against ring: 4096 x 4096 at 24 rows 10.3, 9.3; 2048 x 5632,
+    2560 x 2048 and 2048 x 2048 at 64 rows 10.5, 11.6; 6.9, 7.5; 5.7, 6.2, where the ring leaves half as many parts and whole
+    decode steps take the same), and above 64 MB for fewer (32000 x 2048 at 4 rows 30.9, 28.0; 9216 x 2048 10.5, 10.9).  The
+    gated product of more than 16 rows goes there at any size: it is not split, and deep loads are all that fills a unit."""
+    size = weight.shape[0] * weight.shape[1] * 2
+    return gemm_skinny_takes(x, weight) and weight.shape[1] <= 1 << 24 and ((x.shape[0] > 16 and (gated or size >= 32 << 20)) or size > 64 << 20)
+
+
+def gemm_ring(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, gated: bool = False, gate=None, whole: bool = False,
+              split_len: int | None = None, strips: int | None = None):
+    """y = x . W^T (+ bias) like `gemm_skinny`, by the kernel that keeps W in a ring of registers: float partial sums
+    [nsplit, M, N], or (gated, see `gemm_skinny`) the bfloat16 gate.  whole: K is not split.  split_len, strips: the launch shape
+    (see `ring_plan`, which chooses it when they are not given)."""
+    _device_tensor(x, "x", torch.bfloat16)
+    _device_tensor(weight, "weight", torch.bfloat16)
+    if x.dim() != 2 or weight.dim() != 2 or x.shape[1] != weight.shape[1]:
+        raise invalid_shape(f"gemm_ring: x {list(x.shape)} and weight {list(weight.shape)} do not fit")
+    rows, (out_features, in_features) = x.shape[0], weight.shape
+    if not 0 < rows <= SKINNY_MAX_ROWS or in_features % 8 != 0 or in_features > 1 << 24:
+        raise invalid_argument(f"gemm_ring takes 1..{SKINNY_MAX_ROWS} rows and an inner size that is a multiple of 8, up to 2^24")
+    if bias is not None:
+        _device_tensor(bias, "bias", torch.bfloat16)
+        if bias.shape != (out_features,):
+            raise invalid_shape("gemm_ring: bias needs one entry per output")
+    if gated and out_features % 2 != 0:
+        raise invalid_shape("gemm_ring: the gated product needs an even number of rows of W")
+    if split_len is None or strips is None:
+        split_len, strips = ring_plan(rows, out_features, in_features, _compute_units(x.device), not (gated or whole))
+    if split_len <= 0 or split_len % 64 != 0 or not 1 <= strips <= 8 or (gated and split_len < in_features):
+        raise invalid_argument("gemm_ring: a split's length must be a positive multiple of 64 (gated: all of K), with 1 to 8 strips")
+    nsplit = (in_features + split_len - 1) // split_len
+    act = torch.empty((rows, out_features // 2), dtype=torch.bfloat16, device=x.device) if gated else None
+    out = None if gated else torch.empty((nsplit, rows, out_features), dtype=torch.float32, device=x.device)
+    _check(library().tlie_gemm_skinny_ring(_ptr(x), _ptr(weight), _ptr(bias), _ptr(out), _ptr(act), rows, out_features, in_features,
+                                           split_len, strips, *_gate_args(gate if gated else None), _stream()), "gemm_ring")
+    return act if gated else Product(out, nsplit)
 
 
 def attention_col_tiles(head_dim: int) -> int:

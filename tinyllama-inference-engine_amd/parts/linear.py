@@ -70,6 +70,9 @@ class Linear:
                 return ops.gemm_rows(x, self.weight, self.bias, "store")
         if isinstance(x, ops.NormedRows):
             raise ops.invalid_argument("this product cannot fold the norm before it; ask takes_rows() first")
+        if (ops.gemm_ring_takes(x, self.weight, gated) and (not gated or self.out_features % 2 == 0)
+                and (gated or not whole or out_dtype == torch.float32)):
+            return ops.gemm_ring(x, self.weight, self.bias, gated=gated, gate=gate, whole=whole)
         if gated and ops.gemm_skinny_takes(x, self.weight) and self.out_features % 2 == 0:
             return ops.gemm_skinny(x, self.weight, self.bias, gated=True, gate=gate)     # all of K in a workgroup: the gate is applied there
         if ops.gemm_skinny_takes(x, self.weight) and (not whole or out_dtype == torch.float32):
