@@ -721,6 +721,30 @@ def test_attention_mfma(case):
     assert rel_err(split_portion, want[first:first + count]) < TOL["bfloat16"]
 
 
+@pytest.mark.parametrize("count, nq, nkv, nsplit, waves", [(33, 8, 8, 1, 2), (40, 8, 8, 2, 1), (64, 40, 2, 1, 4), (64, 9, 9, 1, 1), (65, 8, 8, 1, 2),
+                                                           (7, 40, 40, 1, 2)])
+def test_a_decode_step_of_more_workgroups_than_compute_units_serves_every_sequence(count, nq, nkv, nsplit, waves):
+    """Sequences taken longest first: equal lengths, a single position, the most sequences that are ranked and one more, 20 heads a
+    group (two tiles a sequence), a round that is no multiple of the sequences.  Each sequence's result has the bits of that sequence in a step of its own."""
+    from tlie_amd import ops
+    d, page, longest = 64, 16, 300
+    rng = random.Random(count)
+    lens = [rng.choice((1, 17, longest, rng.randint(1, longest))) for _ in range(count)]
+    blocks = longest // page + 1
+    torch.manual_seed(count)
+    order = torch.randperm(count * blocks)
+    table = order.view(count, blocks).int().to(DEV)
+    cache = torch.randn(count * blocks, 2, nkv, page * d).bfloat16().to(DEV)
+    q = torch.randn(count, nq * d).bfloat16().to(DEV)
+    positions = torch.tensor([n - 1 for n in lens], dtype=torch.int32, device=DEV)
+    split_len = (longest // nsplit + 31) // 32 * 32
+    launch = lambda rows: ops.attention_mfma(q[rows].contiguous(), cache, table[rows].contiguous(), None, positions[rows].contiguous(), nq, nkv, d,
+                                             None, 1.0 / math.sqrt(d), nsplit, split_len, 1, waves)
+    together = launch(slice(0, count))
+    for i in range(count):
+        assert torch.equal(launch(slice(i, i + 1))[0], together[i]), (i, lens[i])
+
+
 def test_attention_mfma_finds_one_key_among_hundreds():
     tokens, nq, nkv, d, page = 600, 4, 2, 32, 16
     torch.manual_seed(1)

@@ -143,8 +143,29 @@ attention_mfma_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict
     seq = tile.x, tok0 = tile.y, ntok = tile.z, col0 = tile.w;
     if (ntok <= 0) return;                       // a list of fixed size ends in tiles without tokens (the same for the whole workgroup)
   } else {
-    const int per_seq = (G + 16 * CT - 1) / (16 * CT);
-    seq = tok0 = blockIdx.x / per_seq, ntok = 1, col0 = (blockIdx.x % per_seq) * 16 * CT;
+    const int per_seq = (G + 16 * CT - 1) / (16 * CT), per_token = per_seq * static_cast<int>(gridDim.y);
+    const int tokens = static_cast<int>(gridDim.x) / per_seq, total = tokens * per_token;
+    seq = blockIdx.x / per_seq, col0 = blockIdx.x % per_seq;
+    if (!SHARED && total > round_size && round_size > 0 && tokens <= 64) {
+      // A decode step of more workgroups than compute units, and of sequences of their own lengths: the workgroups of one
+      // unit lie a round apart, and where a round is a multiple of the tokens they would all be the same sequence's, so that
+      // the kernel took as long as the longest sequence on every place (24 sequences of 129 to 1060 positions of 32, 32 heads of
+      // 128: 66 us, in this order 55; 64 of 129 to 1500, 32 heads of 128 on 8: 56, 48).  The sequences are taken longest first, and the rounds forwards
+      // and backwards in turn like a prompt's tiles.  Every wave ranks the sequences itself, a sequence a lane.
+      const int lane_pos = positions[min(lane, tokens - 1)];
+      int rank = 0;
+      for (int j = 0; j < tokens; ++j) {
+        const int other = __builtin_amdgcn_readlane(lane_pos, j);
+        rank += other > lane_pos || (other == lane_pos && j < lane);
+      }
+      const int linear = blockIdx.y * gridDim.x + blockIdx.x, round = linear / round_size, place = linear - round * round_size;
+      const int in_round = min(round_size, total - round * round_size);
+      const int item = round * round_size + ((round & 1) ? in_round - 1 - place : place);
+      const int wanted = item / per_token, rest = item - wanted * per_token;
+      seq = __ffsll(__ballot(lane < tokens && rank == wanted)) - 1;
+      kvh = rest / per_seq, col0 = rest - kvh * per_seq;
+    }
+    tok0 = seq, ntok = 1, col0 *= 16 * CT;
   }
   // everything about the tile is the same for all lanes: keep it in scalar registers, so that the
   // conditions on it below are branches of the wave and not masks over its lanes
