@@ -477,6 +477,41 @@ def test_kernels_refuse_what_they_do_not_take():
 
 # ---- the bfloat16 kernels on the matrix cores ---------------------------------------------------------
 
+@pytest.mark.parametrize("tokens, nq, nkv, d, page", [(256, 4, 2, 64, 16), (257, 3, 3, 24, 8), (400, 2, 1, 128, 64), (330, 4, 4, 40, 16), (300, 2, 2, 32, 4)])
+@pytest.mark.parametrize("dtypes", [("float32", "float32"), ("float32", "bfloat16"), ("bfloat16", "bfloat16")])
+def test_values_placed_by_tiles_lie_where_single_tokens_put_them(dtypes, tokens, nq, nkv, d, page):
+    """Runs of slots that begin and end within a page, tokens without a slot, single slots out of order, tiles with fewer tokens
+    and columns than they hold, pages of too few rows for tiles: the same bytes as the same tokens in steps of less than a tile, in
+    q and in every byte of the cache."""
+    from tlie_amd import ops
+    torch.manual_seed(tokens + d)
+    pages = 2 * tokens // page + 8
+    order = torch.randperm(pages)
+    slots, place = [], 3                                          # (place: a position whose page is looked up, as in a sequence)
+    while len(slots) < tokens:
+        run = random.Random(len(slots)).choice((1, 2, 7, 8, 21, 40))
+        slots += [int(order[p // page]) * page + p % page for p in range(place, place + run)] + [-1]
+        place += run + random.Random(run + place).choice((0, 1, 3))
+    slots = torch.tensor(slots[:tokens], dtype=torch.int32)
+    if tokens == 330:
+        slots = slots[torch.randperm(tokens)]                     # a decode step: every token a sequence of its own
+    extra, rot = 8, d // 8 * 8 // 16 * 16
+    qkv = torch.randn(tokens, (nq + 2 * nkv) * d + extra).to(DT[dtypes[0]]).to(DEV)
+    positions = torch.randint(0, 5000, (tokens,), dtype=torch.int32).to(DEV)
+    inv_freq = torch.pow(torch.tensor(10000.0), -2.0 * torch.arange(rot // 2, dtype=torch.float32) / rot).to(DEV)
+    slots = slots.to(DEV)
+
+    def placed(step):
+        cache = torch.full((pages, 2, nkv, page * d), -3.0).to(DT[dtypes[1]]).to(DEV)
+        q = [ops.rope_cache(ops.Product(qkv[i:i + step].contiguous(), 1), positions[i:i + step].contiguous(), slots[i:i + step].contiguous(), inv_freq,
+                            rot, cache, nq, nkv, d, DT[dtypes[1]], paired=True, extra_cols=extra, runs=True) for i in range(0, tokens, step)]
+        return torch.cat(q), cache
+
+    whole, single = placed(tokens), placed(90)
+    assert torch.equal(whole[0], single[0]) and torch.equal(whole[1], single[1])
+    assert (whole[1][:, 1] != -3.0).any()
+
+
 @pytest.mark.parametrize("shape", [(1, 40, 64), (3, 177, 176), (16, 2560, 2048), (17, 100, 520), (33, 64, 5632),
                                    (64, 515, 1000), (8, 32000, 2048), (5, 16, 8)])
 def test_gemm_skinny(shape):

@@ -80,17 +80,77 @@ __global__ void rope_cache_kernel(const D* __restrict__ qkv, int nsplit, size_t 
 // The same for one summand with eight input columns a thread (16-byte loads): d % 8 == 0 and, where
 // there is rotation, paired columns and rot_dim % 8 == 0, so that a thread holds four whole pairs.
 // One block a token; blockDim.x covers (nq + 2 nkv) * d / 8 groups, or loops.
+// value_tiles > 0: the blocks from `tokens` on place the values instead, each a tile of 64 tokens by 64 value columns (value_tiles of
+// them side by side): a value head lies transposed in its page, so that a token's values are single elements a row of the page
+// apart, and stored from the token's own block each is a request of its own to the L2 (2048 tokens of 32 + 2 x 32 heads of 128:
+// 8.4 million, 57 us where 100 MB take 21).  The tile goes through LDS, and eight tokens in a row whose slots are eight aligned
+// rows of a page become one store a dim (with blocks of 256 threads 22 us; 32 + 2 x 8
+// heads of 128: 21.8 -> 12.5; 32 + 2 x 4 of 64: 10.7 -> 9.3); the ends of a sequence's run keep single elements.
+constexpr int kValueTile = 64;
+
+template <typename D, typename A>
+__device__ __forceinline__ void place_value_tile(const D* __restrict__ qkv, const int* __restrict__ slot_map, A* __restrict__ cache, int tokens,
+                                                 int first_token, int first_column, int nq, int nkv, int d, int page_size, int row_width) {
+  constexpr int kRow = kValueTile + 4 / sizeof(A);               // (a row's end moves the next one bank on)
+  __shared__ A tile[kValueTile * kRow];
+  const int columns = nkv * d, count = min(kValueTile, tokens - first_token);
+  const D* from = qkv + static_cast<size_t>(first_token) * row_width + (nq + nkv) * d + first_column;
+  for (int i = threadIdx.x; i < kValueTile * (kValueTile / 8); i += blockDim.x) {
+    const int token = i / (kValueTile / 8), c = i % (kValueTile / 8) * 8;
+    if (token >= count || first_column + c >= columns) continue;
+    float v[8];
+    load8(from + static_cast<size_t>(token) * row_width + c, v);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) tile[token * kRow + c + j] = from_float<A>(v[j]);
+  }
+  // a run: tokens whose slots follow one another within eight aligned rows; every wave finds the runs' first tokens itself
+  const int lane = threadIdx.x & 63, waves = blockDim.x >> 6;
+  const int slot = lane < count ? slot_map[first_token + lane] : -1;
+  const int before = __shfl_up(slot, 1, 64);
+  const unsigned long long firsts = __ballot(lane == 0 || slot < 0 || slot != before + 1 || (slot & 7) == 0);
+  __syncthreads();
+  const int column = first_column + lane, head = column / d, e = column - head * d;
+  const size_t head_stride = static_cast<size_t>(page_size) * d;
+  unsigned long long left = firsts;
+  for (int run = 0; left != 0; ++run) {
+    const int first = __ffsll(left) - 1;
+    left &= left - 1;
+    if (run % waves != static_cast<int>(threadIdx.x >> 6)) continue;
+    const int length = (left != 0 ? __ffsll(left) - 1 : kValueTile) - first;      // (tokens from `count` on are runs of their own)
+    const int at = __builtin_amdgcn_readlane(slot, first);
+    if (at < 0 || column >= columns) continue;
+    A* out = cache + (static_cast<size_t>(at / page_size) * 2 * nkv + nkv + head) * head_stride + static_cast<size_t>(e) * page_size + at % page_size;
+    const A* values = tile + first * kRow + lane;
+    if (length == 8) {
+      alignas(16) A eight[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) eight[j] = values[j * kRow];
+#pragma unroll
+      for (int j = 0; j < static_cast<int>(sizeof(A)) / 2; ++j)
+        reinterpret_cast<uint4*>(out)[j] = *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(eight) + j * 16);
+    } else {
+      for (int j = 0; j < length; ++j) out[j] = values[j * kRow];
+    }
+  }
+}
+
 template <typename D, typename A>
 __global__ void rope_cache_wide_kernel(const D* __restrict__ qkv, const int* __restrict__ positions,
                                        const int* __restrict__ slot_map, const float* __restrict__ inv_freq,
                                        int rot_dim, A* __restrict__ q_out, A* __restrict__ cache, int nq, int nkv,
-                                       int d, int page_size, int row_width, const float* __restrict__ head_scale) {
+                                       int d, int page_size, int row_width, const float* __restrict__ head_scale, int tokens,
+                                       int value_tiles) {
+  if (static_cast<int>(blockIdx.x) >= tokens) {
+    const int tile = blockIdx.x - tokens;
+    place_value_tile(qkv, slot_map, cache, tokens, tile / value_tiles * kValueTile, tile % value_tiles * kValueTile, nq, nkv, d, page_size, row_width);
+    return;
+  }
   extern __shared__ float lds[];
   const int half = rot_dim / 2;
   float* cosines = lds;                  // half
   float* sines = cosines + half;         // half
   const int t = blockIdx.x;
-  const int heads = nq + 2 * nkv, per_head = d / 8;
+  const int heads = value_tiles > 0 ? nq + nkv : nq + 2 * nkv, per_head = d / 8;
   const int slot = slot_map[t];
   // this thread's first eight columns are asked for before the angles are made: their way from memory
   // is then hidden behind the sines and cosines (and the barrier after them)
@@ -289,10 +349,11 @@ extern "C" int tlie_qkv_place(const void* qkv, int in_dtype, int nsplit, long lo
   return kBadArgument;
 }
 
+// runs: the slots mostly follow one another, as those of a prompt do (only decides how values are stored).
 extern "C" int tlie_rope_cache(const void* qkv, int in_dtype, int nsplit, long long split_stride,
                                const int* positions, const int* slot_map, const float* inv_freq, int rot_dim,
                                void* q_out, void* cache, int act_dtype, int tokens, int nq, int nkv, int d,
-                               int page_size, int paired, int row_width, const float* head_scale, void* stream) {
+                               int page_size, int paired, int row_width, const float* head_scale, int runs, void* stream) {
   if (row_width < (nq + 2 * nkv) * d) return kBadArgument;
   if (tokens <= 0 || nq <= 0 || nkv <= 0 || d <= 0 || d > 1024 || page_size <= 0 || nsplit < 1) return kBadArgument;
   if (rot_dim < 0 || rot_dim > d || rot_dim % 2 != 0) return kBadArgument;
@@ -301,14 +362,22 @@ extern "C" int tlie_rope_cache(const void* qkv, int in_dtype, int nsplit, long l
   const bool aligned = ((reinterpret_cast<uintptr_t>(qkv) | reinterpret_cast<uintptr_t>(q_out) |
                          reinterpret_cast<uintptr_t>(cache)) & 31) == 0;
   if (nsplit == 1 && (d & 7) == 0 && (row_width & 7) == 0 && aligned && (inv_freq == nullptr || (paired && (rot_dim & 7) == 0))) {
-    const int groups = heads * d / 8;
-    const int wide = groups >= 1024 ? 1024 : (groups + 63) / 64 * 64;
+    // Values by tiles where the caller says that slots mostly follow one another, from 256 tokens on (100 tokens of 32 + 2 x 4
+    // heads of 64: 3.9 us without, 5.4 with them, 512: 4.9, 4.6), for pages whose rows come in eights.  Slots on their own stay
+    // with their token's block: 128 of 32 + 2 x 8 heads of 128 take 5.2 us, by tiles 12.9.
+    const int value_tiles = runs && tokens >= 4 * kValueTile && page_size % 8 == 0 ? (nkv * d + kValueTile - 1) / kValueTile : 0;
+    const long long blocks = tokens + static_cast<long long>(value_tiles) * ((tokens + kValueTile - 1) / kValueTile);
+    if (blocks > 0x7fffffffLL) return kBadArgument;
+    const int groups = (value_tiles > 0 ? nq + nkv : heads) * d / 8;
+    // (beside the tiles a token's block has 256 threads: more blocks a unit hide each other's sines and barrier; 1024: 40 us, 512: 26, 256: 22)
+    const int cap = value_tiles > 0 ? 256 : 1024;
+    const int wide = groups >= cap ? cap : (groups + 63) / 64 * 64;
     const size_t wide_lds = static_cast<size_t>(rot_dim) * sizeof(float);
 #define TLIE_WIDE(DC, D, AC, A)                                                                              \
   if (in_dtype == DC && act_dtype == AC) {                                                                   \
-    hipLaunchKernelGGL((rope_cache_wide_kernel<D, A>), dim3(tokens), dim3(wide), wide_lds, s, (const D*)qkv,   \
+    hipLaunchKernelGGL((rope_cache_wide_kernel<D, A>), dim3(static_cast<unsigned>(blocks)), dim3(wide), wide_lds, s, (const D*)qkv,   \
                        positions, slot_map, inv_freq, rot_dim, (A*)q_out, (A*)cache, nq, nkv, d, page_size,   \
-                       row_width, head_scale);                                                               \
+                       row_width, head_scale, tokens, value_tiles);                                          \
     return launch_status();                                                                                  \
   }
     TLIE_WIDE(kF32, float, kF32, float)

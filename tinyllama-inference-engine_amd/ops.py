@@ -239,10 +239,11 @@ def paired_rows(num_heads: int, num_kv_heads: int, head_dim: int, rot_dim: int) 
 def rope_cache(qkv: Product, positions: torch.Tensor, slot_map: torch.Tensor, inv_freq: torch.Tensor | None,
                rot_dim: int, cache: torch.Tensor, num_heads: int, num_kv_heads: int, head_dim: int,
                act_dtype: torch.dtype, paired: bool = False, extra_cols: int = 0,
-               head_scale: torch.Tensor | None = None) -> torch.Tensor:
+               head_scale: torch.Tensor | None = None, runs: bool = False) -> torch.Tensor:
     """Rotates q and k, returns q [T, nq * d], writes k and v into the cache rows of `slot_map`.
     paired: qkv's columns are in the order of `paired_rows`.  extra_cols: columns that the product has after q, k and v, which
     are someone else's to read.  head_scale (float32 [nq]): query head h is multiplied by head_scale[h].
+    runs: most tokens' slots follow one another (a prompt's), which only decides how values are stored.
 
     slot_map[t] = page * page_size + row, or -1 to skip.  The slot map comes from the cache
     manager, which hands out only rows of pages it owns."""
@@ -268,7 +269,7 @@ def rope_cache(qkv: Product, positions: torch.Tensor, slot_map: torch.Tensor, in
                                      ctypes.c_longlong(qkv.split_stride), _ptr(positions), _ptr(slot_map), _ptr(inv_freq),
                                      rot_dim, _ptr(q_out), _ptr(cache), dtype_code(act_dtype), tokens, num_heads,
                                      num_kv_heads, head_dim, page_size, 1 if paired else 0, qkv.cols, _ptr(head_scale),
-                                     _stream()), "rope_cache")
+                                     int(runs), _stream()), "rope_cache")
     return q_out
 
 
