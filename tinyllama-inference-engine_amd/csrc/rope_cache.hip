@@ -363,7 +363,8 @@ extern "C" int tlie_rope_cache(const void* qkv, int in_dtype, int nsplit, long l
                          reinterpret_cast<uintptr_t>(cache)) & 31) == 0;
   if (nsplit == 1 && (d & 7) == 0 && (row_width & 7) == 0 && aligned && (inv_freq == nullptr || (paired && (rot_dim & 7) == 0))) {
     // Values by tiles where the caller says that slots mostly follow one another, from 256 tokens on (100 tokens of 32 + 2 x 4
-    // heads of 64: 3.9 us without, 5.4 with them, 512: 4.9, 4.6), for pages whose rows come in eights.  Slots on their own stay
+    // heads of 64: 3.9 us without, 5.4 with them, 256 in runs of 60: 4.2, 4.5, 512: 5.0, 5.0, in one run 4.9, 4.6; 512 of 32 + 2 x 8 of 128
+    // in runs of 60: 8.7, 6.2), for pages whose rows come in eights.  Slots on their own stay
     // with their token's block: 128 of 32 + 2 x 8 heads of 128 take 5.2 us, by tiles 12.9.
     const int value_tiles = runs && tokens >= 4 * kValueTile && page_size % 8 == 0 ? (nkv * d + kValueTile - 1) / kValueTile : 0;
     const long long blocks = tokens + static_cast<long long>(value_tiles) * ((tokens + kValueTile - 1) / kValueTile);
