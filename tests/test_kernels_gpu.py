@@ -157,6 +157,30 @@ def test_gemm_ring_at_the_edges_of_its_strips_and_turns(rows, n, k):
     assert not y[:, n // 2].isfinite().any() and y[:, n - 1].isnan().all()
 
 
+def added_up(parts):
+    """Partial sums [parts, M, N] as the kernels that take them add them up: float, four interleaved chains."""
+    chains, whole = [torch.zeros_like(parts[0]) for _ in range(4)], parts.shape[0] // 4 * 4
+    for i, part in enumerate(parts):
+        chains[i % 4 if i < whole else 0] += part
+    return parts[0] if len(parts) == 1 else (chains[0] + chains[1]) + (chains[2] + chains[3])
+
+
+@pytest.mark.parametrize("rows, n, k, whole", [(24, 12288, 4096, False), (64, 4096, 11008, False), (64, 2304, 14336, False), (24, 9000, 4096, True),
+                                               (17, 2048, 1536, True)])
+def test_gemm_ring_is_as_exact_as_the_product_it_stands_in_for(rows, n, k, whole):
+    """Float sums of exact products: the error against 64 bits (2-norm over some 1e5 results, which varies by less than 1%), of
+    either kernel as it is launched for these sizes, parts added up as their consumers do."""
+    from tlie_amd import ops
+    torch.manual_seed(n + k)
+    x = torch.randn(rows, k).bfloat16().to(DEV)
+    w = (torch.randn(n, k) / math.sqrt(k)).bfloat16().to(DEV)
+    want = x.double() @ w.double().T
+    error = lambda parts: float((added_up(parts).double() - want).norm() / want.norm())
+    ring = error(ops.gemm_ring(x, w, None, whole=whole).data)
+    skinny = error(ops.gemm_skinny(x, w, None, split_len=(k + 63) // 64 * 64 if whole else None).data)
+    assert ring < 1.02 * skinny, (ring, skinny)
+
+
 @pytest.mark.parametrize("n,k", [(33, 5), (96, 513), (2046, 1026), (2064, 1028), (4200, 512), (500, 7000)])
 def test_gemm_generic_at_the_edges_of_its_kernels_and_gated(n, k):
     """Rows around 8 (two blocks of K at once), 16, 32, 64 (tiles begin) and the tiles' sizes, matrices around 8 and 16 rows a

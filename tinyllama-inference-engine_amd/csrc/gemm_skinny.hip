@@ -243,9 +243,16 @@ gemm_skinny_ring_kernel(const uint16_t* __restrict__ x, const uint16_t* __restri
       *reinterpret_cast<uint4*>(xs + buffer * kHalves * kTile + x_slot[i]) = v;
     }
   };
-  floatx4 acc[NT];
+  // Sums of 512 columns and fewer (2 kDepth turns) join a total: one chain over a half's 2048 columns has
+  // half again the error of the kernel above, which cuts K in more parts (against 64 bits, 12288 x 4096 at 24 rows: 1.9e-7 there,
+  // 2.7e-7 in one chain, 1.35e-7 so; 4096 x 11008 at 64 rows 1.4e-7, 2.2e-7, 1.3e-7).  It costs 0 to 2% of the time.
+  floatx4 acc[NT], total[NT];
 #pragma unroll
-  for (int t = 0; t < NT; ++t) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < NT; ++t) acc[t] = total[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+  auto join = [&]() {
+#pragma unroll
+    for (int t = 0; t < NT; ++t) total[t] += acc[t], acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+  };
   auto turn = [&](int n, int slot, bool next, bool more) {
     if (next) store_x(n + 1, (slot + 1) % kDepth, (slot + 1) & 1);
     const int k = column(n) + grp * 16;
@@ -272,15 +279,19 @@ gemm_skinny_ring_kernel(const uint16_t* __restrict__ x, const uint16_t* __restri
   for (; n + 2 * kDepth - 1 < turns; n += kDepth) {
 #pragma unroll
     for (int u = 0; u < kDepth; ++u) turn(n + u, u, true, true);
+    if (n & kDepth) join();
   }
 #pragma unroll
-  for (int u = 0; u < 2 * kDepth - 1; ++u)
+  for (int u = 0; u < 2 * kDepth - 1; ++u) {
     if (n + u < turns) turn(n + u, u % kDepth, n + u + 1 < turns, n + u + kDepth < turns);
+    if (u == kDepth - 1) join();
+  }
+  join();
 
-  // acc[t][j] = this half's y[token t*16 + (lane & 15)][n_base + grp*4 + j]; the halves meet in LDS, in a fixed order
+  // total[t][j] = this half's y[token t*16 + (lane & 15)][n_base + grp*4 + j]; the halves meet in LDS, in a fixed order
   float4* const sums = reinterpret_cast<float4*>(lds);
 #pragma unroll
-  for (int t = 0; t < NT; ++t) sums[(wave * NT + t) * 64 + lane] = make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]);
+  for (int t = 0; t < NT; ++t) sums[(wave * NT + t) * 64 + lane] = make_float4(total[t][0], total[t][1], total[t][2], total[t][3]);
   lds_barrier();
   for (int pair = wave; pair < S * NT; pair += S * kHalves) {
     const int st = pair % S, t = pair / S;
@@ -376,14 +387,16 @@ extern "C" int tlie_gemm_skinny_ring(const void* x, const void* w, const void* b
   const int nsplit = (K - 1) / split_len + 1;
   if (act != nullptr ? (nsplit != 1 || (N & 1) != 0) : y == nullptr) return kBadArgument;
   if (strips < 1 || strips > 8 || nsplit > 65535) return kBadArgument;
-  const dim3 grid((N - 1) / (16 * strips) + 1, nsplit);
   const int tiles = (M + 15) / 16;
+  if (tiles == 4 && strips == 7) strips = 6;         // (seven would spill: 14 waves have 128 registers each, and stage two pieces)
+  const dim3 grid((N - 1) / (16 * strips) + 1, nsplit);
 #define TLIE_RING(NT, S)                                                                                                      \
   if (tiles == NT && strips == S)                                                                                             \
     return launch_ring<NT, S>(grid, (hipStream_t)stream, (const uint16_t*)x, (const uint16_t*)w, (const uint16_t*)bias, y,    \
                               (uint16_t*)act, M, N, K, split_len, gate_kind, gate_alpha, gate_limit);
 #define TLIE_RINGS(NT) TLIE_RING(NT, 1) TLIE_RING(NT, 2) TLIE_RING(NT, 3) TLIE_RING(NT, 4) TLIE_RING(NT, 5) TLIE_RING(NT, 6) TLIE_RING(NT, 7) TLIE_RING(NT, 8)
-  TLIE_RINGS(1) TLIE_RINGS(2) TLIE_RINGS(3) TLIE_RINGS(4)
+  TLIE_RINGS(1) TLIE_RINGS(2) TLIE_RINGS(3)
+  TLIE_RING(4, 1) TLIE_RING(4, 2) TLIE_RING(4, 3) TLIE_RING(4, 4) TLIE_RING(4, 5) TLIE_RING(4, 6) TLIE_RING(4, 8)
 #undef TLIE_RINGS
 #undef TLIE_RING
   return kBadArgument;

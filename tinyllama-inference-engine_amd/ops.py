@@ -2018,6 +2018,8 @@ def ring_plan(rows: int, out_features: int, in_features: int, compute_units: int
     if key not in _RING_PLANS:
         best = None
         for strips in range(1, 9):
+            if strips == 7 and rows > 48:                  # (spills, see the kernel's entry)
+                continue
             blocks = -(-out_features // (16 * strips))
             for nsplit in range(1, 17 if split else 2):
                 split_len = (-(-in_features // nsplit) + 63) // 64 * 64
