@@ -252,6 +252,8 @@ struct ColumnState {
 // maximum and sum; its values are scaled and wait for the chunk's.
 template <bool CAP>
 __device__ __forceinline__ void take_scores(floatx4 (&dot)[4], ColumnState& state, int start, int lo, int pos, int g, float scale, float softcap) {
+  settle(dot);
+  settle(state.acc);
   float top = -INFINITY;
 #pragma unroll
   for (int t = 0; t < 4; ++t)
@@ -508,6 +510,7 @@ attention_generic_tiled_kernel(const T* __restrict__ q, const T* __restrict__ ca
         }
       }
       if (n1 >= chunks || (n1 & 3) != (n & 3)) {   // the state's last chunk
+        settle(own.acc);
         if ((n & 3) == 0) kept0 = own, own = kept1;
         else if ((n & 3) == 1) kept1 = own, own = kept2;
         else if ((n & 3) == 2) kept2 = own, own = kept3;
@@ -696,6 +699,7 @@ attention_generic_few_kernel(const T* __restrict__ q, const T* __restrict__ cach
       look_up(start + 512);
     }
   }
+  settle(state.acc);
   __syncthreads();
 #pragma unroll
   for (int u = 0; u < 4; ++u)

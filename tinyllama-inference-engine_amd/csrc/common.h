@@ -78,6 +78,29 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// What matrix instructions have left in v, ready to be read.  A result must not be read for up to 12 states after its
+// instruction; the compiler (ROCm 7.2.0, AMD clang 22.0.0git) puts in that wait, but counts it along one path only where two
+// branches meet again: with code for the wait on the longer of the two and none on the shorter, the reader behind them comes too
+// early on the shorter (10 states wanted, 2 left; the last element of the result was wrong).  So whatever reads results behind a
+// branch that came after their instruction asks for them here: the first empty statements stand behind the instructions, the
+// last ones in front of the readers, and the wait between the two.  16 states, some 7 ns.
+template <typename V, int N>
+__device__ __forceinline__ void settle(V (&v)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) asm volatile("" : "+v"(v[i]));
+  asm volatile("s_nop 15");
+#pragma unroll
+  for (int i = 0; i < N; ++i) asm volatile("" : "+v"(v[i]));
+}
+template <typename V, int N, int M>
+__device__ __forceinline__ void settle(V (&v)[N][M]) {
+#pragma unroll
+  for (int i = 0; i < N * M; ++i) asm volatile("" : "+v"(v[i / M][i % M]));
+  asm volatile("s_nop 15");
+#pragma unroll
+  for (int i = 0; i < N * M; ++i) asm volatile("" : "+v"(v[i / M][i % M]));
+}
+
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
   for (int offset = kWave / 2; offset > 0; offset >>= 1) v += __shfl_xor(v, offset, kWave);

@@ -127,7 +127,6 @@ gemm_generic_few_kernel(const X* __restrict__ x, const W* __restrict__ w, const 
         to_quarters(a);
 #pragma unroll
         for (int i = 0; i < MT; ++i) to_quarters(b[i]);
-        // (last, behind every branch: see the kernel of many rows)
 #pragma unroll
         for (int e = 0; e < 4; ++e)
 #pragma unroll
@@ -135,6 +134,7 @@ gemm_generic_few_kernel(const X* __restrict__ x, const W* __restrict__ w, const 
       }
       k0 = next;
     }
+    settle(acc);
     // lane (r, g) holds what the instruction's rows 4 g .. 4 g + 3 (of W) have for its column r (of x)
     if (PAIR) {
       if ((r >> 3) == (g >> 1))
@@ -237,8 +237,6 @@ gemm_generic_kernel(const X* __restrict__ x, const W* __restrict__ w, const W* _
   const int steps = (K + kStepK - 1) / kStepK;
   const float* my_w = ws + ((wave & 1) * (TN / 2) + (lane & 15)) * kStride + (lane >> 4) * 4;
   const float* my_x = xs + ((wave >> 1) * (TM / 2) + (lane & 15)) * kStride + (lane >> 4) * 4;
-  // (the matrix instructions stand last in a turn, behind every branch: this compiler has been seen to read their results
-  // too early, without the wait they need, where a branch lay between)
 #pragma unroll
   for (int j = 0; j < D; ++j)
     if (j < steps) ask(j, j);
@@ -251,6 +249,7 @@ gemm_generic_kernel(const X* __restrict__ x, const W* __restrict__ w, const W* _
       if (s >= steps) break;                               // (the same for the whole workgroup)
       lds_barrier();                                       // this turn's tiles are whole, the last turn's have been read
       if (s > 0 && s % (kBlockK / kStepK) == 0) {          // a block of K has ended: its sums join the totals
+        settle(acc);
 #pragma unroll
         for (int i = 0; i < A; ++i)
 #pragma unroll
@@ -276,6 +275,7 @@ gemm_generic_kernel(const X* __restrict__ x, const W* __restrict__ w, const W* _
       }
     }
   }
+  settle(acc);
 #pragma unroll
   for (int i = 0; i < A; ++i)
 #pragma unroll

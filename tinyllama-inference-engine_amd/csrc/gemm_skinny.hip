@@ -250,6 +250,7 @@ gemm_skinny_ring_kernel(const uint16_t* __restrict__ x, const uint16_t* __restri
 #pragma unroll
   for (int t = 0; t < NT; ++t) acc[t] = total[t] = floatx4{0.f, 0.f, 0.f, 0.f};
   auto join = [&]() {
+    settle(acc);
 #pragma unroll
     for (int t = 0; t < NT; ++t) total[t] += acc[t], acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
   };
