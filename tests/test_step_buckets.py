@@ -52,6 +52,23 @@ def test_what_no_recording_serves():
     assert made.records(entries([5, 3])) is None and not made.replays(entries([1]))
 
 
+def prompt_step(tokens, before, seqs=1):
+    import numpy as np
+    return SimpleNamespace(max_new=tokens, num_seqs=seqs, num_tokens=tokens * seqs, max_context=before + tokens, scratch={}, tile_owner=None,
+                           compute_units=256, tokens=torch.zeros(1),
+                           host={"seq_start": np.arange(seqs + 1) * tokens, "seq_len": np.full(seqs, before + tokens)})
+
+
+@pytest.mark.parametrize("head_dim", [96, 112, 128])
+@pytest.mark.parametrize("tokens, before", [(64, 6000), (128, 4000), (512, 1500), (512, 7000), (1024, 5000), (2048, 0), (2048, 6000), (4096, 0)])
+def test_the_variant_with_sinks_and_caps_takes_columns_that_fit_its_registers(tokens, before, head_dim):
+    """Through LDS, 32 columns a wave of more than 96 dims spill 85 registers and more in the kernel's variant with a sink, chunks,
+    capped scores or shared planes: it takes 16."""
+    from tlie_amd import ops
+    _, col_tiles, _, _, _, shared = ops.attention_plan(prompt_step(tokens, before), 4, 8, head_dim, extra=True)
+    assert not shared or col_tiles == 1 or head_dim <= 96
+
+
 def test_the_skinny_products_launch_shape_is_one_the_kernel_takes():
     """Decided on the host from the sizes alone: every plan is within what the kernel takes, covers
     the inner size exactly, and for matrices that the policy balances the workgroups are no more

@@ -2177,7 +2177,7 @@ def few_rows_route(rows: int, dtype: torch.dtype) -> bool:
     return dtype == torch.bfloat16 and 0 < rows <= ROWS_MAX
 
 
-def attention_plan(ctx, groups_per_kv: int, num_kv_heads: int, head_dim: int, reach: int | None = None):
+def attention_plan(ctx, groups_per_kv: int, num_kv_heads: int, head_dim: int, reach: int | None = None, extra: bool = False):
     """How the tiled attention kernel is launched for the step `ctx` describes: its work list (made
     once per step and group size, kept in `ctx.scratch`; None for a decode step, whose tiles the
     kernel derives itself), and how the keys are cut: into as many parts as it takes to give a step
@@ -2187,7 +2187,8 @@ def attention_plan(ctx, groups_per_kv: int, num_kv_heads: int, head_dim: int, re
     MI355X; the step's context only supplies the host arrays, the number of compute units, and, in a
     recorded step, the owner of work lists at fixed addresses.  reach: the most keys a token sees, itself
     included (a window, a chunk): the parts of a decode step then share those keys (counted from the
-    block of 32 they begin in), not the whole sequence.
+    block of 32 they begin in), not the whole sequence.  extra: the layer's kernel is the variant that takes a sink, chunks,
+    capped scores or shared planes.
     Returns (tiles, col_tiles, nsplit, split_len, waves, shared): `waves` of a workgroup share a
     tile's keys, or with `shared` take columns of their own and get the keys through LDS."""
     decode = ctx.max_new == 1 and ctx.num_seqs == ctx.num_tokens
@@ -2261,6 +2262,10 @@ def attention_plan(ctx, groups_per_kv: int, num_kv_heads: int, head_dim: int, re
                     col_tiles, parts = 1, 4
                 else:
                     shared = False
+            if shared and extra and head_dim > 96:
+                # the variant with sinks, chunks, caps or shared planes spills 97 registers at 32 columns of 128 dims, 85 of 112,
+                # and takes twice the time of 16 columns there (a sink, 32 heads of 128 on 8, 2048 tokens: 205 us against 96)
+                col_tiles = 1
         tiles = tiles_of(col_tiles * (4 if shared else 1))
         count = tiles.shape[0] * (4 if shared else 1)
     tiles_all = count * num_kv_heads

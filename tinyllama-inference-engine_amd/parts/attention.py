@@ -256,7 +256,8 @@ class Attention(Mixer):
                           q_temp=self.q_temp, head_scale=self.temp, extra_cols=self.gate_cols)
         if self.dv == self.d and ops.attention_mfma_takes(self.dtype, self.d, binding.cache.shape[3] // self.d):
             # bfloat16, one head size: the kernel on the matrix cores (scores, softmax and sink float)
-            tiles, col_tiles, nsplit, split_len, waves, shared = ops.attention_plan(ctx, self.nq // self.nkv, self.nkv, self.d, self.reach)
+            extra = self.chunk is not None or self.sink is not None or self.softcap is not None
+            tiles, col_tiles, nsplit, split_len, waves, shared = ops.attention_plan(ctx, self.nq // self.nkv, self.nkv, self.d, self.reach, extra)
             attended = ops.attention_mfma(q, binding.cache, pages.block_table, tiles, ctx.positions, self.nq, self.nkv, self.d,
                                           self.window, self.scale, nsplit, split_len, col_tiles, waves, shared,
                                           chunk=self.chunk, sink=self.sink, softcap=self.softcap)

@@ -141,7 +141,7 @@ class DifferentialAttention(Mixer):
             # the keys' size are kv heads of that kernel: key head k and piece p make kv head k * parts + p, which reads
             # key plane k and, with its map's partner, the group's value planes
             parts = self.dv // self.d
-            tiles, col_tiles, nsplit, split_len, waves, shared = ops.attention_plan(ctx, self.per_group, key_heads * parts, self.d)
+            tiles, col_tiles, nsplit, split_len, waves, shared = ops.attention_plan(ctx, self.per_group, key_heads * parts, self.d, extra=True)
             attended = ops.attention_mfma(q, binding.cache, pages.block_table, tiles, ctx.positions, heads * parts, key_heads * parts,
                                           self.d, None, self.scale, nsplit, split_len, col_tiles, waves, shared,
                                           planes=(parts, 2 * parts, parts), float_out=True)
