@@ -69,6 +69,31 @@ def test_the_variant_with_sinks_and_caps_takes_columns_that_fit_its_registers(to
     assert not shared or col_tiles == 1 or head_dim <= 96
 
 
+@pytest.mark.parametrize("heads, kv_heads, dim, tokens, before, reach, extra, want", [
+    # A window or chunk longer than the context is none: what the same step takes without it (or, in short contexts, no LDS)
+    (16, 2, 128, 512, 6000, 8192, False, (2, 8, True)), (32, 8, 128, 1024, 5000, 8192, False, (2, 2, True)),
+    (32, 8, 128, 64, 6000, 8192, True, (1, 8, True)), (16, 2, 128, 256, 600, 8192, True, (2, 1, False)),
+    # One within the context bounds what is cut
+    (32, 8, 128, 256, 3000, 1024, False, (2, 1, False)), (32, 8, 128, 64, 6000, 1024, True, (2, 4, False)), (32, 8, 128, 512, 6000, 1024, False, (1, 1, True)),
+    (32, 8, 128, 2048, 6000, 1024, False, (2, 1, True)), (32, 8, 128, 2048, 6000, 1024, True, (1, 1, True)),
+    # Heads of up to 32 dims keep their cut keys
+    (16, 8, 32, 64, 6000, None, False, (1, 8, True)), (16, 8, 32, 256, 3000, None, True, (1, 2, True)), (32, 2, 16, 64, 6000, None, False, (1, 4, True)),
+    # One and a half workgroups a unit of 96 dims are served by 16 columns a wave
+    (24, 8, 96, 2048, 0, None, False, (1, 1, True)), (24, 8, 96, 2048, 0, None, True, (1, 1, True)),
+    # Few tiles of their own keys: not cut
+    (24, 8, 96, 256, 600, None, False, (2, 1, False)), (16, 2, 128, 64, 6000, None, False, (1, 8, True)),
+])
+def test_how_the_prompt_attention_is_cut_for_other_heads_and_reaches(heads, kv_heads, dim, tokens, before, reach, extra, want):
+    """Calls that the lines drawn from 128 and 64 dims alone made up to five times slower: (columns a wave / 16, parts of the
+    keys, through LDS) as measured for them."""
+    from tlie_amd import ops
+    _, col_tiles, nsplit, split_len, _, shared = ops.attention_plan(prompt_step(tokens, before), heads // kv_heads, kv_heads, dim, reach, extra)
+    assert (col_tiles, nsplit, shared) == want
+    if nsplit > 1:
+        seen = before + tokens if reach is None else min(before + tokens, reach + 31 + 128 // (heads // kv_heads) + 1)
+        assert split_len % 32 == 0 and nsplit * split_len >= seen
+
+
 def test_the_skinny_products_launch_shape_is_one_the_kernel_takes():
     """Decided on the host from the sizes alone: every plan is within what the kernel takes, covers
     the inner size exactly, and for matrices that the policy balances the workgroups are no more

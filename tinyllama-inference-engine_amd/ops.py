@@ -2186,20 +2186,23 @@ def attention_plan(ctx, groups_per_kv: int, num_kv_heads: int, head_dim: int, re
     multiple of 32 positions and at least 64.  The policy is this kernel's own and measured on the
     MI355X; the step's context only supplies the host arrays, the number of compute units, and, in a
     recorded step, the owner of work lists at fixed addresses.  reach: the most keys a token sees, itself
-    included (a window, a chunk): the parts of a decode step then share those keys (counted from the
-    block of 32 they begin in), not the whole sequence.  extra: the layer's kernel is the variant that takes a sink, chunks,
-    capped scores or shared planes.
+    included (a window, a chunk): the parts then share those keys (counted from the block of 32 they begin in), not the
+    whole sequence.  extra: the layer's kernel is the variant that takes a sink, chunks, capped scores or shared planes.
     Returns (tiles, col_tiles, nsplit, split_len, waves, shared): `waves` of a workgroup share a
     tile's keys, or with `shared` take columns of their own and get the keys through LDS."""
     decode = ctx.max_new == 1 and ctx.num_seqs == ctx.num_tokens
     col_tiles, shared = 1, False
-    context = ctx.max_context
+    context, bounded = ctx.max_context, False
     if decode:
         if reach is not None:
             context = min(context, int(reach) + 31)
         tiles, count = None, ctx.num_tokens * ((groups_per_kv + 15) // 16)
     else:
         col_tiles = attention_col_tiles(head_dim)
+        if reach is not None:                               # what a tile of up to 128 columns sees
+            context = min(context, int(reach) + 31 + (127 + groups_per_kv) // groups_per_kv)
+            bounded = context < ctx.max_context
+            span, context = context, ctx.max_context
         # sequences of some length with portions of many columns: 4 waves take columns of their own
         # of one tile and every block of keys is brought once for all of them, through LDS (a
         # prompt of 1536 tokens: 34 us against 42; of 8192: 450 against 780; of 512: 15 against 13)
@@ -2218,7 +2221,7 @@ def attention_plan(ctx, groups_per_kv: int, num_kv_heads: int, head_dim: int, re
                 else:
                     ctx.scratch[key] = torch.from_numpy(make(ctx.host)).to(ctx.tokens.device)
             return ctx.scratch[key]
-        parts = 1
+        parts, alone = None, False                          # (None: by the number of tiles, below)
         if shared:
             # How many columns a wave takes (32, or 16) and into how many parts the keys are cut, by the workgroups that 32
             # columns a wave make.  A recorded step counts by its tokens (its list also holds empty tiles), and by an eighth
@@ -2230,42 +2233,54 @@ def attention_plan(ctx, groups_per_kv: int, num_kv_heads: int, head_dim: int, re
             else:
                 tiles_wide = (columns + 127) // 128 + ctx.num_seqs // 8
             blocks, units = tiles_wide * num_kv_heads, ctx.compute_units
+            # the variant with sinks, chunks, caps or shared planes spills 97 registers at 32 columns of 128 dims, 85 of 112,
+            # and takes twice the time of 16 columns there (a sink, 32 heads of 128 on 8, 2048 tokens: 205 us against 96)
+            narrow = extra and head_dim > 96
             if head_dim <= 64:
                 # bound by vector arithmetic: 16 columns a wave, four workgroups a unit, while that is at most five for two
                 # units (2048 tokens, 32 heads on 4: 47 us against 60; 3072: 100 against 98; 4096: 162 against 150).  At
-                # 5 for 8 units or fewer, waves that share a tile's keys without LDS (512 tokens behind 500: 20.5 us
+                # 5 for 8 units or fewer, four waves that share a tile's keys without LDS (512 tokens behind 500: 20.5 us
                 # against 25.2, behind 1500: 32.1 against 41.1; 1024 tokens: 25.3 against 24.8; smaller heads not measured)
                 if 8 * blocks <= 5 * units and head_dim > 32:
-                    shared = False
+                    shared, alone = False, True
                 elif 2 * blocks <= 5 * units:
                     col_tiles = 1
-            elif 2 * blocks < 3 * units or (2 * blocks <= 5 * units and ctx.max_context < 2048):
+            elif 2 * blocks > 5 * units:
+                col_tiles = 1 if narrow else 2
+            elif 4 * blocks > units:
                 # heads of more dims are bound by the LDS: a wave of 32 columns reads a block of keys once where two of 16 read it
-                # twice.  Above five workgroups for two units, and from three on where keys are many, 32 columns it is (32 heads of
-                # 128 on 8, 2048 tokens behind 0: 83 us against 89, behind 2000: 152 against 214, behind 6000: 323 against 460;
-                # 1536 behind 0: 64 against 55, behind 2000: 135 against 168).
-                # Fewer are filled up to two a unit by cutting the keys, where these are many: 1024 tokens behind 5000 171 us in
-                # two parts against 189 with 16 columns (behind 2000 103 against 95); 512 behind 1000 46 in four parts against
-                # 48, behind 1500 51 against 60, behind 7000 115 against 199; 128 behind 4000 39 in eight parts against 46
-                # without LDS.  Up to a quarter of a unit each, 16 columns in four parts up to 3072 positions (128 behind 700
-                # 21 us against 24 without LDS, behind 1500 26 against 29; 256 behind 1500 36 against 36, behind 500 28
-                # against 22).  A window's parts would mostly be empty.
-                whole, context_least = reach is not None, 4096 if 2 * blocks > units else 1536
-                if 4 * blocks > units or whole:
-                    if ctx.max_context >= context_least and not whole:
-                        parts = min(4, (2 * units + blocks - 1) // blocks)
-                    else:
-                        col_tiles = 1
-                elif ctx.max_context >= 3072:
-                    parts = min(8, (2 * units + blocks - 1) // blocks)
-                elif ctx.max_context >= 1536 or 8 * blocks <= units:
+                # twice.  From two workgroups a unit on 32 columns it is (32 heads of 128 on 8, 2048 tokens behind 0: 84 us against
+                # 89, behind 2000: 156 against 218, within a window of 1024: 63 to 70 against 74 to 90; of 80 behind 2000: 125
+                # against 174, but behind 0: 67 against 65), from one and a half where heads and contexts are large (1536 tokens
+                # of 128 behind 2000: 135 against 168, behind 0: 64 against 55; 24 heads of 96 on 8, 2048 behind 0: 70 against
+                # 58, behind 6000: 266 against 262).
+                # Fewer are filled up to two a unit by cutting the keys, where these are many: 1024 tokens of 128 behind 5000
+                # 171 us in two parts against 196 with 16 columns (behind 1000 81 against 64); 512 behind 1500 52 in four parts
+                # against 61, behind 7000 116 against 200, with a sink in four parts of 16 columns 157 against 206.
+                few = blocks <= (3 * units - 1) // 2 and not bounded
+                if blocks >= 2 * units and not narrow and (head_dim > 96 or bounded or ctx.max_context >= 3072):
+                    col_tiles = 2
+                elif 2 * blocks >= 3 * units and head_dim > 96 and not narrow and not bounded and ctx.max_context >= 3072:
+                    col_tiles = 2
+                elif few and not narrow and ctx.max_context >= (4096 if 2 * blocks > units else 1536):
+                    parts = min(4, (2 * units + blocks - 1) // blocks)
+                elif few and 2 * blocks <= units and ctx.max_context >= 4096:
                     col_tiles, parts = 1, 4
                 else:
-                    shared = False
-            if shared and extra and head_dim > 96:
-                # the variant with sinks, chunks, caps or shared planes spills 97 registers at 32 columns of 128 dims, 85 of 112,
-                # and takes twice the time of 16 columns there (a sink, 32 heads of 128 on 8, 2048 tokens: 205 us against 96)
-                col_tiles = 1
+                    col_tiles = 1
+            # Up to a quarter of a unit each.  In a window or chunk four waves that share a tile's keys without LDS (128 tokens
+            # of 128 behind 4000 in a window of 1024: 28 us against 36 with 16 columns through LDS).  Else cut keys: 128 tokens
+            # behind 4000 41 us in eight parts against 66 without LDS and 45 in four; 128 behind 700 21.8 us in four parts of 16
+            # columns against 24 without LDS; 256 behind 1500 38 against 36, behind 600 31 against 24.5.  Up to an eighth of
+            # a unit 16 columns a wave also where keys are many (16 heads of 112 on 4, 128 behind 4000: 29.5 us against 34).
+            elif bounded or (reach is not None and ctx.max_context < 3072):
+                shared, alone = False, True
+            elif ctx.max_context >= 3072:
+                col_tiles, parts = 1 if narrow or 8 * blocks <= units else 2, min(8, (2 * units + blocks - 1) // blocks)
+            elif ctx.max_context >= 1536 or 8 * blocks <= units:
+                col_tiles, parts = 1, 4
+            else:
+                shared, alone = False, True
         tiles = tiles_of(col_tiles * (4 if shared else 1))
         count = tiles.shape[0] * (4 if shared else 1)
     tiles_all = count * num_kv_heads
@@ -2277,8 +2292,13 @@ def attention_plan(ctx, groups_per_kv: int, num_kv_heads: int, head_dim: int, re
         # Up to 4 waves share a tile's keys, each with 128 or more: a tile that sees the whole of
         # a long sequence then takes a quarter of the time, and it is the longest tiles that
         # the step waits for (a prompt of 2048 tokens: 70 us against 87 with one wave a tile)
-        # From 256 tiles on four waves each do (256 tokens, 32 heads of 128 on 8, behind 500: 22 us against 30 in two parts)
-        nsplit = parts if shared else max(1, min((512 + tiles_all - 1) // tiles_all if tiles_all < 256 else 1, 16, ctx.max_context // 256))
+        # From 256 tiles on four waves each do (256 tokens, 32 heads of 128 on 8, behind 500: 22 us against 30 in two parts), and
+        # from 128 on for steps that could share keys through LDS (24 heads of 96 on 8, 256 behind 600: 19 us against 29 in three).
+        # Through LDS from 384 waves on (16 heads of 32 on 8, 256 behind 3000, 256 waves: 35 us in two parts against 55)
+        if bounded and (shared or alone):
+            context = span
+        full = 128 if alone else (384 if shared else 256)
+        nsplit = parts or max(1, min((512 + tiles_all - 1) // tiles_all if tiles_all < full else 1, 16, context // 256))
         waves = 4 if shared else 1
         while (not shared and waves < 4 and waves * 2 <= attention_max_waves(head_dim, col_tiles)
                and ctx.max_context >= nsplit * waves * 2 * 128):
