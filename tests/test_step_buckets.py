@@ -94,6 +94,16 @@ def test_how_the_prompt_attention_is_cut_for_other_heads_and_reaches(heads, kv_h
         assert split_len % 32 == 0 and nsplit * split_len >= seen
 
 
+@pytest.mark.parametrize("batch, kv_heads, dim, context, parts", [
+    (1, 8, 128, 8100, 29), (1, 8, 128, 16000, 32), (1, 8, 128, 5000, 16), (1, 4, 64, 5000, 16), (3, 4, 64, 16000, 16), (1, 4, 64, 16000, 32),
+    (1, 8, 32, 16000, 16), (1, 8, 96, 8100, 29), (4, 2, 256, 8100, 29), (8, 2, 128, 16000, 16), (8, 4, 64, 2000, 8)])
+def test_into_how_many_parts_a_decode_step_cuts_its_keys(batch, kv_heads, dim, context, parts):
+    """More than 16 only for few tiles of many keys of large heads (elsewhere the merge takes longer than the parts give)."""
+    from tlie_amd import ops
+    _, _, nsplit, split_len, _, _ = ops.attention_plan(prompt_step(1, context - 1, batch), 4, kv_heads, dim)
+    assert nsplit == parts and split_len % 32 == 0 and nsplit * split_len >= context
+
+
 def test_the_skinny_products_launch_shape_is_one_the_kernel_takes():
     """Decided on the host from the sizes alone: every plan is within what the kernel takes, covers
     the inner size exactly, and for matrices that the policy balances the workgroups are no more

@@ -2308,9 +2308,11 @@ def attention_plan(ctx, groups_per_kv: int, num_kv_heads: int, head_dim: int, re
         # meet in the merge kernel); then the waves of a workgroup share them, which costs no
         # launch, while a wave keeps 128 keys or more and the step has 2048 waves at most
         # (measured inside whole steps at 2048 positions: batch 1 16 parts x 1 wave, batch 8
-        # 8 x 2, batch 64 1 x 8).  More than 16 parts only of 256 keys or more (8000 positions, 8 key heads of 128, batch 1,
-        # with the merge: 17.4 us in 32 parts against 19.4 in 16)
-        nsplit = max(1, min((256 + tiles_all - 1) // tiles_all, max(16, min(32, context // 256)), (context + 63) // 64))
+        # 8 x 2, batch 64 1 x 8).  More than 16 parts, of 256 keys or more, for up to 8 tiles from 8000 positions of 96 dims (16000
+        # of 48) on (batch 1, 8 key heads of 128, with the merge, in 16 parts and in up to 32: 8100 positions 18.7 us and 17.6,
+        # 5000 14.9 and 15.4; of 64 on 4: 16000 14.6 and 13.8, 5000 10.1 and 11.2, 12 tiles of 16000 18.0 and 19.7)
+        most = min(32, context // 256) if tiles_all <= 8 and context >= 8000 and context * head_dim >= 768000 else 16
+        nsplit = max(1, min((256 + tiles_all - 1) // tiles_all, most, (context + 63) // 64))
         waves = 1
         while (waves * 2 <= attention_max_waves(head_dim) and tiles_all * nsplit * waves * 2 <= 2048
                and context >= nsplit * waves * 2 * 128):
