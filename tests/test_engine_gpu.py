@@ -587,6 +587,42 @@ def test_benchmark_layer_sizes_cut_three_ways(tmp_path, dtype):
         assert bad is None, f"recorded portions of {request}: position {places[bad]} is wrong"
 
 
+def test_decode_steps_list_their_sequences_longest_first(tmp_path):
+    """33 sequences of 3 to 300 positions on 16 key heads: more workgroups in the attention than compute units, which then goes by
+    the list; replays of one recording while lengths grow and sequences end, so that padding takes their rows."""
+    from tlie_amd import Engine, StepEntry
+    raw = dict(BENCH_SHAPE, hidden_size=256, intermediate_size=512, num_attention_heads=16, num_key_value_heads=16, vocab_size=300,
+               max_position_embeddings=512)
+    folder = make_model(tmp_path / "model", raw, seed=9, dtype_name="bfloat16", std=0.03)
+    stored, weights = load_plain(folder)
+    rng = random.Random(4)
+    lengths = [300] + [rng.randint(3, 299) for _ in range(32)]
+    texts = [random_tokens(600 + i, length, 300) for i, length in enumerate(lengths)]
+    engine = Engine(folder, dtype="bfloat16", max_tokens=33 * 320, page_size=16, max_requests=33)
+    replay, live = Replayer(engine), list(range(33))
+    for first in range(0, 33, 11):
+        replay.step([(i, texts[i][:-3], []) for i in range(first, first + 11) if lengths[i] > 3])
+    for turn in range(3):
+        replay.step([(i, [texts[i][turn - 3]], [0]) for i in live], end=live[1::4])
+        live = [i for i in live if i not in live[1::4]]
+        graph = engine.runner._graphs[(64 if turn == 0 else 32, 512)]
+        order, held = graph.ctx.seq_order.cpu().long(), graph.ctx.seq_len.cpu()
+        assert torch.equal(order.sort().values, torch.arange(len(held))) and (held[order].diff() <= 0).all()
+    for i in range(0, 33, 4):
+        places = sorted(place for name, place in replay.rows if name == i)
+        bad = first_bad_row(replay.logits_of(i, places), plain_forward(stored, weights, texts[i])[places], TOLERANCE["bfloat16"])
+        assert bad is None, f"position {places[bad]} of sequence {i} is wrong"
+    # launched steps bring the list too, where it has a reader
+    for i in live:
+        engine.cache.reserve(i, 1)
+    for count, listed in ((9, True), (8, False)):
+        ctx = engine.runner.build_context([StepEntry(i, [1], [0]) for i in live[:count]])
+        assert live[0] == 0 and (ctx.seq_order is not None) == listed
+        if listed:
+            held = ctx.seq_len.cpu()[ctx.seq_order.cpu().long()]
+            assert held[0] == 301 and (held.diff() <= 0).all()
+
+
 # The layer sizes of the two larger shapes that bench.py offers (width 4096, head size 128; one with
 # as many key heads as query heads and a feed-forward of 11008, one with 4 query heads a key head, a
 # feed-forward of 14336 and rope_theta 500000), one layer each and a small vocabulary: other

@@ -804,6 +804,40 @@ def test_a_decode_step_of_more_workgroups_than_compute_units_serves_every_sequen
         assert torch.equal(launch(slice(i, i + 1))[0], together[i]), (i, lens[i])
 
 
+@pytest.mark.parametrize("count, nq, nkv, d, nsplit, waves, ordered", [
+    (33, 32, 8, 64, 1, 2, True), (64, 60, 3, 64, 1, 4, True), (40, 80, 4, 64, 1, 2, True), (64, 32, 8, 128, 1, 4, True), (9, 40, 40, 32, 1, 2, True),
+    (40, 24, 8, 64, 2, 1, True), (65, 16, 8, 64, 1, 2, True), (64, 40, 2, 64, 1, 4, False), (33, 14, 7, 64, 1, 2, False)])
+def test_a_decode_step_serves_its_sequences_in_any_order(count, nq, nkv, d, nsplit, waves, ordered):
+    """The list of sequences, longest first, backwards and shuffled: the bits of the step without it, and of each sequence alone.
+    Grouped heads, two tiles a sequence (more than 16 heads a group), rounds that are no multiple of the sequences.  ordered:
+    whether the step has more workgroups than the device has compute units, which are the ones that look at the list."""
+    from tlie_amd import ops
+    assert ordered == (count * -(-nq // nkv // 16) * nkv > torch.cuda.get_device_properties(0).multi_processor_count)
+    page, longest, rng = 16, 300, random.Random(count)
+    lens = [rng.choice((1, 17, longest, rng.randint(1, longest))) for _ in range(count)]
+    blocks = longest // page + 1
+    torch.manual_seed(count)
+    table = torch.randperm(count * blocks).view(count, blocks).int().to(DEV)
+    cache = torch.randn(count * blocks, 2, nkv, page * d).bfloat16().to(DEV)
+    q = torch.randn(count, nq * d).bfloat16().to(DEV)
+    positions = torch.tensor([n - 1 for n in lens], dtype=torch.int32, device=DEV)
+    split_len = (longest // nsplit + 31) // 32 * 32
+
+    def launch(rows, order=None):
+        order = None if order is None else torch.tensor(order, dtype=torch.int32, device=DEV)
+        return ops.attention_mfma(q[rows].contiguous(), cache, table[rows].contiguous(), None, positions[rows].contiguous(), nq, nkv, d, None,
+                                  1.0 / math.sqrt(d), nsplit, split_len, 1, waves, order=order)
+    every = slice(0, count)
+    plain = launch(every)
+    longest_first = sorted(range(count), key=lambda i: -lens[i])
+    for order in (longest_first, longest_first[::-1], rng.sample(range(count), count)):
+        assert torch.equal(launch(every, order), plain)
+    for i in range(0, count, 5):
+        assert torch.equal(launch(slice(i, i + 1))[0], plain[i]), (i, lens[i])
+    with pytest.raises(Exception):
+        launch(every, longest_first[:-1])
+
+
 def test_attention_mfma_finds_one_key_among_hundreds():
     tokens, nq, nkv, d, page = 600, 4, 2, 32, 16
     torch.manual_seed(1)

@@ -106,7 +106,8 @@ attention_mfma_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict
                       const int* __restrict__ block_table, int max_blocks, const int4* __restrict__ tiles,
                       const int* __restrict__ positions, uint16_t* __restrict__ out, float* __restrict__ part_o,
                       float* __restrict__ part_ml, int nsplit, int split_len, int nq, int nkv, int page_size,
-                      int window, int chunk, const float* __restrict__ sink, float scale_log2, int round_size, int plane_map, float cap_pre) {
+                      int window, int chunk, const float* __restrict__ sink, float scale_log2, int round_size, int plane_map, float cap_pre,
+                      const int* __restrict__ order) {
   constexpr int D = DT * 16;
   // the first key that the token at position p sees: the window's edge, or the start of the token's own
   // chunk of positions (chunks are counted from position 0), whichever is later; 0 without either
@@ -144,25 +145,20 @@ attention_mfma_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict
     if (ntok <= 0) return;                       // a list of fixed size ends in tiles without tokens (the same for the whole workgroup)
   } else {
     const int per_seq = (G + 16 * CT - 1) / (16 * CT), per_token = per_seq * static_cast<int>(gridDim.y);
-    const int tokens = static_cast<int>(gridDim.x) / per_seq, total = tokens * per_token;
+    const int total = static_cast<int>(gridDim.x * gridDim.y);
     seq = blockIdx.x / per_seq, col0 = blockIdx.x % per_seq;
-    if (!SHARED && total > round_size && round_size > 0 && tokens <= 64) {
+    if (!SHARED && order != nullptr && total > round_size && round_size > 0) {
       // A decode step of more workgroups than compute units, and of sequences of their own lengths: the workgroups of one
       // unit lie a round apart, and where a round is a multiple of the tokens they would all be the same sequence's, so that
-      // the kernel took as long as the longest sequence on every place (24 sequences of 129 to 1060 positions of 32, 32 heads of
-      // 128: 66 us, in this order 55; 64 of 129 to 1500, 32 heads of 128 on 8: 56, 48).  The sequences are taken longest first, and the rounds forwards
-      // and backwards in turn like a prompt's tiles.  Every wave ranks the sequences itself, a sequence a lane.
-      const int lane_pos = positions[min(lane, tokens - 1)];
-      int rank = 0;
-      for (int j = 0; j < tokens; ++j) {
-        const int other = __builtin_amdgcn_readlane(lane_pos, j);
-        rank += other > lane_pos || (other == lane_pos && j < lane);
-      }
+      // the kernel took as long as the longest sequence on every place (64 sequences of 50 to 1500 positions, 32 heads of 128 on
+      // 8: 51.5 us, in this order 43.5; 16 of them on 32 key heads 53.2, 41.5; of equal lengths the list costs 0.3 us).  The sequences are taken longest first, as `order` lists
+      // them, and the rounds forwards and backwards in turn like a prompt's tiles.  (Ranked by every wave from the positions
+      // instead, the keys wait for that: 64 sequences of 60 positions, 32 heads of 128 on 8, 10.1 us against 7.1.)
       const int linear = blockIdx.y * gridDim.x + blockIdx.x, round = linear / round_size, place = linear - round * round_size;
       const int in_round = min(round_size, total - round * round_size);
       const int item = round * round_size + ((round & 1) ? in_round - 1 - place : place);
       const int wanted = item / per_token, rest = item - wanted * per_token;
-      seq = __ffsll(__ballot(lane < tokens && rank == wanted)) - 1;
+      seq = order[wanted];
       kvh = rest / per_seq, col0 = rest - kvh * per_seq;
     }
     tok0 = seq, ntok = 1, col0 *= 16 * CT;
@@ -742,7 +738,7 @@ template <int DT, int CT, bool SHARED = false>
 static int launch_attention(const void* q, const void* cache, const int* block_table, int max_blocks, const void* tiles,
                             int num_tiles, const int* positions, void* out, float* part_o, float* part_ml, int nsplit,
                             int split_len, int nq, int nkv, int page_size, int window, int chunk, const float* sink, float scale,
-                            int waves, hipStream_t stream, int plane_map, float softcap) {
+                            int waves, hipStream_t stream, int plane_map, float softcap, const int* order) {
   // (capped scores: the kernel forms tanh(score * scale / cap), and the cap takes the scale's place in the exponent)
   const float scale_log2 = (softcap > 0.f ? softcap : scale) * 1.4426950408889634f;
   const float cap_pre = softcap > 0.f ? scale / softcap : 0.f;
@@ -752,11 +748,11 @@ static int launch_attention(const void* q, const void* cache, const int* block_t
   if (chunk > 0 || sink != nullptr || plane_map != 0 || softcap > 0.f)
     hipLaunchKernelGGL((attention_mfma_kernel<DT, CT, SHARED, true>), dim3(num_tiles, nkv, nsplit), dim3(64 * waves), lds, stream, (const uint16_t*)q,
                        (const uint16_t*)cache, block_table, max_blocks, (const int4*)tiles, positions, (uint16_t*)out, part_o,
-                       part_ml, nsplit, split_len, nq, nkv, page_size, window, chunk, sink, scale_log2, compute_units(), plane_map, cap_pre);
+                       part_ml, nsplit, split_len, nq, nkv, page_size, window, chunk, sink, scale_log2, compute_units(), plane_map, cap_pre, order);
   else
     hipLaunchKernelGGL((attention_mfma_kernel<DT, CT, SHARED, false>), dim3(num_tiles, nkv, nsplit), dim3(64 * waves), lds, stream, (const uint16_t*)q,
                        (const uint16_t*)cache, block_table, max_blocks, (const int4*)tiles, positions, (uint16_t*)out, part_o,
-                       part_ml, nsplit, split_len, nq, nkv, page_size, window, 0, nullptr, scale_log2, compute_units(), 0, 0.f);
+                       part_ml, nsplit, split_len, nq, nkv, page_size, window, 0, nullptr, scale_log2, compute_units(), 0, 0.f, order);
   return launch_status();
 }
 
@@ -775,11 +771,13 @@ using namespace tlie;
 // takes 16 * col_tiles of them, and keys and values reach the waves through LDS.  Otherwise:
 // waves: 1, 2, 4 or 8 waves of a workgroup share a tile's keys; waves * col_tiles * d <= 1024 (their merge's LDS), and
 // at most 4 when col_tiles * d > 128.
+// order (or null; only looked at without tiles): the step's sequences 0 .. tokens - 1 in the order in which their workgroups
+// start, best the longest first.  It changes no result.
 static int attention_entry(const void* q, const void* cache, const int* block_table, int max_blocks,
                            const void* tiles, int num_tiles, int col_tiles, const int* positions, void* out,
                            float* part_o, float* part_ml, int nsplit, int split_len, int tokens, int nq, int nkv,
                            int d, int page_size, int window, int chunk, const float* sink, float scale, int waves, int shared,
-                           void* stream, int plane_map = 0, float softcap = 0.f) {
+                           const int* order, void* stream, int plane_map = 0, float softcap = 0.f) {
   if (chunk < 0 || softcap < 0.f) return kBadArgument;
   if (plane_map != 0) {
     const int kdiv = plane_map & 255, vgroup = (plane_map >> 8) & 255, vmod = (plane_map >> 16) & 255;
@@ -802,7 +800,7 @@ static int attention_entry(const void* q, const void* cache, const int* block_ta
   hipStream_t s = (hipStream_t)stream;
   int status = kBadArgument;
 #define TLIE_ARGS q, cache, block_table, max_blocks, tiles, num_tiles, positions, out, part_o, part_ml, nsplit, split_len, nq, \
-                  nkv, page_size, window, chunk, sink, scale, waves, s, plane_map, softcap
+                  nkv, page_size, window, chunk, sink, scale, waves, s, plane_map, softcap, order
 #define TLIE_CASE(DT)                                        \
   case DT:                                                   \
     status = launch_attention<DT, 1>(TLIE_ARGS);             \
@@ -851,11 +849,11 @@ extern "C" int tlie_attention_mfma(const void* q, const void* cache, const int* 
                                    const void* tiles, int num_tiles, int col_tiles, const int* positions, void* out,
                                    float* part_o, float* part_ml, int nsplit, int split_len, int tokens, int nq, int nkv,
                                    int d, int page_size, int window, int chunk, const float* sink, float scale, int waves,
-                                   int shared, void* stream) {
+                                   int shared, const int* order, void* stream) {
   // chunk > 0: a token sees only the keys of its own chunk of so many positions (counted from position 0);
   // sink (or null): float [nq], a number per head whose exponential joins the softmax's denominator
   return attention_entry(q, cache, block_table, max_blocks, tiles, num_tiles, col_tiles, positions, out, part_o, part_ml, nsplit,
-                         split_len, tokens, nq, nkv, d, page_size, window, chunk, sink, scale, waves, shared, stream);
+                         split_len, tokens, nq, nkv, d, page_size, window, chunk, sink, scale, waves, shared, order, stream);
 }
 
 // The same with capped scores: softcap > 0, a scaled score s enters the softmax as softcap * tanh(s / softcap).
@@ -863,9 +861,9 @@ extern "C" int tlie_attention_mfma_capped(const void* q, const void* cache, cons
                                           const void* tiles, int num_tiles, int col_tiles, const int* positions, void* out,
                                           float* part_o, float* part_ml, int nsplit, int split_len, int tokens, int nq, int nkv,
                                           int d, int page_size, int window, int chunk, const float* sink, float scale, int waves,
-                                          int shared, float softcap, void* stream) {
+                                          int shared, float softcap, const int* order, void* stream) {
   return attention_entry(q, cache, block_table, max_blocks, tiles, num_tiles, col_tiles, positions, out, part_o, part_ml, nsplit,
-                         split_len, tokens, nq, nkv, d, page_size, window, chunk, sink, scale, waves, shared, stream, 0, softcap);
+                         split_len, tokens, nq, nkv, d, page_size, window, chunk, sink, scale, waves, shared, order, stream, 0, softcap);
 }
 
 // The same with planes of a page that several kv heads share (see the kernel's plane_map): key_share kv heads in a row
@@ -876,12 +874,12 @@ extern "C" int tlie_attention_mfma_planes(const void* q, const void* cache, cons
                                           float* part_o, float* part_ml, int nsplit, int split_len, int tokens, int nq, int nkv,
                                           int d, int page_size, int window, int chunk, const float* sink, float scale, int waves,
                                           int shared, int key_share, int value_group, int value_planes, int float_out,
-                                          void* stream) {
+                                          const int* order, void* stream) {
   if (key_share <= 0 || key_share > 255 || value_group <= 0 || value_group > 255 || value_planes <= 0 || value_planes > 255)
     return kBadArgument;
   const int plane_map = key_share | (value_group << 8) | (value_planes << 16) | ((float_out ? 1 : 0) << 24);
   return attention_entry(q, cache, block_table, max_blocks, tiles, num_tiles, col_tiles, positions, out, part_o, part_ml, nsplit,
-                         split_len, tokens, nq, nkv, d, page_size, window, chunk, sink, scale, waves, shared, stream, plane_map);
+                         split_len, tokens, nq, nkv, d, page_size, window, chunk, sink, scale, waves, shared, order, stream, plane_map);
 }
 
 // ---- the same attention for callers that cannot allocate (declared and described in no_alloc.h) ----------
@@ -925,5 +923,5 @@ extern "C" int tlie_attention_mfma_no_alloc(const void* q, const void* cache, co
     part_ml = reinterpret_cast<float*>(base + o_bytes);
   }
   return attention_entry(q, cache, block_table, max_blocks, tiles, num_tiles, col_tiles, positions, out, part_o, part_ml, nsplit,
-                         split_len, tokens, nq, nkv, d, page_size, window, 0, nullptr, scale, waves, shared, stream);
+                         split_len, tokens, nq, nkv, d, page_size, window, 0, nullptr, scale, waves, shared, nullptr, stream);
 }

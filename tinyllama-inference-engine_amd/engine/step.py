@@ -85,6 +85,8 @@ class StepContext:
     host: dict                     # the same arrays as numpy, by name
     wants_all_rows: bool = False   # the wanted rows are all the step's tokens, in order
     compute_units: int = 256       # of the device: how many workgroups start at once
+    # int32 [S], a step of single tokens (see `orders_sequences`): its sequences, longest first; None: any order will do
+    seq_order: torch.Tensor | None = None
     # a recorded step of prompt portions: work lists that parts make on the host live at fixed
     # addresses, at a fixed size (the recording's owner keeps them: `tiles_for(key, list) -> tensor`,
     # and makes them again for every replay); None: a list per step
@@ -253,6 +255,14 @@ class ModelRunner:
         return logits
 
 
+def orders_sequences(seqs: int, longest: int) -> bool:
+    """Whether a step of single tokens lists its sequences by length (4 us of the host).  Up to 8 sequences the attention of up to 32
+    key heads has no more workgroups than the device has compute units, and the list would have no reader; within 256 positions it
+    costs the kernel as much as it gives (64 sequences of 4 to 100, 32 heads of 128 on 8: 9.3 us and 9.2; of 14 to 400 20.6 and 17.7);
+    beyond 64 sequences it was not measured."""
+    return 8 < seqs <= 64 and longest > 256
+
+
 class DecodeGraph:
     """A decode step for up to `bucket` sequences, one token each, every token's logits wanted:
     the step's arrays live at fixed addresses, the model's kernels are recorded once into a HIP
@@ -287,6 +297,8 @@ class DecodeGraph:
         layout = [("tokens", (bucket,)), ("positions", (bucket,)), ("token_seq", (bucket,)), ("no_slots", (bucket,)),
                   ("seq_start", (seqs + 1,)), ("seq_first_pos", (seqs,)), ("seq_len", (seqs,)), ("seq_slot", (seqs,)),
                   ("token_slot", (bucket,)), ("want_rows", (seqs,)), ("token_source", (bucket,))]
+        if single and orders_sequences(seqs, longest):
+            layout.append(("seq_order", (seqs,)))
         for group, width in enumerate(self.widths):
             layout += [(f"block_table{group}", (seqs, width)), (f"slot_map{group}", (bucket,))]
         total = sum(int(np.prod(shape)) for _, shape in layout)
@@ -318,7 +330,7 @@ class DecodeGraph:
             seq_start=views["seq_start"], seq_first_pos=views["seq_first_pos"], seq_len=views["seq_len"],
             seq_slot=views["seq_slot"], token_slot=views["token_slot"], want_rows=views["want_rows"], groups=groups,
             host=self.host, wants_all_rows=single,
-            compute_units=_compute_units(runner.device), tile_owner=None if single else self)
+            compute_units=_compute_units(runner.device), tile_owner=None if single else self, seq_order=views.get("seq_order"))
         self.graph = None
         self.logits = None
         self._rows_filled = bucket                           # rows that may hold a step's values
@@ -359,6 +371,8 @@ class DecodeGraph:
         host["positions"][:count] = positions
         host["seq_first_pos"][:count] = positions
         host["seq_len"][:count] = [position + 1 for position in positions]
+        if "seq_order" in host:
+            host["seq_order"][:] = np.argsort(-host["seq_len"], kind="stable")
         host["seq_slot"][:count] = [info.slot for info in held]
         host["token_slot"][:count] = host["seq_slot"][:count]
         for group in range(len(cache.groups)):
@@ -535,6 +549,8 @@ def build_context(cache: CacheManager, entries: Sequence[StepEntry], device) -> 
         "want_rows": want_rows,
     }
     host["token_slot"] = np.repeat(host["seq_slot"], counts)
+    if total == seqs and orders_sequences(seqs, int(host["seq_len"].max())):
+        host["seq_order"] = np.argsort(-host["seq_len"], kind="stable").astype(np.int32)
     group_shapes = []
     for group in range(len(cache.groups)):
         lists = [cache.page_list(entry.request, group) for entry in entries]
@@ -565,5 +581,5 @@ def build_context(cache: CacheManager, entries: Sequence[StepEntry], device) -> 
         seq_first_pos=views["seq_first_pos"], seq_len=views["seq_len"], seq_slot=views["seq_slot"],
         token_slot=views["token_slot"], want_rows=views["want_rows"], groups=groups, host=host,
         wants_all_rows=bool(want_rows.size == total and np.array_equal(want_rows, np.arange(total))),
-        compute_units=_compute_units(device))
+        compute_units=_compute_units(device), seq_order=views.get("seq_order"))
 

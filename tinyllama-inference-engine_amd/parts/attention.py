@@ -260,7 +260,7 @@ class Attention(Mixer):
             tiles, col_tiles, nsplit, split_len, waves, shared = ops.attention_plan(ctx, self.nq // self.nkv, self.nkv, self.d, self.reach, extra)
             attended = ops.attention_mfma(q, binding.cache, pages.block_table, tiles, ctx.positions, self.nq, self.nkv, self.d,
                                           self.window, self.scale, nsplit, split_len, col_tiles, waves, shared,
-                                          chunk=self.chunk, sink=self.sink, softcap=self.softcap)
+                                          chunk=self.chunk, sink=self.sink, softcap=self.softcap, order=ctx.seq_order)
         else:
             attended = ops.attention_generic(q, binding.cache, pages.block_table, ctx.token_seq, ctx.positions, self.nq, self.nkv,
                                              self.d, self.window, self.scale, tiled=ops.attention_generic_plan(ctx, self.nq, self.nkv, self.d, self.dv),
@@ -296,7 +296,7 @@ class Attention(Mixer):
         if ops.attention_mfma_takes(self.dtype, self.d, page_size):
             tiles, col_tiles, nsplit, split_len, waves, shared = ops.attention_plan(ctx, self.nq // self.nkv, self.nkv, self.d, self.reach)
             attended = ops.attention_mfma(q, binding.cache, pages.block_table, tiles, ctx.positions, self.nq, self.nkv,
-                                          self.d, self.window, self.scale, nsplit, split_len, col_tiles, waves, shared)
+                                          self.d, self.window, self.scale, nsplit, split_len, col_tiles, waves, shared, order=ctx.seq_order)
         else:
             attended = ops.attention_generic(q, binding.cache, pages.block_table, ctx.token_seq, ctx.positions, self.nq,
                                              self.nkv, self.d, self.window, self.scale,

@@ -144,7 +144,7 @@ class DifferentialAttention(Mixer):
             tiles, col_tiles, nsplit, split_len, waves, shared = ops.attention_plan(ctx, self.per_group, key_heads * parts, self.d, extra=True)
             attended = ops.attention_mfma(q, binding.cache, pages.block_table, tiles, ctx.positions, heads * parts, key_heads * parts,
                                           self.d, None, self.scale, nsplit, split_len, col_tiles, waves, shared,
-                                          planes=(parts, 2 * parts, parts), float_out=True)
+                                          planes=(parts, 2 * parts, parts), float_out=True, order=ctx.seq_order)
         else:
             attended = ops.attention_generic(q, binding.cache, pages.block_table, ctx.token_seq, ctx.positions, heads, key_heads,
                                              self.d, None, self.scale, tiled=ops.attention_generic_plan(ctx, heads, key_heads, self.d, self.dv),

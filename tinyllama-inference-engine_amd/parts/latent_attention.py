@@ -155,7 +155,7 @@ class LatentAttention(Mixer):
         if self.dv == self.plain and ops.attention_mfma_takes(self.dtype, self.plain, binding.cache.shape[3] // self.plain):
             tiles, col_tiles, nsplit, split_len, waves, shared = ops.attention_plan(ctx, 1, self.heads, self.plain, self.window, self.sink is not None)
             attended = ops.attention_mfma(q, binding.cache, pages.block_table, tiles, ctx.positions, self.heads, self.heads, self.plain,
-                                          self.window, self.scale, nsplit, split_len, col_tiles, waves, shared, sink=self.sink)
+                                          self.window, self.scale, nsplit, split_len, col_tiles, waves, shared, sink=self.sink, order=ctx.seq_order)
         else:
             attended = ops.attention_generic(q, binding.cache, pages.block_table, ctx.token_seq, ctx.positions, self.heads, self.heads,
                                              self.plain, self.window, self.scale, tiled=ops.attention_generic_plan(ctx, self.heads, self.heads, self.plain, self.dv),
@@ -181,7 +181,7 @@ class LatentAttention(Mixer):
         if self.wide_values and ops.attention_mfma_takes(self.dtype, key, binding.cache.shape[-1] // key):
             tiles, col_tiles, nsplit, split_len, waves, shared = ops.attention_plan(ctx, self.heads, 1, key, self.window, self.sink is not None)
             attended = ops.attention_mfma(q_wide, binding.cache, pages.block_table, tiles, ctx.positions, self.heads, 1, key,
-                                          self.window, self.scale, nsplit, split_len, col_tiles, waves, shared, sink=self.sink)
+                                          self.window, self.scale, nsplit, split_len, col_tiles, waves, shared, sink=self.sink, order=ctx.seq_order)
         else:
             attended = ops.attention_generic(q_wide, binding.cache, pages.block_table, ctx.token_seq, ctx.positions, self.heads, 1,
                                              key, self.window, self.scale, tiled=ops.attention_generic_plan(ctx, self.heads, 1, key, value_dim),
