@@ -104,6 +104,19 @@ def test_into_how_many_parts_a_decode_step_cuts_its_keys(batch, kv_heads, dim, c
     assert nsplit == parts and split_len % 32 == 0 and nsplit * split_len >= context
 
 
+@pytest.mark.parametrize("rows, outputs, inputs, gated, want", [
+    (24, 22016, 4096, True, True), (16, 22016, 4096, True, True), (16, 11264, 2048, True, False), (17, 2048, 128, True, True), (64, 8192, 128, True, True),
+    (64, 8193, 256, True, False), (32, 32768, 512, True, True), (32, 32769, 512, True, False), (64, 50000, 1024, False, False),
+    (64, 50000, 1536, False, True), (4, 131072, 1024, False, False), (4, 32000, 2048, False, True), (64, 2048, 2048, False, False),
+    (64, 1 << 10, (1 << 24) + 8, False, False)])
+def test_which_products_keep_their_weights_in_a_ring(rows, outputs, inputs, gated, want):
+    from tlie_amd import ops
+    assert ops.ring_fits(rows, outputs, inputs, gated) is want
+    if want:
+        split_len, strips = ops.ring_plan(rows, outputs, inputs, 256, not gated)
+        assert split_len % 64 == 0 and 1 <= strips <= 8 and (rows <= 48 or strips != 7) and (split_len >= inputs or not gated)
+
+
 def test_the_skinny_products_launch_shape_is_one_the_kernel_takes():
     """Decided on the host from the sizes alone: every plan is within what the kernel takes, covers
     the inner size exactly, and for matrices that the policy balances the workgroups are no more

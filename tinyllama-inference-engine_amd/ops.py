@@ -2091,13 +2091,22 @@ def gemm_skinny(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None
     return Product(out, nsplit)
 
 
-def gemm_ring_takes(x: torch.Tensor, weight: torch.Tensor, gated: bool = False) -> bool:
+def ring_fits(rows: int, out_features: int, in_features: int, gated: bool, compute_units: int = 256) -> bool:
     """Matrices of 32 MB or more for more than 16 rows (us, skinny against ring: 4096 x 4096 at 24 rows 10.3, 9.3; 2048 x 5632,
     2560 x 2048 and 2048 x 2048 at 64 rows 10.5, 11.6; 6.9, 7.5; 5.7, 6.2, where the ring leaves half as many parts and whole
     decode steps take the same), and above 64 MB for fewer (32000 x 2048 at 4 rows 30.9, 28.0; 9216 x 2048 10.5, 10.9).  The
-    gated product of more than 16 rows goes there at any size: it is not split, and deep loads are all that fills a unit."""
-    size = weight.shape[0] * weight.shape[1] * 2
-    return gemm_skinny_takes(x, weight) and weight.shape[1] <= 1 << 24 and ((x.shape[0] > 16 and (gated or size >= 32 << 20)) or size > 64 << 20)
+    gated product of more than 16 rows goes there at any size: it is not split, and deep loads are all that fills a unit.
+    A workgroup's first loads are a wait that its turns must outweigh, once a round: inner sizes below 1536 only where 128 outputs a unit
+    make one round (50000 x 768 at 64 rows 25.2, 30.6, gated 32 rows 20.0, 22.4; 131072 x 1024 at 64 rows 65.8, 75.5; 32768 x
+    1024 17.6, 15.1), below 512 only where 32 outputs a unit do (gated, 32768 x 256 at 32 rows 6.7, 8.2; 8192 x 128 4.0, 3.5)."""
+    size = out_features * in_features * 2
+    if in_features > 1 << 24 or not ((rows > 16 and (gated or size >= 32 << 20)) or size > 64 << 20):
+        return False
+    return in_features >= 1536 or out_features <= (128 if in_features >= 512 else 32) * compute_units
+
+
+def gemm_ring_takes(x: torch.Tensor, weight: torch.Tensor, gated: bool = False) -> bool:
+    return gemm_skinny_takes(x, weight) and ring_fits(x.shape[0], weight.shape[0], weight.shape[1], gated, _compute_units(x.device))
 
 
 def gemm_ring(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, gated: bool = False, gate=None, whole: bool = False,
