@@ -501,7 +501,10 @@ def test_kernels_refuse_what_they_do_not_take():
 
 # ---- the bfloat16 kernels on the matrix cores ---------------------------------------------------------
 
-@pytest.mark.parametrize("tokens, nq, nkv, d, page", [(256, 4, 2, 64, 16), (257, 3, 3, 24, 8), (400, 2, 1, 128, 64), (330, 4, 4, 40, 16), (300, 2, 2, 32, 4)])
+@pytest.mark.parametrize("tokens, nq, nkv, d, page", [(256, 4, 2, 64, 16), (257, 3, 3, 24, 8), (400, 2, 1, 128, 64), (330, 4, 4, 40, 16), (300, 2, 2, 32, 4),
+                                                      # (tiles want 2^18 values, 256 columns and 256 threads' worth of heads, those above have fewer)
+                                                      (256, 8, 8, 128, 16), (257, 10, 8, 128, 8), (400, 12, 6, 128, 64), (331, 50, 20, 40, 16),
+                                                      (730, 24, 5, 72, 16), (1030, 32, 4, 64, 32), (600, 8, 8, 128, 4)])
 @pytest.mark.parametrize("dtypes", [("float32", "float32"), ("float32", "bfloat16"), ("bfloat16", "bfloat16")])
 def test_values_placed_by_tiles_lie_where_single_tokens_put_them(dtypes, tokens, nq, nkv, d, page):
     """Runs of slots that begin and end within a page, tokens without a slot, single slots out of order, tiles with fewer tokens
@@ -517,7 +520,7 @@ def test_values_placed_by_tiles_lie_where_single_tokens_put_them(dtypes, tokens,
         slots += [int(order[p // page]) * page + p % page for p in range(place, place + run)] + [-1]
         place += run + random.Random(run + place).choice((0, 1, 3))
     slots = torch.tensor(slots[:tokens], dtype=torch.int32)
-    if tokens == 330:
+    if tokens in (330, 331):
         slots = slots[torch.randperm(tokens)]                     # a decode step: every token a sequence of its own
     extra, rot = 8, d // 8 * 8 // 16 * 16
     qkv = torch.randn(tokens, (nq + 2 * nkv) * d + extra).to(DT[dtypes[0]]).to(DEV)

@@ -104,6 +104,18 @@ def test_into_how_many_parts_a_decode_step_cuts_its_keys(batch, kv_heads, dim, c
     assert nsplit == parts and split_len % 32 == 0 and nsplit * split_len >= context
 
 
+@pytest.mark.parametrize("counts, recorded, want", [
+    ([512], False, True), ([7] * 60, False, False), ([8] * 60, False, True), ([400] + [1] * 8, False, True), ([400] + [1] * 9, False, False),
+    ([2000] + [1] * 16, False, False), ([2048] + [1] * 16, False, True), ([1] * 300, False, False), ([300] + [0] * 7, True, True),
+    ([300] + [0] * 63, True, False), ([1] * 64, True, False)])
+def test_which_steps_bring_tokens_whose_slots_follow_one_another(counts, recorded, want):
+    import numpy as np
+    from tlie_amd import ops
+    ctx = SimpleNamespace(max_new=max(counts), num_tokens=sum(counts), num_seqs=len(counts), tile_owner=object() if recorded else None,
+                          host={"seq_start": np.concatenate([[0], np.cumsum(counts)])})
+    assert ops.slots_follow(ctx) is want
+
+
 @pytest.mark.parametrize("rows, outputs, inputs, gated, want", [
     (24, 22016, 4096, True, True), (16, 22016, 4096, True, True), (16, 11264, 2048, True, False), (17, 2048, 128, True, True), (64, 8192, 128, True, True),
     (64, 8193, 256, True, False), (32, 32768, 512, True, True), (32, 32769, 512, True, False), (64, 50000, 1024, False, False),

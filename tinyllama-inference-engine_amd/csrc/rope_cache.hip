@@ -362,11 +362,15 @@ extern "C" int tlie_rope_cache(const void* qkv, int in_dtype, int nsplit, long l
   const bool aligned = ((reinterpret_cast<uintptr_t>(qkv) | reinterpret_cast<uintptr_t>(q_out) |
                          reinterpret_cast<uintptr_t>(cache)) & 31) == 0;
   if (nsplit == 1 && (d & 7) == 0 && (row_width & 7) == 0 && aligned && (inv_freq == nullptr || (paired && (rot_dim & 7) == 0))) {
-    // Values by tiles where the caller says that slots mostly follow one another, from 256 tokens on (100 tokens of 32 + 2 x 4
-    // heads of 64: 3.9 us without, 5.4 with them, 256 in runs of 60: 4.2, 4.5, 512: 5.0, 5.0, in one run 4.9, 4.6; 512 of 32 + 2 x 8 of 128
-    // in runs of 60: 8.7, 6.2), for pages whose rows come in eights.  Slots on their own stay
-    // with their token's block: 128 of 32 + 2 x 8 heads of 128 take 5.2 us, by tiles 12.9.
-    const int value_tiles = runs && tokens >= 4 * kValueTile && page_size % 8 == 0 ? (nkv * d + kValueTile - 1) / kValueTile : 0;
+    // Values by tiles where the caller says that slots mostly follow one another, from 256 tokens and 2^18 values on (in runs of 60,
+    // without them and with them: 256 tokens of 32 + 2 x 8 heads of 128 5.8 us, 4.9; 512 of 32 + 2 x 4 of 64 4.9, 5.0, 1024 6.5, 6.2;
+    // 300 4.3, 5.2), for pages whose rows come in eights.  A tile wants the four waves of 256 threads, and its columns be full: with
+    // heads that make fewer threads, or fewer than four tiles side by side, single elements (1024 of 4 + 2 x 2 of 64 4.5, 6.9; of 8 + 2 x
+    // 8 of 32 5.8, 7.0; 2048 of 32 + 2 x 1 of 64 8.8, 9.3).  Slots on their own stay with their token's block: 128 of 32 + 2 x 8 heads
+    // of 128 take 5.2 us, by tiles 12.9.
+    const bool tiled = runs && page_size % 8 == 0 && tokens >= 4 * kValueTile && nkv * d >= 4 * kValueTile &&
+                       static_cast<long long>(tokens) * nkv * d >= 1 << 18 && (nq + nkv) * d / 8 >= 256;
+    const int value_tiles = tiled ? (nkv * d + kValueTile - 1) / kValueTile : 0;
     const long long blocks = tokens + static_cast<long long>(value_tiles) * ((tokens + kValueTile - 1) / kValueTile);
     if (blocks > 0x7fffffffLL) return kBadArgument;
     const int groups = (value_tiles > 0 ? nq + nkv : heads) * d / 8;

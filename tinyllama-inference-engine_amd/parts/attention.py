@@ -291,7 +291,7 @@ class Attention(Mixer):
             if other_positions:
                 q = self._apply_other_positions(q, ctx)
             q = ops.rope_cache(q, ctx.positions, slot_map, inv_freq, rot_dim, binding.cache, self.nq, self.nkv, self.d,
-                               self.dtype, paired=self.paired, extra_cols=self.gate_cols, head_scale=self.temp, runs=ctx.max_new >= 8)
+                               self.dtype, paired=self.paired, extra_cols=self.gate_cols, head_scale=self.temp, runs=ops.slots_follow(ctx))
         page_size = binding.cache.shape[3] // self.d
         if ops.attention_mfma_takes(self.dtype, self.d, page_size):
             tiles, col_tiles, nsplit, split_len, waves, shared = ops.attention_plan(ctx, self.nq // self.nkv, self.nkv, self.d, self.reach)
