@@ -209,6 +209,23 @@ def test_gemm_generic_at_the_edges_of_its_kernels_and_gated(n, k):
             ops.gemm_generic(x, w, b, torch.float32, gated=True)
 
 
+@pytest.mark.parametrize("n, k, gated", [(18, 32768, False), (18, 32776, True), (20, 33795, False), (16, 70000, True)])
+def test_gemm_generic_of_more_blocks_than_fit_at_once(n, k, gated):
+    """At most 16 rows and K from 64 blocks of 512 on: the blocks' sums are added up in passes.  The same bits as among many rows."""
+    from tlie_amd import ops
+    torch.manual_seed(k)
+    x = torch.randn(70, k, device=DEV)
+    w = torch.randn(n, k, device=DEV) / math.sqrt(k)
+    b = torch.randn(n, device=DEV)
+    many = ops.gemm_generic(x, w, b, torch.float32, gated=gated)
+    many = many if gated else many.dense()
+    if not gated:
+        assert rel_err(many, x.double() @ w.double().T + b.double()) < 2e-5      # (K 2^-24 of what |x| |w| add up to, 2.6 sqrt(K) here)
+    for m in (1, 8, 9, 16):
+        few = ops.gemm_generic(x[:m].contiguous(), w, b, torch.float32, gated=gated)
+        assert torch.equal(few if gated else few.dense(), many[:m]), m
+
+
 @pytest.mark.parametrize("shape", [(65, 96, 64), (200, 2560, 2048), (333, 177, 200), (70, 129, 333), (1024, 2048, 5632)])
 def test_library_product_of_many_rows(shape):
     """The vendor library's product, called directly where it offers an algorithm (and through

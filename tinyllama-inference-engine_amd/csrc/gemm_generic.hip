@@ -71,7 +71,7 @@ __device__ __forceinline__ void to_quarters(float4& v) {
 template <typename X, typename W, typename O, int MT, int R, bool PAIR, int RING, int WAVES, bool WIDE>
 __global__ void __launch_bounds__(64 * WAVES)
 gemm_generic_few_kernel(const X* __restrict__ x, const W* __restrict__ w, const W* __restrict__ bias,
-                        O* __restrict__ y, int M, int N, int K, int gate, float alpha, float limit) {
+                        O* __restrict__ y, int M, int N, int K, int gate, float alpha, float limit, int jobs_at_once) {
   static_assert(!PAIR || (MT == 1 && R == 8), "two blocks at once: 8 rows of W, 8 of x");
   constexpr int SC = 8 / MT < RING / 2 ? 8 / MT : RING / 2;      // loads of x asked for together
   constexpr int kJobK = PAIR ? 2 * kBlockK : kBlockK, kPartK = 16 * RING;
@@ -95,83 +95,95 @@ gemm_generic_few_kernel(const X* __restrict__ x, const W* __restrict__ w, const 
 #pragma unroll
     for (int c = 0; c < RING; ++c) ring[c] = fetch4<WIDE>(w_row, k0 + first + 16 * c, K);
   }
-  for (int job = wave; job < jobs; job += waves) {
-    const int end = min(job * kJobK + kBlockK, K);
-    floatx4 acc[MT];
-#pragma unroll
-    for (int i = 0; i < MT; ++i) acc[i] = floatx4{0.f, 0.f, 0.f, 0.f};
-    while (k0 < end) {                                     // (all of these the same for the whole wave)
-      const int next = k0 + kPartK < end ? k0 + kPartK : (job + waves) * kJobK;
-      const bool more = next < K, edge = k0 + kPartK + (PAIR ? kBlockK : 0) > K;
-#pragma unroll
-      for (int c = 0; c < RING; ++c) {
-        if (c % SC == 0) {                                 // the next few pieces of x
-          const int to = (c / SC + 1) & 1;
-          const int from = (c + SC < RING ? k0 + 16 * (c + SC) : next) + first;
-          if (c + SC < RING || more) {
-#pragma unroll
-            for (int e = 0; e < SC; ++e)
-#pragma unroll
-              for (int i = 0; i < MT; ++i) xs[to][e][i] = fetch4<WIDE>(x_row[i], from + 16 * e, K);
-          }
-        }
-        float4 a = ring[c], b[MT];
-#pragma unroll
-        for (int i = 0; i < MT; ++i) b[i] = xs[(c / SC) & 1][c % SC][i];
-        if (edge) {                                        // past the end of K: zeros
-          a = inside(a, k0 + first + 16 * c, K);
-#pragma unroll
-          for (int i = 0; i < MT; ++i) b[i] = inside(b[i], k0 + first + 16 * c, K);
-        }
-        if (more) ring[c] = fetch4<WIDE>(w_row, next + first + 16 * c, K);
-        to_quarters(a);
-#pragma unroll
-        for (int i = 0; i < MT; ++i) to_quarters(b[i]);
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-#pragma unroll
-          for (int i = 0; i < MT; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32((&a.x)[e], (&b[i].x)[e], acc[i], 0, 0, 0);
-      }
-      k0 = next;
-    }
-    settle(acc);
-    // lane (r, g) holds what the instruction's rows 4 g .. 4 g + 3 (of W) have for its column r (of x)
-    if (PAIR) {
-      if ((r >> 3) == (g >> 1))
-        *reinterpret_cast<float4*>(sums + (2 * job + (r >> 3)) * 64 + (r & 7) * 8 + 4 * (g & 1)) = make_float4(acc[0][0], acc[0][1], acc[0][2], acc[0][3]);
-    } else {
-#pragma unroll
-      for (int i = 0; i < MT; ++i)
-        *reinterpret_cast<float4*>(sums + (job * MT + i) * 256 + r * 16 + 4 * g) = make_float4(acc[i][0], acc[i][1], acc[i][2], acc[i][3]);
-    }
-  }
-  __syncthreads();
-  const int blocks = (K + kBlockK - 1) / kBlockK;
+  // (the blocks' sums of one pass fit LDS; only a K of more than 64 blocks, with MT = 1, takes several)
   constexpr int kQuads = R / 4, kRows = PAIR ? 8 : 16 * MT;
-  for (int t = threadIdx.x; t < kQuads * kRows; t += blockDim.x) {
-    const int m = t / kQuads, j = t % kQuads * 4, n = n0 + j;       // four neighbouring columns of y
-    if (m >= M || n >= N) continue;
-    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int b = 0; b < blocks; ++b) {                     // in index order
-      const float4 s = *reinterpret_cast<const float4*>(sums + (b * kRows + m) * R + j);
-      v.x += s.x, v.y += s.y, v.z += s.z, v.w += s.w;
-    }
-    const float out[4] = {v.x, v.y, v.z, v.w};
+  const int blocks = (K + kBlockK - 1) / kBlockK, pass = min(jobs, jobs_at_once);
+  float4 before = make_float4(0.f, 0.f, 0.f, 0.f);         // this thread's sums of earlier passes (then it has one place at most)
+  int job = wave;
+  for (int first_job = 0; first_job < jobs; first_job += pass) {
+    for (; job < min(jobs, first_job + pass); job += waves) {
+      const int end = min(job * kJobK + kBlockK, K), slot = job - first_job;
+      floatx4 acc[MT];
 #pragma unroll
-    for (int e = 0; e < 4; e += 2) {
-      float p = out[e], u = out[e + 1];
-      if (n + e >= N) break;
-      if (bias) {
-        p += to_float(bias[n + e]);
-        if (n + e + 1 < N) u += to_float(bias[n + e + 1]);
+      for (int i = 0; i < MT; ++i) acc[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+      while (k0 < end) {                                     // (all of these the same for the whole wave)
+        const int next = k0 + kPartK < end ? k0 + kPartK : (job + waves) * kJobK;
+        const bool more = next < K, edge = k0 + kPartK + (PAIR ? kBlockK : 0) > K;
+#pragma unroll
+        for (int c = 0; c < RING; ++c) {
+          if (c % SC == 0) {                                 // the next few pieces of x
+            const int to = (c / SC + 1) & 1;
+            const int from = (c + SC < RING ? k0 + 16 * (c + SC) : next) + first;
+            if (c + SC < RING || more) {
+#pragma unroll
+              for (int e = 0; e < SC; ++e)
+#pragma unroll
+                for (int i = 0; i < MT; ++i) xs[to][e][i] = fetch4<WIDE>(x_row[i], from + 16 * e, K);
+            }
+          }
+          float4 a = ring[c], b[MT];
+#pragma unroll
+          for (int i = 0; i < MT; ++i) b[i] = xs[(c / SC) & 1][c % SC][i];
+          if (edge) {                                        // past the end of K: zeros
+            a = inside(a, k0 + first + 16 * c, K);
+#pragma unroll
+            for (int i = 0; i < MT; ++i) b[i] = inside(b[i], k0 + first + 16 * c, K);
+          }
+          if (more) ring[c] = fetch4<WIDE>(w_row, next + first + 16 * c, K);
+          to_quarters(a);
+#pragma unroll
+          for (int i = 0; i < MT; ++i) to_quarters(b[i]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int i = 0; i < MT; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32((&a.x)[e], (&b[i].x)[e], acc[i], 0, 0, 0);
+        }
+        k0 = next;
       }
-      if (gate != kNoGate) {
-        y[static_cast<size_t>(m) * (N / 2) + (n + e) / 2] = from_float<O>(gated_value(p, u, gate, alpha, limit));
+      settle(acc);
+      // lane (r, g) holds what the instruction's rows 4 g .. 4 g + 3 (of W) have for its column r (of x)
+      if (PAIR) {
+        if ((r >> 3) == (g >> 1))
+          *reinterpret_cast<float4*>(sums + (2 * slot + (r >> 3)) * 64 + (r & 7) * 8 + 4 * (g & 1)) = make_float4(acc[0][0], acc[0][1], acc[0][2], acc[0][3]);
       } else {
-        y[static_cast<size_t>(m) * N + n + e] = from_float<O>(p);
-        if (n + e + 1 < N) y[static_cast<size_t>(m) * N + n + e + 1] = from_float<O>(u);
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+          *reinterpret_cast<float4*>(sums + (slot * MT + i) * 256 + r * 16 + 4 * g) = make_float4(acc[i][0], acc[i][1], acc[i][2], acc[i][3]);
       }
     }
+    __syncthreads();
+    const bool last = first_job + pass >= jobs;
+    const int blocks_here = last ? blocks - first_job * (kJobK / kBlockK) : pass * (kJobK / kBlockK);
+    for (int t = threadIdx.x; t < kQuads * kRows; t += blockDim.x) {
+      const int m = t / kQuads, j = t % kQuads * 4, n = n0 + j;       // four neighbouring columns of y
+      if (m >= M || n >= N) continue;
+      float4 v = before;
+      for (int b = 0; b < blocks_here; ++b) {                // in index order
+        const float4 s = *reinterpret_cast<const float4*>(sums + (b * kRows + m) * R + j);
+        v.x += s.x, v.y += s.y, v.z += s.z, v.w += s.w;
+      }
+      if (!last) {
+        before = v;
+        continue;
+      }
+      const float out[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+      for (int e = 0; e < 4; e += 2) {
+        float p = out[e], u = out[e + 1];
+        if (n + e >= N) break;
+        if (bias) {
+          p += to_float(bias[n + e]);
+          if (n + e + 1 < N) u += to_float(bias[n + e + 1]);
+        }
+        if (gate != kNoGate) {
+          y[static_cast<size_t>(m) * (N / 2) + (n + e) / 2] = from_float<O>(gated_value(p, u, gate, alpha, limit));
+        } else {
+          y[static_cast<size_t>(m) * N + n + e] = from_float<O>(p);
+          if (n + e + 1 < N) y[static_cast<size_t>(m) * N + n + e + 1] = from_float<O>(u);
+        }
+      }
+    }
+    if (!last) __syncthreads();                              // (the sums have been read)
   }
 }
 
@@ -313,9 +325,11 @@ template <typename X, typename W, typename O, int MT, int R, bool PAIR, int RING
 int launch_few(const X* x, const W* w, const W* bias, O* y, int M, int N, int K, int gate, float alpha, float limit, hipStream_t s) {
   const int job_k = PAIR ? 2 * kBlockK : kBlockK, jobs = (K + job_k - 1) / job_k, turns = (jobs + WAVES - 1) / WAVES;
   const int waves = (jobs + turns - 1) / turns;            // as many for each turn
-  const int bytes = jobs * (PAIR ? 2 * 64 : 16 * MT * R) * static_cast<int>(sizeof(float));
+  const int job_bytes = (PAIR ? 2 * 64 : 16 * MT * R) * static_cast<int>(sizeof(float));
+  const int at_once = jobs <= 64 * 1024 / job_bytes ? jobs : 64 * 1024 / job_bytes;
+  const int bytes = at_once * job_bytes;
   hipLaunchKernelGGL((gemm_generic_few_kernel<X, W, O, MT, R, PAIR, RING, WAVES, WIDE>), dim3((N + R - 1) / R), dim3(64 * waves), bytes, s,
-                     x, w, bias, y, M, N, K, gate, alpha, limit);
+                     x, w, bias, y, M, N, K, gate, alpha, limit, at_once);
   return launch_status();
 }
 
@@ -334,13 +348,13 @@ template <typename X, typename W, typename O, bool WIDE>
 int launch_product(const X* x, const W* w, const W* bias, O* y, int M, int N, int K, int gate, float alpha, float limit,
                    int compute_units, hipStream_t s) {
   const long long blocks = (K + kBlockK - 1) / kBlockK;
-  // Few rows of x: the kernel that reads W straight into registers, while the sums of the blocks fit LDS.  A matrix of at
+  // Few rows of x: the kernel that reads W straight into registers; more than 16, while the sums of the blocks fit LDS.  A matrix of at
   // most 8 rows a compute unit takes two blocks at once (2048 x 2048, 8 rows of x: 10.1 us against 12.0; 2560 x 2048, where
   // some units would get two workgroups: 14.8 against 12.3).  More than 16 rows of x go there only while W has at most 16 rows
   // a unit: every workgroup reads all of x (64 rows, 2048 x 2048: 24.7 us against 34.4 in tiles; 11264 x 2048: 70.1 against 46.1).
   // One block of K or less gives a workgroup one wave: such products go in tiles (96 x 96, 16 rows: 3.3 us against 4.0).
   const int mt = M <= 16 ? 1 : (M <= 32 ? 2 : 4);
-  if (M <= 64 && blocks > 1 && blocks * mt * 1024 <= 64 * 1024 && (mt == 1 || (N + 15) / 16 <= compute_units)) {
+  if (M <= 64 && blocks > 1 && (mt == 1 || (blocks * mt * 1024 <= 64 * 1024 && (N + 15) / 16 <= compute_units))) {
     constexpr int kRing = WIDE ? 16 : 8;
     if (mt == 4) return launch_few<X, W, O, 4, 16, false, 8, 8, WIDE>(x, w, bias, y, M, N, K, gate, alpha, limit, s);
     if (mt == 2) return launch_few<X, W, O, 2, 16, false, 8, WIDE ? 12 : 8, WIDE>(x, w, bias, y, M, N, K, gate, alpha, limit, s);
