@@ -587,6 +587,36 @@ def test_benchmark_layer_sizes_cut_three_ways(tmp_path, dtype):
         assert bad is None, f"recorded portions of {request}: position {places[bad]} is wrong"
 
 
+def test_recorded_steps_of_both_forms_of_the_plain_attention(tmp_path):
+    """32-bit steps of portions beside single tokens at the benchmark's layer sizes: recorded at 320 tokens, where both forms of the
+    plain attention are launched and each sequence's token count on the device decides; replayed with other cuts, with padding
+    tokens, and with sequences whose part changes from one form to the other; against the plain implementation."""
+    from tlie_amd import Engine, ops
+    folder = make_model(tmp_path / "model", BENCH_SHAPE, seed=5, dtype_name="float32", std=0.02, norm_std=0.1)
+    raw, weights = load_plain(folder)
+    length = 400
+    tokens = random_tokens(78, length, BENCH_SHAPE["vocab_size"])
+    want = plain_forward(raw, weights, tokens)
+    del weights
+    engine = Engine(folder, dtype="float32", max_tokens=2048, page_size=16, max_requests=6)
+    replay, starts = Replayer(engine), {}
+    for cut in ({"a": 150, "b": 100, "c": 1, "d": 20}, {"a": 1, "b": 130, "c": 120, "d": 8}, {"a": 2, "b": 1, "c": 1, "d": 260},
+                {"a": 120, "b": 7, "c": 150, "d": 1}, {"a": 3, "b": 92, "c": 91, "d": 100}):
+        items = []
+        for request, size in cut.items():
+            first = starts.get(request, 0)
+            items.append((request, tokens[first:first + size], sorted({0, size - 1})))
+            starts[request] = first + size
+        replay.step(items)
+    assert sorted(engine.runner._portion_graphs) == [(320, 8, 256), (320, 8, 512)]
+    for graph in engine.runner._portion_graphs.values():
+        assert graph.graph is not None and ops.attention_generic_plan(graph.ctx, 32, 4, 64) == 2
+    for request in starts:
+        places = sorted(place for name, place in replay.rows if name == request)
+        bad = first_bad_row(replay.logits_of(request, places), want[places], TOLERANCE["float32"])
+        assert bad is None, f"position {places[bad]} of {request} is wrong"
+
+
 def test_decode_steps_list_their_sequences_longest_first(tmp_path):
     """33 sequences of 3 to 300 positions on 16 key heads: more workgroups in the attention than compute units, which then goes by
     the list; replays of one recording while lengths grow and sequences end, so that padding takes their rows."""

@@ -365,6 +365,38 @@ def test_the_three_forms_of_the_plain_attention_kernel_give_the_same_bits(dtype,
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("nq, nkv, d, page", [(16, 2, 8, 16), (16, 4, 24, 24), (6, 6, 40, 16), (5, 5, 20, 8), (8, 4, 64, 16), (7, 7, 32, 32), (70, 1, 16, 16)])
+def test_the_sharing_form_of_the_plain_attention_in_pieces(dtype, nq, nkv, d, page):
+    """A workgroup's tokens cut to those of one sequence, to fewer, and as they come: the same bits as a workgroup a token and head,
+    for head sizes of one to four sixteens of dims, pages of no power of two, sequences of one to 65 tokens side by side."""
+    from tlie_amd import ops
+    counts, before = [65, 1, 16, 7, 33, 8], [3, 70, 0, 200, 64, 129]
+    torch.manual_seed(nq + d)
+    tables, caches, base = [], [], 0
+    for count, first in zip(counts, before):
+        cache, pages = build_cache(torch.randn(first + count, nkv, d), torch.randn(first + count, nkv, d), page, DT[dtype], shuffle_seed=d)
+        tables.append([base + number for number in pages])
+        caches.append(cache)
+        base += cache.shape[0]
+    width = max(len(table) for table in tables)
+    table = torch.tensor([row + [0] * (width - len(row)) for row in tables], dtype=torch.int32, device=DEV)
+    cache = torch.cat(caches).to(DEV)
+    tokens = sum(counts)
+    token_seq = torch.repeat_interleave(torch.arange(len(counts), dtype=torch.int32), torch.tensor(counts)).to(DEV)
+    positions = torch.cat([torch.arange(first, first + count, dtype=torch.int32) for count, first in zip(counts, before)]).to(DEV)
+    seq_start = torch.tensor([sum(counts[:i]) for i in range(len(counts) + 1)], dtype=torch.int32, device=DEV)
+    q = torch.randn(tokens, nq * d).to(DT[dtype]).to(DEV)
+
+    def run(tiled, **kw):
+        return ops.attention_generic(q, cache, table, token_seq, positions, nq, nkv, d, None, 1.0 / math.sqrt(d), tiled=tiled, seq_start=seq_start, **kw)
+    plain = run(0)
+    assert torch.isfinite(plain.float()).all()
+    for pieces in (None, 0, 1, 5, 16, 33, 1000):
+        assert torch.equal(run(1, tile_tokens=pieces), plain), pieces
+        assert torch.equal(run(2, tile_tokens=pieces), plain), pieces
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("case", [
     dict(nq=8, nkv=2, d=64, page=16, window=None), dict(nq=6, nkv=3, d=48, page=16, window=70),
     dict(nq=5, nkv=5, d=7, page=8, window=None), dict(nq=40, nkv=1, d=16, page=16, window=300),   # 40 heads a group: two blocks of heads

@@ -129,6 +129,35 @@ def test_which_products_keep_their_weights_in_a_ring(rows, outputs, inputs, gate
         assert split_len % 64 == 0 and 1 <= strips <= 8 and (rows <= 48 or strips != 7) and (split_len >= inputs or not gated)
 
 
+@pytest.mark.parametrize("counts, heads, kv_heads, dim, dtype, recorded, how, want", [
+    # groups and sizes that the kernels know
+    ([256], 32, 4, 64, "float32", False, {}, 1), ([255], 32, 4, 64, "float32", False, {}, 0), ([250, 1, 5], 32, 4, 64, "float32", False, {}, 2),
+    ([4] * 64, 32, 4, 64, "float32", False, {}, 1), ([3] * 86, 32, 4, 64, "float32", False, {}, 0), ([256], 32, 4, 64, "bfloat16", False, {}, 1),
+    ([256], 32, 4, 64, "float32", True, {}, 2), ([255], 32, 4, 64, "float32", True, {}, 0), ([1] * 300, 32, 4, 64, "float32", True, {}, 0),
+    # sizes that they do not know, or no groups
+    ([64], 32, 4, 64, "float32", False, dict(softcap=30.0), 1), ([63], 32, 4, 64, "float32", False, dict(softcap=30.0), 0),
+    ([64], 32, 4, 64, "float32", False, dict(page_size=24), 1), ([64], 32, 4, 64, "float32", False, dict(page_size=8), 1),
+    ([86], 32, 4, 32, "float32", False, dict(value_dim=48), 1), ([85], 32, 4, 32, "float32", False, dict(value_dim=48), 0),
+    ([16], 32, 32, 64, "bfloat16", False, {}, 1), ([15], 32, 32, 64, "bfloat16", False, {}, 0), ([64], 32, 32, 64, "float32", False, {}, 1),
+    ([7] * 64, 32, 32, 64, "float32", False, {}, 0), ([8] * 64, 32, 32, 64, "float32", False, {}, 1),
+    ([86], 16, 2, 8, "bfloat16", False, {}, 1), ([85], 16, 2, 8, "bfloat16", False, {}, 0),
+    # heads too large for it
+    ([500], 32, 4, 65, "float32", False, {}, 0), ([500], 32, 4, 64, "float32", False, dict(value_dim=65), 0)])
+def test_which_form_of_the_plain_attention_a_step_takes(counts, heads, kv_heads, dim, dtype, recorded, how, want):
+    """0: a workgroup a token and head; 1: keys shared among a sequence's tokens; 2: both."""
+    import numpy as np
+    from tlie_amd import ops
+    ctx = SimpleNamespace(num_tokens=sum(counts), max_new=max(counts), tile_owner=object() if recorded else None,
+                          host={"seq_start": np.concatenate([[0], np.cumsum(counts)])})
+    assert ops.attention_generic_plan(ctx, heads, kv_heads, dim, dtype=getattr(torch, dtype), **how) == want
+    for group in (1, 3, 4, 16, 70):                           # pieces: equal ones of a sequence, as many columns as fit
+        full = 64 // min(64, group)
+        for tokens, seqs in ((1, 1), (100, 1), (60, 1), (128, 16), (1000, 64)):
+            size = ops.generic_tile_tokens(tokens, seqs, group, 1)
+            mean = -(-tokens // seqs)
+            assert 1 <= size <= full and (mean > full or size == mean) and (mean <= full or 2 * size >= full or full == 1)
+
+
 def test_the_skinny_products_launch_shape_is_one_the_kernel_takes():
     """Decided on the host from the sizes alone: every plan is within what the kernel takes, covers
     the inner size exactly, and for matrices that the policy balances the workgroups are no more

@@ -243,15 +243,16 @@ __device__ __forceinline__ void row4(float (&v)[4], const T* __restrict__ row, i
 }
 
 // One running state of a column: lane (column l & 15, quarter g) keeps the dims 16 t + 4 g .. + 3 of its sum of values.
+template <int KD>
 struct ColumnState {
   float top = -INFINITY, sum = 0.f;
-  floatx4 acc[4] = {};
+  floatx4 acc[KD] = {};
 };
 
 // A chunk's scores (dot[t]: keys 16 t + 4 g .. + 3, from `start`) become probabilities, in place, and the state takes in their
 // maximum and sum; its values are scaled and wait for the chunk's.
-template <bool CAP>
-__device__ __forceinline__ void take_scores(floatx4 (&dot)[4], ColumnState& state, int start, int lo, int pos, int g, float scale, float softcap) {
+template <bool CAP, int KD>
+__device__ __forceinline__ void take_scores(floatx4 (&dot)[4], ColumnState<KD>& state, int start, int lo, int pos, int g, float scale, float softcap) {
   settle(dot);
   settle(state.acc);
   float top = -INFINITY;
@@ -282,7 +283,7 @@ __device__ __forceinline__ void take_scores(floatx4 (&dot)[4], ColumnState& stat
   state.sum = state.sum * alpha + chunk_sum;
   state.top = new_max;
 #pragma unroll
-  for (int t = 0; t < 4; ++t) state.acc[t] *= alpha;
+  for (int u = 0; u < KD; ++u) state.acc[u] *= alpha;
 }
 
 // ---- many tokens a sequence ----
@@ -300,8 +301,9 @@ __device__ __forceinline__ void take_scores(floatx4 (&dot)[4], ColumnState& stat
 // Tokens of a workgroup that belong to different sequences are served one run of equal sequences after the other.
 // C > 0: both head sizes are 16 C, a page holds a power of two of rows, 16 at least, cache and queries are aligned for loads of
 // four, and scores have no cap: a chunk's sixteen rows a piece then lie on one page.  C = 0: everything else.
+// KD: sixteens of dims that either head size has at most.
 constexpr int kTiledCols = 64, kTiledWaves = 4, kRowStride = 68;
-template <typename T, int C>
+template <typename T, int C, int KD>
 __global__ void __launch_bounds__(64 * kTiledWaves)
 attention_generic_tiled_kernel(const T* __restrict__ q, const T* __restrict__ cache, const int* __restrict__ block_table,
                                int max_blocks, const int* __restrict__ token_seq, const int* __restrict__ positions,
@@ -322,8 +324,12 @@ attention_generic_tiled_kernel(const T* __restrict__ q, const T* __restrict__ ca
   const size_t page_stride = static_cast<size_t>(page_size) * (static_cast<size_t>(nkv) * d + static_cast<size_t>(nkv / vshare) * dv);
   const T* keys = cache + static_cast<size_t>(kv_head) * page_size * d;
   const T* values = cache + static_cast<size_t>(nkv) * page_size * d + static_cast<size_t>(kv_head / vshare) * page_size * dv;
-  constexpr int kDims = C > 0 ? C : 4;             // sixteens of dims
-  const int page_bits = 31 - __builtin_clz(page_size), in_page = page_size - 1;        // (where pages hold a power of two)
+  static_assert(C == 0 || C == KD, "known sizes");
+    const int page_bits = 31 - __builtin_clz(page_size), in_page = page_size - 1;        // (where pages hold a power of two)
+  const bool whole_bits = (page_size & in_page) == 0;
+  // where key j lies: its page's place in the table, its row there
+  auto page_at = [&](int j) { return whole_bits ? j >> page_bits : j / page_size; };
+  auto row_in = [&](int j) { return whole_bits ? j & in_page : j % page_size; };
   // whole loads of four where rows allow them
   const bool aligned = C > 0 || ((reinterpret_cast<uintptr_t>(cache) % (4 * sizeof(T))) == 0 && (page_size & 3) == 0);
   const bool wide_k = aligned && (d & 3) == 0, wide_q = C > 0 || ((d & 3) == 0 && (reinterpret_cast<uintptr_t>(q) % (4 * sizeof(T))) == 0);
@@ -335,13 +341,13 @@ attention_generic_tiled_kernel(const T* __restrict__ q, const T* __restrict__ ca
   const int col_pos = col_tok >= 0 ? positions[tok0 + col_tok] : -1;
   int col_lo = window > 0 ? max(0, col_pos - window + 1) : 0;
   if (chunk > 0 && col_pos >= 0) col_lo = max(col_lo, col_pos - col_pos % chunk);
-  float query[kDims][4];                           // dims 16 c + 4 j + g
+  float query[KD][4];                           // dims 16 c + 4 j + g
 #pragma unroll
-  for (int c = 0; c < kDims; ++c) {
+  for (int c = 0; c < KD; ++c) {
     row4(query[c], q + (static_cast<size_t>(tok0 + max(col_tok, 0)) * nq + col_head) * d, 16 * c + 4 * g, C > 0 ? 16 * C : (col_tok >= 0 ? d : 0), wide_q);
     to_quarters(query[c]);
   }
-  ColumnState kept0, kept1, kept2, kept3;          // (not an array: the compiler would keep it in memory)
+  ColumnState<KD> kept0, kept1, kept2, kept3;          // (not an array: the compiler would keep it in memory)
 
   int stamp = 0;                                   // chunks so far
   int run_first = 0;
@@ -403,16 +409,17 @@ attention_generic_tiled_kernel(const T* __restrict__ q, const T* __restrict__ ca
       for (int p = 0; p < 4; ++p) {
         const int row = (threadIdx.x >> 4) + 16 * p;
         const int j = min(max(start + row, lo), hi);                       // (a key outside is masked: any that was written will do)
-        row4(k_next[p], keys + static_cast<size_t>(pages[j / page_size]) * page_stride + static_cast<size_t>(j % page_size) * d, 4 * piece, d, wide_k);
+        row4(k_next[p], keys + static_cast<size_t>(pages[page_at(j)]) * page_stride + static_cast<size_t>(row_in(j)) * d, 4 * piece, d, wide_k);
+        if (p >= KD) continue;                     // (no dims there)
         const int jv = start + 4 * piece;          // keys jv .. jv + 3 of dim `row`
         if (aligned && jv >= lo && jv + 3 <= hi) {
-          row4(v_next[p], values + static_cast<size_t>(pages[jv / page_size]) * page_stride + static_cast<size_t>(row) * page_size + jv % page_size, 0, row < dv ? 4 : 0, true);
+          row4(v_next[p], values + static_cast<size_t>(pages[page_at(jv)]) * page_stride + static_cast<size_t>(row) * page_size + row_in(jv), 0, row < dv ? 4 : 0, true);
         } else {
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const int je = jv + e;
             v_next[p][e] = row < dv && je >= lo && je <= hi
-                ? to_float(values[static_cast<size_t>(pages[je / page_size]) * page_stride + static_cast<size_t>(row) * page_size + je % page_size]) : 0.f;
+                ? to_float(values[static_cast<size_t>(pages[page_at(je)]) * page_stride + static_cast<size_t>(row) * page_size + row_in(je)]) : 0.f;
           }
         }
       }
@@ -424,11 +431,11 @@ attention_generic_tiled_kernel(const T* __restrict__ q, const T* __restrict__ ca
 #pragma unroll
       for (int p = 0; p < 4; ++p) {
         const int at = ((threadIdx.x >> 4) + 16 * p) * kRowStride + (piece >> 2) * 16 + (piece & 3);
-        if (4 * piece < 16 * kDims) {
+        if (4 * piece < 16 * KD) {
 #pragma unroll
           for (int e = 0; e < 4; ++e) k_tile[half][at + 4 * e] = k_next[p][e];
         }
-        if (p < kDims) {
+        if (p < KD) {
           if (C > 0 && outside) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) v_next[p][e] = start + 4 * piece + e >= lo && start + 4 * piece + e <= hi ? v_next[p][e] : 0.f;
@@ -453,7 +460,7 @@ attention_generic_tiled_kernel(const T* __restrict__ q, const T* __restrict__ ca
     look_up(n1);
     put(0, 0);
     if (n1 < chunks) ask(n1);
-    ColumnState own = kept0;
+    ColumnState<KD> own = kept0;
     while (n < chunks) {                           // (uniform)
       const int n2 = n1 < chunks ? after(n1) : n1;
       lds_barrier();                               // chunk n is whole, the one before has been read
@@ -465,7 +472,7 @@ attention_generic_tiled_kernel(const T* __restrict__ q, const T* __restrict__ ca
         floatx4 dot[4] = {};
         const float* key = k_tile[half] + r * kRowStride + 4 * g;
 #pragma unroll
-        for (int c = 0; c < kDims; ++c) {
+        for (int c = 0; c < KD; ++c) {
           if (16 * c >= d) break;                  // (dims past d are zeros)
           float4 a[4];
 #pragma unroll
@@ -482,13 +489,13 @@ attention_generic_tiled_kernel(const T* __restrict__ q, const T* __restrict__ ca
           for (int t = 0; t < 4; ++t) {
             float weight[4] = {dot[t][0], dot[t][1], dot[t][2], dot[t][3]};
             to_quarters(weight);
-            float4 a[kDims];
+            float4 a[KD];
 #pragma unroll
-            for (int u = 0; u < kDims; ++u) a[u] = *reinterpret_cast<const float4*>(value + 16 * u * kRowStride + 16 * t);
+            for (int u = 0; u < KD; ++u) a[u] = *reinterpret_cast<const float4*>(value + 16 * u * kRowStride + 16 * t);
 #pragma unroll
             for (int e = 0; e < 4; ++e)
 #pragma unroll
-              for (int u = 0; u < kDims; ++u) own.acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32((&a[u].x)[e], weight[e], own.acc[u], 0, 0, 0);
+              for (int u = 0; u < KD; ++u) own.acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32((&a[u].x)[e], weight[e], own.acc[u], 0, 0, 0);
           }
         } else {
           // a value that is not finite, among keys that some column must not see: zero times it would be no zero there, so every
@@ -502,7 +509,7 @@ attention_generic_tiled_kernel(const T* __restrict__ q, const T* __restrict__ ca
                 const float weight = __shfl(dot[t][i], 16 * from + r, 64);
                 if (j < col_lo || j > my_pos) continue;
 #pragma unroll
-                for (int u = 0; u < kDims; ++u)
+                for (int u = 0; u < KD; ++u)
 #pragma unroll
                   for (int e = 0; e < 4; ++e)
                     own.acc[u][e] = fmaf(weight, v_tile[half][(16 * u + 4 * g + e) * kRowStride + 16 * t + 4 * i + from], own.acc[u][e]);
@@ -528,17 +535,17 @@ attention_generic_tiled_kernel(const T* __restrict__ q, const T* __restrict__ ca
   }
   // the four states of a column into one, in their order
   float top = fmaxf(fmaxf(kept0.top, kept1.top), fmaxf(kept2.top, kept3.top)), total = 0.f;
-  floatx4 result[kDims] = {};
+  floatx4 result[KD] = {};
   if (sink != nullptr) {
     top = fmaxf(top, sink[col_head]);
     total = expf(sink[col_head] - top);
   }
-  auto join = [&](const ColumnState& one) {
+  auto join = [&](const ColumnState<KD>& one) {
     if (one.top == -INFINITY) return;
     const float w = expf(one.top - top);
     total += w * one.sum;
 #pragma unroll
-    for (int u = 0; u < kDims; ++u)
+    for (int u = 0; u < KD; ++u)
 #pragma unroll
       for (int e = 0; e < 4; ++e) result[u][e] += w * one.acc[u][e];
   };
@@ -548,7 +555,7 @@ attention_generic_tiled_kernel(const T* __restrict__ q, const T* __restrict__ ca
   join(kept3);
   const size_t row = (static_cast<size_t>(tok0 + col_tok) * nq + col_head) * dv;
 #pragma unroll
-  for (int u = 0; u < kDims; ++u)
+  for (int u = 0; u < KD; ++u)
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int dim = 16 * u + 4 * g + e;
@@ -561,7 +568,8 @@ attention_generic_tiled_kernel(const T* __restrict__ q, const T* __restrict__ ca
 // and values straight from the cache into registers (a lane asks for 16 bytes of a key or of a dim's row of values), the next
 // chunk's asked for while this one's products run.  The kernel of one head a workgroup reads a key once for each of the heads that
 // share it; what a chunk takes here (some 4 us) does not fall with the number of heads, so that kernel stays for steps of little
-// work (the line is drawn where it is launched).
+// work (the line is drawn where it is launched).  C as above, but never 0: with sizes that are not known beforehand it is the slower
+// one throughout (64 tokens of 200 keys, 16 heads of 48 on 8: 36 us against 15).
 template <typename T, int C>
 __global__ void __launch_bounds__(256)
 attention_generic_few_kernel(const T* __restrict__ q, const T* __restrict__ cache, const int* __restrict__ block_table,
@@ -581,69 +589,41 @@ attention_generic_few_kernel(const T* __restrict__ q, const T* __restrict__ cach
   const size_t page_stride = static_cast<size_t>(page_size) * (static_cast<size_t>(nkv) * d + static_cast<size_t>(nkv / vshare) * dv);
   const T* keys = cache + static_cast<size_t>(kv_head) * page_size * d;
   const T* values = cache + static_cast<size_t>(nkv) * page_size * d + static_cast<size_t>(kv_head / vshare) * page_size * dv;
-  constexpr int kDims = C > 0 ? C : 4;
   const int page_bits = 31 - __builtin_clz(page_size), in_page = page_size - 1;
-  const bool aligned = C > 0 || ((reinterpret_cast<uintptr_t>(cache) % (4 * sizeof(T))) == 0 && (page_size & 3) == 0);
-  const bool wide_k = aligned && (d & 3) == 0, wide_q = C > 0 || ((d & 3) == 0 && (reinterpret_cast<uintptr_t>(q) % (4 * sizeof(T))) == 0);
-  const int kc = C > 0 ? C : (d + 15) / 16, vc = C > 0 ? C : (dv + 15) / 16;
-  float query[kDims][4];
+  float query[C][4];
 #pragma unroll
-  for (int c = 0; c < kDims; ++c) {
-    row4(query[c], q + (static_cast<size_t>(t0) * nq + kv_head * G + head0 + min(r, nheads - 1)) * d, 16 * c + 4 * g, C > 0 ? 16 * C : d, wide_q);
+  for (int c = 0; c < C; ++c) {
+    row4(query[c], q + (static_cast<size_t>(t0) * nq + kv_head * G + head0 + min(r, nheads - 1)) * d, 16 * c + 4 * g, 16 * C, true);
     to_quarters(query[c]);
   }
   const int first = lo / 256 * 256 + 64 * wave;
-  float k_next[4][kDims][4], v_next[4][kDims][4];
-  int page_of[4];                                  // (C > 0) the pages of the four sixteens of the chunk that is asked for next
+  float k_next[4][C][4], v_next[4][C][4];
+  int page_of[4];                                  // the pages of the four sixteens of the chunk that is asked for next
   auto look_up = [&](int start) {
-    if (C > 0) {
 #pragma unroll
-      for (int t = 0; t < 4; ++t) page_of[t] = pages[min(max(start + 16 * t, lo), pos) >> page_bits];
-    }
+    for (int t = 0; t < 4; ++t) page_of[t] = pages[min(max(start + 16 * t, lo), pos) >> page_bits];
   };
   auto ask_keys = [&](int start) {
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-      const T* row;
-      if (C > 0) {
-        row = keys + static_cast<size_t>(page_of[t]) * page_stride + static_cast<size_t>((start + 16 * t + r) & in_page) * (16 * C);
-      } else {
-        const int j = min(max(start + 16 * t + r, lo), pos);
-        row = keys + static_cast<size_t>(pages[j / page_size]) * page_stride + static_cast<size_t>(j % page_size) * d;
-      }
+      const T* row = keys + static_cast<size_t>(page_of[t]) * page_stride + static_cast<size_t>((start + 16 * t + r) & in_page) * (16 * C);
 #pragma unroll
-      for (int c = 0; c < kDims; ++c) {
-        if (C > 0) {
-          const float4 f = load4(row + 16 * c + 4 * g);
-          k_next[t][c][0] = f.x, k_next[t][c][1] = f.y, k_next[t][c][2] = f.z, k_next[t][c][3] = f.w;
-        } else if (c < kc) {
-          row4(k_next[t][c], row, 16 * c + 4 * g, d, wide_k);
-        }
+      for (int c = 0; c < C; ++c) {
+        const float4 f = load4(row + 16 * c + 4 * g);
+        k_next[t][c][0] = f.x, k_next[t][c][1] = f.y, k_next[t][c][2] = f.z, k_next[t][c][3] = f.w;
       }
     }
   };
-  // (a value outside lo .. pos counts as zero; C > 0: `hide` sets it to zero before it is used)
+  // (a value outside lo .. pos counts as zero: `hide` sets it to zero before it is used)
   auto ask_values = [&](int start) {
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       const int jv = start + 16 * t + 4 * g;
-      if (C > 0) {
-        const T* at = values + static_cast<size_t>(page_of[t]) * page_stride + static_cast<size_t>(r) * page_size + (jv & in_page);
+      const T* at = values + static_cast<size_t>(page_of[t]) * page_stride + static_cast<size_t>(r) * page_size + (jv & in_page);
 #pragma unroll
-        for (int u = 0; u < kDims; ++u) {
-          const float4 f = load4(at + static_cast<size_t>(16 * u) * page_size);
-          v_next[t][u][0] = f.x, v_next[t][u][1] = f.y, v_next[t][u][2] = f.z, v_next[t][u][3] = f.w;
-        }
-      } else {
-#pragma unroll
-        for (int u = 0; u < kDims; ++u)
-          if (u < vc)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const int je = jv + e;
-              v_next[t][u][e] = je >= lo && je <= pos
-                  ? to_float(values[static_cast<size_t>(pages[je / page_size]) * page_stride + static_cast<size_t>(min(16 * u + r, dv - 1)) * page_size + je % page_size]) : 0.f;
-            }
+      for (int u = 0; u < C; ++u) {
+        const float4 f = load4(at + static_cast<size_t>(16 * u) * page_size);
+        v_next[t][u][0] = f.x, v_next[t][u][1] = f.y, v_next[t][u][2] = f.z, v_next[t][u][3] = f.w;
       }
     }
   };
@@ -651,14 +631,14 @@ attention_generic_few_kernel(const T* __restrict__ q, const T* __restrict__ cach
 #pragma unroll
     for (int t = 0; t < 4; ++t)
 #pragma unroll
-      for (int u = 0; u < kDims; ++u)
+      for (int u = 0; u < C; ++u)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int j = start + 16 * t + 4 * g + e;
           v_next[t][u][e] = j >= lo && j <= pos ? v_next[t][u][e] : 0.f;
         }
   };
-  ColumnState state;
+  ColumnState<C> state;
   if (first <= pos) {
     look_up(first);
     ask_keys(first);
@@ -669,8 +649,7 @@ attention_generic_few_kernel(const T* __restrict__ q, const T* __restrict__ cach
     const bool more = start + 256 <= pos, partial = start < lo || start + 63 > pos;      // (uniform)
     floatx4 dot[4] = {};
 #pragma unroll
-    for (int c = 0; c < kDims; ++c) {
-      if (c >= kc) break;
+    for (int c = 0; c < C; ++c) {
 #pragma unroll
       for (int t = 0; t < 4; ++t) to_quarters(k_next[t][c]);
 #pragma unroll
@@ -679,20 +658,18 @@ attention_generic_few_kernel(const T* __restrict__ q, const T* __restrict__ cach
         for (int t = 0; t < 4; ++t) dot[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(k_next[t][c][e], query[c][e], dot[t], 0, 0, 0);
     }
     if (more) ask_keys(start + 256);
-    take_scores<C == 0>(dot, state, start, lo, pos, g, scale, softcap);
-    if (C > 0 && partial) hide(start);
+    take_scores<false>(dot, state, start, lo, pos, g, scale, softcap);
+    if (partial) hide(start);
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       float weight[4] = {dot[t][0], dot[t][1], dot[t][2], dot[t][3]};
       to_quarters(weight);
 #pragma unroll
-      for (int u = 0; u < kDims; ++u)
-        if (u < vc) to_quarters(v_next[t][u]);
+      for (int u = 0; u < C; ++u) to_quarters(v_next[t][u]);
 #pragma unroll
       for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int u = 0; u < kDims; ++u)
-          if (u < vc) state.acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(v_next[t][u][e], weight[e], state.acc[u], 0, 0, 0);
+        for (int u = 0; u < C; ++u) state.acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(v_next[t][u][e], weight[e], state.acc[u], 0, 0, 0);
     }
     if (more) {
       ask_values(start + 256);
@@ -702,7 +679,7 @@ attention_generic_few_kernel(const T* __restrict__ q, const T* __restrict__ cach
   settle(state.acc);
   __syncthreads();
 #pragma unroll
-  for (int u = 0; u < 4; ++u)
+  for (int u = 0; u < C; ++u)
     *reinterpret_cast<float4*>(&states[wave][r][16 * u + 4 * g]) = make_float4(state.acc[u][0], state.acc[u][1], state.acc[u][2], state.acc[u][3]);
   if (g == 0) states[wave][r][64] = state.top, states[wave][r][65] = state.sum;
   __syncthreads();
@@ -736,12 +713,15 @@ using namespace tlie;
 extern "C" int tlie_attention_generic(const void* q, const void* cache, int dtype, const int* block_table,
                                       int max_blocks, const int* token_seq, const int* positions, void* out,
                                       int tokens, int nq, int nkv, int d, int dv, int page_size, int window, int chunk,
-                                      const float* sink, float scale, int tiled, const int* seq_start, int min_tokens,
+                                      const float* sink, float scale, int tiled, int tile_tokens, const int* seq_start, int min_tokens,
                                       int vshare, int out_f32, float softcap, int compute_units, void* stream) {
   // tiled 0: the kernel of one (token, head) a workgroup; 1: the kernel that shares keys among a
   // sequence's tokens (head sizes up to 64); 2: both, each token served by one of them: the second
   // takes the sequences that bring min_tokens tokens or more (seq_start: int32 [sequences + 1], the
   // step's cumulative token counts), the first the others.  A token gets the same bits from either.
+  // tile_tokens: at most so many tokens a workgroup of the second (0: as many as its 64 columns hold).  It serves the sequences
+  // that its tokens belong to one after the other, so where they bring few tokens each, a workgroup of one sequence ends the
+  // sooner: 16 sequences of 32 tokens behind 200, 16 heads of 20, 33 us with 32 tokens a workgroup against 59 with 64.
   // (d only bounds the length of a dot product; dv is served by one thread a dim of a group of at most 256)
   if (tokens <= 0 || nq <= 0 || nkv <= 0 || nq % nkv != 0 || d <= 0 || d > 4096 || dv <= 0 || dv > 256 || page_size <= 0 ||
       max_blocks <= 0 || chunk < 0 || compute_units <= 0 || vshare <= 0 || nkv % vshare != 0 || softcap < 0.f)
@@ -754,46 +734,50 @@ extern "C" int tlie_attention_generic(const void* q, const void* cache, int dtyp
   const bool known = d == dv && d % 16 == 0 && d <= 64 && page_size >= 16 && (page_size & (page_size - 1)) == 0 &&
                      (reinterpret_cast<uintptr_t>(cache) | reinterpret_cast<uintptr_t>(q)) % (dtype == kF32 ? 16 : 8) == 0 && softcap == 0.f;
   const int sixteens = known && d != 48 ? d / 16 : 0;
-#define TLIE_BY_SIZE(LAUNCH)                                                                                  \
-  if (dtype == kF32) {                                                                                        \
-    if (sixteens == 1) LAUNCH(float, 1);                                                                      \
-    else if (sixteens == 2) LAUNCH(float, 2);                                                                 \
-    else if (sixteens == 4) LAUNCH(float, 4);                                                                 \
-    else LAUNCH(float, 0);                                                                                    \
-  } else {                                                                                                    \
-    if (sixteens == 1) LAUNCH(bf16, 1);                                                                       \
-    else if (sixteens == 2) LAUNCH(bf16, 2);                                                                  \
-    else if (sixteens == 4) LAUNCH(bf16, 4);                                                                  \
-    else LAUNCH(bf16, 0);                                                                                     \
-  }
+#define TLIE_BY_TYPE(LAUNCH, C, KD) \
+  { if (dtype == kF32) LAUNCH(float, C, KD); else LAUNCH(bf16, C, KD); }
   if (tiled) {
     // (the same bits as the kernel below, for steps whose sequences bring several tokens each)
     const int G = nq / nkv;
     const int heads_per_block = G < kTiledCols ? G : kTiledCols;
-    const int tokens_per_block = kTiledCols / heads_per_block;
+    int tokens_per_block = kTiledCols / heads_per_block;
+    const int least = (16 + heads_per_block - 1) / heads_per_block;                // (a wave's columns)
+    if (tile_tokens > 0) tokens_per_block = tile_tokens >= tokens_per_block ? tokens_per_block : (tile_tokens > least ? tile_tokens : least);
     const long long blocks = static_cast<long long>((tokens + tokens_per_block - 1) / tokens_per_block) * nkv;
     if (blocks > 0x7fffffff) return kBadArgument;
     const dim3 grid(static_cast<unsigned>(blocks), 1, (G + heads_per_block - 1) / heads_per_block);
-#define TLIE_TILED(T, C)                                                                                                       \
-  hipLaunchKernelGGL((attention_generic_tiled_kernel<T, C>), grid, dim3(64 * kTiledWaves), 0, (hipStream_t)stream, (const T*)q,      \
+    const int widest = d > dv ? d : dv;
+#define TLIE_TILED(T, C, KD)                                                                                                   \
+  hipLaunchKernelGGL((attention_generic_tiled_kernel<T, C, KD>), grid, dim3(64 * kTiledWaves), 0, (hipStream_t)stream, (const T*)q,      \
                      (const T*)cache, block_table, max_blocks, token_seq, positions, (T*)out, tokens, nq, nkv, d, dv, page_size,      \
                      window, chunk, sink, scale, softcap, tokens_per_block, heads_per_block, select, min_tokens, vshare, out_f32, compute_units)
-    TLIE_BY_SIZE(TLIE_TILED)
+    if (sixteens == 1) TLIE_BY_TYPE(TLIE_TILED, 1, 1)
+    else if (sixteens == 2) TLIE_BY_TYPE(TLIE_TILED, 2, 2)
+    else if (sixteens == 4) TLIE_BY_TYPE(TLIE_TILED, 4, 4)
+    else if (widest <= 16) TLIE_BY_TYPE(TLIE_TILED, 0, 1)
+    else if (widest <= 32) TLIE_BY_TYPE(TLIE_TILED, 0, 2)
+    else if (widest <= 48) TLIE_BY_TYPE(TLIE_TILED, 0, 3)
+    else TLIE_BY_TYPE(TLIE_TILED, 0, 4)
 #undef TLIE_TILED
     const int status = launch_status();
     if (status != kOk || tiled == 1) return status;
   }
-  // Head sizes up to 64: the kernel that serves a kv head's query heads together, where they are several and the step has
-  // work for four workgroups a compute unit in the kernel of one head each (64 tokens of 500 keys, 32 heads on 4: 17.4 us against
-  // 54; 8 tokens of 100 keys 9.0 against 6.7; 64 tokens of 500 keys, 32 heads on 32: 144 against 116).
-  if (d <= 64 && dv <= 64 && nq / nkv >= 2 && static_cast<long long>(tokens) * nq >= 4LL * compute_units) {
+  // Known sizes: the kernel that serves a kv head's query heads together, where they are several and the step has work for four
+  // workgroups a compute unit in the kernel of one head each (64 tokens of 500 keys, 32 heads on 4: 17.4 us against
+  // 54; 8 tokens of 100 keys 9.0 against 6.7; 64 tokens of 500 keys, 32 heads on 32: 144 against 116).  A single chunk of keys
+  // takes it longer (48 tokens of 3 keys, 32 heads on 4: 9.6 us against 8.7), so that where no sequence has more, it wants
+  // sixteen a unit.
+  const long long enough = static_cast<long long>(max_blocks) * page_size <= 64 ? 16LL * compute_units : 4LL * compute_units;
+  if (sixteens > 0 && nq / nkv >= 2 && static_cast<long long>(tokens) * nq >= enough) {
     const dim3 grid(tokens, nkv, (nq / nkv + 15) / 16);
     if (grid.y > 65535 || grid.z > 65535) return kBadArgument;
-#define TLIE_FEW(T, C)                                                                                                         \
+#define TLIE_FEW(T, C, KD)                                                                                                         \
   hipLaunchKernelGGL((attention_generic_few_kernel<T, C>), grid, dim3(256), 0, (hipStream_t)stream, (const T*)q, (const T*)cache,    \
                      block_table, max_blocks, token_seq, positions, (T*)out, nq, nkv, d, dv, page_size, window, chunk, sink, scale,  \
                      softcap, select, min_tokens, vshare, out_f32)
-    TLIE_BY_SIZE(TLIE_FEW)
+    if (sixteens == 1) TLIE_BY_TYPE(TLIE_FEW, 1, 1)
+    else if (sixteens == 2) TLIE_BY_TYPE(TLIE_FEW, 2, 2)
+    else TLIE_BY_TYPE(TLIE_FEW, 4, 4)
 #undef TLIE_FEW
     return launch_status();
   }
@@ -817,6 +801,6 @@ extern "C" int tlie_attention_generic(const void* q, const void* cache, int dtyp
   else
     return kBadArgument;
 #undef TLIE_LAUNCH
-#undef TLIE_BY_SIZE
+#undef TLIE_BY_TYPE
   return launch_status();
 }

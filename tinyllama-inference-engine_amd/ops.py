@@ -293,7 +293,7 @@ def attention_generic(q: torch.Tensor, cache: torch.Tensor, block_table: torch.T
                       window: int | None, scale: float, tiled: bool | int = False, seq_start: torch.Tensor | None = None,
                       min_tokens: int | None = None, value_dim: int | None = None, chunk: int | None = None,
                       sink: torch.Tensor | None = None, value_heads: int | None = None, float_out: bool = False,
-                      softcap: float | None = None) -> torch.Tensor:
+                      softcap: float | None = None, tile_tokens: int | None = None) -> torch.Tensor:
     """Causal attention of every token over its sequence's cached keys; any number of tokens per
     sequence.  block_table: [sequences, max_blocks] pages; token_seq[t]: the token's row of it.
     tiled 1 (True): the step's sequences bring several tokens each (consecutive in the step, at
@@ -335,6 +335,8 @@ def attention_generic(q: torch.Tensor, cache: torch.Tensor, block_table: torch.T
         raise invalid_shape("attention: the number of heads must be a multiple of the number of kv heads")
     tiled = int(tiled)
     min_tokens = generic_tiled_min_tokens(num_heads, num_kv_heads) if min_tokens is None else int(min_tokens)
+    if tile_tokens is None:
+        tile_tokens = generic_tile_tokens(tokens, max(1, block_table.shape[0]), num_heads // num_kv_heads, tiled)
     if tiled == 2:
         _device_tensor(seq_start, "seq_start", torch.int32)
         if seq_start.dim() != 1 or seq_start.shape[0] != block_table.shape[0] + 1 or min_tokens < 1:
@@ -346,7 +348,7 @@ def attention_generic(q: torch.Tensor, cache: torch.Tensor, block_table: torch.T
                                             block_table.shape[1], _ptr(token_seq), _ptr(positions), _ptr(out), tokens,
                                             num_heads, num_kv_heads, head_dim, value_dim, page_size,
                                             int(window) if window else 0, int(chunk) if chunk else 0, _ptr(sink),
-                                            ctypes.c_float(scale), tiled,
+                                            ctypes.c_float(scale), tiled, int(tile_tokens),
                                             _ptr(seq_start if tiled == 2 else None), min_tokens,
                                             num_kv_heads // value_heads, 1 if float_out else 0,
                                             ctypes.c_float(float(softcap) if softcap else 0.0), _compute_units(q.device), _stream()),
@@ -355,25 +357,47 @@ def attention_generic(q: torch.Tensor, cache: torch.Tensor, block_table: torch.T
 
 
 def generic_tiled_min_tokens(heads: int, kv_heads: int) -> int:
-    """A sequence's tokens in a step from which the plain attention may share its reads of the keys among them: half the
-    tokens that a workgroup of 64 columns holds, 8 at least (a workgroup serves the sequences in it one after the other:
-    64 sequences of 4 tokens, 32 heads on 4, 500 keys: 75 us against 47)."""
-    return max(8, 32 // (heads // kv_heads))
+    """A sequence's tokens in a step from which the plain attention may share its reads of the keys among them: 4, and 8 columns
+    of (token, query head of a group) pairs, half of a wave's."""
+    return max(4, 8 // (heads // kv_heads))
 
 
-def attention_generic_plan(ctx, heads: int, kv_heads: int, head_dim: int, value_dim: int | None = None) -> int:
+def generic_tile_tokens(tokens: int, seqs: int, group: int, tiled: int) -> int:
+    """How many tokens a workgroup of the plain attention's sharing form takes: those of one sequence, in equal pieces, so that
+    it has no second sequence's keys to walk (see the kernel's entry), going by the sequences' mean.  A step of both forms mixes
+    single tokens, which it skips, with portions: 16 at least."""
+    full = 64 // min(64, group)
+    mean = -(-tokens // seqs)
+    if tiled == 2:
+        mean = max(mean, 16)
+    if mean <= full:
+        return mean
+    return next((size for size in range(full, full // 2, -1) if mean % size == 0), -(-mean // -(-mean // full)))
+
+
+def attention_generic_plan(ctx, heads: int, kv_heads: int, head_dim: int, value_dim: int | None = None, dtype: torch.dtype = torch.float32,
+                           page_size: int = 16, softcap: float | None = None) -> int:
     """Which form of the plain attention kernel a step takes (the `tiled` of `attention_generic`): the one that shares each
     read of the keys among a sequence's tokens pays where its workgroups fill the chip.  A chunk of keys takes a
-    workgroup of it some 4 us however few they are; the form of a workgroup a token and key head (a token and query head,
-    without groups) takes as long as it has work.  Measured on an MI355X, the two meet at some 256 tokens of 4 key heads of
-    64 (4 x 64 tokens behind 1500: 114 us against 110, 1 x 400 199 against 130, 16 x 8 68 against 107), at more than 1600 of one
-    key head of 32, some 2500 of two of 16, and, without groups, at some 64 of 32 heads of 64 (4 x 64: 40 against 21).
+    workgroup of it some 4 us however few they are; the others take as long as they have work.  Measured on an MI355X over 1 to
+    64 sequences of 1 to 300 tokens behind 0, 200 and 1500 positions and 23 kinds of heads:
+    Where the form of a workgroup a token and key head exists (groups; sizes that the kernels know, see the kernel's entry),
+    the two meet at some 2^16 dims of key heads (tokens x key heads x head size; behind 200, 32 heads of 64 on 4: 100 tokens 21 us and
+    29, 4 x 60 32 and 29, 300 50 and 43).  Else, against a workgroup a token and query head, at 2^17 dims of query heads, in
+    bfloat16, whose keys that form reads singly, at 2^15; a head counts as 24 dims at least (behind 200, 32 heads of 64: 60
+    tokens 32 us and 38, 100 52 and 36).
     A launched step is decided from its host arrays; a recorded step of portions, whose cut changes from replay to replay,
     launches both and lets each sequence's token count on the device decide."""
-    widest = max(head_dim, value_dim or head_dim)
+    value_dim = value_dim or head_dim
+    widest = max(head_dim, value_dim)
     least = generic_tiled_min_tokens(heads, kv_heads)
-    work = ctx.num_tokens * (kv_heads if heads > kv_heads else (heads + 1) // 2) * widest
-    if widest > 64 or ctx.max_new < least or work < 1 << 16:
+    if widest > 64 or ctx.max_new < least:
+        return 0
+    if heads > kv_heads and head_dim == value_dim and head_dim in (16, 32, 64) and page_size >= 16 and page_size & (page_size - 1) == 0 and not softcap:
+        enough = ctx.num_tokens * kv_heads * widest >= 1 << 16
+    else:
+        enough = ctx.num_tokens * heads * max(widest, 24) >= (1 << 15 if dtype == torch.bfloat16 else 1 << 17)
+    if not enough:
         return 0
     if ctx.tile_owner is not None:
         return 2

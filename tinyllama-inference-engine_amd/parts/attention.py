@@ -262,10 +262,10 @@ class Attention(Mixer):
                                           self.window, self.scale, nsplit, split_len, col_tiles, waves, shared,
                                           chunk=self.chunk, sink=self.sink, softcap=self.softcap, order=ctx.seq_order)
         else:
+            tiled = ops.attention_generic_plan(ctx, self.nq, self.nkv, self.d, self.dv, self.dtype, binding.cache.shape[-1] // self.d, self.softcap)
             attended = ops.attention_generic(q, binding.cache, pages.block_table, ctx.token_seq, ctx.positions, self.nq, self.nkv,
-                                             self.d, self.window, self.scale, tiled=ops.attention_generic_plan(ctx, self.nq, self.nkv, self.d, self.dv),
-                                             seq_start=ctx.seq_start, value_dim=self.dv, chunk=self.chunk, sink=self.sink,
-                                             softcap=self.softcap)
+                                             self.d, self.window, self.scale, tiled=tiled, seq_start=ctx.seq_start, value_dim=self.dv,
+                                             chunk=self.chunk, sink=self.sink, softcap=self.softcap)
         if self.head_gate:
             attended = ops.head_gate(attended, fused, fused.cols - self.gate_cols, self.nq)
         return self.o(attended)
@@ -298,9 +298,9 @@ class Attention(Mixer):
             attended = ops.attention_mfma(q, binding.cache, pages.block_table, tiles, ctx.positions, self.nq, self.nkv,
                                           self.d, self.window, self.scale, nsplit, split_len, col_tiles, waves, shared, order=ctx.seq_order)
         else:
+            tiled = ops.attention_generic_plan(ctx, self.nq, self.nkv, self.d, dtype=self.dtype, page_size=page_size)
             attended = ops.attention_generic(q, binding.cache, pages.block_table, ctx.token_seq, ctx.positions, self.nq,
-                                             self.nkv, self.d, self.window, self.scale,
-                                             tiled=ops.attention_generic_plan(ctx, self.nq, self.nkv, self.d), seq_start=ctx.seq_start)
+                                             self.nkv, self.d, self.window, self.scale, tiled=tiled, seq_start=ctx.seq_start)
         if self.head_gate:
             attended = ops.head_gate(attended, gates, gates.cols - self.gate_cols, self.nq)
         return self.o(attended, into=into)

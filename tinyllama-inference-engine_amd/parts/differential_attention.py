@@ -147,7 +147,7 @@ class DifferentialAttention(Mixer):
                                           planes=(parts, 2 * parts, parts), float_out=True, order=ctx.seq_order)
         else:
             attended = ops.attention_generic(q, binding.cache, pages.block_table, ctx.token_seq, ctx.positions, heads, key_heads,
-                                             self.d, None, self.scale, tiled=ops.attention_generic_plan(ctx, heads, key_heads, self.d, self.dv),
+                                             self.d, None, self.scale, tiled=ops.attention_generic_plan(ctx, heads, key_heads, self.d, self.dv, self.dtype),
                                              seq_start=ctx.seq_start, value_dim=self.dv, value_heads=self.groups, float_out=True)
         combined = ops.head_combine(attended, self.heads, self.dv, self.eps, self.dtype, pair_group=self.per_group,
                                     pair_lambda=self.pair_lambda, mult=1.0 - self.diff,

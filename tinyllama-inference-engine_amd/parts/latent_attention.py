@@ -158,7 +158,7 @@ class LatentAttention(Mixer):
                                           self.window, self.scale, nsplit, split_len, col_tiles, waves, shared, sink=self.sink, order=ctx.seq_order)
         else:
             attended = ops.attention_generic(q, binding.cache, pages.block_table, ctx.token_seq, ctx.positions, self.heads, self.heads,
-                                             self.plain, self.window, self.scale, tiled=ops.attention_generic_plan(ctx, self.heads, self.heads, self.plain, self.dv),
+                                             self.plain, self.window, self.scale, tiled=ops.attention_generic_plan(ctx, self.heads, self.heads, self.plain, self.dv, self.dtype),
                                              seq_start=ctx.seq_start, value_dim=self.dv, sink=self.sink)
         if self.output_gate:
             ops.sigmoid_gate(attended, fused, fused.cols - self.heads * self.dv)
@@ -184,7 +184,7 @@ class LatentAttention(Mixer):
                                           self.window, self.scale, nsplit, split_len, col_tiles, waves, shared, sink=self.sink, order=ctx.seq_order)
         else:
             attended = ops.attention_generic(q_wide, binding.cache, pages.block_table, ctx.token_seq, ctx.positions, self.heads, 1,
-                                             key, self.window, self.scale, tiled=ops.attention_generic_plan(ctx, self.heads, 1, key, value_dim),
+                                             key, self.window, self.scale, tiled=ops.attention_generic_plan(ctx, self.heads, 1, key, value_dim, self.dtype),
                                              seq_start=ctx.seq_start, value_dim=value_dim, sink=self.sink)
         # (of every head's attended vector the first rank dims: with wide values the rest are zeros)
         values = torch.empty((tokens, self.heads * self.dv), dtype=self.dtype, device=attended.device)
