@@ -209,6 +209,29 @@ def test_gemm_generic_at_the_edges_of_its_kernels_and_gated(n, k):
             ops.gemm_generic(x, w, b, torch.float32, gated=True)
 
 
+@pytest.mark.parametrize("n, k", [(11262, 1030), (11262, 1028), (4610, 517)])
+def test_gemm_generic_in_tiles_of_64_by_64(n, k):
+    """The largest tiles, which the launch takes where several of them come to every compute unit (256 of these): ragged rows, columns
+    and blocks of K, no 16-byte loads, bias and gate.  The same bits as the same rows in smaller tiles or alone."""
+    from tlie_amd import ops
+    rows = 1025 if n < 8000 else 577
+    units = torch.cuda.get_device_properties(0).multi_processor_count
+    cost = {64: 28.6 / 0.75, 32: 14.3 / 0.69}                    # (a tile's time on its unit, as the launch reckons)
+    tiles = {columns: -(-n // 64) * -(-rows // columns) for columns in cost}
+    assert all(count > 2 * units for count in tiles.values()) and cost[64] * -(-tiles[64] // units) < cost[32] * -(-tiles[32] // units)
+    torch.manual_seed(n + k)
+    x = torch.randn(rows, k, device=DEV)
+    w = torch.randn(n, k, device=DEV) / math.sqrt(k)
+    b = torch.randn(n, device=DEV)
+    many = ops.gemm_generic(x, w, b, torch.float32)
+    assert rel_err(many.dense(), x.double() @ w.double().T + b.double()) < 5e-6
+    for first, count in ((0, 7), (rows - 40, 40), (100, 129)):
+        few = ops.gemm_generic(x[first:first + count].contiguous(), w, b, torch.float32)
+        assert torch.equal(few.dense(), many.dense()[first:first + count])
+    gated = ops.gemm_generic(x, w, b, torch.float32, gated=True)
+    assert rel_err(gated, ops.silu_mul(many, torch.float32, interleaved=True)) < 1e-6
+
+
 @pytest.mark.parametrize("n, k, gated", [(18, 32768, False), (18, 32776, True), (20, 33795, False), (16, 70000, True)])
 def test_gemm_generic_of_more_blocks_than_fit_at_once(n, k, gated):
     """At most 16 rows and K from 64 blocks of 512 on: the blocks' sums are added up in passes.  The same bits as among many rows."""
