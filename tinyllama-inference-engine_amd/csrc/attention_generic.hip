@@ -197,22 +197,6 @@ attention_generic_kernel(const T* __restrict__ q, const T* __restrict__ cache, c
 // take whichever is faster.
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ void swap32(float& a, float& b) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-  a = __uint_as_float(r[0]), b = __uint_as_float(r[1]);
-}
-__device__ __forceinline__ void swap16(float& a, float& b) {
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-  a = __uint_as_float(r[0]), b = __uint_as_float(r[1]);
-}
-// A lane of the quarter g (lanes 16 g ..) holds the values 4 g .. 4 g + 3 of sixteen; afterwards it holds g, 4 + g, 8 + g,
-// 12 + g: what it gives to four instructions of four k each, so that these take the k in their order.
-__device__ __forceinline__ void to_quarters(float (&v)[4]) {
-  swap32(v[0], v[2]);
-  swap32(v[1], v[3]);
-  swap16(v[0], v[1]);
-  swap16(v[2], v[3]);
-}
 // The sum and the maximum with the lane 32 (then 16) away: for keys, with the key whose bit 3 (then bit 2) differs.
 __device__ __forceinline__ float sum_quarters(float v) {
   float a = v, b = v;
@@ -294,8 +278,7 @@ __device__ __forceinline__ void take_scores(floatx4 (&dot)[4], ColumnState<KD>& 
 // next stored behind a barrier, before a chunk's products.  Rows lie in LDS 16 dims (keys) at a time as 0 4 8 12 1 5 ..: one
 // 16-byte read gives a lane what four instructions take from it; 68 floats apart, sixteen rows' reads cover the banks once.
 // Later tokens see more keys: workgroups are taken from the step's end, in rounds of one for each compute unit, every second
-// round backwards, so that the two that share a unit add up to the same length (in an earlier form of this kernel 103 us against 146
-// for a prompt of 1000 tokens).
+// round backwards, so that the two that share a unit add up to the same length.
 // 32 heads of 64 on 4, beside the form of plain multiply-adds before: a prompt of 1000 tokens 75 us against 493, of 2048 237 (73
 // TFLOP/s) against 1756; without groups 84 against 942.
 // Tokens of a workgroup that belong to different sequences are served one run of equal sequences after the other.

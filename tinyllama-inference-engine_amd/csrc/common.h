@@ -101,6 +101,26 @@ __device__ __forceinline__ void settle(V (&v)[N][M]) {
   for (int i = 0; i < N * M; ++i) asm volatile("" : "+v"(v[i / M][i % M]));
 }
 
+// a's lanes 32 .. 63 with b's 0 .. 31; a's odd sixteens of lanes with b's even ones.
+__device__ __forceinline__ void swap32(float& a, float& b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  a = __uint_as_float(r[0]), b = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ void swap16(float& a, float& b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  a = __uint_as_float(r[0]), b = __uint_as_float(r[1]);
+}
+// A lane of the quarter g (lanes 16 g ..) holds the values 4 g .. 4 g + 3 of sixteen; afterwards it holds g, 4 + g, 8 + g,
+// 12 + g: what it gives to four matrix instructions of four k each, so that these take the k in their order.
+__device__ __forceinline__ void to_quarters(float& a, float& b, float& c, float& d) {
+  swap32(a, c);
+  swap32(b, d);
+  swap16(a, b);
+  swap16(c, d);
+}
+__device__ __forceinline__ void to_quarters(float (&v)[4]) { to_quarters(v[0], v[1], v[2], v[3]); }
+__device__ __forceinline__ void to_quarters(float4& v) { to_quarters(v.x, v.y, v.z, v.w); }
+
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
   for (int offset = kWave / 2; offset > 0; offset >>= 1) v += __shfl_xor(v, offset, kWave);

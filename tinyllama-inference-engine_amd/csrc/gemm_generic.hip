@@ -42,23 +42,6 @@ __device__ __forceinline__ float4 inside(float4 v, int k, int K) {
   return make_float4(k < K ? v.x : 0.f, k + 1 < K ? v.y : 0.f, k + 2 < K ? v.z : 0.f, k + 3 < K ? v.w : 0.f);
 }
 
-__device__ __forceinline__ void swap32(float& a, float& b) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-  a = __uint_as_float(r[0]), b = __uint_as_float(r[1]);
-}
-__device__ __forceinline__ void swap16(float& a, float& b) {
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
-  a = __uint_as_float(r[0]), b = __uint_as_float(r[1]);
-}
-// A lane of the quarter g (lanes 16 g ..) holds the values 4 g .. 4 g + 3 of sixteen; afterwards it holds g, 4 + g, 8 + g,
-// 12 + g: what it gives to four matrix instructions of four k each, so that these take the k in their order.
-__device__ __forceinline__ void to_quarters(float4& v) {
-  swap32(v.x, v.z);
-  swap32(v.y, v.w);
-  swap16(v.x, v.y);
-  swap16(v.z, v.w);
-}
-
 // ---- few rows of x (decoding, short portions) ------------------------------------------------------------
 // Bound by reading W.  A workgroup owns R rows of W (columns of y) and all M <= 16 MT rows of x; its waves take the blocks
 // of K in turn, each block one chain of matrix instructions whose operands go straight from memory into registers: a
