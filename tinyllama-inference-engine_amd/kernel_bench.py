@@ -198,7 +198,8 @@ def bench_kernels(cfg: dict, batch: int = 8, context: int = 2048, prompt: int = 
             positions_p = torch.arange(prompt, dtype=torch.int32, device=device)
             qkv = ops.Product(rand(prompt, (nq + 2 * nkv) * d, scale=1.0), 1)
             rows.append(_row(f"{label}: rotation + cache write",
-                             _timed(lambda i: ops.rope_cache(qkv, positions_p, positions_p, inv_freq, d, cache_p, nq, nkv, d, bf, paired=True),
+                             _timed(lambda i: ops.rope_cache(qkv, positions_p, positions_p, inv_freq, d, cache_p, nq, nkv, d, bf, paired=True,
+                                                      runs=True),
                                     4, samples), read_bytes=prompt * (nq + 2 * nkv) * d * 4))
     return rows
 
@@ -260,8 +261,9 @@ def bench_design_kernels(sizes: dict, batch: int = 8, context: int = 2048, promp
         cache = rand(seqs * blocks, 2, nkv, page_size * d, scale=0.5)
         q = rand(tokens, nq * d, scale=1.0)
         sink = rand(nq, scale=1.0, dtype=f32)
-        tiles, col_tiles, nsplit, split_len, waves, shared = ops.attention_plan(ctx, nq // nkv, nkv, d)
         for name, extra, keys in (("attention, causal (Llama's)", {}, length), (f"attention, sink + chunks of {chunk}", {"chunk": chunk, "sink": sink}, seen)):
+            ctx.scratch = {}
+            tiles, col_tiles, nsplit, split_len, waves, shared = ops.attention_plan(ctx, nq // nkv, nkv, d, extra.get("chunk"), bool(extra))
             launch = lambda i: ops.attention_mfma(q, cache, table, tiles, positions, nq, nkv, d, None, d ** -0.5, nsplit, split_len,
                                                   col_tiles, waves, shared, **extra)
             if decode:
@@ -286,7 +288,7 @@ def bench_design_kernels(sizes: dict, batch: int = 8, context: int = 2048, promp
         row(f"{label}: heads' queries onto the latent space [{lh} x {ldim} x {rank}]", _timed(launch, 4, samples),
             **({"read_bytes": lh * ldim * rank * 2 + tokens * lh * (ldim + rank) * 2} if decode else {"flops": 2.0 * tokens * lh * ldim * rank}))
         latent_sink = rand(lh, scale=1.0, dtype=f32)
-        ltiles, lcol_tiles, lnsplit, lsplit_len, lwaves, lshared = ops.attention_plan(ctx, lh, 1, key)
+        ltiles, lcol_tiles, lnsplit, lsplit_len, lwaves, lshared = ops.attention_plan(ctx, lh, 1, key, extra=True)
         launch = lambda i: ops.attention_mfma(q_wide, latent_cache, table, ltiles, positions, lh, 1, key, None, 0.1, lnsplit, lsplit_len,
                                               lcol_tiles, lwaves, lshared, sink=latent_sink)
         if decode:
@@ -336,7 +338,7 @@ def bench_design_kernels(sizes: dict, batch: int = 8, context: int = 2048, promp
         qkv = ops.Product(rand(tokens, (nq + 2 * nkv) * d, scale=1.0), 1)
         rot_freq = torch.pow(torch.tensor(10000.0), -2.0 * torch.arange(d // 2, dtype=f32) / d).to(device)
         row(f"{label}: rotation + cache write (Llama's)",
-            _timed(lambda i: ops.rope_cache(qkv, positions, slot_map, rot_freq, d, cache, nq, nkv, d, bf, paired=True), 4, samples),
+            _timed(lambda i: ops.rope_cache(qkv, positions, slot_map, rot_freq, d, cache, nq, nkv, d, bf, paired=True, runs=not decode), 4, samples),
             read_bytes=tokens * (nq + 2 * nkv) * d * 4)
         row(f"{label}: placement of q, k, v (no rotation)",
             _timed(lambda i: ops.qkv_place(qkv, positions, slot_map, None, 0, cache, nq, nkv, d, d, bf), 4, samples),
@@ -410,7 +412,7 @@ def bench_raketar_kernels(sizes: dict, batch: int = 8, context: int = 2048, prom
         ctx.scratch = {}
         cache2 = rand(seqs * blocks, G, page_size * (2 * d + dv), scale=0.5)
         q2 = rand(tokens, 2 * H * d, scale=1.0)
-        tiles, col_tiles, nsplit, split_len, waves, shared = ops.attention_plan(ctx, H // G, 2 * G * parts, d)
+        tiles, col_tiles, nsplit, split_len, waves, shared = ops.attention_plan(ctx, H // G, 2 * G * parts, d, extra=True)
         times = _timed(lambda i: ops.attention_mfma(q2, cache2, table, tiles, positions, 2 * H * parts, 2 * G * parts, d, None, d ** -0.5,
                                                     nsplit, split_len, col_tiles, waves, shared, planes=(parts, 2 * parts, parts),
                                                     float_out=True), 8, samples)
@@ -427,7 +429,8 @@ def bench_raketar_kernels(sizes: dict, batch: int = 8, context: int = 2048, prom
                                                bf, value_heads=G, extra_cols=H * dv), 8, samples)
         row(f"{label}: placement of q, k, v (shared value heads)", times, tokens * (2 * H * d * 2 + 2 * G * d + G * dv) * 2 * 2)
         qkv = ops.Product(rand(tokens, (lq + 2 * lkv) * d, scale=1.0), 1)
-        times = _timed(lambda i: ops.rope_cache(qkv, positions, slot_map, torch.ones(d // 2, device=device), d, cache, lq, lkv, d, bf), 8, samples)
+        times = _timed(lambda i: ops.rope_cache(qkv, positions, slot_map, torch.ones(d // 2, device=device), d, cache, lq, lkv, d, bf,
+                                                 runs=not decode), 8, samples)
         row(f"{label}: rotation + cache write (Llama's)", times, tokens * (lq * 2 + 2 * lkv) * d * 2 * 2)
         # ---- the matrix memory -------------------------------------------------------------------------------------
         memory_in = ops.Product(rand(tokens, 2 * mh * md + 2 * mh * mv, scale=1.0), 1)
@@ -546,7 +549,7 @@ def bench_narolorn_kernels(sizes: dict, batch: int = 8, context: int = 2048, pro
         cache_bytes, flops = seqs * length * G * 2 * d * 2, 4.0 * tokens * H * d * keys_seen
         for name, options in (("causal (Llama's)", {}), ("capped scores", {"softcap": sizes["softcap"]}), (f"chunks of {sizes['chunk']}", {"chunk": sizes["chunk"]})):
             ctx.scratch = {}
-            tiles, col_tiles, nsplit, split_len, waves, shared = ops.attention_plan(ctx, H // G, G, d)
+            tiles, col_tiles, nsplit, split_len, waves, shared = ops.attention_plan(ctx, H // G, G, d, options.get("chunk"), bool(options))
             times = _timed(lambda i: ops.attention_mfma(q, cache, table, tiles, positions, H, G, d, None, d ** -0.5, nsplit, split_len,
                                                         col_tiles, waves, shared, **options), 8, samples)
             seen = min(keys_seen, sizes["chunk"] if decode else sizes["chunk"] / 2) if "chunk" in options else keys_seen
@@ -556,7 +559,7 @@ def bench_narolorn_kernels(sizes: dict, batch: int = 8, context: int = 2048, pro
         latent_cache = rand(seqs * blocks, 2, 1, page_size * key, scale=0.5)
         q_wide = rand(tokens, lh * key, scale=1.0)
         ctx.scratch = {}
-        tiles, col_tiles, nsplit, split_len, waves, shared = ops.attention_plan(ctx, lh, 1, key)
+        tiles, col_tiles, nsplit, split_len, waves, shared = ops.attention_plan(ctx, lh, 1, key, sizes["window"])
         times = _timed(lambda i: ops.attention_mfma(q_wide, latent_cache, table, tiles, positions, lh, 1, key, sizes["window"], ld ** -0.5,
                                                     nsplit, split_len, col_tiles, waves, shared), 8, samples)
         seen = min(keys_seen, sizes["window"])
@@ -565,7 +568,7 @@ def bench_narolorn_kernels(sizes: dict, batch: int = 8, context: int = 2048, pro
         # ---- placement ---------------------------------------------------------------------------------------------------
         inv_freq = torch.ones(d // 2, device=device)
         qkv = ops.Product(rand(tokens, (H + 2 * G) * d, scale=1.0), 1)
-        times = _timed(lambda i: ops.rope_cache(qkv, positions, slot_map, inv_freq, d, cache, H, G, d, bf), 8, samples)
+        times = _timed(lambda i: ops.rope_cache(qkv, positions, slot_map, inv_freq, d, cache, H, G, d, bf, runs=not decode), 8, samples)
         row(f"{label}: rotation + cache write (Llama's)", times, tokens * (H * 2 + 2 * G) * d * 2 * 2)
         times = _timed(lambda i: ops.qkv_place(qkv, positions, slot_map, None, 0, cache, H, G, d, d, bf, q_temp=(0.1, 512.0)), 8, samples)
         row(f"{label}: placement of q, k, v with a query temperature", times, tokens * (H * 2 + 2 * G) * d * 2 * 2)
@@ -814,12 +817,13 @@ def bench_paluzen_kernels(sizes: dict, batch: int = 8, context: int = 2048, prom
             row(f"{label}: attention, {name}, {H} heads of {d} on {G}", times, seqs * seen * 2 * G * d * 2 if decode else 0, flops)
         qkv = ops.Product(rand(tokens, (H + 2 * G) * d, scale=1.0), 1)
         inv_freq = torch.ones(d // 2, device=device)
-        times = _timed(lambda i: ops.rope_cache(qkv, positions, slot_map, inv_freq, d, cache, H, G, d, bf, paired=True), 8, samples)
+        times = _timed(lambda i: ops.rope_cache(qkv, positions, slot_map, inv_freq, d, cache, H, G, d, bf, paired=True, runs=not decode), 8,
+                       samples)
         row(f"{label}: rotation + cache write (Llama's)", times, tokens * (H * 2 + 2 * G) * d * 2 * 2)
         gated = ops.Product(rand(tokens, (H + 2 * G) * d + H, scale=1.0), 1)       # (H is a multiple of 8: no column between)
         temp, part_freq = rand(H, scale=1.0, dtype=f32), torch.ones(d // 4, device=device)
         times = _timed(lambda i: ops.rope_cache(gated, positions, slot_map, part_freq, d // 2, cache, H, G, d, bf, paired=True, extra_cols=H,
-                                                head_scale=temp), 8, samples)
+                                                head_scale=temp, runs=not decode), 8, samples)
         row(f"{label}: rotation + cache write with a number a head, gates' columns beside", times, tokens * (H * 2 + 2 * G) * d * 2 * 2)
         values = rand(tokens, H * d, scale=1.0)
         times = _timed(lambda i: ops.head_gate(values, gated, (H + 2 * G) * d, H), 8, samples)
@@ -998,7 +1002,8 @@ def bench_barilix_kernels(sizes: dict, batch: int = 8, context: int = 2048, prom
         columns = (H + 2 * G) * d
         qkv = ops.Product(rand(tokens, columns, scale=1.0), 1)
         inv_freq = torch.ones(d // 2, device=device)
-        times = _timed(lambda i: ops.rope_cache(qkv, positions, slot_map, inv_freq, d, cache, H, G, d, bf, paired=True), 8, samples)
+        times = _timed(lambda i: ops.rope_cache(qkv, positions, slot_map, inv_freq, d, cache, H, G, d, bf, paired=True, runs=not decode), 8,
+                       samples)
         row(f"{label}: rotation + cache write (Llama's)", times, tokens * columns * 2 * 2)
         held = lambda channels: torch.zeros(seqs, ops.short_conv_state_floats(channels, taps), dtype=f32, device=device)      # noqa: E731
         conv, state, norm_d = rand(columns, taps, scale=0.5), held(columns), rand(d, scale=1.0, dtype=f32)
