@@ -166,7 +166,7 @@ def added_up(parts):
 
 
 @pytest.mark.parametrize("rows, n, k, whole", [(24, 12288, 4096, False), (64, 4096, 11008, False), (64, 2304, 14336, False), (24, 9000, 4096, True),
-                                               (17, 2048, 1536, True)])
+                                               (17, 2048, 1536, True), (20, 11264, 2048, False), (33, 4096, 14336, False)])
 def test_gemm_ring_is_as_exact_as_the_product_it_stands_in_for(rows, n, k, whole):
     """Float sums of exact products: the error against 64 bits (2-norm over some 1e5 results, which varies by less than 1%), of
     either kernel as it is launched for these sizes, parts added up as their consumers do."""

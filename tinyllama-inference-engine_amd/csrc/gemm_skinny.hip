@@ -185,10 +185,10 @@ gemm_skinny_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ 
 //     turns, which ask for nothing, are code of their own: with a condition around the loads the compiler would wait for all);
 //   * workgroup b begins at turn (b / 8) % turns and goes round, so that the workgroups of a die ask for different columns;
 //   * x goes through LDS in two buffers, one barrier a turn that waits for LDS alone.
-// Measured with cold weights (us, the kernel above -> this): gated 11264 x 2048 at 64 rows 20.3 -> 15.0, at 32 16.0 -> 13.6;
-// gated 22016 x 4096 at 24 rows 48.5 -> 36.3; gated 28672 x 4096 at 64 rows 63.8 -> 49.6; 32000 x 2048 at 64 rows 38.1 -> 31.5;
-// 4096 x 11008 at 24 rows 25.7 in 11 parts -> 20.2 in 2.  Without the loads of x the first takes 12.7: W's 46 MB at 6 TB/s and
-// the launch.  Four waves a strip are slower (17.8), as is a ring of 8 (17.0) or 2 (17.3 with four waves).
+// Measured with cold weights (us, the kernel above -> this): gated 11264 x 2048 at 64 rows 20.7 -> 16.2, at 24 16.3 -> 12.8;
+// gated 22016 x 4096 at 24 rows 49.4 -> 35.4; gated 28672 x 4096 at 64 rows 65.2 -> 50.0; 32000 x 2048 at 64 rows 37.9 -> 31.7;
+// 4096 x 11008 at 24 rows 25.5 in 11 parts -> 20.3 in 2.  Of the first, in one chain of sums 15.0: without the loads of x 12.7
+// (W's 46 MB at 6 TB/s and the launch), with four waves a strip 17.8, a ring of 8 17.0, of 2 and four waves 17.3.
 constexpr int kDepth = 4, kHalves = 2;
 
 template <int NT, int S, bool GATED>
@@ -243,9 +243,10 @@ gemm_skinny_ring_kernel(const uint16_t* __restrict__ x, const uint16_t* __restri
       *reinterpret_cast<uint4*>(xs + buffer * kHalves * kTile + x_slot[i]) = v;
     }
   };
-  // Sums of 512 columns and fewer (2 kDepth turns) join a total: one chain over a half's 2048 columns has
-  // half again the error of the kernel above, which cuts K in more parts (against 64 bits, 12288 x 4096 at 24 rows: 1.9e-7 there,
-  // 2.7e-7 in one chain, 1.35e-7 so; 4096 x 11008 at 64 rows 1.4e-7, 2.2e-7, 1.3e-7).  It costs 0 to 2% of the time.
+  // Sums of 256 columns and fewer (kDepth turns) join a total: one chain over a half's 2048 columns has half again the error of
+  // the kernel above, which cuts K in more parts (against 64 bits, 12288 x 4096 at 24 rows: 1.84e-7 there, 2.7e-7 in one chain,
+  // 1.35e-7 in sums of 512, 1.07e-7 so; 11264 x 2048 at 20 rows, four parts there, 1.25e-7, 1.31e-7 in sums of 512, 0.98e-7 so).
+  // It costs 0 to 3% of the time.
   floatx4 acc[NT], total[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) acc[t] = total[t] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -280,7 +281,7 @@ gemm_skinny_ring_kernel(const uint16_t* __restrict__ x, const uint16_t* __restri
   for (; n + 2 * kDepth - 1 < turns; n += kDepth) {
 #pragma unroll
     for (int u = 0; u < kDepth; ++u) turn(n + u, u, true, true);
-    if (n & kDepth) join();
+    join();
   }
 #pragma unroll
   for (int u = 0; u < 2 * kDepth - 1; ++u) {
