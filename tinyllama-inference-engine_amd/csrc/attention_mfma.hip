@@ -26,9 +26,9 @@
 //    among the waves of a workgroup (up to 16): wave w takes the blocks w, w + W, ... and the
 //    waves' results are merged through LDS, so the kernel still writes final results.  Then, for
 //    long contexts, among nsplit workgroups of split_len positions each, which write unnormalised
-//    partial results with their maxima and sums for a second kernel to merge.  The parts are fixed ranges of positions, so a wave can fetch its first keys
-//    before it knows how long the sequence is: the position, the block table and the keys are not
-//    three loads in a row.
+//    partial results with their maxima and sums for a second kernel to merge.  The parts are fixed
+//    ranges of positions, so a wave can fetch its first keys before it knows how long the sequence
+//    is: the position, the block table and the keys are not three loads in a row.
 #include "common.h"
 #include "no_alloc.h"
 
@@ -151,9 +151,10 @@ attention_mfma_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict
       // A decode step of more workgroups than compute units, and of sequences of their own lengths: the workgroups of one
       // unit lie a round apart, and where a round is a multiple of the tokens they would all be the same sequence's, so that
       // the kernel took as long as the longest sequence on every place (64 sequences of 50 to 1500 positions, 32 heads of 128 on
-      // 8: 51.5 us, in this order 43.5; 16 of them on 32 key heads 53.2, 41.5; of equal lengths the list costs 0.3 us).  The sequences are taken longest first, as `order` lists
-      // them, and the rounds forwards and backwards in turn like a prompt's tiles.  (Ranked by every wave from the positions
-      // instead, the keys wait for that: 64 sequences of 60 positions, 32 heads of 128 on 8, 10.1 us against 7.1.)
+      // 8: 51.5 us, in this order 43.5; 16 of them on 32 key heads 53.2, 41.5; of equal lengths the list costs 0.3 us).  The
+      // sequences are taken longest first, as `order` lists them, and the rounds forwards and backwards in turn like a prompt's
+      // tiles.  (Ranked by every wave from the positions instead, the keys wait for that: 64 sequences of 60 positions, 32
+      // heads of 128 on 8, 10.1 us against 7.1.)
       const int linear = blockIdx.y * gridDim.x + blockIdx.x, round = linear / round_size, place = linear - round * round_size;
       const int in_round = min(round_size, total - round * round_size);
       const int item = round * round_size + ((round & 1) ? in_round - 1 - place : place);

@@ -8,7 +8,9 @@ Which kernel runs is decided here and nowhere else:
   bfloat16, at most 16 rows      the rows kernel when the caller folds something in: the norm before the
                                  product, the SiLU gate or the add into the residual after it
   bfloat16, at most 64 rows      the skinny MFMA kernel (W streamed once, split-K partial sums; the gated
-                                 feed-forward's first product keeps K whole and applies the SiLU gate itself)
+                                 feed-forward's first product keeps K whole and applies the SiLU gate itself), with W in a
+                                 ring of registers where the matrix is large, or gated and of more than 16 rows
+                                 (`ops.ring_fits`)
   bfloat16, more rows            the library's product (as the reference uses a library for its
                                  products: cublasGemmEx, src/cuda/kernels.cu:342-368), bfloat16 out, or
                                  float32 for the output head: hipBLASLt called directly
