@@ -80,6 +80,7 @@ def test_the_variant_with_sinks_and_caps_takes_columns_that_fit_its_registers(to
     (16, 8, 32, 64, 6000, None, False, (1, 8, True)), (16, 8, 32, 256, 3000, None, True, (1, 2, True)), (32, 2, 16, 64, 6000, None, False, (1, 4, True)),
     # One and a half workgroups a unit of 96 dims are served by 16 columns a wave
     (24, 8, 96, 2048, 0, None, False, (1, 1, True)), (24, 8, 96, 2048, 0, None, True, (1, 1, True)),
+    (24, 8, 96, 2048, 6000, None, True, (2, 1, True)), (32, 8, 80, 1536, 3000, None, True, (2, 1, True)), (24, 8, 96, 2048, 6000, None, False, (1, 1, True)),
     # Few tiles of their own keys: not cut
     (24, 8, 96, 256, 600, None, False, (2, 1, False)), (16, 2, 128, 64, 6000, None, False, (1, 8, True)),
 ])

@@ -2301,14 +2301,15 @@ def attention_plan(ctx, groups_per_kv: int, num_kv_heads: int, head_dim: int, re
                 # 89, behind 2000: 156 against 218, within a window of 1024: 63 to 70 against 74 to 90; of 80 behind 2000: 125
                 # against 174, but behind 0: 67 against 65), from one and a half where heads and contexts are large (1536 tokens
                 # of 128 behind 2000: 135 against 168, behind 0: 64 against 55; 24 heads of 96 on 8, 2048 behind 0: 70 against
-                # 58, behind 6000: 266 against 262).
+                # 58, behind 6000: 266 against 262) or the kernel is the variant (of 96 with a sink, 2048 behind 1600: 131
+                # against 144, behind 6000: 296 against 350; of 80 with capped scores behind 3000: 219 against 231).
                 # Fewer are filled up to two a unit by cutting the keys, where these are many: 1024 tokens of 128 behind 5000
                 # 171 us in two parts against 196 with 16 columns (behind 1000 81 against 64); 512 behind 1500 52 in four parts
                 # against 61, behind 7000 116 against 200, with a sink in four parts of 16 columns 157 against 206.
                 few = blocks <= (3 * units - 1) // 2 and not bounded
                 if blocks >= 2 * units and not narrow and (head_dim > 96 or bounded or ctx.max_context >= 3072):
                     col_tiles = 2
-                elif 2 * blocks >= 3 * units and head_dim > 96 and not narrow and not bounded and ctx.max_context >= 3072:
+                elif 2 * blocks >= 3 * units and (head_dim > 96 or extra) and not narrow and not bounded and ctx.max_context >= 3072:
                     col_tiles = 2
                 elif few and not narrow and ctx.max_context >= (4096 if 2 * blocks > units else 1536):
                     parts = min(4, (2 * units + blocks - 1) // blocks)
