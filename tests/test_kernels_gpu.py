@@ -209,6 +209,69 @@ def test_gemm_generic_at_the_edges_of_its_kernels_and_gated(n, k):
             ops.gemm_generic(x, w, b, torch.float32, gated=True)
 
 
+@pytest.mark.parametrize("rows", [1, 7, 8, 9, 16])
+@pytest.mark.parametrize("k, n, heads", [(32, 96, (3, 1, 10, 4)), (96, 256, (3, 1, 32, 32)), (256, 64, (2, 2, 16, 16)), (288, 2048, (4, 2, 6, 0)),
+                                         (512, 544, (2, 1, 66, 64)), (544, 2080, (32, 4, 64, 64)), (2048, 2048, (24, 4, 80, 40)),
+                                         (8224, 64, (1, 1, 16, 16))])
+def test_gemm_generic_rows_gives_the_bits_of_the_kernels_it_stands_in_for(rows, k, n, heads):
+    """At most 16 rows in 32 bits with the norm before and the gate, the add or the rotation and cache write after: one part of the ring
+    and more, one block of K, two at once, more blocks than waves, shares of rows (2560 and 2080 columns), heads that no
+    group of four columns divides; against the norm, the product and the rotation as kernels of their own, bit for bit."""
+    from tlie_amd import ops
+    torch.manual_seed(rows * n + k)
+    f32 = torch.float32
+
+    def matrix(outs, ins):
+        return torch.randn(outs, ins, device=DEV) / math.sqrt(ins)
+    table, weight, next_weight, bias = torch.randn(20, k, device=DEV), torch.randn(k, device=DEV), torch.randn(n, device=DEV), torch.randn(n, device=DEV)
+    w, after = matrix(n, k), matrix(72, n)
+    tokens = torch.randperm(20, device=DEV)[:rows].to(torch.int32)
+    residual, lazy = ops.embed_rows(tokens, table, (weight, 1e-5), f32)
+    assert torch.equal(residual, table[tokens.long()])
+    normed = ops.add_rmsnorm(residual.clone(), None, weight, 1e-5, f32)
+    want = ops.gemm_generic(normed, w, bias, f32)
+    assert rel_err(want.dense(), plain_linear(plain_rms_norm(residual.double().cpu(), weight.double().cpu(), 1e-5), w.double().cpu(), bias.double().cpu())) < 5e-6
+    for x in (lazy, normed):
+        assert torch.equal(ops.gemm_generic_rows(x, w, bias).dense(), want.dense())
+        for gate in (None, ("clamped_swish", 1.7, 0.8)):
+            assert torch.equal(ops.gemm_generic_rows(x, w, bias, "gate", gate=gate), ops.gemm_generic(normed, w, bias, f32, gated=True, gate=gate))
+    start = torch.randn(rows, n, device=DEV)
+    sums, plain = start.clone(), start.clone()
+    left = ops.gemm_generic_rows(lazy, w, bias, "residual", residual=sums, next_norm=(next_weight, 1e-6))
+    next_normed = ops.add_rmsnorm(plain, want, next_weight, 1e-6, f32)
+    assert torch.equal(sums, plain)
+    assert torch.equal(ops.gemm_generic_rows(left.normed, after, None).dense(), ops.gemm_generic(next_normed, after, None, f32).dense())
+    sums = start.clone()
+    assert ops.gemm_generic_rows(normed, w, bias, "residual", residual=sums).normed is None and torch.equal(sums, plain)
+    nq, nkv, d, rot = heads
+    columns = (nq + 2 * nkv) * d
+    w, bias = matrix(columns, k), torch.randn(columns, device=DEV)
+    positions = torch.randint(0, 3000, (rows,), device=DEV, dtype=torch.int32)
+    slots = torch.randperm(3 * 8, device=DEV)[:rows].to(torch.int32)
+    slots[rows // 2] = -1
+    inv_freq = (10000.0 ** (-torch.arange(0, rot, 2, device=DEV) / max(rot, 1))).float() if rot else None
+    caches = [torch.zeros(3, 2, nkv, 8 * d, device=DEV) for _ in range(2)]
+    got = ops.gemm_generic_rows(lazy, w, bias, "rope", rope=ops.RopeTarget(positions, slots, inv_freq, rot, caches[0], nq, nkv, d))
+    want = ops.rope_cache(ops.gemm_generic(normed, w, bias, f32), positions, slots, inv_freq, rot, caches[1], nq, nkv, d, f32, paired=rot > 0)
+    assert torch.equal(got, want) and torch.equal(caches[0], caches[1])
+
+
+def test_gemm_generic_rows_refuses_what_it_does_not_take():
+    from tlie_amd import ops
+    w, x = torch.randn(24, 16, device=DEV), torch.randn(17, 16, device=DEV)
+    with pytest.raises(Exception):
+        ops.gemm_generic_rows(x, w, None)                                                           # 17 rows
+    with pytest.raises(Exception):
+        ops.gemm_generic_rows(x[:4, :14].contiguous(), w[:, :14].contiguous(), None)                # no 16-byte rows
+    with pytest.raises(Exception):
+        ops.gemm_generic_rows(x[:4], w, None, "residual", residual=torch.zeros(5, 24, device=DEV))
+    with pytest.raises(Exception):
+        ops.gemm_generic_rows(ops.NormedRows(x[:4], torch.zeros(4, 3, device=DEV), 1e-5), w, None)  # sums of squares of another width
+    narrow = torch.randn(24, device=DEV)
+    assert ops.gemm_generic_rows(x[:4], w, None, "residual", residual=torch.zeros(4, 24, device=DEV),
+                                 next_norm=(narrow, 1e-5)).normed is None                           # 24 columns: no 32
+
+
 @pytest.mark.parametrize("n, k", [(11262, 1030), (11262, 1028), (4610, 517)])
 def test_gemm_generic_in_tiles_of_64_by_64(n, k):
     """The largest tiles, which the launch takes where several of them come to every compute unit (256 of these): ragged rows, columns

@@ -175,6 +175,12 @@ __device__ __forceinline__ float sum_splits(const D* __restrict__ first, int nsp
   return (a + b) + (c + d);
 }
 
+// The sum of squares of four, or eight, neighbouring columns of the 32-bit path's norms: one order for every kernel that forms it.
+__device__ __forceinline__ float squares_of4(float a, float b, float c, float d) { return fmaf(d, d, fmaf(c, c, fmaf(b, b, a * a))); }
+__device__ __forceinline__ float squares_of8(const float (&v)[8]) {
+  return squares_of4(v[0], v[1], v[2], v[3]) + squares_of4(v[4], v[5], v[6], v[7]);
+}
+
 // The gate of a gated feed-forward, from a gate g and an up u (both float).
 // kind 0: silu(g) * u (reference: (g / (1 + exp(-g))) * u in float, src/cuda/kernels.cu:198-206).
 // kind 1: g and u clamped first, g from above only (g = min(g, limit), u in [-limit, limit]), then

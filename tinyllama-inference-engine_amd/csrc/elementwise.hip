@@ -54,14 +54,42 @@ __global__ void add_rmsnorm_kernel(float* __restrict__ residual, const D* __rest
   }
 }
 
+// The sum of squares of a row of the 32-bit path, of which every thread has left the sums of its chunks of eight columns in
+// `eights` [chunks]: by blocks of 64 chunks (512 columns, the product's blocks of K), a block's quarters (every fourth group of four
+// chunks) summed group by group, the blocks in their order.  The products of few rows that fold this norm in form the same sum
+// (gemm_generic.hip).  blocks [(chunks + 63) / 64] floats of LDS; every thread gets the result.
+__device__ __forceinline__ float block_squares(const float* eights, float* blocks, int chunks) {
+  __syncthreads();
+  const int count = (chunks + 63) / 64;
+  for (int i = threadIdx.x; i < count * 4; i += blockDim.x) {        // (whole groups of four lanes)
+    float sum = 0.f;
+    for (int j = 0; j < 4; ++j) {
+      const int c = (i >> 2) * 64 + 16 * j + 4 * (i & 3);
+      float v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = c + e < chunks ? eights[c + e] : 0.f;
+      sum += (v[0] + v[1]) + (v[2] + v[3]);
+    }
+    sum += __shfl_xor(sum, 1, 64);
+    sum += __shfl_xor(sum, 2, 64);
+    if ((i & 3) == 0) blocks[i >> 2] = sum;
+  }
+  __syncthreads();
+  float total = 0.f;
+  for (int b = 0; b < count; ++b) total += blocks[b];
+  return total;
+}
+
 // The same with eight elements a thread (16-byte loads and stores): hidden % 8 == 0; the summands
-// of a split product are added in the order of their index.
+// of a split product are added in the order of their index.  With a float result the squares are summed as `block_squares` says
+// and the weight comes before the scale.
 template <typename D, typename W, typename O>
 __global__ void add_rmsnorm_wide_kernel(float* __restrict__ residual, const D* __restrict__ delta, int nsplit,
                                         size_t split_stride, const W* __restrict__ weight, float eps,
                                         O* __restrict__ out, const int* __restrict__ rows, int hidden) {
-  extern __shared__ float row_cache[];           // hidden floats, then 16 for the reduction
-  float* scratch = row_cache + hidden;
+  extern __shared__ float row_cache[];           // hidden floats, then 16 for the reduction (a float result: hidden / 8 sums and their blocks)
+  float* eights = row_cache + hidden;
+  float* scratch = eights + (sizeof(O) == sizeof(float) ? hidden / 8 : 0);
   const int r = blockIdx.x;
   const int src = rows ? rows[r] : r;
   float* res = residual + static_cast<size_t>(src) * hidden;
@@ -84,10 +112,16 @@ __global__ void add_rmsnorm_wide_kernel(float* __restrict__ residual, const D* _
       if (!rows) store8(res + i, v);
     }
     store8(row_cache + i, v);
+    if constexpr (sizeof(O) == sizeof(float)) {
+      eights[i / 8] = squares_of8(v);
+    } else {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) square += v[j] * v[j];
+      for (int j = 0; j < 8; ++j) square += v[j] * v[j];
+    }
   }
-  const float total = block_sum(square, scratch);
+  float total;
+  if constexpr (sizeof(O) == sizeof(float)) total = block_squares(eights, scratch, hidden / 8);
+  else total = block_sum(square, scratch);
   const float scale = rsqrtf(total / static_cast<float>(hidden) + eps);
   if (out) {
     O* o = out + static_cast<size_t>(r) * hidden;
@@ -96,7 +130,7 @@ __global__ void add_rmsnorm_wide_kernel(float* __restrict__ residual, const D* _
       load8(row_cache + i, v);                   // the thread's own entries
       load8(weight + i, w);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] = v[j] * scale * w[j];
+      for (int j = 0; j < 8; ++j) v[j] = sizeof(O) == sizeof(float) ? v[j] * w[j] * scale : v[j] * scale * w[j];
       store8(o + i, v);
     }
   }
@@ -346,13 +380,14 @@ static int launch_add_rmsnorm(float* residual, const void* delta, int nsplit, si
                               const void* weight, float eps, void* out,
                               const int* rows, int num_rows, int hidden, hipStream_t stream) {
   const size_t lds = (static_cast<size_t>(hidden) + 16) * sizeof(float);
+  const size_t wide_lds = sizeof(O) == sizeof(float) ? (hidden + hidden / 8 + (hidden + 511) / 512) * sizeof(float) : lds;
   if (lds > 160 * 1024) return kBadArgument;
   const bool aligned = ((reinterpret_cast<uintptr_t>(residual) | reinterpret_cast<uintptr_t>(delta) |
                          reinterpret_cast<uintptr_t>(weight) | reinterpret_cast<uintptr_t>(out)) & 31) == 0;
-  if ((hidden & 7) == 0 && aligned && (nsplit == 1 || (split_stride * sizeof(D)) % 32 == 0)) {
+  if ((hidden & 7) == 0 && aligned && wide_lds <= 160 * 1024 && (nsplit == 1 || (split_stride * sizeof(D)) % 32 == 0)) {
     const int chunks = hidden / 8;
     const int wide = chunks >= 1024 ? 1024 : (chunks + 63) / 64 * 64;
-    hipLaunchKernelGGL((add_rmsnorm_wide_kernel<D, W, O>), dim3(num_rows), dim3(wide), lds, stream, residual,
+    hipLaunchKernelGGL((add_rmsnorm_wide_kernel<D, W, O>), dim3(num_rows), dim3(wide), wide_lds, stream, residual,
                        (const D*)delta, nsplit, split_stride, (const W*)weight, eps, (O*)out, rows, hidden);
     return launch_status();
   }

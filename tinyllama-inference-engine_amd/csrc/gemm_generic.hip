@@ -42,6 +42,105 @@ __device__ __forceinline__ float4 inside(float4 v, int k, int K) {
   return make_float4(k < K ? v.x : 0.f, k + 1 < K ? v.y : 0.f, k + 2 < K ? v.z : 0.f, k + 3 < K ? v.w : 0.f);
 }
 
+// ---- what a product of few rows may do beside (a layer's neighbouring arithmetic) ---------------------------
+// Each saves a launch of 5 us whose own work is some kilobytes, and gives the bits of the kernel that it stands in for:
+//   before   x is residual * norm weight and `ssq` [M][K / 8] the sums of squares of the residual's rows by eights; the rows of x are
+//            multiplied by rsqrt(mean of squares + eps), the sum formed as in the norm kernel (`block_squares` in elementwise.hip)
+//   after    kFoldResidual: residual [M][N] += result; with next_weight also xg = residual * next_weight and `ssq_out` for the
+//            product that the next norm stands before.  kFoldRotation: W is a fused q/k/v weight with rows in paired order; rotation
+//            and cache write of rope_cache.hip
+constexpr int kFoldStore = 0, kFoldResidual = 1, kFoldRotation = 2;
+
+struct RowsFold {
+  const float* ssq;
+  float eps;
+  int kind;
+  int squares_at;                     // where the blocks' sums of squares lie in LDS
+  int rows;                           // rows of W a workgroup: even, at most the kernel's R; for ssq_out a multiple of 8
+  float* residual;
+  const float* next_weight;
+  float* xg;
+  float* ssq_out;
+  const int* positions;
+  const int* slot_map;
+  const float* inv_freq;
+  float* q_out;
+  float* cache;
+  int rot_dim, nq, nkv, d, page_size;
+};
+
+// What a thread's four neighbouring columns n .. n + 3 of row m need beside their sums, asked for before W (behind it the wait for
+// these would be a way to memory of its own, twice for the rotation).
+struct FoldAhead {
+  float4 bias, residual, weight;
+  float sine[2], cosine[2];
+  int slot;
+};
+
+__device__ __forceinline__ FoldAhead fold_ahead(const RowsFold& fold, const float* __restrict__ bias, int m, int n, int N) {
+  FoldAhead a;
+  a.bias = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (bias) a.bias = make_float4(bias[n], bias[min(n + 1, N - 1)], bias[min(n + 2, N - 1)], bias[min(n + 3, N - 1)]);
+  if (fold.kind == kFoldResidual) {
+    a.residual = *reinterpret_cast<const float4*>(fold.residual + static_cast<size_t>(m) * N + n);
+    if (fold.next_weight != nullptr) a.weight = *reinterpret_cast<const float4*>(fold.next_weight + n);
+  } else if (fold.kind == kFoldRotation) {
+    a.slot = fold.slot_map[m];
+    a.cosine[0] = static_cast<float>(fold.positions[m]);   // (turned into sines by `fold_angles`)
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int c = (n + 2 * e) % fold.d;
+      a.sine[e] = fold.inv_freq != nullptr && c < fold.rot_dim ? fold.inv_freq[c / 2] : 0.f;
+    }
+  }
+  return a;
+}
+
+__device__ __forceinline__ void fold_angles(const RowsFold& fold, FoldAhead& a) {
+  if (fold.kind != kFoldRotation || fold.inv_freq == nullptr) return;
+  const float position = a.cosine[0];
+#pragma unroll
+  for (int e = 0; e < 2; ++e) sincosf(position * a.sine[e], &a.sine[e], &a.cosine[e]);
+}
+
+// N a multiple of 4; with next_weight of 8, and the neighbouring thread holds the other half of the eight.
+__device__ __forceinline__ void fold_residual(const RowsFold& fold, const FoldAhead& a, const float (&sum)[4], int m, int n, int N) {
+  const float v[4] = {a.residual.x + sum[0], a.residual.y + sum[1], a.residual.z + sum[2], a.residual.w + sum[3]};
+  store4(fold.residual + static_cast<size_t>(m) * N + n, v[0], v[1], v[2], v[3]);
+  if (fold.next_weight == nullptr) return;                 // (the same for the whole grid)
+  store4(fold.xg + static_cast<size_t>(m) * N + n, v[0] * a.weight.x, v[1] * a.weight.y, v[2] * a.weight.z, v[3] * a.weight.w);
+  const float half = squares_of4(v[0], v[1], v[2], v[3]), other = __shfl_xor(half, 1, 64);
+  if ((n & 4) == 0) fold.ssq_out[static_cast<size_t>(m) * (N / 8) + n / 8] = half + other;
+}
+
+// Two pairs of columns n, n + 1 and n + 2, n + 3 of token m (n and d even).
+__device__ __forceinline__ void fold_rotation(const RowsFold& fold, const FoldAhead& a, const float (&sum)[4], int m, int n, int n_end) {
+  const int slot = a.slot, half = fold.rot_dim / 2;
+  const size_t head_stride = static_cast<size_t>(fold.page_size) * fold.d;
+  float* page = fold.cache + static_cast<size_t>(slot < 0 ? 0 : slot / fold.page_size) * 2 * fold.nkv * head_stride;
+  const int row = slot < 0 ? 0 : slot % fold.page_size;
+#pragma unroll
+  for (int e = 0; e < 4; e += 2) {
+    if (n + e >= n_end) break;
+    const int head = (n + e) / fold.d, c = (n + e) % fold.d;
+    if (head >= fold.nq && slot < 0) continue;
+    if (head >= fold.nq + fold.nkv) {                      // a value head lies transposed, after the key heads
+      float* out = page + (head - fold.nq) * head_stride + static_cast<size_t>(c) * fold.page_size + row;
+      out[0] = sum[e], out[fold.page_size] = sum[e + 1];
+      continue;
+    }
+    float* out = head < fold.nq ? fold.q_out + (static_cast<size_t>(m) * fold.nq + head) * fold.d
+                                : page + (head - fold.nq) * head_stride + static_cast<size_t>(row) * fold.d;
+    if (fold.inv_freq != nullptr && c < fold.rot_dim) {
+      const float sn = a.sine[e / 2], cs = a.cosine[e / 2];
+      out[c / 2] = sum[e] * cs - sum[e + 1] * sn;
+      out[c / 2 + half] = sum[e + 1] * cs + sum[e] * sn;
+    } else {
+      out[c] = sum[e], out[c + 1] = sum[e + 1];
+    }
+  }
+}
+
 // ---- few rows of x (decoding, short portions) ------------------------------------------------------------
 // Bound by reading W.  A workgroup owns R rows of W (columns of y) and all M <= 16 MT rows of x; its waves take the blocks
 // of K in turn, each block one chain of matrix instructions whose operands go straight from memory into registers: a
@@ -51,36 +150,96 @@ __device__ __forceinline__ float4 inside(float4 v, int k, int K) {
 // PAIR (at most 8 rows of x, R = 8): of the instruction's 16 x 16 results two quarters of 8 x 8 are used, one for each of
 // two blocks of K: lanes 0 .. 7 of a sixteen bring both operands' rows from the one block, lanes 8 .. 15 from the other.
 // Twice the workgroups of R = 16, and no lane brings what another one has.
-template <typename X, typename W, typename O, int MT, int R, bool PAIR, int RING, int WAVES, bool WIDE>
+// FOLD: a layer's neighbouring arithmetic in the same kernel, described by `RowsFold` (at most 16 rows of x, all in 32 bits; the bits
+// are those of the kernels it stands in for).  SHORT: K is at most 256, one part of the ring: what lies past K is neither asked
+// for nor multiplied (96 x 96: 24 instructions of a chain in place of 64).
+template <typename X, typename W, typename O, int MT, int R, bool PAIR, int RING, int WAVES, bool WIDE, bool FOLD = false, bool SHORT = false>
 __global__ void __launch_bounds__(64 * WAVES)
 gemm_generic_few_kernel(const X* __restrict__ x, const W* __restrict__ w, const W* __restrict__ bias,
-                        O* __restrict__ y, int M, int N, int K, int gate, float alpha, float limit, int jobs_at_once) {
+                        O* __restrict__ y, int M, int N, int K, int gate, float alpha, float limit, int jobs_at_once, RowsFold fold) {
   static_assert(!PAIR || (MT == 1 && R == 8), "two blocks at once: 8 rows of W, 8 of x");
-  constexpr int SC = 8 / MT < RING / 2 ? 8 / MT : RING / 2;      // loads of x asked for together
+  static_assert(!FOLD || (MT == 1 && WIDE), "folds: at most 16 rows of x, 16-byte loads");
+  static_assert(!SHORT || (!PAIR && MT == 1 && RING == 16), "K of one part: one block");
+  // Folded: x goes through a ring of its own, both rings 8 deep and asked for four pieces at a time.  Loads come back in the order they
+  // were asked for, so that with W 16 groups ahead and x 8 the wait for x leaves only 8 of W's on their way; and a shorter ring is
+  // half the code, most of which runs once or twice and comes from memory itself.  8 rows: 11264 x 2048 gated 26.9 us (rings of 16 with
+  // x 8 ahead 31.7, one piece at a time 29.3), 2048 x 5632 17.6 (22.1, 19.1; two blocks at once with rings of 16 19.7), 2560 x 2048 11.2.
+  constexpr bool kTogether = FOLD;
+  constexpr int SC = kTogether ? RING : (8 / MT < RING / 2 ? 8 / MT : RING / 2);     // loads of x asked for together
   constexpr int kJobK = PAIR ? 2 * kBlockK : kBlockK, kPartK = 16 * RING;
   extern __shared__ __attribute__((aligned(16))) float sums[];   // [block][rows of x][R rows of W]
+  constexpr int kNormRows = PAIR ? 8 : 16;
+  float* squares = sums + fold.squares_at;                       // [block][rows of x]
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
   const int r = lane & 15, g = lane >> 4;
-  const int n0 = blockIdx.x * R;
-  const W* w_row = w + static_cast<size_t>(min(n0 + r % R, N - 1)) * K;
+  const int here = FOLD ? fold.rows : R;                   // rows of W of this workgroup (even, at most R)
+  const int n0 = blockIdx.x * here, n_end = min(N, n0 + here);
+  const W* w_row = w + static_cast<size_t>(min(n0 + (FOLD ? min(r % R, here - 1) : r % R), N - 1)) * K;
   const X* x_row[MT];
 #pragma unroll
   for (int i = 0; i < MT; ++i) x_row[i] = x + static_cast<size_t>(min(16 * i + (PAIR ? r & 7 : r), M - 1)) * K;
   const int jobs = (K + kJobK - 1) / kJobK;                // of one block of K, or of two
   const int first = (PAIR ? (r >> 3) * kBlockK : 0) + 4 * g;     // this lane's k within a job's first 16
-  float4 ring[RING], xs[2][SC][MT];
+  float4 ring[RING], xs[kTogether ? 1 : 2][SC][MT];
   int k0 = wave * kJobK;
+  constexpr int kQuads = R / 4, kRows = PAIR ? 8 : 16 * MT;
+  FoldAhead ahead;
+  // the norm before this product: a lane sums the squares of its row of x over its quarter of a block of K, asked for ahead of W (its
+  // first job's; those of further ones behind); code that runs once is kept short, its way from memory is what it costs
+  const int chunks = K / 8;
+  const bool normed = FOLD && fold.ssq != nullptr;         // (the same for the whole grid)
+  auto part_of_block = [&](int k, float4 (&v)[4]) {
+    const float* row = fold.ssq + static_cast<size_t>(min(PAIR ? r & 7 : r, M - 1)) * chunks;
+    const int c0 = (k + first - 4 * g) / 8 + 4 * g;
+#pragma unroll
+    for (int j = 0; j < (SHORT ? 2 : 4); ++j) v[j] = load4(row + min(c0 + 16 * j, chunks - 4));
+  };
+  float4 square[4];
+  if constexpr (FOLD) {
+    const int m = threadIdx.x / kQuads, n = n0 + threadIdx.x % kQuads * 4;
+    if (m < M && n < n_end && threadIdx.x < kQuads * kRows) ahead = fold_ahead(fold, bias, m, n, N);
+    if (normed && k0 < K) part_of_block(k0, square);
+  }
   if (k0 < K) {
+    if (!kTogether) {
 #pragma unroll
-    for (int c = 0; c < SC; ++c)
+      for (int c = 0; c < SC; ++c)
 #pragma unroll
-      for (int i = 0; i < MT; ++i) xs[0][c][i] = fetch4<WIDE>(x_row[i], k0 + first + 16 * c, K);
+        for (int i = 0; i < MT; ++i) xs[0][c][i] = fetch4<WIDE>(x_row[i], k0 + first + 16 * c, K);
+    }
 #pragma unroll
-    for (int c = 0; c < RING; ++c) ring[c] = fetch4<WIDE>(w_row, k0 + first + 16 * c, K);
+    for (int c = 0; c < RING; ++c) {
+      if (SHORT && 16 * c >= K) break;
+      ring[c] = fetch4<WIDE>(w_row, k0 + first + 16 * c, K);
+      if (kTogether) xs[0][c][0] = fetch4<WIDE>(x_row[0], k0 + first + 16 * c, K);
+    }
+  }
+  float x_scale = 1.f;                                     // of this lane's row of x
+  if constexpr (FOLD) {
+    if (normed) {
+      for (int job = wave; job < (K + kJobK - 1) / kJobK; job += waves) {
+        if (job != wave) part_of_block(job * kJobK, square);
+        const int c0 = (job * kJobK + first - 4 * g) / 8 + 4 * g;
+        float sum = 0.f;
+#pragma unroll
+        for (int j = 0; j < (SHORT ? 2 : 4); ++j)
+          sum += c0 + 16 * j < chunks ? (square[j].x + square[j].y) + (square[j].z + square[j].w) : 0.f;
+        float a = sum, b = sum;
+        swap16(a, b);
+        a = b = a + b;
+        swap32(a, b);
+        if (lane < 16) squares[(PAIR ? 2 * job + (r >> 3) : job) * kNormRows + (PAIR ? r & 7 : r)] = a + b;
+      }
+      lds_barrier();
+      float total = 0.f;
+#pragma unroll 4
+      for (int b = 0; b < (K + kBlockK - 1) / kBlockK; ++b) total += squares[b * kNormRows + (PAIR ? r & 7 : r)];
+      x_scale = rsqrtf(total / static_cast<float>(K) + fold.eps);
+    }
+    if (wave == 0) fold_angles(fold, ahead);
   }
   // (the blocks' sums of one pass fit LDS; only a K of more than 64 blocks, with MT = 1, takes several: 512 x 40000 at 1 row 63 us,
   // at 16 rows 155, in tiles 540; 128 x 33000 46, 358)
-  constexpr int kQuads = R / 4, kRows = PAIR ? 8 : 16 * MT;
   const int blocks = (K + kBlockK - 1) / kBlockK, pass = min(jobs, jobs_at_once);
   float4 before = make_float4(0.f, 0.f, 0.f, 0.f);         // this thread's sums of earlier passes (then it has one place at most)
   int job = wave;
@@ -95,7 +254,8 @@ gemm_generic_few_kernel(const X* __restrict__ x, const W* __restrict__ w, const 
         const bool more = next < K, edge = k0 + kPartK + (PAIR ? kBlockK : 0) > K;
 #pragma unroll
         for (int c = 0; c < RING; ++c) {
-          if (c % SC == 0) {                                 // the next few pieces of x
+          if (SHORT && 16 * c >= K) break;
+          if (!kTogether && c % SC == 0) {                   // the next few pieces of x
             const int to = (c / SC + 1) & 1;
             const int from = (c + SC < RING ? k0 + 16 * (c + SC) : next) + first;
             if (c + SC < RING || more) {
@@ -107,13 +267,16 @@ gemm_generic_few_kernel(const X* __restrict__ x, const W* __restrict__ w, const 
           }
           float4 a = ring[c], b[MT];
 #pragma unroll
-          for (int i = 0; i < MT; ++i) b[i] = xs[(c / SC) & 1][c % SC][i];
+          for (int i = 0; i < MT; ++i) {
+            b[i] = xs[kTogether ? 0 : (c / SC) & 1][c % SC][i];
+            if (FOLD) b[i].x *= x_scale, b[i].y *= x_scale, b[i].z *= x_scale, b[i].w *= x_scale;
+          }
           if (edge) {                                        // past the end of K: zeros
             a = inside(a, k0 + first + 16 * c, K);
 #pragma unroll
             for (int i = 0; i < MT; ++i) b[i] = inside(b[i], k0 + first + 16 * c, K);
           }
-          if (more) ring[c] = fetch4<WIDE>(w_row, next + first + 16 * c, K);
+          if (!SHORT && more && !kTogether) ring[c] = fetch4<WIDE>(w_row, next + first + 16 * c, K);
           to_quarters(a);
 #pragma unroll
           for (int i = 0; i < MT; ++i) to_quarters(b[i]);
@@ -121,6 +284,12 @@ gemm_generic_few_kernel(const X* __restrict__ x, const W* __restrict__ w, const 
           for (int e = 0; e < 4; ++e)
 #pragma unroll
             for (int i = 0; i < MT; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32((&a.x)[e], (&b[i].x)[e], acc[i], 0, 0, 0);
+          if (kTogether && !SHORT && more && c % 4 == 3) {
+#pragma unroll
+            for (int e = c - 3; e <= c; ++e) ring[e] = fetch4<WIDE>(w_row, next + first + 16 * e, K);
+#pragma unroll
+            for (int e = c - 3; e <= c; ++e) xs[0][e][0] = fetch4<WIDE>(x_row[0], next + first + 16 * e, K);
+          }
         }
         k0 = next;
       }
@@ -140,7 +309,7 @@ gemm_generic_few_kernel(const X* __restrict__ x, const W* __restrict__ w, const 
     const int blocks_here = last ? blocks - first_job * (kJobK / kBlockK) : pass * (kJobK / kBlockK);
     for (int t = threadIdx.x; t < kQuads * kRows; t += blockDim.x) {
       const int m = t / kQuads, j = t % kQuads * 4, n = n0 + j;       // four neighbouring columns of y
-      if (m >= M || n >= N) continue;
+      if (m >= M || n >= n_end) continue;
       float4 v = before;
       for (int b = 0; b < blocks_here; ++b) {                // in index order
         const float4 s = *reinterpret_cast<const float4*>(sums + (b * kRows + m) * R + j);
@@ -151,19 +320,31 @@ gemm_generic_few_kernel(const X* __restrict__ x, const W* __restrict__ w, const 
         continue;
       }
       const float out[4] = {v.x, v.y, v.z, v.w};
+      if constexpr (FOLD) {
+        if (fold.kind != kFoldStore) {
+          float sum[4] = {out[0], out[1], out[2], out[3]};
+          if (bias) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sum[e] += (&ahead.bias.x)[e];
+          }
+          if (fold.kind == kFoldResidual) fold_residual(fold, ahead, sum, m, n, N);
+          else fold_rotation(fold, ahead, sum, m, n, n_end);
+          continue;
+        }
+      }
 #pragma unroll
       for (int e = 0; e < 4; e += 2) {
         float p = out[e], u = out[e + 1];
-        if (n + e >= N) break;
+        if (n + e >= n_end) break;
         if (bias) {
           p += to_float(bias[n + e]);
-          if (n + e + 1 < N) u += to_float(bias[n + e + 1]);
+          if (n + e + 1 < n_end) u += to_float(bias[n + e + 1]);
         }
         if (gate != kNoGate) {
           y[static_cast<size_t>(m) * (N / 2) + (n + e) / 2] = from_float<O>(gated_value(p, u, gate, alpha, limit));
         } else {
           y[static_cast<size_t>(m) * N + n + e] = from_float<O>(p);
-          if (n + e + 1 < N) y[static_cast<size_t>(m) * N + n + e + 1] = from_float<O>(u);
+          if (n + e + 1 < n_end) y[static_cast<size_t>(m) * N + n + e + 1] = from_float<O>(u);
         }
       }
     }
@@ -313,8 +494,40 @@ int launch_few(const X* x, const W* w, const W* bias, O* y, int M, int N, int K,
   const int at_once = jobs <= 64 * 1024 / job_bytes ? jobs : 64 * 1024 / job_bytes;
   const int bytes = at_once * job_bytes;
   hipLaunchKernelGGL((gemm_generic_few_kernel<X, W, O, MT, R, PAIR, RING, WAVES, WIDE>), dim3((N + R - 1) / R), dim3(64 * waves), bytes, s,
-                     x, w, bias, y, M, N, K, gate, alpha, limit, at_once);
+                     x, w, bias, y, M, N, K, gate, alpha, limit, at_once, RowsFold{});
   return launch_status();
+}
+
+template <int R, bool PAIR, int WAVES, bool SHORT>
+int launch_folded(const float* x, const float* w, const float* bias, float* y, int M, int N, int K, int gate, float alpha, float limit,
+                  const RowsFold& fold, hipStream_t s) {
+  const int job_k = PAIR ? 2 * kBlockK : kBlockK, jobs = (K + job_k - 1) / job_k, turns = (jobs + WAVES - 1) / WAVES;
+  const int waves = (jobs + turns - 1) / turns;
+  const int job_bytes = (PAIR ? 2 * 64 : 16 * R) * static_cast<int>(sizeof(float));
+  const int squares = fold.ssq != nullptr ? jobs * 16 * static_cast<int>(sizeof(float)) : 0, room = 64 * 1024 - squares;
+  if (room < job_bytes) return kBadArgument;               // (K of half a million)
+  const int at_once = jobs <= room / job_bytes ? jobs : room / job_bytes;
+  RowsFold placed = fold;
+  placed.squares_at = at_once * job_bytes / static_cast<int>(sizeof(float));
+  hipLaunchKernelGGL((gemm_generic_few_kernel<float, float, float, 1, R, PAIR, SHORT ? 16 : 8, WAVES, true, true, SHORT>), dim3((N + fold.rows - 1) / fold.rows),
+                     dim3(64 * waves), at_once * job_bytes + squares, s, x, w, bias, y, M, N, K, gate, alpha, limit, at_once, placed);
+  return launch_status();
+}
+
+// ---- embedding of few rows with the first norm's inputs ------------------------------------------------------
+__global__ void embed_rows_float_kernel(const int* __restrict__ tokens, const float* __restrict__ table, const float* __restrict__ weight,
+                                        float* __restrict__ residual, float* __restrict__ xg, float* __restrict__ ssq, int hidden) {
+  const int t = blockIdx.y, chunk = blockIdx.x * blockDim.x + threadIdx.x;
+  if (chunk * 8 >= hidden) return;
+  const size_t at = static_cast<size_t>(t) * hidden + chunk * 8;
+  float v[8], w[8];
+  load8(table + static_cast<size_t>(tokens[t]) * hidden + chunk * 8, v);
+  load8(weight + chunk * 8, w);
+  store8(residual + at, v);
+  ssq[static_cast<size_t>(t) * (hidden / 8) + chunk] = squares_of8(v);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) v[j] *= w[j];
+  store8(xg + at, v);
 }
 
 template <typename X, typename W, typename O, int TN, int TM, int D, bool WIDE>
@@ -385,4 +598,50 @@ extern "C" int tlie_gemm_generic(const void* x, int x_dtype, const void* w, int 
   TLIE_CASE(kBF16, bf16, kF32, float, kF32, float)
 #undef TLIE_CASE
   return kBadArgument;
+}
+
+// The product of at most 16 rows with a layer's neighbouring arithmetic, all in 32 bits (see `RowsFold`).  K % 4 == 0 (ssq: % 32) and
+// 16-byte aligned rows; N % 4 == 0 for the residual, % 8 with next_weight; d even for the rotation.
+extern "C" int tlie_gemm_generic_rows(const float* x, const float* w, const float* bias, float* y, int M, int N, int K, int gate, float alpha,
+                                      float limit, const float* ssq, float eps, int kind, float* residual, const float* next_weight, float* xg,
+                                      float* ssq_out, const int* positions, const int* slot_map, const float* inv_freq, int rot_dim, float* q_out,
+                                      float* cache, int nq, int nkv, int d, int page_size, int compute_units, void* stream) {
+  if (M <= 0 || M > 16 || N <= 0 || K <= 0 || K % 4 != 0 || compute_units <= 0) return kBadArgument;
+  if (gate < kNoGate || gate > kGateClampedSwish || (gate != kNoGate && (N % 2 != 0 || kind != kFoldStore))) return kBadArgument;
+  if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) % 16 != 0 || (ssq != nullptr && (K % 32 != 0 || reinterpret_cast<uintptr_t>(ssq) % 16 != 0))) return kBadArgument;
+  if (kind == kFoldStore) {
+    if (y == nullptr) return kBadArgument;
+  } else if (kind == kFoldResidual) {
+    if (residual == nullptr || N % 4 != 0 || (next_weight != nullptr && (N % 8 != 0 || xg == nullptr || ssq_out == nullptr))) return kBadArgument;
+    if ((reinterpret_cast<uintptr_t>(residual) | reinterpret_cast<uintptr_t>(next_weight) | reinterpret_cast<uintptr_t>(xg)) % 16 != 0) return kBadArgument;
+  } else if (kind == kFoldRotation) {
+    if (positions == nullptr || slot_map == nullptr || q_out == nullptr || cache == nullptr || nq <= 0 || nkv <= 0 || d <= 0 || d % 2 != 0 ||
+        page_size <= 0 || rot_dim < 0 || rot_dim > d || rot_dim % 2 != 0 || N != (nq + 2 * nkv) * d)
+      return kBadArgument;
+  } else {
+    return kBadArgument;
+  }
+  hipStream_t s = (hipStream_t)stream;
+  RowsFold fold{ssq, eps, kind, 0, 16, residual, next_weight, xg, ssq_out, positions, slot_map, inv_freq, q_out, cache, rot_dim, nq, nkv, d, page_size};
+  if (K <= 256) return launch_folded<16, false, 1, true>(x, w, bias, y, M, N, K, gate, alpha, limit, fold, s);
+  if (M <= 8 && K > kBlockK && (N + 7) / 8 <= compute_units) {       // (the lines of `launch_product`)
+    fold.rows = 8;
+    return launch_folded<8, true, 12, false>(x, w, bias, y, M, N, K, gate, alpha, limit, fold, s);
+  }
+  // where strips of 16 rows leave units without a workgroup, even shares of the rows instead
+  const int strips = (N + 15) / 16, share = ((N + compute_units - 1) / compute_units + 1) / 2 * 2;
+  if (kind != kFoldResidual && strips < compute_units && 2 * strips > compute_units && share < 16) fold.rows = share < 8 ? 8 : share;
+  return launch_folded<16, false, 12, false>(x, w, bias, y, M, N, K, gate, alpha, limit, fold, s);
+}
+
+// The embedding of few rows with the first norm's inputs: residual [rows][hidden] = table's rows, xg = residual * weight, ssq the sums
+// of squares by eights; hidden % 8 == 0, 32-byte aligned arrays.
+extern "C" int tlie_embed_rows_float(const int* tokens, const float* table, const float* weight, float* residual, float* xg, float* ssq,
+                                     int rows, int hidden, void* stream) {
+  if (rows <= 0 || rows > 65535 || hidden <= 0 || hidden % 8 != 0) return kBadArgument;
+  if ((reinterpret_cast<uintptr_t>(table) | reinterpret_cast<uintptr_t>(weight) | reinterpret_cast<uintptr_t>(residual) | reinterpret_cast<uintptr_t>(xg)) & 31)
+    return kBadArgument;
+  hipLaunchKernelGGL(embed_rows_float_kernel, dim3((hidden / 8 + 63) / 64, rows), dim3(64), 0, (hipStream_t)stream, tokens, table, weight, residual,
+                     xg, ssq, hidden);
+  return launch_status();
 }

@@ -96,7 +96,7 @@ class DecoderModel:
         trace = getattr(ctx, "trace", None)
         if runs[0].depth_mix is not None:
             return self._forward_depth_mixed(ctx, bindings)
-        few = ops.few_rows_route(ctx.num_tokens, self.dtype) and (trace is None or getattr(ctx, "trace_serving_route", False))
+        few = ops.folded_route(ctx.num_tokens, self.dtype, trace, getattr(ctx, "trace_serving_route", False))
 
         def entry_norm(block):
             # a block may say which norm reads the residual first (its writer can then leave that
@@ -104,7 +104,8 @@ class DecoderModel:
             return block.entry_norm() if hasattr(block, "entry_norm") else None
         first_norm = entry_norm(self.blocks[runs[0].layer]) if runs[0].pass_input is None else None
         lazy = first_norm.lazy_params() if first_norm is not None else None
-        if few and hasattr(self.embedding, "forward_rows") and lazy is not None and getattr(self.embedding, "scale", 1.0) == 1.0:
+        if (few and hasattr(self.embedding, "forward_rows") and lazy is not None and getattr(self.embedding, "scale", 1.0) == 1.0
+                and getattr(self.embedding, "norm", None) is None):
             residual, normed = self.embedding.forward_rows(ctx.tokens, lazy)
             pending = ResidualUpdated(normed)
         elif (self.dtype == torch.bfloat16 and getattr(self.blocks[runs[0].layer], "reads_residual", False)
@@ -134,6 +135,8 @@ class DecoderModel:
                     pending = None
                 vector = self.run_vectors[run.add_vector[0]][run.add_vector[1]] if run.add_vector is not None else None
                 ops.residual_inject(residual, ctx.tokens, self.embedding.table if run.add_embedding else None, vector)
+                if isinstance(pending, ResidualUpdated):
+                    pending = ResidualUpdated(None)          # (what its writer left for the next norm is of the residual before)
             if run.pass_input is not None:
                 # a pass begins with a residual of its own: a product of the residual so far and the embedding's output
                 if pending is not None:

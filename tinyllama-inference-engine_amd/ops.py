@@ -1681,6 +1681,96 @@ def gemm_generic(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | Non
     return out if gated else Product(out, 1)
 
 
+def gemm_generic_rows_takes(rows: int, weight: torch.Tensor, dtype: torch.dtype, bias: torch.Tensor | None = None) -> bool:
+    """Whether `gemm_generic_rows` takes a step of `rows` tokens: everything in 32 bits, rows that 16-byte loads fit."""
+    return (dtype == torch.float32 and weight.dtype == torch.float32 and 0 < rows <= ROWS_MAX and weight.shape[1] % 4 == 0
+            and weight.data_ptr() % 16 == 0 and (bias is None or bias.dtype == torch.float32))
+
+
+def _float_norm_folds(weight: torch.Tensor, width: int) -> bool:
+    """Whether a product of few rows may leave and take this norm's inputs: the sums of squares by eight columns in fours, and the norm
+    kernel sums by eights too."""
+    return weight.dtype == torch.float32 and width % 32 == 0 and weight.data_ptr() % 32 == 0
+
+
+def gemm_generic_rows(x, weight: torch.Tensor, bias: torch.Tensor | None, epilogue: str = "store", residual: torch.Tensor | None = None,
+                      next_norm: tuple | None = None, rope: "RopeTarget | None" = None, gate=None):
+    """y = x . W^T (+ bias) for at most 16 rows in true 32-bit, with what stands beside it in a layer: the bits of `gemm_generic` and of
+    the kernels it stands in for.  x: float32 [M, K], or a float32 `NormedRows`.  epilogue "store": a `Product`; "gate": W's rows
+    alternate gate and up, returns the gated [M, N / 2] (gate: see `silu_mul`); "residual": residual [M, N] += y in place, returns a
+    `ResidualUpdated`, with the next norm's inputs when next_norm = (weight [N], eps) is given and its sums go by eight columns;
+    "rope": W is a fused q/k/v weight with rows in the order of `paired_rows`: rotation and cache write as `rope_cache` does, q is returned."""
+    normed = x if isinstance(x, NormedRows) else None
+    data = normed.xg if normed is not None else x
+    _device_tensor(data, "x", torch.float32)
+    _device_tensor(weight, "weight", torch.float32)
+    if data.dim() != 2 or weight.dim() != 2 or data.shape[1] != weight.shape[1]:
+        raise invalid_shape(f"gemm: x {list(data.shape)} and weight {list(weight.shape)} do not fit")
+    rows, (out_features, in_features) = data.shape[0], weight.shape
+    if not gemm_generic_rows_takes(rows, weight, data.dtype, bias):
+        raise invalid_argument(f"gemm_generic_rows takes 1..{ROWS_MAX} rows of float32 and an inner size that is a multiple of 4")
+    if bias is not None:
+        _device_tensor(bias, "bias", torch.float32)
+        if bias.shape != (out_features,):
+            raise invalid_shape("gemm: bias needs one entry per output")
+    ssq, eps = None, 0.0
+    if normed is not None:
+        _device_tensor(normed.ssq, "ssq", torch.float32)
+        if in_features % 32 != 0 or normed.ssq.shape != (rows, in_features // 8):
+            raise invalid_shape(f"gemm: sums of squares {list(normed.ssq.shape)} are not [{rows}, {in_features} / 8]")
+        ssq, eps = normed.ssq, float(normed.eps)
+    device, code = data.device, 0
+    y = xg = ssq_out = next_weight = q_out = None
+    gate_kind, alpha, limit = _gate_args(gate if epilogue == "gate" else None)
+    rope_args = (_ptr(None), _ptr(None), _ptr(None), 0, _ptr(None), _ptr(None), 0, 0, 0, 0)
+    if epilogue == "store":
+        gate_kind, y = -1, torch.empty((rows, out_features), dtype=torch.float32, device=device)
+    elif epilogue == "gate":
+        if out_features % 2 != 0:
+            raise invalid_shape("gemm: the gated product needs an even number of rows of W")
+        y = torch.empty((rows, out_features // 2), dtype=torch.float32, device=device)
+    elif epilogue == "residual":
+        gate_kind, code = -1, 1
+        _device_tensor(residual, "residual", torch.float32)
+        if residual.shape != (rows, out_features) or out_features % 4 != 0:
+            raise invalid_shape(f"gemm: residual {list(residual.shape)} is not [{rows}, {out_features}], or not a multiple of 4 columns")
+        if next_norm is not None and _float_norm_folds(next_norm[0], out_features):
+            next_weight = next_norm[0]
+            _device_tensor(next_weight, "next norm weight", torch.float32)
+            if next_weight.shape != (out_features,):
+                raise invalid_shape("gemm: the next norm's weight needs one entry per output")
+            xg = torch.empty((rows, out_features), dtype=torch.float32, device=device)
+            ssq_out = torch.empty((rows, out_features // 8), dtype=torch.float32, device=device)
+    elif epilogue == "rope":
+        gate_kind, code = -1, 2
+        _device_tensor(rope.positions, "positions", torch.int32)
+        _device_tensor(rope.slot_map, "slot_map", torch.int32)
+        _device_tensor(rope.cache, "cache", torch.float32)
+        if rope.extra_cols or rope.head_scale is not None or rope.head_dim % 2 != 0:
+            raise invalid_argument("gemm: the rotation takes an even head size, no further columns and no numbers a head")
+        if out_features != (rope.num_heads + 2 * rope.num_kv_heads) * rope.head_dim:
+            raise invalid_shape(f"gemm: {out_features} rows of W are not (nq + 2 nkv) * d")
+        if rope.positions.shape != (rows,) or rope.slot_map.shape != (rows,):
+            raise invalid_shape("gemm: positions and slot_map need one entry per token")
+        page_size = _check_cache(rope.cache, rope.num_kv_heads, rope.head_dim, "gemm")
+        rot_dim = rope.rot_dim if rope.inv_freq is not None else 0
+        if rope.inv_freq is not None:
+            _device_tensor(rope.inv_freq, "inv_freq", torch.float32)
+            if rot_dim % 2 != 0 or not 0 < rot_dim <= rope.head_dim or rope.inv_freq.shape != (rot_dim // 2,):
+                raise invalid_shape("gemm: inv_freq needs rot_dim / 2 entries, rot_dim even and at most d")
+        q_out = torch.empty((rows, rope.num_heads * rope.head_dim), dtype=torch.float32, device=device)
+        rope_args = (_ptr(rope.positions), _ptr(rope.slot_map), _ptr(rope.inv_freq), rot_dim, _ptr(q_out), _ptr(rope.cache),
+                     rope.num_heads, rope.num_kv_heads, rope.head_dim, page_size)
+    else:
+        raise invalid_argument(f"gemm: unknown epilogue '{epilogue}'")
+    _check(library().tlie_gemm_generic_rows(_ptr(data), _ptr(weight), _ptr(bias), _ptr(y), rows, out_features, in_features, gate_kind, alpha, limit,
+                                            _ptr(ssq), ctypes.c_float(eps), code, _ptr(residual if code == 1 else None), _ptr(next_weight),
+                                            _ptr(xg), _ptr(ssq_out), *rope_args, _compute_units(device), _stream()), "gemm_generic_rows")
+    if epilogue == "residual":
+        return ResidualUpdated(NormedRows(xg, ssq_out, float(next_norm[1])) if next_weight is not None else None)
+    return q_out if epilogue == "rope" else (y if epilogue == "gate" else Product(y, 1))
+
+
 # state: None (not tried), True, False (not there); fallbacks: products that took this library's plain kernel instead
 _library_gemm = {"state": None, "workspace": {}, "fallbacks": 0, "warned": set(), "no_bias_epilogue": set()}
 LIBRARY_WORKSPACE_BYTES = 32 << 20
@@ -2225,6 +2315,14 @@ def few_rows_route(rows: int, dtype: torch.dtype) -> bool:
     return dtype == torch.bfloat16 and 0 < rows <= ROWS_MAX
 
 
+def folded_route(rows: int, dtype: torch.dtype, trace=None, trace_serving_route: bool = False) -> bool:
+    """`few_rows_route`, or the same route in 32 bits (`gemm_generic_rows`, as far as each product of the step takes it).  A step
+    that keeps a trace takes it in bfloat16 alone, and when asked to: in 32 bits the other route gives the same bits and leaves every tensor."""
+    if dtype == torch.float32:
+        return trace is None and 0 < rows <= ROWS_MAX
+    return few_rows_route(rows, dtype) and (trace is None or trace_serving_route)
+
+
 def attention_plan(ctx, groups_per_kv: int, num_kv_heads: int, head_dim: int, reach: int | None = None, extra: bool = False):
     """How the tiled attention kernel is launched for the step `ctx` describes: its work list (made
     once per step and group size, kept in `ctx.scratch`; None for a decode step, whose tiles the
@@ -2517,7 +2615,8 @@ class NormedRows:
     partial sums of squares of the residual's rows, ssq [parts, 16] (each part covers some of the
     columns; their sum over the parts is the row's sum of squares).  The product applies
     rsqrt(sum(ssq) / width + eps) to its result's rows, which is the same as having normed the
-    input."""
+    input.  In a 32-bit step xg is float32 and ssq [T, width / 8] the sums of squares by eight columns; the product
+    scales its rows of xg, which gives the bits of the norm kernel."""
     xg: torch.Tensor
     ssq: torch.Tensor
     eps: float
@@ -2713,9 +2812,10 @@ def gemm_rows_batch(x: torch.Tensor, weight: torch.Tensor) -> list[Product]:
     return [Product(y[index], 1) for index in range(batch)]
 
 
-def embed_rows(tokens: torch.Tensor, table: torch.Tensor, next_norm: tuple):
+def embed_rows(tokens: torch.Tensor, table: torch.Tensor, next_norm: tuple, dtype: torch.dtype = torch.bfloat16):
     """The embedding for at most 16 tokens with the first norm's inputs: returns (float32
-    residual [T, hidden], NormedRows)."""
+    residual [T, hidden], NormedRows).  dtype: of the step; in 32 bits the second is None where the norm's sums do not go by
+    eight columns (or the table is kept in another type)."""
     _device_tensor(tokens, "tokens", torch.int32)
     _device_tensor(table, "embedding table", (torch.float32, torch.bfloat16))
     next_weight, next_eps = next_norm
@@ -2723,6 +2823,14 @@ def embed_rows(tokens: torch.Tensor, table: torch.Tensor, next_norm: tuple):
     if tokens.dim() != 1 or table.dim() != 2 or next_weight.shape != (table.shape[1],) or not 0 < tokens.shape[0] <= ROWS_MAX:
         raise invalid_shape("embed_rows takes 1..16 tokens, a table [vocab, hidden] and a norm weight [hidden]")
     count, hidden = tokens.shape[0], table.shape[1]
+    if dtype == torch.float32:
+        if table.dtype != torch.float32 or table.data_ptr() % 32 != 0 or not _float_norm_folds(next_weight, hidden):
+            return embed_gather(tokens, table), None
+        residual, xg = (torch.empty((count, hidden), dtype=torch.float32, device=table.device) for _ in range(2))
+        ssq = torch.empty((count, hidden // 8), dtype=torch.float32, device=table.device)
+        _check(library().tlie_embed_rows_float(_ptr(tokens), _ptr(table), _ptr(next_weight), _ptr(residual), _ptr(xg), _ptr(ssq), count, hidden,
+                                               _stream()), "embed_rows")
+        return residual, NormedRows(xg, ssq, float(next_eps))
     residual = torch.empty((count, hidden), dtype=torch.float32, device=table.device)
     xg = torch.empty((count, hidden), dtype=torch.bfloat16, device=table.device)
     ssq = torch.empty(((hidden + 15) // 16, 16), dtype=torch.float32, device=table.device)

@@ -201,7 +201,7 @@ class Attention(Mixer):
         return not self.general
 
     def takes_normed_rows(self, rows: int) -> bool:
-        return not self.general and self.qkv.takes_rows(rows)
+        return not self.general and self.qkv.takes_normed(rows)
 
     def cache_need(self):
         """A page holds two planes per kv head, [2, nkv, page_size * d]: the rotated keys as

@@ -118,7 +118,7 @@ class PreNormBlock:
         rows = residual.shape[0]
         if not self.plain:
             return self._forward_general(residual, pending, ctx, binding, first_normed)
-        few = ops.few_rows_route(rows, self.dtype) and (trace is None or getattr(ctx, "trace_serving_route", False))
+        few = ops.folded_route(rows, self.dtype, trace, getattr(ctx, "trace_serving_route", False))
         if trace is not None and not few:
             return self._forward_traced(residual, pending, ctx, binding)
 

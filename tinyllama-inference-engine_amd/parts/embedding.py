@@ -65,7 +65,7 @@ class TokenEmbedding(Part):
 
     def forward_rows(self, tokens: torch.Tensor, next_norm: tuple):
         """For a step of few rows: the residual and the first norm's inputs in one launch."""
-        return ops.embed_rows(tokens, self.table, next_norm)
+        return ops.embed_rows(tokens, self.table, next_norm, self.dtype)
 
 
 @register("head", "lm_head")
@@ -97,7 +97,7 @@ class LMHead(Part):
         self.linear = Linear(matrix, None, self.dtype, keep=partial(keep_in, weights))
 
     def takes_normed_rows(self, rows: int) -> bool:
-        return self.linear.takes_rows(rows)
+        return self.linear.takes_normed(rows)
 
     def forward(self, normed) -> torch.Tensor:
         logits = self.linear(normed, out_dtype=torch.float32, whole=True).dense(torch.float32)

@@ -3,7 +3,8 @@
 
 Which kernel runs is decided here and nowhere else:
   float32 activations            the true 32-bit kernel (32-bit matrix instructions: the bits of plain FMAs), which also
-                                 applies the gated feed-forward's gate itself
+                                 applies the gated feed-forward's gate itself; for at most 16 rows with the norm before, the add
+                                 into the residual or the rotation and cache write folded in
   bfloat16, weight kept float32  the same kernel on widened values
   bfloat16, at most 16 rows      the rows kernel when the caller folds something in: the norm before the
                                  product, the SiLU gate or the add into the residual after it
@@ -42,6 +43,10 @@ class Linear:
         ask for the gate, or for the add into the residual)."""
         return ops.gemm_rows_takes(rows, self.weight, self.dtype)
 
+    def takes_normed(self, rows: int) -> bool:
+        """Whether a step of `rows` rows may bring a `NormedRows`: to the rows kernel, or to the 32-bit product of few rows."""
+        return self.takes_rows(rows) or (self.in_features % 32 == 0 and ops.gemm_generic_rows_takes(rows, self.weight, self.dtype, self.bias))
+
     def relu_squared(self, x, scale: torch.Tensor | None = None, block: int = 1) -> torch.Tensor:
         """s * max(y, 0)^2 in the activation type, y the product with x: applied by the product's own kernel for a step of few
         rows, else by the kernel that adds its parts up.  scale, block: see `ops.relu_squared`."""
@@ -70,8 +75,18 @@ class Linear:
                 return ops.gemm_rows(x, self.weight, self.bias, "rope", rope=rope)
             if isinstance(x, ops.NormedRows):
                 return ops.gemm_rows(x, self.weight, self.bias, "store")
-        if isinstance(x, ops.NormedRows):
-            raise ops.invalid_argument("this product cannot fold the norm before it; ask takes_rows() first")
+        normed = isinstance(x, ops.NormedRows)
+        if (normed or into is not None or rope is not None) and (normed or x.dtype == torch.float32) and ops.gemm_generic_rows_takes(
+                x.shape[0], self.weight, self.dtype, self.bias):
+            if into is not None and self.out_features % 4 == 0:
+                return ops.gemm_generic_rows(x, self.weight, self.bias, "residual", residual=into.residual, next_norm=into.next_norm)
+            if rope is not None and not rope.extra_cols and rope.head_scale is None:
+                return ops.gemm_generic_rows(x, self.weight, self.bias, "rope", rope=rope)
+            if normed:
+                gated = gated and self.out_features % 2 == 0
+                return ops.gemm_generic_rows(x, self.weight, self.bias, "gate" if gated else "store", gate=gate)
+        if normed:
+            raise ops.invalid_argument("this product cannot fold the norm before it; ask takes_normed() first")
         if (ops.gemm_ring_takes(x, self.weight, gated) and (not gated or self.out_features % 2 == 0)
                 and (gated or not whole or out_dtype == torch.float32)):
             return ops.gemm_ring(x, self.weight, self.bias, gated=gated, gate=gate, whole=whole)

@@ -68,7 +68,7 @@ class GatedMLP(FeedForward):
         return True
 
     def takes_normed_rows(self, rows: int) -> bool:
-        return self.activation == "silu" and self.gate_up.takes_rows(rows)
+        return self.activation == "silu" and self.gate_up.takes_normed(rows)
 
     def forward(self, x, ctx, into=None):
         gate = None if self.activation == "silu" else (self.activation, self.alpha, self.limit)
