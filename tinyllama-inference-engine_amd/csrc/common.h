@@ -176,7 +176,7 @@ __device__ __forceinline__ float sum_splits(const D* __restrict__ first, int nsp
 }
 
 // The sum of squares of four, or eight, neighbouring columns of the 32-bit path's norms: one order for every kernel that forms it.
-__device__ __forceinline__ float squares_of4(float a, float b, float c, float d) { return fmaf(d, d, fmaf(c, c, fmaf(b, b, a * a))); }
+__device__ __forceinline__ float squares_of4(float a, float b, float c, float d) { return fmaf(a, a, b * b) + fmaf(c, c, d * d); }
 __device__ __forceinline__ float squares_of8(const float (&v)[8]) {
   return squares_of4(v[0], v[1], v[2], v[3]) + squares_of4(v[4], v[5], v[6], v[7]);
 }

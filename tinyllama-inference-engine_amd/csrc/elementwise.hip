@@ -68,7 +68,7 @@ __device__ __forceinline__ float block_squares(const float* eights, float* block
       float v[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[e] = c + e < chunks ? eights[c + e] : 0.f;
-      sum += (v[0] + v[1]) + (v[2] + v[3]);
+      sum += (v[0] + v[2]) + (v[1] + v[3]);
     }
     sum += __shfl_xor(sum, 1, 64);
     sum += __shfl_xor(sum, 2, 64);

@@ -223,7 +223,7 @@ gemm_generic_few_kernel(const X* __restrict__ x, const W* __restrict__ w, const 
         float sum = 0.f;
 #pragma unroll
         for (int j = 0; j < (SHORT ? 2 : 4); ++j)
-          sum += c0 + 16 * j < chunks ? (square[j].x + square[j].y) + (square[j].z + square[j].w) : 0.f;
+          sum += c0 + 16 * j < chunks ? (square[j].x + square[j].z) + (square[j].y + square[j].w) : 0.f;
         float a = sum, b = sum;
         swap16(a, b);
         a = b = a + b;
