@@ -121,15 +121,29 @@ __device__ __forceinline__ void to_quarters(float& a, float& b, float& c, float&
 __device__ __forceinline__ void to_quarters(float (&v)[4]) { to_quarters(v[0], v[1], v[2], v[3]); }
 __device__ __forceinline__ void to_quarters(float4& v) { to_quarters(v.x, v.y, v.z, v.w); }
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int offset = kWave / 2; offset > 0; offset >>= 1) v += __shfl_xor(v, offset, kWave);
+// Reductions over a whole wave (every lane active), a value with that of lane ^ 32, then ^ 16, 8, 4, 2 and 1, between registers: a
+// shuffle goes through the LDS unit and waits for it six times in a row, 0.25 us that a kernel of 4 us feels.  Once a step has made the
+// lanes of a sixteen repeat, a rotation within the sixteen is the exchange that the next step wants.
+template <typename Join>
+__device__ __forceinline__ float wave_join(float v, Join join) {
+  float a = v, b = v;
+  swap32(a, b);
+  v = a = join(a, b), b = v;
+  swap16(a, b);
+  v = join(a, b);
+#define TLIE_STEP(control) v = join(v, __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), control, 0xf, 0xf, true)));
+  TLIE_STEP(0x128)                                       // row_ror:8
+  TLIE_STEP(0x124)                                       // row_ror:4
+  TLIE_STEP(0x4e)                                        // quad_perm 2 3 0 1
+  TLIE_STEP(0xb1)                                        // quad_perm 1 0 3 2
+#undef TLIE_STEP
   return v;
 }
+__device__ __forceinline__ float wave_sum(float v) {
+  return wave_join(v, [](float a, float b) { return a + b; });
+}
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int offset = kWave / 2; offset > 0; offset >>= 1) v = fmaxf(v, __shfl_xor(v, offset, kWave));
-  return v;
+  return wave_join(v, [](float a, float b) { return fmaxf(a, b); });
 }
 
 // Block-wide reductions over up to 16 waves; `scratch` holds at least 16 floats of LDS.
@@ -173,6 +187,28 @@ __device__ __forceinline__ float sum_splits(const D* __restrict__ first, int nsp
   }
   for (; s < nsplit; ++s) a += to_float(first[s * stride]);
   return (a + b) + (c + d);
+}
+
+// Eight neighbouring elements summed over the parts of a split product, in the order of their index.  The parts are asked for eight at a
+// time: one after the other, each waits for the one before, and a kernel of few rows is little else than that chain (the norm after a
+// product of 64 rows in 8 parts, 2048 columns, 5.2 us one by one, 4.7 so).
+template <typename D>
+__device__ __forceinline__ void load8_splits(const D* __restrict__ part, int nsplit, size_t stride, float (&d)[8]) {
+  load8(part, d);
+  if (sizeof(D) < sizeof(float)) return;                     // (parts are floats: this is a whole product)
+  constexpr int kTogether = 8;
+  for (int s = 1; s < nsplit; s += kTogether) {
+    float more[kTogether][8];
+#pragma unroll
+    for (int u = 0; u < kTogether; ++u)
+      if (s + u < nsplit) load8(part + (s + u) * stride, more[u]);       // (the same for the whole grid)
+#pragma unroll
+    for (int u = 0; u < kTogether; ++u) {
+      if (s + u >= nsplit) break;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) d[j] += more[u][j];
+    }
+  }
 }
 
 // The sum of squares of four, or eight, neighbouring columns of the 32-bit path's norms: one order for every kernel that forms it.

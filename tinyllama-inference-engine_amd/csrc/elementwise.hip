@@ -93,20 +93,16 @@ __global__ void add_rmsnorm_wide_kernel(float* __restrict__ residual, const D* _
   const int r = blockIdx.x;
   const int src = rows ? rows[r] : r;
   float* res = residual + static_cast<size_t>(src) * hidden;
-  float square = 0.f;
+  float square = 0.f, first_weight[8];
+  const int first = threadIdx.x * 8;
+  const bool ahead = sizeof(D) == sizeof(float) && out && first < hidden;       // (few rows: the weight is asked for ahead of the sums)
+  if (ahead) load8(weight + first, first_weight);
   for (int i = threadIdx.x * 8; i < hidden; i += blockDim.x * 8) {
     float v[8];
     load8(res + i, v);
     if (delta) {
-      const D* part = delta + static_cast<size_t>(src) * hidden + i;
       float d[8];
-      load8(part, d);
-      for (int s = 1; s < nsplit; ++s) {
-        float more[8];
-        load8(part + s * split_stride, more);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) d[j] += more[j];
-      }
+      load8_splits(delta + static_cast<size_t>(src) * hidden + i, nsplit, split_stride, d);
 #pragma unroll
       for (int j = 0; j < 8; ++j) v[j] += d[j];
       if (!rows) store8(res + i, v);
@@ -126,11 +122,11 @@ __global__ void add_rmsnorm_wide_kernel(float* __restrict__ residual, const D* _
   if (out) {
     O* o = out + static_cast<size_t>(r) * hidden;
     for (int i = threadIdx.x * 8; i < hidden; i += blockDim.x * 8) {
-      float v[8], w[8];
+      float v[8];
       load8(row_cache + i, v);                   // the thread's own entries
-      load8(weight + i, w);
+      if (!ahead || i != first) load8(weight + i, first_weight);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] = sizeof(O) == sizeof(float) ? v[j] * w[j] * scale : v[j] * scale * w[j];
+      for (int j = 0; j < 8; ++j) v[j] = sizeof(O) == sizeof(float) ? v[j] * first_weight[j] * scale : v[j] * scale * first_weight[j];
       store8(o + i, v);
     }
   }
@@ -167,17 +163,8 @@ __global__ void silu_mul_wide_kernel(const D* __restrict__ gate_up, int nsplit, 
     const D* base = gate_up + t * 2 * inter;
     float a[8], b[8], g[8], u[8];
     const int first = interleaved ? 2 * i : i, second = interleaved ? 2 * i + 8 : inter + i;
-    load8(base + first, a);
-    load8(base + second, b);
-    for (int s = 1; s < nsplit; ++s) {
-      float more[8];
-      load8(base + s * split_stride + first, more);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) a[j] += more[j];
-      load8(base + s * split_stride + second, more);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) b[j] += more[j];
-    }
+    load8_splits(base + first, nsplit, split_stride, a);
+    load8_splits(base + second, nsplit, split_stride, b);
     if (interleaved) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -243,15 +230,8 @@ __global__ void norm_add_rmsnorm_wide_kernel(float* __restrict__ residual, const
   float* res = residual + static_cast<size_t>(src) * hidden;
   float square = 0.f;
   for (int i = threadIdx.x * 8; i < hidden; i += blockDim.x * 8) {
-    const D* part = delta + static_cast<size_t>(src) * hidden + i;
     float d[8];
-    load8(part, d);
-    for (int s = 1; s < nsplit; ++s) {
-      float more[8];
-      load8(part + s * split_stride, more);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) d[j] += more[j];
-    }
+    load8_splits(delta + static_cast<size_t>(src) * hidden + i, nsplit, split_stride, d);
     store8(row_cache + i, d);                    // (a thread reads back only what it wrote itself)
 #pragma unroll
     for (int j = 0; j < 8; ++j) square += d[j] * d[j];
