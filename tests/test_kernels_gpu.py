@@ -165,6 +165,47 @@ def added_up(parts):
     return parts[0] if len(parts) == 1 else (chains[0] + chains[1]) + (chains[2] + chains[3])
 
 
+@pytest.mark.parametrize("nsplit", [2, 3, 4, 5, 8, 9, 10, 17, 18, 32, 37])
+def test_parts_of_a_split_product_meet_in_their_order(nsplit):
+    """The kernels that ask for many parts together add them up as one after the other: the bits of the same call on the sum, formed
+    beforehand in that order (four interleaved chains, or one part after the other), around the numbers asked for at once."""
+    from tlie_amd import ops
+    torch.manual_seed(nsplit)
+
+    def in_turn(parts):
+        total = parts[0].clone()
+        for part in parts[1:]:
+            total += part
+        return total
+    for tokens, hidden in ((1, 8), (3, 272), (2, 2064)):
+        parts = torch.randn(nsplit, tokens, hidden, device=DEV)
+        weight, bias, start = torch.randn(hidden, device=DEV), torch.randn(hidden, device=DEV), torch.randn(tokens, hidden, device=DEV)
+        split, whole = ops.Product(parts, nsplit), ops.Product(in_turn(parts), 1)
+        for norm in (lambda residual, delta: ops.add_rmsnorm(residual, delta, weight, 1e-5, torch.float32),
+                     lambda residual, delta: ops.add_rmsnorm(residual, delta, weight, 1e-5, torch.bfloat16),
+                     lambda residual, delta: ops.layer_norm(residual, delta, weight, bias, 1e-5, torch.float32),
+                     lambda residual, delta: ops.norm_add_rmsnorm(residual, delta, weight, 1e-5, weight, 1e-5, torch.float32)):
+            one, other = start.clone(), start.clone()
+            assert torch.equal(norm(one, split), norm(other, whole)) and torch.equal(one, other), (tokens, hidden)
+        gated = whole if hidden % 16 == 0 else ops.Product(added_up(parts), 1)
+        assert torch.equal(ops.silu_mul(split, torch.float32), ops.silu_mul(gated, torch.float32))
+    for heads, dv in ((3, 40), (2, 64), (5, 72), (1, 200), (2, 512), (1, 520), (2, 604)):
+        together = in_turn if dv == 520 else added_up            # (a head of more than 512 dims in eights: one part after the other)
+        parts, a = torch.randn(nsplit, 3, heads * dv + 8, device=DEV), torch.randn(3, heads * dv, device=DEV)
+        weight = torch.randn(heads * dv, device=DEV)
+        for first in (False, True):
+            one, other = (ops.head_combine(a, heads, dv, 1e-5, torch.float32, weight=weight, gate=gate, gate_col=8, gate_kind="silu", gate_first=first)
+                          for gate in (ops.Product(parts, nsplit), ops.Product(together(parts), 1)))
+            assert torch.equal(one, other), (heads, dv, first)
+    for rank in (1, 7, 64, 72):
+        parts = torch.randn(nsplit, 2, rank, device=DEV)
+        weight = torch.randn(300, rank, device=DEV) / math.sqrt(rank)
+        one, other = (ops.low_rank_decay(low, weight, None, "exp_neg_exp", inner_tanh=True)
+                      for low in (ops.Product(parts, nsplit), ops.Product(added_up(parts), 1)))
+        assert torch.equal(one, other), rank
+        assert rel_err(one, torch.exp(-torch.exp(torch.tanh(parts.double().sum(0)) @ weight.double().T))) < 1e-5
+
+
 @pytest.mark.parametrize("rows, n, k, whole", [(24, 12288, 4096, False), (64, 4096, 11008, False), (64, 2304, 14336, False), (24, 9000, 4096, True),
                                                (17, 2048, 1536, True), (20, 11264, 2048, False), (33, 4096, 14336, False)])
 def test_gemm_ring_is_as_exact_as_the_product_it_stands_in_for(rows, n, k, whole):
