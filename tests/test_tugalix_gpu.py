@@ -190,6 +190,52 @@ def test_the_input_convolution_carries_its_last_inputs(taps, channels, plan, out
         assert torch.equal(state[2].cpu(), inputs[0][-(taps - 1):])
 
 
+@pytest.mark.parametrize("hidden,nsplit,entries", [(8, 1, 0), (104, 3, 2), (2048, 9, 6), (2056, 1, 1), (4104, 2, 5)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_the_norm_applies_the_convolution_behind_it(hidden, nsplit, entries, dtype):
+    """One token a sequence, slots in no order, one token that pads the step, rows of one pass of the threads and more: the bits of the norm
+    and the convolution one after the other, results, residual and state, and a slot that is nobody's stays as it is."""
+    from tlie_amd import ops
+    generator = torch.Generator(device=DEVICE).manual_seed(hidden)
+    tokens, slots = 4, [3, -1, 0, 4]
+
+    def drawn(*shape):
+        return torch.randn(*shape, generator=generator, device=DEVICE)
+    weight, bias, taps = drawn(hidden).to(dtype), drawn(hidden).to(dtype), drawn(hidden, 4).to(dtype)
+    parts, history = drawn(nsplit, tokens, hidden), drawn(max(entries, 1), tokens, hidden)
+    shares, areas = drawn(entries).to(dtype), drawn(5, 2, 3, hidden)
+    place = torch.tensor(slots, dtype=torch.int32, device=DEVICE)
+    ctx = SimpleNamespace(max_new=1, num_seqs=tokens, num_tokens=tokens, token_slot=place, seq_slot=place, trace=None,
+                          token_seq=torch.arange(tokens, dtype=torch.int32, device=DEVICE),
+                          seq_start=torch.arange(tokens + 1, dtype=torch.int32, device=DEVICE))
+    results = []
+    for together in (False, True):
+        earlier, area = history.clone(), areas.clone()
+        state, residual, mixed = area[:, 1], earlier[-1], torch.zeros(tokens, hidden, device=DEVICE)
+        mix = dict(history=earlier, history_count=entries, history_weight=shares, mixed=mixed) if entries else {}
+        conv = ops.conv_after(taps, state, ctx, ops.NormParams(weight, bias, 1e-5, True), dtype)
+        assert conv is not None
+        out = ops.layer_norm(residual, ops.Product(parts, nsplit), weight, bias, 1e-5, torch.float32, conv=conv if together else None, **mix)
+        results.append((out if together else ops.input_conv(out, taps, state, ctx, dtype), residual, mixed, area))
+    for one, other in zip(*results):
+        assert one.dtype == other.dtype and torch.equal(one, other)
+    assert torch.equal(results[1][3][[1, 2]], areas[[1, 2]]) and torch.equal(results[1][3][:, 0], areas[:, 0])
+
+
+def test_the_norm_leaves_the_convolution_where_it_cannot_apply_it():
+    from tlie_amd import ops
+    weight, taps, state = (torch.zeros(shape, device=DEVICE) for shape in ((16,), (16, 4), (2, 3, 16)))
+    norm = ops.NormParams(weight, None, 1e-5, True)
+
+    def ctx(max_new=1, seqs=2):
+        return SimpleNamespace(max_new=max_new, num_seqs=seqs, num_tokens=2, token_slot=torch.zeros(2, dtype=torch.int32, device=DEVICE))
+    assert ops.conv_after(taps, state, ctx(), norm, torch.float32) is not None
+    assert ops.conv_after(taps, state, ctx(max_new=2, seqs=1), norm, torch.float32) is None          # two tokens of one sequence
+    assert ops.conv_after(taps, state, ctx(), norm, torch.bfloat16) is None                          # a result of another type
+    assert ops.conv_after(taps[:, :2].contiguous(), state[:, :1], ctx(), norm, torch.float32) is None
+    assert ops.conv_after(taps[:12], state[..., :12], ctx(), ops.NormParams(weight[:12], None, 1e-5, True), torch.float32) is None
+
+
 @pytest.mark.parametrize("width,mixes,plan,dtype", [(80, 5, SHORT_STEPS, torch.float32), (44, 1, LONG_STEPS, torch.float32),
                                                     (203, 5, SHORT_STEPS, torch.bfloat16)])
 def test_the_token_shift_blends_with_the_token_before(width, mixes, plan, dtype):

@@ -72,14 +72,24 @@ layer_norm_kernel(float* __restrict__ residual, const D1* __restrict__ d1, int n
 // product lie a multiple of eight elements apart; the summands of a split product are added in the order of their index.
 // A few rows are bound by the way of their loads: what a thread's first eight elements need is asked for at once, the earlier results of
 // a depth mix four at a time, weight and bias ahead of the sums they are used behind (4 rows of 2048, 8 parts, up to 5 results: 7.4 -> 6.4 us).
-template <typename D1, typename D2, typename W, typename O>
+// CONV: what leaves is h + conv(h) of the normed row h, the input convolution below of four taps, in a step in which every sequence
+// brings one token (decoding): a channel's earlier inputs are the sequence's state, which takes the new one, and a launch of 4 us with
+// a way to memory of its own goes (4 rows of 2048: 8.1 us in place of 6.4 + 4.1).  Same sums in the same order, the same bits.
+struct ConvAfter {
+  const void* taps;          // [hidden, 4] in the norm's weights' type
+  float* state;              // [slots, 3, hidden], the slots slot_stride floats apart
+  const int* token_slot;     // [tokens]; negative: a token that pads a recorded step, zeros leave
+  size_t slot_stride;
+};
+
+template <typename D1, typename D2, typename W, typename O, bool CONV>
 __global__ void __launch_bounds__(256)
 layer_norm_wide_kernel(float* __restrict__ residual, const D1* __restrict__ d1, int n1, size_t stride1, float s1,
                        const D2* __restrict__ d2, int n2, size_t stride2, float s2, const float* __restrict__ row_scale,
                        int row_scale_stride, int centred, const float* __restrict__ history, size_t history_stride,
                   int history_count, const W* __restrict__ history_weight, float* __restrict__ mixed,
                        const W* __restrict__ weight, const W* __restrict__ bias, float eps, O* __restrict__ out,
-                       const int* __restrict__ rows, int hidden) {
+                       const int* __restrict__ rows, int hidden, ConvAfter conv) {
   extern __shared__ float row_values[];
   __shared__ float scratch[16];
   const int t = rows != nullptr ? rows[blockIdx.x] : blockIdx.x;
@@ -90,6 +100,20 @@ layer_norm_wide_kernel(float* __restrict__ residual, const D1* __restrict__ d1, 
   if (out != nullptr && first < hidden) {
     load8(weight + first, first_weight);
     if (bias != nullptr) load8(bias + first, first_bias);
+  }
+  const W* taps = static_cast<const W*>(conv.taps);
+  float first_taps[CONV ? 4 : 1][8], first_held[CONV ? 3 : 1][8];
+  int slot = 0;
+  auto ask_conv = [&](int c) {                         // (a channel's four taps lie side by side: eight channels are four pieces)
+#pragma unroll
+    for (int p = 0; p < (CONV ? 4 : 0); ++p) load8(taps + static_cast<size_t>(c) * 4 + 8 * p, first_taps[p]);
+#pragma unroll
+    for (int j = 0; j < (CONV ? 3 : 0); ++j)
+      if (slot >= 0) load8(conv.state + slot * conv.slot_stride + static_cast<size_t>(j) * hidden + c, first_held[j]);
+  };
+  if (CONV) {
+    slot = conv.token_slot[t];
+    if (first < hidden) ask_conv(first);
   }
   float sum = 0.f;                                     // of x, or (not centred) of x^2
   for (int c = threadIdx.x * 8; c < hidden; c += blockDim.x * 8) {
@@ -161,6 +185,25 @@ layer_norm_wide_kernel(float* __restrict__ residual, const D1* __restrict__ d1, 
       if (c != first) load8(bias + c, first_bias);
 #pragma unroll
       for (int j = 0; j < 8; ++j) x[j] += first_bias[j];
+    }
+    if constexpr (CONV) {
+      if (c != first) ask_conv(c);
+      float y[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        float acc = x[j];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc += first_taps[(4 * j + i) / 8][(4 * j + i) % 8] * (i < 3 ? first_held[i < 3 ? i : 0][j] : x[j]);
+        y[j] = slot < 0 ? 0.f : acc;
+      }
+      if (slot >= 0) {
+        float* held = conv.state + slot * conv.slot_stride + c;
+        store8(held, first_held[1]);
+        store8(held + hidden, first_held[2]);
+        store8(held + 2 * static_cast<size_t>(hidden), x);
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[j] = y[j];
     }
     store8(dst + c, x);
   }
@@ -419,12 +462,12 @@ static inline bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>
 // row_scale); centred: take the mean off (0: an RMS norm); history (or null, with history_count 0): float, entry j at history + j * history_stride, the last
 // entry being the residual itself; history_weight: [history_count] of w_dtype; mixed: float [tokens, hidden]; weight,
 // bias (bias may be null) [hidden] of w_dtype; out (or null) [count, hidden] of out_dtype; rows (or null): int [count].
-extern "C" int tlie_layer_norm(float* residual, const void* d1, int d1_dtype, int n1, long long stride1, float s1,
+static int layer_norm_entry(float* residual, const void* d1, int d1_dtype, int n1, long long stride1, float s1,
                                const void* d2, int d2_dtype, int n2, long long stride2, float s2, const float* row_scale,
                                int row_scale_stride, int centred, const float* history, long long history_stride,
                                int history_count, const void* history_weight, float* mixed,
                                const void* weight, const void* bias, int w_dtype, float eps, void* out, int out_dtype,
-                               const int* rows, int count, int hidden, void* stream) {
+                               const int* rows, int count, int hidden, const ConvAfter& conv, void* stream) {
   if (count <= 0 || hidden <= 0 || hidden > 16000 || history_count < 0 || n1 < 1 || n2 < 1) return kBadArgument;
   if (row_scale != nullptr && row_scale_stride < 1) return kBadArgument;
   if (history_count > 0 && (history == nullptr || history_weight == nullptr || (rows == nullptr && mixed == nullptr))) return kBadArgument;
@@ -435,15 +478,26 @@ extern "C" int tlie_layer_norm(float* residual, const void* d1, int d1_dtype, in
   const bool wide = hidden % 8 == 0 && (d1 == nullptr || n1 == 1 || stride1 % 8 == 0) && (d2 == nullptr || n2 == 1 || stride2 % 8 == 0) &&
                     (history_count == 0 || history_stride % 8 == 0) && aligned16(residual) && aligned16(d1) && aligned16(d2) &&
                     aligned16(history) && aligned16(mixed) && aligned16(weight) && aligned16(bias) && aligned16(out);
+  if (conv.taps != nullptr && (!wide || out == nullptr || rows != nullptr || conv.state == nullptr || conv.token_slot == nullptr ||
+                               !aligned16(conv.taps) || !aligned16(conv.state) || conv.slot_stride % 4 != 0))
+    return kBadArgument;
   int threads = 64;                                    // as many waves as the row has work for (at most four)
   while (threads < 256 && threads * 8 < hidden) threads *= 2;
 #define TLIE_CASE(C1, D1, C2, D2, WC, W, OC, O)                                                                          \
   if (d1_dtype == C1 && d2_dtype == C2 && w_dtype == WC && out_dtype == OC) {                                            \
-    if (wide)                                                                                                            \
-      hipLaunchKernelGGL((layer_norm_wide_kernel<D1, D2, W, O>), dim3(count), dim3(threads), lds, s, residual,            \
+    if (conv.taps != nullptr) {                                                                                          \
+      if constexpr (sizeof(W) == sizeof(O))                                                                              \
+        hipLaunchKernelGGL((layer_norm_wide_kernel<D1, D2, W, O, true>), dim3(count), dim3(threads), lds, s, residual,   \
+                           (const D1*)d1, n1, (size_t)stride1, s1, (const D2*)d2, n2, (size_t)stride2, s2, row_scale,    \
+                           row_scale_stride, centred, history, (size_t)history_stride, history_count,                    \
+                           (const W*)history_weight, mixed, (const W*)weight, (const W*)bias, eps, (O*)out, rows, hidden, conv);  \
+      else                                                                                                               \
+        return kBadArgument;                                                                                             \
+    } else if (wide)                                                                                                     \
+      hipLaunchKernelGGL((layer_norm_wide_kernel<D1, D2, W, O, false>), dim3(count), dim3(threads), lds, s, residual,            \
                          (const D1*)d1, n1, (size_t)stride1, s1, (const D2*)d2, n2, (size_t)stride2, s2, row_scale,     \
                          row_scale_stride, centred, history, (size_t)history_stride, history_count,                        \
-                         (const W*)history_weight, mixed, (const W*)weight, (const W*)bias, eps, (O*)out, rows, hidden);  \
+                         (const W*)history_weight, mixed, (const W*)weight, (const W*)bias, eps, (O*)out, rows, hidden, conv);  \
     else                                                                                                                 \
       hipLaunchKernelGGL((layer_norm_kernel<D1, D2, W, O>), dim3(count), dim3(256), lds, s, residual, (const D1*)d1, n1,  \
                          (size_t)stride1, s1, (const D2*)d2, n2, (size_t)stride2, s2, row_scale, row_scale_stride, centred,       \
@@ -462,6 +516,19 @@ extern "C" int tlie_layer_norm(float* residual, const void* d1, int d1_dtype, in
   TLIE_CASE(kBF16, bf16, kBF16, bf16, kBF16, bf16, kBF16, bf16)
 #undef TLIE_CASE
   return kBadArgument;
+}
+
+extern "C" int tlie_layer_norm(float* residual, const void* d1, int d1_dtype, int n1, long long stride1, float s1,
+                               const void* d2, int d2_dtype, int n2, long long stride2, float s2, const float* row_scale,
+                               int row_scale_stride, int centred, const float* history, long long history_stride,
+                               int history_count, const void* history_weight, float* mixed,
+                               const void* weight, const void* bias, int w_dtype, float eps, void* out, int out_dtype,
+                               const int* rows, int count, int hidden, const void* taps, float* state, const int* token_slot,
+                               long long slot_stride, void* stream) {
+  // taps (or null), state, token_slot, slot_stride: see ConvAfter; weights and result are then of one type
+  return layer_norm_entry(residual, d1, d1_dtype, n1, stride1, s1, d2, d2_dtype, n2, stride2, s2, row_scale, row_scale_stride, centred, history,
+                          history_stride, history_count, history_weight, mixed, weight, bias, w_dtype, eps, out, out_dtype, rows, count, hidden,
+                          ConvAfter{taps, state, token_slot, static_cast<size_t>(slot_stride)}, stream);
 }
 
 extern "C" int tlie_input_conv(const float* h, const void* taps, int taps_dtype, float* state, const int* token_seq,

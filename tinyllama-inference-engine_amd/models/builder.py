@@ -202,7 +202,11 @@ class DecoderModel:
                 rows = None if ctx.wants_all_rows else ctx.want_rows
                 normed = next_norm.add_forward(history[index + 1], pending, rows=rows, mixed=history[index + 2], **mix)
             else:
-                normed = next_norm.add_forward(history[index + 1], pending, mixed=history[index + 2], **mix)
+                # (what stands between that norm and the next run's mixer it may apply too)
+                after = self.blocks[runs[index + 1].layer] if not last else None
+                conv = after.entry_conv(ctx, bindings[index + 1]) if hasattr(after, "entry_conv") else None
+                behind = {"conv": conv} if conv is not None else {}
+                normed = next_norm.add_forward(history[index + 1], pending, mixed=history[index + 2], **mix, **behind)
                 if trace is not None:
                     trace[f"layer{index}.mixed"] = history[index + 2].clone()
                     if last:

@@ -792,13 +792,19 @@ class ScaledSum:
 def layer_norm(residual: torch.Tensor, delta, weight: torch.Tensor | None, bias: torch.Tensor | None, eps: float,
                out_dtype: torch.dtype, rows: torch.Tensor | None = None, history: torch.Tensor | None = None,
                history_count: int = 0, history_weight: torch.Tensor | None = None, mixed: torch.Tensor | None = None,
-               want_out: bool = True, centred: bool = True) -> torch.Tensor | None:
+               want_out: bool = True, centred: bool = True, conv: "ConvAfter | None" = None) -> torch.Tensor | None:
     """residual += delta (a Product, a ScaledSum or None; all rows, in place), then out = (x - mean) / sqrt(var + eps)
     * weight + bias of every row, means and variances float (centred False: an RMS norm, x / sqrt(mean(x^2) + eps) * weight).  With `history` (float32 [entries, tokens, hidden] of which
     the first history_count are read, the last of them being `residual` itself) what is normed is the weighted sum
     sum_j history_weight[j] * history[j], which is also written to `mixed`.  With `rows` (int32 indices) only those
-    rows are normed and nothing but the result is written.  want_out False: only the sums."""
+    rows are normed and nothing but the result is written.  want_out False: only the sums.  conv (of `conv_after`, without `rows`):
+    the result is `input_conv` of the normed rows, in the norm's weights' type."""
     _device_tensor(residual, "residual", torch.float32)
+    if conv is not None:
+        out_dtype = weight.dtype
+        if (rows is not None or not want_out or conv.taps.dtype != weight.dtype or conv.taps.shape != (residual.shape[-1], 4)
+                or conv.token_slot.shape != (residual.shape[0],) or tuple(conv.state.shape[1:]) != (3, residual.shape[-1])):
+            raise invalid_shape("layer_norm: the convolution behind it takes all rows, four taps in the weights' type and a state of three rows")
     if residual.dim() != 2:
         raise invalid_shape("layer_norm: the residual is [tokens, hidden]")
     tokens, hidden = residual.shape
@@ -865,8 +871,35 @@ def layer_norm(residual: torch.Tensor, delta, weight: torch.Tensor | None, bias:
         _ptr(history if history_count > 0 else None), ctypes.c_longlong(tokens * hidden), int(history_count),
         _ptr(history_weight if history_count > 0 else None), _ptr(mixed if history_count > 0 and rows is None else None),
         _ptr(weight if want_out else None), _ptr(bias if want_out else None), w_code, ctypes.c_float(eps if want_out else 1.0),
-        _ptr(out), dtype_code(out_dtype), _ptr(rows), count, hidden, _stream()), "layer_norm")
+        _ptr(out), dtype_code(out_dtype), _ptr(rows), count, hidden, _ptr(conv.taps if conv is not None else None),
+        _ptr(conv.state if conv is not None else None), _ptr(conv.token_slot if conv is not None else None),
+        ctypes.c_longlong(conv.state.stride(0) if conv is not None else 0), _stream()), "layer_norm")
     return out
+
+
+@dataclass
+class ConvAfter:
+    """An input convolution of four taps for the norm before it to apply, in a step of one token a sequence."""
+    taps: torch.Tensor
+    state: torch.Tensor
+    token_slot: torch.Tensor
+
+
+@dataclass
+class Convolved:
+    """A sublayer's input: the norm before it has applied the convolution too."""
+    rows: torch.Tensor
+
+
+def conv_after(taps: torch.Tensor, state: torch.Tensor, ctx, norm: "NormParams", out_dtype: torch.dtype) -> "ConvAfter | None":
+    """What `layer_norm` needs to apply `input_conv` to its own result, where its kernel can: every sequence of the step brings one
+    token (the convolution of several reads rows that other workgroups norm), four taps, and taps, norm and result of one type in
+    rows that 16-byte loads fit; else None."""
+    tensors = [norm.weight, taps, state] + ([norm.bias] if norm.bias is not None else [])
+    if (ctx.max_new != 1 or ctx.num_seqs != ctx.num_tokens or taps.shape[1] != 4 or taps.shape[0] % 8 != 0 or state.stride(0) % 4 != 0
+            or taps.dtype != norm.weight.dtype or taps.dtype != out_dtype or any(tensor.data_ptr() % 16 != 0 for tensor in tensors)):
+        return None
+    return ConvAfter(taps, state, ctx.token_slot)
 
 
 @dataclass

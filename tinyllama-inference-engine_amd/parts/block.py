@@ -97,6 +97,16 @@ class PreNormBlock:
         the block (the embedding, the block before) may leave that norm's inputs with it."""
         return self.mixer_norm
 
+    def entry_conv(self, ctx, binding):
+        """What stands between the first norm and the mixer, for the norm to apply, or None (see `ops.conv_after`)."""
+        return self.mixer_input.behind(self.mixer_norm, ctx, binding.block_state[:, 0]) if self.mixer_input is not None else None
+
+    @staticmethod
+    def _normed(norm, residual, delta, conv):
+        if conv is None or isinstance(delta, (ops.PostNormed, ops.NormedDelta)):
+            return norm.add_forward(residual, delta)
+        return norm.add_forward(residual, delta, conv=conv)
+
     @property
     def graph_safe(self) -> bool:
         return all(getattr(getattr(self, attribute), "graph_safe", False) for attribute, _, _ in self._parts(self.layer))
@@ -155,16 +165,23 @@ class PreNormBlock:
         def keep(name, tensor):
             if trace is not None:
                 trace[ctx.trace_prefix + name] = tensor.float().clone()
-        normed = first_normed if first_normed is not None else self.mixer_norm.add_forward(residual, pending)
-        if self.mixer_input is not None:
+        normed = first_normed if first_normed is not None else self._normed(self.mixer_norm, residual, pending, self.entry_conv(ctx, binding))
+        if isinstance(normed, ops.Convolved):
+            normed = normed.rows
+        elif self.mixer_input is not None:
             normed = self.mixer_input.forward(normed, ctx, binding.block_state[:, 0])
         keep("input_norm", normed)
         out = self.mixer.forward(normed, ctx, binding)
         if trace is not None:
             keep("attention_output", as_product(out).dense(torch.float32))
         if self.feed_forward is not None:
-            normed = self.feed_forward_norm.add_forward(residual, out)
+            conv = None
             if self.feed_forward_input is not None:
+                conv = self.feed_forward_input.behind(self.feed_forward_norm, ctx, binding.block_state[:, -1])
+            normed = self._normed(self.feed_forward_norm, residual, out, conv)
+            if isinstance(normed, ops.Convolved):
+                normed = normed.rows
+            elif self.feed_forward_input is not None:
                 normed = self.feed_forward_input.forward(normed, ctx, binding.block_state[:, -1])
             keep("post_attention_norm", normed)
             out = self.feed_forward.forward(normed, ctx)

@@ -39,6 +39,12 @@ class ResidualConv(Part):
         """Of a request's state: the last taps - 1 inputs, oldest first (one row at least)."""
         return (max(self.taps - 1, 1), self.size)
 
+    def behind(self, norm, ctx, state: torch.Tensor) -> "ops.ConvAfter | None":
+        """For the norm before it to apply this convolution in its own kernel, where both can (`ops.conv_after`)."""
+        if getattr(ctx, "trace", None) is not None or not getattr(norm, "applies_conv", False):
+            return None
+        return ops.conv_after(self.weight, state, ctx, norm.params(), self.dtype)
+
     def forward(self, h: torch.Tensor, ctx, state: torch.Tensor) -> torch.Tensor:
         return ops.input_conv(h, self.weight, state, ctx, self.dtype)
 

@@ -115,9 +115,17 @@ class LayerNorm(Norm):
     def params(self) -> ops.NormParams:
         return ops.NormParams(self.weight, self.bias, self.eps, True)
 
-    def add_forward(self, residual, delta, rows=None, lazy=False, **history):
+    applies_conv = True           # (`conv` of `add_forward`)
+
+    def add_forward(self, residual, delta, rows=None, lazy=False, conv=None, **history):
         """history: `history`, `history_count`, `history_weight`, `mixed` of `ops.layer_norm`: the norm then reads a
-        weighted sum over earlier residuals in the residual's place."""
+        weighted sum over earlier residuals in the residual's place.  conv (an `ops.ConvAfter`; of a sublayer's result or none): what
+        stands behind this norm, applied here; an `ops.Convolved` then comes back."""
+        if conv is not None:
+            if isinstance(delta, (ops.PostNormed, NormedDelta)):
+                raise ops.invalid_argument("a convolution behind a norm goes with results that join the residual as they are")
+            delta = None if isinstance(delta, ResidualUpdated) else delta
+            return ops.Convolved(ops.layer_norm(residual, delta, self.weight, self.bias, self.eps, self.out_dtype, rows=rows, conv=conv, **history))
         if isinstance(delta, ops.PostNormed) and not history:
             return ops.post_norm(residual, delta, self.out_dtype, last=self.params(), rows=rows)
         if isinstance(delta, ResidualUpdated):
