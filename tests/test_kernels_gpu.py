@@ -251,12 +251,12 @@ def test_gemm_generic_at_the_edges_of_its_kernels_and_gated(n, k):
 
 
 @pytest.mark.parametrize("rows", [1, 7, 8, 9, 16])
-@pytest.mark.parametrize("k, n, heads", [(32, 96, (3, 1, 10, 4)), (96, 256, (3, 1, 32, 32)), (256, 64, (2, 2, 16, 16)), (288, 2048, (4, 2, 6, 0)),
-                                         (512, 544, (2, 1, 66, 64)), (544, 2080, (32, 4, 64, 64)), (2048, 2048, (24, 4, 80, 40)),
-                                         (8224, 64, (1, 1, 16, 16))])
+@pytest.mark.parametrize("k, n, heads", [(544, 576, (3, 1, 10, 4)), (576, 608, (3, 1, 32, 32)), (1024, 640, (2, 2, 16, 16)), (1056, 2048, (4, 2, 6, 0)),
+                                         (1504, 544, (2, 1, 66, 64)), (544, 2080, (32, 4, 64, 64)), (2048, 2048, (24, 4, 80, 40)),
+                                         (8224, 544, (1, 1, 16, 16))])
 def test_gemm_generic_rows_gives_the_bits_of_the_kernels_it_stands_in_for(rows, k, n, heads):
-    """At most 16 rows in 32 bits with the norm before and the gate, the add or the rotation and cache write after: one part of the ring
-    and more, one block of K, two at once, more blocks than waves, shares of rows (2560 and 2080 columns), heads that no
+    """At most 16 rows in 32 bits with the norm before and the gate, the add or the rotation and cache write after: ragged blocks
+    of K, two at once, more blocks than waves, shares of rows (2560 and 2080 columns), heads that no
     group of four columns divides; against the norm, the product and the rotation as kernels of their own, bit for bit."""
     from tlie_amd import ops
     torch.manual_seed(rows * n + k)
@@ -299,18 +299,20 @@ def test_gemm_generic_rows_gives_the_bits_of_the_kernels_it_stands_in_for(rows, 
 
 def test_gemm_generic_rows_refuses_what_it_does_not_take():
     from tlie_amd import ops
-    w, x = torch.randn(24, 16, device=DEV), torch.randn(17, 16, device=DEV)
+    w, x = torch.randn(24, 544, device=DEV), torch.randn(17, 544, device=DEV)
     with pytest.raises(Exception):
         ops.gemm_generic_rows(x, w, None)                                                           # 17 rows
     with pytest.raises(Exception):
-        ops.gemm_generic_rows(x[:4, :14].contiguous(), w[:, :14].contiguous(), None)                # no 16-byte rows
+        ops.gemm_generic_rows(x[:4, :542].contiguous(), w[:, :542].contiguous(), None)              # no 16-byte rows
+    with pytest.raises(Exception):
+        ops.gemm_generic_rows(x[:4, :512].contiguous(), w[:, :512].contiguous(), None)              # one block of K
     with pytest.raises(Exception):
         ops.gemm_generic_rows(x[:4], w, None, "residual", residual=torch.zeros(5, 24, device=DEV))
     with pytest.raises(Exception):
         ops.gemm_generic_rows(ops.NormedRows(x[:4], torch.zeros(4, 3, device=DEV), 1e-5), w, None)  # sums of squares of another width
     narrow = torch.randn(24, device=DEV)
     assert ops.gemm_generic_rows(x[:4], w, None, "residual", residual=torch.zeros(4, 24, device=DEV),
-                                 next_norm=(narrow, 1e-5)).normed is None                           # 24 columns: no 32
+                                 next_norm=(narrow, 1e-5)).normed is None                           # 24 columns
 
 
 @pytest.mark.parametrize("n, k", [(11262, 1030), (11262, 1028), (4610, 517)])

@@ -151,15 +151,13 @@ __device__ __forceinline__ void fold_rotation(const RowsFold& fold, const FoldAh
 // two blocks of K: lanes 0 .. 7 of a sixteen bring both operands' rows from the one block, lanes 8 .. 15 from the other.
 // Twice the workgroups of R = 16, and no lane brings what another one has.
 // FOLD: a layer's neighbouring arithmetic in the same kernel, described by `RowsFold` (at most 16 rows of x, all in 32 bits; the bits
-// are those of the kernels it stands in for).  SHORT: K is at most 256, one part of the ring: what lies past K is neither asked
-// for nor multiplied (96 x 96: 24 instructions of a chain in place of 64).
-template <typename X, typename W, typename O, int MT, int R, bool PAIR, int RING, int WAVES, bool WIDE, bool FOLD = false, bool SHORT = false>
+// are those of the kernels it stands in for). 
+template <typename X, typename W, typename O, int MT, int R, bool PAIR, int RING, int WAVES, bool WIDE, bool FOLD = false>
 __global__ void __launch_bounds__(64 * WAVES)
 gemm_generic_few_kernel(const X* __restrict__ x, const W* __restrict__ w, const W* __restrict__ bias,
                         O* __restrict__ y, int M, int N, int K, int gate, float alpha, float limit, int jobs_at_once, RowsFold fold) {
   static_assert(!PAIR || (MT == 1 && R == 8), "two blocks at once: 8 rows of W, 8 of x");
   static_assert(!FOLD || (MT == 1 && WIDE), "folds: at most 16 rows of x, 16-byte loads");
-  static_assert(!SHORT || (!PAIR && MT == 1 && RING == 16), "K of one part: one block");
   // Folded: x goes through a ring of its own, both rings 8 deep and asked for four pieces at a time.  Loads come back in the order they
   // were asked for, so that with W 16 groups ahead and x 8 the wait for x leaves only 8 of W's on their way; and a shorter ring is
   // half the code, most of which runs once or twice and comes from memory itself.  8 rows: 11264 x 2048 gated 26.9 us (rings of 16 with
@@ -192,7 +190,7 @@ gemm_generic_few_kernel(const X* __restrict__ x, const W* __restrict__ w, const 
     const float* row = fold.ssq + static_cast<size_t>(min(PAIR ? r & 7 : r, M - 1)) * chunks;
     const int c0 = (k + first - 4 * g) / 8 + 4 * g;
 #pragma unroll
-    for (int j = 0; j < (SHORT ? 2 : 4); ++j) v[j] = load4(row + min(c0 + 16 * j, chunks - 4));
+    for (int j = 0; j < 4; ++j) v[j] = load4(row + min(c0 + 16 * j, chunks - 4));
   };
   float4 square[4];
   if constexpr (FOLD) {
@@ -209,7 +207,6 @@ gemm_generic_few_kernel(const X* __restrict__ x, const W* __restrict__ w, const 
     }
 #pragma unroll
     for (int c = 0; c < RING; ++c) {
-      if (SHORT && 16 * c >= K) break;
       ring[c] = fetch4<WIDE>(w_row, k0 + first + 16 * c, K);
       if (kTogether) xs[0][c][0] = fetch4<WIDE>(x_row[0], k0 + first + 16 * c, K);
     }
@@ -222,7 +219,7 @@ gemm_generic_few_kernel(const X* __restrict__ x, const W* __restrict__ w, const 
         const int c0 = (job * kJobK + first - 4 * g) / 8 + 4 * g;
         float sum = 0.f;
 #pragma unroll
-        for (int j = 0; j < (SHORT ? 2 : 4); ++j)
+        for (int j = 0; j < 4; ++j)
           sum += c0 + 16 * j < chunks ? (square[j].x + square[j].z) + (square[j].y + square[j].w) : 0.f;
         float a = sum, b = sum;
         swap16(a, b);
@@ -254,7 +251,6 @@ gemm_generic_few_kernel(const X* __restrict__ x, const W* __restrict__ w, const 
         const bool more = next < K, edge = k0 + kPartK + (PAIR ? kBlockK : 0) > K;
 #pragma unroll
         for (int c = 0; c < RING; ++c) {
-          if (SHORT && 16 * c >= K) break;
           if (!kTogether && c % SC == 0) {                   // the next few pieces of x
             const int to = (c / SC + 1) & 1;
             const int from = (c + SC < RING ? k0 + 16 * (c + SC) : next) + first;
@@ -276,7 +272,7 @@ gemm_generic_few_kernel(const X* __restrict__ x, const W* __restrict__ w, const 
 #pragma unroll
             for (int i = 0; i < MT; ++i) b[i] = inside(b[i], k0 + first + 16 * c, K);
           }
-          if (!SHORT && more && !kTogether) ring[c] = fetch4<WIDE>(w_row, next + first + 16 * c, K);
+          if (more && !kTogether) ring[c] = fetch4<WIDE>(w_row, next + first + 16 * c, K);
           to_quarters(a);
 #pragma unroll
           for (int i = 0; i < MT; ++i) to_quarters(b[i]);
@@ -284,7 +280,7 @@ gemm_generic_few_kernel(const X* __restrict__ x, const W* __restrict__ w, const 
           for (int e = 0; e < 4; ++e)
 #pragma unroll
             for (int i = 0; i < MT; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32((&a.x)[e], (&b[i].x)[e], acc[i], 0, 0, 0);
-          if (kTogether && !SHORT && more && c % 4 == 3) {
+          if (kTogether && more && c % 4 == 3) {
 #pragma unroll
             for (int e = c - 3; e <= c; ++e) ring[e] = fetch4<WIDE>(w_row, next + first + 16 * e, K);
 #pragma unroll
@@ -498,7 +494,7 @@ int launch_few(const X* x, const W* w, const W* bias, O* y, int M, int N, int K,
   return launch_status();
 }
 
-template <int R, bool PAIR, int WAVES, bool SHORT>
+template <int R, bool PAIR, int WAVES>
 int launch_folded(const float* x, const float* w, const float* bias, float* y, int M, int N, int K, int gate, float alpha, float limit,
                   const RowsFold& fold, hipStream_t s) {
   const int job_k = PAIR ? 2 * kBlockK : kBlockK, jobs = (K + job_k - 1) / job_k, turns = (jobs + WAVES - 1) / WAVES;
@@ -509,7 +505,7 @@ int launch_folded(const float* x, const float* w, const float* bias, float* y, i
   const int at_once = jobs <= room / job_bytes ? jobs : room / job_bytes;
   RowsFold placed = fold;
   placed.squares_at = at_once * job_bytes / static_cast<int>(sizeof(float));
-  hipLaunchKernelGGL((gemm_generic_few_kernel<float, float, float, 1, R, PAIR, SHORT ? 16 : 8, WAVES, true, true, SHORT>), dim3((N + fold.rows - 1) / fold.rows),
+  hipLaunchKernelGGL((gemm_generic_few_kernel<float, float, float, 1, R, PAIR, 8, WAVES, true, true>), dim3((N + fold.rows - 1) / fold.rows),
                      dim3(64 * waves), at_once * job_bytes + squares, s, x, w, bias, y, M, N, K, gate, alpha, limit, at_once, placed);
   return launch_status();
 }
@@ -623,15 +619,14 @@ extern "C" int tlie_gemm_generic_rows(const float* x, const float* w, const floa
   }
   hipStream_t s = (hipStream_t)stream;
   RowsFold fold{ssq, eps, kind, 0, 16, residual, next_weight, xg, ssq_out, positions, slot_map, inv_freq, q_out, cache, rot_dim, nq, nkv, d, page_size};
-  if (K <= 256) return launch_folded<16, false, 1, true>(x, w, bias, y, M, N, K, gate, alpha, limit, fold, s);
   if (M <= 8 && K > kBlockK && (N + 7) / 8 <= compute_units) {       // (the lines of `launch_product`)
     fold.rows = 8;
-    return launch_folded<8, true, 12, false>(x, w, bias, y, M, N, K, gate, alpha, limit, fold, s);
+    return launch_folded<8, true, 12>(x, w, bias, y, M, N, K, gate, alpha, limit, fold, s);
   }
   // where strips of 16 rows leave units without a workgroup, even shares of the rows instead
   const int strips = (N + 15) / 16, share = ((N + compute_units - 1) / compute_units + 1) / 2 * 2;
   if (kind != kFoldResidual && strips < compute_units && 2 * strips > compute_units && share < 16) fold.rows = share < 8 ? 8 : share;
-  return launch_folded<16, false, 12, false>(x, w, bias, y, M, N, K, gate, alpha, limit, fold, s);
+  return launch_folded<16, false, 12>(x, w, bias, y, M, N, K, gate, alpha, limit, fold, s);
 }
 
 // The embedding of few rows with the first norm's inputs: residual [rows][hidden] = table's rows, xg = residual * weight, ssq the sums

@@ -1715,15 +1715,17 @@ def gemm_generic(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | Non
 
 
 def gemm_generic_rows_takes(rows: int, weight: torch.Tensor, dtype: torch.dtype, bias: torch.Tensor | None = None) -> bool:
-    """Whether `gemm_generic_rows` takes a step of `rows` tokens: everything in 32 bits, rows that 16-byte loads fit."""
-    return (dtype == torch.float32 and weight.dtype == torch.float32 and 0 < rows <= ROWS_MAX and weight.shape[1] % 4 == 0
+    """Whether `gemm_generic_rows` takes a step of `rows` tokens: everything in 32 bits, rows that 16-byte loads fit, more than one
+    block of K.  (Up to 512 a workgroup has one wave, whose folded work stands in a row: a layer of 96 to 256 columns 25 us in five
+    launches, 24 in eight, and whole requests 5 to 8% slower.)"""
+    return (dtype == torch.float32 and weight.dtype == torch.float32 and 0 < rows <= ROWS_MAX and weight.shape[1] % 4 == 0 and weight.shape[1] > 512
             and weight.data_ptr() % 16 == 0 and (bias is None or bias.dtype == torch.float32))
 
 
 def _float_norm_folds(weight: torch.Tensor, width: int) -> bool:
     """Whether a product of few rows may leave and take this norm's inputs: the sums of squares by eight columns in fours, and the norm
-    kernel sums by eights too."""
-    return weight.dtype == torch.float32 and width % 32 == 0 and weight.data_ptr() % 32 == 0
+    kernel sums by eights too (and the product that reads them is one of `gemm_generic_rows`)."""
+    return weight.dtype == torch.float32 and width % 32 == 0 and width > 512 and weight.data_ptr() % 32 == 0
 
 
 def gemm_generic_rows(x, weight: torch.Tensor, bias: torch.Tensor | None, epilogue: str = "store", residual: torch.Tensor | None = None,
@@ -1741,7 +1743,7 @@ def gemm_generic_rows(x, weight: torch.Tensor, bias: torch.Tensor | None, epilog
         raise invalid_shape(f"gemm: x {list(data.shape)} and weight {list(weight.shape)} do not fit")
     rows, (out_features, in_features) = data.shape[0], weight.shape
     if not gemm_generic_rows_takes(rows, weight, data.dtype, bias):
-        raise invalid_argument(f"gemm_generic_rows takes 1..{ROWS_MAX} rows of float32 and an inner size that is a multiple of 4")
+        raise invalid_argument(f"gemm_generic_rows takes 1..{ROWS_MAX} rows of float32 and an inner size from 516 on, a multiple of 4")
     if bias is not None:
         _device_tensor(bias, "bias", torch.float32)
         if bias.shape != (out_features,):
