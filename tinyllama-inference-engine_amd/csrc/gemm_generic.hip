@@ -151,7 +151,7 @@ __device__ __forceinline__ void fold_rotation(const RowsFold& fold, const FoldAh
 // two blocks of K: lanes 0 .. 7 of a sixteen bring both operands' rows from the one block, lanes 8 .. 15 from the other.
 // Twice the workgroups of R = 16, and no lane brings what another one has.
 // FOLD: a layer's neighbouring arithmetic in the same kernel, described by `RowsFold` (at most 16 rows of x, all in 32 bits; the bits
-// are those of the kernels it stands in for). 
+// are those of the kernels it stands in for).
 template <typename X, typename W, typename O, int MT, int R, bool PAIR, int RING, int WAVES, bool WIDE, bool FOLD = false>
 __global__ void __launch_bounds__(64 * WAVES)
 gemm_generic_few_kernel(const X* __restrict__ x, const W* __restrict__ w, const W* __restrict__ bias,
