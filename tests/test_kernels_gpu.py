@@ -206,6 +206,32 @@ def test_parts_of_a_split_product_meet_in_their_order(nsplit):
         assert rel_err(one, torch.exp(-torch.exp(torch.tanh(parts.double().sum(0)) @ weight.double().T))) < 1e-5
 
 
+@pytest.mark.parametrize("nsplit", [2, 3, 9])
+def test_kernels_add_up_parts_of_sixteen_bits_too(monkeypatch, nsplit):
+    """No product of this library leaves its parts in bfloat16 and the Python faces refuse them; the kernels behind take them: the
+    bits of the same values as floats."""
+    from tlie_amd import ops
+    monkeypatch.setattr(ops, "_check_product", lambda product, name: None)
+    torch.manual_seed(nsplit)
+    bf = torch.bfloat16
+
+    def drawn(*shape):
+        return torch.randn(*shape, device=DEV).to(bf)
+    parts, weight, bias, start, numbers = drawn(nsplit, 3, 272), drawn(272), drawn(272), torch.randn(3, 272, device=DEV), drawn(2)
+    for kernel in (lambda residual, delta: ops.add_rmsnorm(residual, delta, weight, 1e-5, bf),
+                   lambda residual, delta: ops.layer_norm(residual, delta, weight, bias, 1e-5, bf),
+                   lambda residual, delta: ops.norm_add_rmsnorm(residual, delta, weight, 1e-5, weight, 1e-5, bf),
+                   lambda residual, delta: ops.xielu(delta, numbers, bf)):
+        one, other = start.clone(), start.clone()
+        assert torch.equal(kernel(one, ops.Product(parts, nsplit)), kernel(other, ops.Product(parts.float(), nsplit))) and torch.equal(one, other)
+    for heads, dv in ((3, 40), (2, 200), (1, 512), (1, 520)):
+        a, gate, weight = torch.randn(3, heads * dv, device=DEV), drawn(nsplit, 3, heads * dv), drawn(heads * dv)
+        for first in (False, True):
+            one, other = (ops.head_combine(a, heads, dv, 1e-5, bf, weight=weight, gate=ops.Product(data, nsplit), gate_kind="silu", gate_first=first)
+                          for data in (gate, gate.float()))
+            assert torch.equal(one, other), (heads, dv, first)
+
+
 @pytest.mark.parametrize("rows, n, k, whole", [(24, 12288, 4096, False), (64, 4096, 11008, False), (64, 2304, 14336, False), (24, 9000, 4096, True),
                                                (17, 2048, 1536, True), (20, 11264, 2048, False), (33, 4096, 14336, False)])
 def test_gemm_ring_is_as_exact_as_the_product_it_stands_in_for(rows, n, k, whole):

@@ -195,8 +195,7 @@ __device__ __forceinline__ float sum_splits(const D* __restrict__ first, int nsp
 template <typename D>
 __device__ __forceinline__ void load8_splits(const D* __restrict__ part, int nsplit, size_t stride, float (&d)[8]) {
   load8(part, d);
-  if (sizeof(D) < sizeof(float)) return;                     // (parts are floats: this is a whole product)
-  constexpr int kTogether = 8;
+  constexpr int kTogether = sizeof(D) < sizeof(float) ? 1 : 8;       // (the products of this library leave their parts as floats)
   for (int s = 1; s < nsplit; s += kTogether) {
     float more[kTogether][8];
 #pragma unroll

@@ -53,11 +53,12 @@ head_combine_kernel(const float* __restrict__ a, int heads, int dv, int pair_gro
   // their gates' parts are asked for together, four parts of all dims at a time, each dim's added up as `sum_splits` does
   // (4 rows of 4 heads of 512 dims, 8 parts: one dim after the other behind the norm 11.7 us, so 8.8)
   float gates[kKept];
-  if (fits && gate != nullptr && (gate_nsplit == 1 || dv <= 64)) {
+  constexpr bool kTogether = sizeof(D) == sizeof(float);                  // (the products of this library leave their parts as floats)
+  if (fits && gate != nullptr && (!kTogether || gate_nsplit == 1 || dv <= 64)) {
 #pragma unroll
     for (int k = 0; k < kKept; ++k)
       if (64 * k < dv) gates[k] = gate_value(min(lane + 64 * k, dv - 1));
-  } else if (sizeof(D) == sizeof(float) && fits && gate != nullptr) {     // (parts are floats)
+  } else if (kTogether && fits && gate != nullptr) {
     const D* from = gate + static_cast<size_t>(t) * gate_row + gate_col + h * dv;
     float chain[4][kKept] = {};
     int s = 0;
