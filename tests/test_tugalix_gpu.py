@@ -236,6 +236,19 @@ def test_the_norm_leaves_the_convolution_where_it_cannot_apply_it():
     assert ops.conv_after(taps[:12], state[..., :12], ctx(), ops.NormParams(weight[:12], None, 1e-5, True), torch.float32) is None
 
 
+def test_the_norm_refuses_a_convolution_whose_arrays_it_would_read_wrongly():
+    from tlie_amd import ops
+    from tlie_amd.errors import EngineError
+    weight, residual, wide = torch.ones(16, device=DEVICE), torch.zeros(2, 16, device=DEVICE), torch.zeros(16, 8, device=DEVICE)
+    taps, state, place = wide[:, :4].contiguous(), torch.zeros(2, 3, 16, device=DEVICE), torch.zeros(2, dtype=torch.int32, device=DEVICE)
+    for wrong in (dict(taps=wide[:, :4]), dict(taps=taps.cpu()), dict(state=state.bfloat16()), dict(state=state.cpu()),
+                  dict(state=torch.zeros(2, 16, 3, device=DEVICE).transpose(1, 2)), dict(state=torch.zeros(2, 3, 32, device=DEVICE)[..., :16]),
+                  dict(token_slot=place.long()), dict(token_slot=place.cpu())):
+        with pytest.raises(EngineError):
+            ops.layer_norm(residual, None, weight, None, 1e-5, torch.float32, conv=ops.ConvAfter(**{"taps": taps, "state": state, "token_slot": place, **wrong}))
+    ops.layer_norm(residual, None, weight, None, 1e-5, torch.float32, conv=ops.ConvAfter(taps, state, place))
+
+
 @pytest.mark.parametrize("width,mixes,plan,dtype", [(80, 5, SHORT_STEPS, torch.float32), (44, 1, LONG_STEPS, torch.float32),
                                                     (203, 5, SHORT_STEPS, torch.bfloat16)])
 def test_the_token_shift_blends_with_the_token_before(width, mixes, plan, dtype):

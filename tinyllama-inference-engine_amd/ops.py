@@ -802,9 +802,14 @@ def layer_norm(residual: torch.Tensor, delta, weight: torch.Tensor | None, bias:
     _device_tensor(residual, "residual", torch.float32)
     if conv is not None:
         out_dtype = weight.dtype
+        _device_tensor(conv.taps, "taps", (torch.float32, torch.bfloat16))
+        _device_tensor(conv.token_slot, "token_slot", torch.int32)
+        if not conv.state.is_cuda or conv.state.dtype != torch.float32:
+            raise invalid_argument("layer_norm: the convolution's state is a float32 tensor on the GPU")
         if (rows is not None or not want_out or conv.taps.dtype != weight.dtype or conv.taps.shape != (residual.shape[-1], 4)
-                or conv.token_slot.shape != (residual.shape[0],) or tuple(conv.state.shape[1:]) != (3, residual.shape[-1])):
-            raise invalid_shape("layer_norm: the convolution behind it takes all rows, four taps in the weights' type and a state of three rows")
+                or conv.token_slot.shape != (residual.shape[0],) or tuple(conv.state.shape[1:]) != (3, residual.shape[-1])
+                or conv.state.stride()[1:] != (residual.shape[-1], 1)):
+            raise invalid_shape("layer_norm: the convolution behind it takes all rows, four taps in the weights' type and a state of three rows side by side")
     if residual.dim() != 2:
         raise invalid_shape("layer_norm: the residual is [tokens, hidden]")
     tokens, hidden = residual.shape
