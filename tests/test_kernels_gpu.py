@@ -336,6 +336,14 @@ def test_gemm_generic_rows_refuses_what_it_does_not_take():
         ops.gemm_generic_rows(x[:4], w, None, "residual", residual=torch.zeros(5, 24, device=DEV))
     with pytest.raises(Exception):
         ops.gemm_generic_rows(ops.NormedRows(x[:4], torch.zeros(4, 3, device=DEV), 1e-5), w, None)  # sums of squares of another width
+    one = torch.ones(544, device=DEV)
+    for eps in (0.0, -1e-5, float("nan")):                                                          # as the norm's own kernel refuses it
+        with pytest.raises(Exception, match="epsilon"):
+            ops.embed_rows(torch.zeros(2, dtype=torch.int32, device=DEV), x, (one, eps), torch.float32)
+        with pytest.raises(Exception, match="epsilon"):
+            ops.gemm_generic_rows(ops.NormedRows(x[:4], torch.ones(4, 68, device=DEV), eps), w, None)
+        with pytest.raises(Exception, match="epsilon"):
+            ops.gemm_generic_rows(x[:4], torch.randn(544, 544, device=DEV), None, "residual", residual=torch.zeros(4, 544, device=DEV), next_norm=(one, eps))
     narrow = torch.randn(24, device=DEV)
     assert ops.gemm_generic_rows(x[:4], w, None, "residual", residual=torch.zeros(4, 24, device=DEV),
                                  next_norm=(narrow, 1e-5)).normed is None                           # 24 columns

@@ -1759,6 +1759,8 @@ def gemm_generic_rows(x, weight: torch.Tensor, bias: torch.Tensor | None, epilog
         if in_features % 32 != 0 or normed.ssq.shape != (rows, in_features // 8):
             raise invalid_shape(f"gemm: sums of squares {list(normed.ssq.shape)} are not [{rows}, {in_features} / 8]")
         ssq, eps = normed.ssq, float(normed.eps)
+    if (normed is not None and not eps > 0.0) or (epilogue == "residual" and next_norm is not None and not next_norm[1] > 0.0):
+        raise EngineError(ErrorCode.NUMERICAL, "RMSNorm requires a positive epsilon")
     device, code = data.device, 0
     y = xg = ssq_out = next_weight = q_out = None
     gate_kind, alpha, limit = _gate_args(gate if epilogue == "gate" else None)
@@ -2864,6 +2866,8 @@ def embed_rows(tokens: torch.Tensor, table: torch.Tensor, next_norm: tuple, dtyp
         raise invalid_shape("embed_rows takes 1..16 tokens, a table [vocab, hidden] and a norm weight [hidden]")
     count, hidden = tokens.shape[0], table.shape[1]
     if dtype == torch.float32:
+        if not next_eps > 0.0:
+            raise EngineError(ErrorCode.NUMERICAL, "RMSNorm requires a positive epsilon")
         if table.dtype != torch.float32 or table.data_ptr() % 32 != 0 or not _float_norm_folds(next_weight, hidden):
             return embed_gather(tokens, table), None
         residual, xg = (torch.empty((count, hidden), dtype=torch.float32, device=table.device) for _ in range(2))
