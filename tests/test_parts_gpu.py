@@ -179,6 +179,29 @@ def test_embedding_and_head_parts(dtype, tied):
     assert_close(logits, plain_linear(x.double(), matrix.double()), TOL[dtype])
 
 
+@pytest.mark.parametrize("shifted", ["x", "residual"])
+def test_a_product_of_few_rows_takes_float_rows_wherever_they_lie(shifted):
+    """Rows of x or of the residual between 16-byte boundaries: the product that adds into the residual, or rotates, itself does not
+    take them, so the result comes back as usual."""
+    from tlie_amd.parts.base import ResidualTarget, ResidualUpdated, as_product
+    from tlie_amd.parts.linear import Linear
+    torch.manual_seed(5)
+
+    def lying(where, *shape):
+        count = math.prod(shape)
+        return torch.randn(count + 4, device=DEV)[1 if shifted == where else 0:][:count].view(*shape)
+    weight, x, residual = torch.randn(64, 544, device=DEV), lying("x", 3, 544), lying("residual", 3, 64)
+    linear, want = Linear(weight, None, torch.float32), x.double() @ weight.double().T
+    before = residual.double()
+    out = linear(x, into=ResidualTarget(residual))
+    got = residual.double() - before if isinstance(out, ResidualUpdated) else as_product(out).dense(torch.float32).double()
+    assert float((got - want).norm() / want.norm()) < 1e-6
+    positions, cache = torch.arange(3, dtype=torch.int32, device=DEV), torch.zeros(1, 2, 1, 8 * 16, device=DEV)
+    out = linear(x, rope=ops.RopeTarget(positions, positions, None, 0, cache, 2, 1, 16))
+    got, columns = (out.dense(torch.float32), 64) if isinstance(out, ops.Product) else (out, 32)
+    assert float((got.double() - want[:, :columns]).norm() / want.norm()) < 1e-6
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("rows", [40, 7])
 def test_pre_norm_block_part(dtype, rows):

@@ -76,9 +76,10 @@ class Linear:
             if isinstance(x, ops.NormedRows):
                 return ops.gemm_rows(x, self.weight, self.bias, "store")
         normed = isinstance(x, ops.NormedRows)
-        if (normed or into is not None or rope is not None) and (normed or x.dtype == torch.float32) and ops.gemm_generic_rows_takes(
+        # (rows that are not brought normed may lie anywhere: what 16-byte loads do not fit takes the kernels one by one)
+        if (normed or ((into is not None or rope is not None) and x.dtype == torch.float32 and x.data_ptr() % 16 == 0)) and ops.gemm_generic_rows_takes(
                 x.shape[0], self.weight, self.dtype, self.bias):
-            if into is not None and self.out_features % 4 == 0:
+            if into is not None and self.out_features % 4 == 0 and into.residual.data_ptr() % 16 == 0:
                 return ops.gemm_generic_rows(x, self.weight, self.bias, "residual", residual=into.residual, next_norm=into.next_norm)
             if rope is not None and not rope.extra_cols and rope.head_scale is None:
                 return ops.gemm_generic_rows(x, self.weight, self.bias, "rope", rope=rope)
