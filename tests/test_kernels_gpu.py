@@ -279,10 +279,10 @@ def test_gemm_generic_at_the_edges_of_its_kernels_and_gated(n, k):
 @pytest.mark.parametrize("rows", [1, 7, 8, 9, 16])
 @pytest.mark.parametrize("k, n, heads", [(544, 576, (3, 1, 10, 4)), (576, 608, (3, 1, 32, 32)), (1024, 640, (2, 2, 16, 16)), (1056, 2048, (4, 2, 6, 0)),
                                          (1504, 544, (2, 1, 66, 64)), (544, 2080, (32, 4, 64, 64)), (2048, 2048, (24, 4, 80, 40)),
-                                         (8224, 544, (1, 1, 16, 16))])
+                                         (8224, 544, (1, 1, 16, 16)), (33792, 544, (1, 1, 16, 16))])
 def test_gemm_generic_rows_gives_the_bits_of_the_kernels_it_stands_in_for(rows, k, n, heads):
     """At most 16 rows in 32 bits with the norm before and the gate, the add or the rotation and cache write after: ragged blocks
-    of K, two at once, more blocks than waves, shares of rows (2560 and 2080 columns), heads that no
+    of K, two at once, more blocks than waves and than LDS holds the sums of (several passes), shares of rows (2560 and 2080 columns), heads that no
     group of four columns divides; against the norm, the product and the rotation as kernels of their own, bit for bit."""
     from tlie_amd import ops
     torch.manual_seed(rows * n + k)
