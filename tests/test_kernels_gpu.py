@@ -323,6 +323,21 @@ def test_gemm_generic_rows_gives_the_bits_of_the_kernels_it_stands_in_for(rows, 
     assert torch.equal(got, want) and torch.equal(caches[0], caches[1])
 
 
+@pytest.mark.parametrize("width", [544, 1056, 4104, 14560, 16384, 36416, 40864, 40896])
+def test_float_rows_are_normed_alike_folded_or_not(width):
+    """The sums of squares by eights, in the norm's kernel and in the product that folds it in, up to the widest row that the kernel
+    keeps in LDS; a wider one is not folded.  Against 64 bits: a chain of a few dozen sums."""
+    from tlie_amd import ops
+    torch.manual_seed(width)
+    table, weight, w = torch.randn(3, width, device=DEV), torch.randn(width, device=DEV), torch.randn(40, width, device=DEV) / math.sqrt(width)
+    residual, lazy = ops.embed_rows(torch.arange(3, device=DEV, dtype=torch.int32), table, (weight, 1e-5), torch.float32)
+    normed = ops.add_rmsnorm(residual.clone(), None, weight, 1e-5, torch.float32)
+    assert rel_err(normed, plain_rms_norm(table.double().cpu(), weight.double().cpu(), 1e-5)) < 1e-6
+    assert (lazy is None) == (width % 32 != 0 or width > 40880)
+    if lazy is not None:
+        assert torch.equal(ops.gemm_generic_rows(lazy, w, None).dense(), ops.gemm_generic(normed, w, None, torch.float32).dense())
+
+
 def test_gemm_generic_rows_refuses_what_it_does_not_take():
     from tlie_amd import ops
     w, x = torch.randn(24, 544, device=DEV), torch.randn(17, 544, device=DEV)

@@ -54,42 +54,35 @@ __global__ void add_rmsnorm_kernel(float* __restrict__ residual, const D* __rest
   }
 }
 
-// The sum of squares of a row of the 32-bit path, of which every thread has left the sums of its chunks of eight columns in
-// `eights` [chunks]: by blocks of 64 chunks (512 columns, the product's blocks of K), a block's quarters (every fourth group of four
-// chunks) summed group by group, the blocks in their order.  The products of few rows that fold this norm in form the same sum
-// (gemm_generic.hip).  blocks [(chunks + 63) / 64] floats of LDS; every thread gets the result.
-__device__ __forceinline__ float block_squares(const float* eights, float* blocks, int chunks) {
-  __syncthreads();
-  const int count = (chunks + 63) / 64;
-  for (int i = threadIdx.x; i < count * 4; i += blockDim.x) {        // (whole groups of four lanes)
-    float sum = 0.f;
-    for (int j = 0; j < 4; ++j) {
-      const int c = (i >> 2) * 64 + 16 * j + 4 * (i & 3);
-      float v[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = c + e < chunks ? eights[c + e] : 0.f;
-      sum += (v[0] + v[2]) + (v[1] + v[3]);
-    }
-    sum += __shfl_xor(sum, 1, 64);
-    sum += __shfl_xor(sum, 2, 64);
-    if ((i & 3) == 0) blocks[i >> 2] = sum;
-  }
-  __syncthreads();
-  float total = 0.f;
-  for (int b = 0; b < count; ++b) total += blocks[b];
-  return total;
+// The sum of squares of a row of the 32-bit path goes by blocks of 512 columns (the product's blocks of K): sums of eight columns, a
+// wave's 64 lanes those of a block; a block's quarters (every fourth group of four sums) summed group by group; the blocks in their
+// order.  The products of few rows that fold this norm in form the same sum (gemm_generic.hip).  Between registers: through LDS, with
+// the sums of eight kept there, 8 rows of 2048 took 3.8 us (3.4 so), 64 of 8192 5.5 (5.1), and rows from 36416 columns on did not fit.
+__device__ __forceinline__ float block_of_squares(float v) {
+#define TLIE_FROM(control) __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), control, 0xf, 0xf, true))
+  v += TLIE_FROM(0x4e);                                  // quad_perm 2 3 0 1: (0 + 2) and (1 + 3) of a group of four
+  v += TLIE_FROM(0xb1);                                  // quad_perm 1 0 3 2
+  float a = v, c = v;
+  swap32(a, c);
+  float b = a, d = c;
+  swap16(a, b);
+  swap16(c, d);
+  v = ((a + b) + c) + d;
+  v += TLIE_FROM(0x141);                                 // row_half_mirror: the other quarter of a pair
+  v += TLIE_FROM(0x128);                                 // row_ror:8: the other pair
+#undef TLIE_FROM
+  return v;
 }
 
 // The same with eight elements a thread (16-byte loads and stores): hidden % 8 == 0; the summands
-// of a split product are added in the order of their index.  With a float result the squares are summed as `block_squares` says
+// of a split product are added in the order of their index.  With a float result the squares are summed as `block_of_squares` says
 // and the weight comes before the scale.
 template <typename D, typename W, typename O>
 __global__ void add_rmsnorm_wide_kernel(float* __restrict__ residual, const D* __restrict__ delta, int nsplit,
                                         size_t split_stride, const W* __restrict__ weight, float eps,
                                         O* __restrict__ out, const int* __restrict__ rows, int hidden) {
-  extern __shared__ float row_cache[];           // hidden floats, then 16 for the reduction (a float result: hidden / 8 sums and their blocks)
-  float* eights = row_cache + hidden;
-  float* scratch = eights + (sizeof(O) == sizeof(float) ? hidden / 8 : 0);
+  extern __shared__ float row_cache[];           // hidden floats, then 16 for the reduction (a float result: the blocks' sums)
+  float* scratch = row_cache + hidden;
   const int r = blockIdx.x;
   const int src = rows ? rows[r] : r;
   float* res = residual + static_cast<size_t>(src) * hidden;
@@ -97,27 +90,38 @@ __global__ void add_rmsnorm_wide_kernel(float* __restrict__ residual, const D* _
   const int first = threadIdx.x * 8;
   const bool ahead = sizeof(D) == sizeof(float) && out && first < hidden;       // (few rows: the weight is asked for ahead of the sums)
   if (ahead) load8(weight + first, first_weight);
-  for (int i = threadIdx.x * 8; i < hidden; i += blockDim.x * 8) {
-    float v[8];
-    load8(res + i, v);
-    if (delta) {
-      float d[8];
-      load8_splits(delta + static_cast<size_t>(src) * hidden + i, nsplit, split_stride, d);
+  for (int i = threadIdx.x * 8; i - first % 512 < hidden; i += blockDim.x * 8) {       // (whole waves)
+    float eights = 0.f;
+    if (i < hidden) {
+      float v[8];
+      load8(res + i, v);
+      if (delta) {
+        float d[8];
+        load8_splits(delta + static_cast<size_t>(src) * hidden + i, nsplit, split_stride, d);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] += d[j];
-      if (!rows) store8(res + i, v);
+        for (int j = 0; j < 8; ++j) v[j] += d[j];
+        if (!rows) store8(res + i, v);
+      }
+      store8(row_cache + i, v);
+      if constexpr (sizeof(O) == sizeof(float)) {
+        eights = squares_of8(v);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) square += v[j] * v[j];
+      }
     }
-    store8(row_cache + i, v);
     if constexpr (sizeof(O) == sizeof(float)) {
-      eights[i / 8] = squares_of8(v);
-    } else {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) square += v[j] * v[j];
+      const float block = block_of_squares(eights);
+      if (first % 512 == 0) scratch[i / 512] = block;
     }
   }
-  float total;
-  if constexpr (sizeof(O) == sizeof(float)) total = block_squares(eights, scratch, hidden / 8);
-  else total = block_sum(square, scratch);
+  float total = 0.f;
+  if constexpr (sizeof(O) == sizeof(float)) {
+    __syncthreads();
+    for (int b = 0; b < (hidden + 511) / 512; ++b) total += scratch[b];
+  } else {
+    total = block_sum(square, scratch);
+  }
   const float scale = rsqrtf(total / static_cast<float>(hidden) + eps);
   if (out) {
     O* o = out + static_cast<size_t>(r) * hidden;
@@ -360,7 +364,7 @@ static int launch_add_rmsnorm(float* residual, const void* delta, int nsplit, si
                               const void* weight, float eps, void* out,
                               const int* rows, int num_rows, int hidden, hipStream_t stream) {
   const size_t lds = (static_cast<size_t>(hidden) + 16) * sizeof(float);
-  const size_t wide_lds = sizeof(O) == sizeof(float) ? (hidden + hidden / 8 + (hidden + 511) / 512) * sizeof(float) : lds;
+  const size_t wide_lds = sizeof(O) == sizeof(float) ? (hidden + (hidden + 511) / 512) * sizeof(float) : lds;     // (up to 40880 columns)
   if (lds > 160 * 1024) return kBadArgument;
   const bool aligned = ((reinterpret_cast<uintptr_t>(residual) | reinterpret_cast<uintptr_t>(delta) |
                          reinterpret_cast<uintptr_t>(weight) | reinterpret_cast<uintptr_t>(out)) & 31) == 0;

@@ -45,7 +45,7 @@ __device__ __forceinline__ float4 inside(float4 v, int k, int K) {
 // ---- what a product of few rows may do beside (a layer's neighbouring arithmetic) ---------------------------
 // Each saves a launch of 5 us whose own work is some kilobytes, and gives the bits of the kernel that it stands in for:
 //   before   x is residual * norm weight and `ssq` [M][K / 8] the sums of squares of the residual's rows by eights; the rows of x are
-//            multiplied by rsqrt(mean of squares + eps), the sum formed as in the norm kernel (`block_squares` in elementwise.hip)
+//            multiplied by rsqrt(mean of squares + eps), the sum formed as in the norm kernel (`block_of_squares` in elementwise.hip)
 //   after    kFoldResidual: residual [M][N] += result; with next_weight also xg = residual * next_weight and `ssq_out` for the
 //            product that the next norm stands before.  kFoldRotation: W is a fused q/k/v weight with rows in paired order; rotation
 //            and cache write of rope_cache.hip

@@ -1727,10 +1727,13 @@ def gemm_generic_rows_takes(rows: int, weight: torch.Tensor, dtype: torch.dtype,
             and weight.data_ptr() % 16 == 0 and (bias is None or bias.dtype == torch.float32))
 
 
+FLOAT_NORM_MAX = 40880         # the widest row that the norm kernel sums by eights (what it keeps of a row in LDS)
+
+
 def _float_norm_folds(weight: torch.Tensor, width: int) -> bool:
     """Whether a product of few rows may leave and take this norm's inputs: the sums of squares by eight columns in fours, and the norm
     kernel sums by eights too (and the product that reads them is one of `gemm_generic_rows`)."""
-    return weight.dtype == torch.float32 and width % 32 == 0 and width > 512 and weight.data_ptr() % 32 == 0
+    return weight.dtype == torch.float32 and width % 32 == 0 and 512 < width <= FLOAT_NORM_MAX and weight.data_ptr() % 32 == 0
 
 
 def gemm_generic_rows(x, weight: torch.Tensor, bias: torch.Tensor | None, epilogue: str = "store", residual: torch.Tensor | None = None,
