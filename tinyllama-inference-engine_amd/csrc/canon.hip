@@ -121,13 +121,13 @@ layer_norm_wide_kernel(float* __restrict__ residual, const D1* __restrict__ d1, 
     load8(residual + at + c, x);
     if (d1 != nullptr) {
       float d[8];
-      load8_splits(d1 + at + c, n1, stride1, d);
+      load8_splits<true>(d1 + at + c, n1, stride1, d);
 #pragma unroll
       for (int j = 0; j < 8; ++j) x[j] += s1 * d[j];
     }
     if (d2 != nullptr) {
       float d[8];
-      load8_splits(d2 + at + c, n2, stride2, d);
+      load8_splits<true>(d2 + at + c, n2, stride2, d);
 #pragma unroll
       for (int j = 0; j < 8; ++j) x[j] += s2 * d[j];
     }
@@ -437,14 +437,14 @@ xielu_kernel(const D* __restrict__ in, int nsplit, size_t split_stride, const W*
 }
 
 // The same with eight elements a thread: count % 8 == 0 and the parts of a split product a multiple of eight apart.
-template <typename D, typename W, typename O>
+template <typename D, typename W, typename O, bool PARTS>
 __global__ void __launch_bounds__(256)
 xielu_wide_kernel(const D* __restrict__ in, int nsplit, size_t split_stride, const W* __restrict__ numbers, O* __restrict__ out,
                   size_t count) {
   const float up = softplus_of(to_float(numbers[0])), down = 0.5f + softplus_of(to_float(numbers[1]));
   for (size_t i = (static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x) * 8; i < count; i += static_cast<size_t>(gridDim.x) * blockDim.x * 8) {
     float z[8];
-    load8_splits(in + i, nsplit, split_stride, z);
+    load8_splits<PARTS>(in + i, nsplit, split_stride, z);
 #pragma unroll
     for (int j = 0; j < 8; ++j) z[j] = z[j] > 0.f ? up * z[j] * z[j] + 0.5f * z[j] : down * (expm1f(z[j]) - z[j]) + 0.5f * z[j];
     store8(out + i, z);
@@ -597,7 +597,7 @@ extern "C" int tlie_xielu(const void* in, int in_dtype, int nsplit, long long sp
 #define TLIE_CASE(IC, D, NC, W, OC, O)                                                                                   \
   if (in_dtype == IC && n_dtype == NC && out_dtype == OC) {                                                              \
     if (wide)                                                                                                            \
-      hipLaunchKernelGGL((xielu_wide_kernel<D, W, O>), dim3((unsigned)((blocks + 7) / 8)), dim3(256), 0, s, (const D*)in,  \
+      hipLaunchKernelGGL(TLIE_PARTS_FORM(nsplit, D, xielu_wide_kernel, D, W, O), dim3((unsigned)((blocks + 7) / 8)), dim3(256), 0, s, (const D*)in,  \
                          nsplit, (size_t)split_stride, (const W*)numbers, (O*)out, (size_t)count);                        \
     else                                                                                                                 \
       hipLaunchKernelGGL((xielu_kernel<D, W, O>), dim3((unsigned)blocks), dim3(256), 0, s, (const D*)in, nsplit,          \

@@ -191,10 +191,12 @@ __device__ __forceinline__ float sum_splits(const D* __restrict__ first, int nsp
 
 // Eight neighbouring elements summed over the parts of a split product, in the order of their index.  The parts are asked for eight at a
 // time: one after the other, each waits for the one before, and a kernel of few rows is little else than that chain (the norm after a
-// product of 64 rows in 8 parts, 2048 columns, 5.2 us one by one, 4.7 so).
-template <typename D>
+// product of 64 rows in 8 parts, 2048 columns, 5.2 us one by one, 4.7 so).  They take 64 registers, with which half as many waves fit a
+// compute unit: PARTS false for a product that comes whole, as those of many rows do (2048 x 2048 floats normed 14.7 us with them, 12.0 without).
+template <bool PARTS, typename D>
 __device__ __forceinline__ void load8_splits(const D* __restrict__ part, int nsplit, size_t stride, float (&d)[8]) {
   load8(part, d);
+  if (!PARTS) return;
   constexpr int kTogether = sizeof(D) < sizeof(float) ? 1 : 8;       // (the products of this library leave their parts as floats)
   for (int s = 1; s < nsplit; s += kTogether) {
     float more[kTogether][8];
@@ -209,6 +211,9 @@ __device__ __forceinline__ void load8_splits(const D* __restrict__ part, int nsp
     }
   }
 }
+
+// Of a kernel's two forms, the one for this product (one of 16 bits takes no registers for parts: it has one form).
+#define TLIE_PARTS_FORM(nsplit, D, KERNEL, ...) ((nsplit) == 1 ? &KERNEL<__VA_ARGS__, (sizeof(D) < sizeof(float))> : &KERNEL<__VA_ARGS__, true>)
 
 // The sum of squares of four, or eight, neighbouring columns of the 32-bit path's norms: one order for every kernel that forms it.
 __device__ __forceinline__ float squares_of4(float a, float b, float c, float d) { return fmaf(a, a, b * b) + fmaf(c, c, d * d); }

@@ -77,7 +77,7 @@ __device__ __forceinline__ float block_of_squares(float v) {
 // The same with eight elements a thread (16-byte loads and stores): hidden % 8 == 0; the summands
 // of a split product are added in the order of their index.  With a float result the squares are summed as `block_of_squares` says
 // and the weight comes before the scale.
-template <typename D, typename W, typename O>
+template <typename D, typename W, typename O, bool PARTS>
 __global__ void add_rmsnorm_wide_kernel(float* __restrict__ residual, const D* __restrict__ delta, int nsplit,
                                         size_t split_stride, const W* __restrict__ weight, float eps,
                                         O* __restrict__ out, const int* __restrict__ rows, int hidden) {
@@ -97,7 +97,7 @@ __global__ void add_rmsnorm_wide_kernel(float* __restrict__ residual, const D* _
       load8(res + i, v);
       if (delta) {
         float d[8];
-        load8_splits(delta + static_cast<size_t>(src) * hidden + i, nsplit, split_stride, d);
+        load8_splits<PARTS>(delta + static_cast<size_t>(src) * hidden + i, nsplit, split_stride, d);
 #pragma unroll
         for (int j = 0; j < 8; ++j) v[j] += d[j];
         if (!rows) store8(res + i, v);
@@ -167,8 +167,8 @@ __global__ void silu_mul_wide_kernel(const D* __restrict__ gate_up, int nsplit, 
     const D* base = gate_up + t * 2 * inter;
     float a[8], b[8], g[8], u[8];
     const int first = interleaved ? 2 * i : i, second = interleaved ? 2 * i + 8 : inter + i;
-    load8_splits(base + first, nsplit, split_stride, a);
-    load8_splits(base + second, nsplit, split_stride, b);
+    load8_splits<true>(base + first, nsplit, split_stride, a);
+    load8_splits<true>(base + second, nsplit, split_stride, b);
     if (interleaved) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -222,7 +222,7 @@ __global__ void norm_add_rmsnorm_kernel(float* __restrict__ residual, const D* _
 
 // The same with eight elements a thread (16-byte loads and stores): hidden % 8 == 0; the summands of a split
 // product are added in the order of their index.
-template <typename D, typename W, typename O>
+template <typename D, typename W, typename O, bool PARTS>
 __global__ void norm_add_rmsnorm_wide_kernel(float* __restrict__ residual, const D* __restrict__ delta, int nsplit,
                                              size_t split_stride, const W* __restrict__ post_weight, float post_eps,
                                              const W* __restrict__ weight, float eps, O* __restrict__ out,
@@ -235,7 +235,7 @@ __global__ void norm_add_rmsnorm_wide_kernel(float* __restrict__ residual, const
   float square = 0.f;
   for (int i = threadIdx.x * 8; i < hidden; i += blockDim.x * 8) {
     float d[8];
-    load8_splits(delta + static_cast<size_t>(src) * hidden + i, nsplit, split_stride, d);
+    load8_splits<PARTS>(delta + static_cast<size_t>(src) * hidden + i, nsplit, split_stride, d);
     store8(row_cache + i, d);                    // (a thread reads back only what it wrote itself)
 #pragma unroll
     for (int j = 0; j < 8; ++j) square += d[j] * d[j];
@@ -371,7 +371,7 @@ static int launch_add_rmsnorm(float* residual, const void* delta, int nsplit, si
   if ((hidden & 7) == 0 && aligned && wide_lds <= 160 * 1024 && (nsplit == 1 || (split_stride * sizeof(D)) % 32 == 0)) {
     const int chunks = hidden / 8;
     const int wide = chunks >= 1024 ? 1024 : (chunks + 63) / 64 * 64;
-    hipLaunchKernelGGL((add_rmsnorm_wide_kernel<D, W, O>), dim3(num_rows), dim3(wide), wide_lds, stream, residual,
+    hipLaunchKernelGGL(TLIE_PARTS_FORM(nsplit, D, add_rmsnorm_wide_kernel, D, W, O), dim3(num_rows), dim3(wide), wide_lds, stream, residual,
                        (const D*)delta, nsplit, split_stride, (const W*)weight, eps, (O*)out, rows, hidden);
     return launch_status();
   }
@@ -423,8 +423,8 @@ extern "C" int tlie_norm_add_rmsnorm(float* residual, const void* delta, int del
 #define TLIE_CASE(DC, D, WC, W, OC, O)                                                                              \
   if (delta_dtype == DC && weight_dtype == WC && out_dtype == OC) {                                                 \
     if (wide) {                                                                                                     \
-      hipLaunchKernelGGL((norm_add_rmsnorm_wide_kernel<D, W, O>), dim3(num_rows), dim3(wide_threads), lds, s, residual, \
-                         (const D*)delta, nsplit, (size_t)split_stride, (const W*)post_weight, post_eps,            \
+      hipLaunchKernelGGL(TLIE_PARTS_FORM(nsplit, D, norm_add_rmsnorm_wide_kernel, D, W, O), dim3(num_rows), dim3(wide_threads), \
+                         lds, s, residual, (const D*)delta, nsplit, (size_t)split_stride, (const W*)post_weight, post_eps,            \
                          (const W*)weight, eps, (O*)out, rows, hidden);                                              \
       return launch_status();                                                                                       \
     }                                                                                                               \

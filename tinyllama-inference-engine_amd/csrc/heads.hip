@@ -117,7 +117,7 @@ head_combine_kernel(const float* __restrict__ a, int heads, int dv, int pair_gro
 // are one head here): a workgroup a head, eight dims a thread and access, a thread's first kKept groups kept between the
 // sum of squares and the output.  dv a multiple of 8, rows of `a`, weight, gate and out at multiples of 32 bytes, the
 // gate's parts a multiple of 8 apart.
-template <typename D, typename W, typename A>
+template <typename D, typename W, typename A, bool PARTS>
 __global__ void __launch_bounds__(256)
 head_combine_wide_kernel(const float* __restrict__ a, int heads, int dv, float eps, const W* __restrict__ weight, float mult,
                          const D* __restrict__ gate, int gate_nsplit, size_t gate_split_stride, int gate_row, int gate_col,
@@ -131,7 +131,7 @@ head_combine_wide_kernel(const float* __restrict__ a, int heads, int dv, float e
   auto gates = [&](int e, float (&v)[8]) {             // v *= f(gate) of dims e .. e + 7
     float z[8];
     const D* from = gate + static_cast<size_t>(t) * gate_row + gate_col + h * dv + e;
-    load8_splits(from, gate_nsplit, gate_split_stride, z);
+    load8_splits<PARTS>(from, gate_nsplit, gate_split_stride, z);
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] *= (gate_kind == 1 ? z[j] : 1.f) / (1.f + expf(-z[j]));
   };
@@ -204,7 +204,7 @@ extern "C" int tlie_head_combine(const float* a, int tokens, int heads, int dv, 
 #define TLIE_CASE(GC, D, WC, W, AC, A)                                                                                   \
   if (gate_dtype == GC && weight_dtype == WC && out_dtype == AC) {                                                       \
     if (wide) {                                                                                                          \
-      hipLaunchKernelGGL((head_combine_wide_kernel<D, W, A>), dim3(tokens, heads), dim3(256), 0, s, a, heads, dv, eps,    \
+      hipLaunchKernelGGL(TLIE_PARTS_FORM(gate_nsplit, D, head_combine_wide_kernel, D, W, A), dim3(tokens, heads), dim3(256), 0, s, a, heads, dv, eps,    \
                          (const W*)weight, mult, (const D*)gate, gate_nsplit, (size_t)gate_split_stride, gate_row,       \
                          gate_col, gate_kind, gate_first, (A*)out);                                                                  \
       return launch_status();                                                                                            \
