@@ -88,7 +88,7 @@ __global__ void add_rmsnorm_wide_kernel(float* __restrict__ residual, const D* _
   float* res = residual + static_cast<size_t>(src) * hidden;
   float square = 0.f, first_weight[8];
   const int first = threadIdx.x * 8;
-  const bool ahead = sizeof(D) == sizeof(float) && out && first < hidden;       // (few rows: the weight is asked for ahead of the sums)
+  const bool ahead = PARTS && sizeof(D) == sizeof(float) && out && first < hidden;       // (few rows: the weight is asked for ahead of the sums)
   if (ahead) load8(weight + first, first_weight);
   for (int i = threadIdx.x * 8; i - first % 512 < hidden; i += blockDim.x * 8) {       // (whole waves)
     float eights = 0.f;
