@@ -70,8 +70,11 @@ layer_norm_kernel(float* __restrict__ residual, const D1* __restrict__ d1, int n
 
 // The same with eight elements a thread (16- and 32-byte loads and stores): hidden % 8 == 0, and the parts of a split
 // product lie a multiple of eight elements apart; the summands of a split product are added in the order of their index.
-// A few rows are bound by the way of their loads: what a thread's first eight elements need is asked for at once, the earlier results of
-// a depth mix four at a time, weight and bias ahead of the sums they are used behind (4 rows of 2048, 8 parts, up to 5 results: 7.4 -> 6.4 us).
+// PARTS (split products, which few rows leave): a row is bound by the way of its loads: what a thread's first eight elements need is
+// asked for at once, the earlier results of a depth mix four at a time, weight and bias ahead of the sums they are used behind (4 rows of
+// 2048, 8 parts, up to 5 results: 7.4 -> 6.4 us).  Whole products take the form without, at 26 to 35 registers in place of 80 to 135, with which
+// three times the waves fit a unit: 2048 x 2048 with a bfloat16 product 11.4 us against 15.6, with five results mixed in 23.3 against
+// 26.2; 264 rows 5.0 against 5.3 and 5.9 against 6.2.
 // CONV: what leaves is h + conv(h) of the normed row h, the input convolution below of four taps, in a step in which every sequence
 // brings one token (decoding): a channel's earlier inputs are the sequence's state, which takes the new one, and a launch of 4 us with
 // a way to memory of its own goes (4 rows of 2048: 8.1 us in place of 6.4 + 4.1).  Same sums in the same order, the same bits.
@@ -82,7 +85,7 @@ struct ConvAfter {
   size_t slot_stride;
 };
 
-template <typename D1, typename D2, typename W, typename O, bool CONV>
+template <typename D1, typename D2, typename W, typename O, bool PARTS, bool CONV>
 __global__ void __launch_bounds__(256)
 layer_norm_wide_kernel(float* __restrict__ residual, const D1* __restrict__ d1, int n1, size_t stride1, float s1,
                        const D2* __restrict__ d2, int n2, size_t stride2, float s2, const float* __restrict__ row_scale,
@@ -96,8 +99,8 @@ layer_norm_wide_kernel(float* __restrict__ residual, const D1* __restrict__ d1, 
   const size_t at = static_cast<size_t>(t) * hidden;
   if (row_scale != nullptr) s2 *= row_scale[static_cast<size_t>(t) * row_scale_stride];
   float first_weight[8], first_bias[8];
-  const int first = threadIdx.x * 8;
-  if (out != nullptr && first < hidden) {
+  const int first = PARTS ? threadIdx.x * 8 : -1;        // the columns whose weight and bias are asked for ahead of the sums
+  if (PARTS && out != nullptr && first < hidden) {
     load8(weight + first, first_weight);
     if (bias != nullptr) load8(bias + first, first_bias);
   }
@@ -121,13 +124,13 @@ layer_norm_wide_kernel(float* __restrict__ residual, const D1* __restrict__ d1, 
     load8(residual + at + c, x);
     if (d1 != nullptr) {
       float d[8];
-      load8_splits<true>(d1 + at + c, n1, stride1, d);
+      load8_splits<PARTS>(d1 + at + c, n1, stride1, d);
 #pragma unroll
       for (int j = 0; j < 8; ++j) x[j] += s1 * d[j];
     }
     if (d2 != nullptr) {
       float d[8];
-      load8_splits<true>(d2 + at + c, n2, stride2, d);
+      load8_splits<PARTS>(d2 + at + c, n2, stride2, d);
 #pragma unroll
       for (int j = 0; j < 8; ++j) x[j] += s2 * d[j];
     }
@@ -135,17 +138,18 @@ layer_norm_wide_kernel(float* __restrict__ residual, const D1* __restrict__ d1, 
     if (history_count > 0) {
       float y[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
       const float w = to_float(history_weight[history_count - 1]);
-      for (int j = 0; j + 1 < history_count; j += 4) {
-        float earlier[4][8], share[4];
+      constexpr int kTogether = PARTS ? 4 : 1;
+      for (int j = 0; j + 1 < history_count; j += kTogether) {
+        float earlier[kTogether][8], share[kTogether];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
+        for (int u = 0; u < kTogether; ++u) {
           if (j + u + 1 < history_count) {             // (the same for the whole grid)
             load8(history + (j + u) * history_stride + at + c, earlier[u]);
             share[u] = to_float(history_weight[j + u]);
           }
         }
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
+        for (int u = 0; u < kTogether; ++u) {
           if (j + u + 1 >= history_count) break;
 #pragma unroll
           for (int e = 0; e < 8; ++e) y[e] += share[u] * earlier[u][e];
@@ -481,23 +485,24 @@ static int layer_norm_entry(float* residual, const void* d1, int d1_dtype, int n
   if (conv.taps != nullptr && (!wide || out == nullptr || rows != nullptr || conv.state == nullptr || conv.token_slot == nullptr ||
                                !aligned16(conv.taps) || !aligned16(conv.state) || conv.slot_stride % 4 != 0))
     return kBadArgument;
+  const bool parts = n1 > 1 || n2 > 1;
   int threads = 64;                                    // as many waves as the row has work for (at most four)
   while (threads < 256 && threads * 8 < hidden) threads *= 2;
 #define TLIE_CASE(C1, D1, C2, D2, WC, W, OC, O)                                                                          \
   if (d1_dtype == C1 && d2_dtype == C2 && w_dtype == WC && out_dtype == OC) {                                            \
     if (conv.taps != nullptr) {                                                                                          \
       if constexpr (sizeof(W) == sizeof(O))                                                                              \
-        hipLaunchKernelGGL((layer_norm_wide_kernel<D1, D2, W, O, true>), dim3(count), dim3(threads), lds, s, residual,   \
+        hipLaunchKernelGGL((layer_norm_wide_kernel<D1, D2, W, O, true, true>), dim3(count), dim3(threads), lds, s, residual,   \
                            (const D1*)d1, n1, (size_t)stride1, s1, (const D2*)d2, n2, (size_t)stride2, s2, row_scale,    \
                            row_scale_stride, centred, history, (size_t)history_stride, history_count,                    \
                            (const W*)history_weight, mixed, (const W*)weight, (const W*)bias, eps, (O*)out, rows, hidden, conv);  \
       else                                                                                                               \
         return kBadArgument;                                                                                             \
     } else if (wide)                                                                                                     \
-      hipLaunchKernelGGL((layer_norm_wide_kernel<D1, D2, W, O, false>), dim3(count), dim3(threads), lds, s, residual,            \
-                         (const D1*)d1, n1, (size_t)stride1, s1, (const D2*)d2, n2, (size_t)stride2, s2, row_scale,     \
-                         row_scale_stride, centred, history, (size_t)history_stride, history_count,                        \
-                         (const W*)history_weight, mixed, (const W*)weight, (const W*)bias, eps, (O*)out, rows, hidden, conv);  \
+      hipLaunchKernelGGL((parts ? &layer_norm_wide_kernel<D1, D2, W, O, true, false> : &layer_norm_wide_kernel<D1, D2, W, O, false, false>), \
+                         dim3(count), dim3(threads), lds, s, residual, (const D1*)d1, n1, (size_t)stride1, s1, (const D2*)d2, n2,   \
+                         (size_t)stride2, s2, row_scale, row_scale_stride, centred, history, (size_t)history_stride, history_count, \
+                         (const W*)history_weight, mixed, (const W*)weight, (const W*)bias, eps, (O*)out, rows, hidden, conv);      \
     else                                                                                                                 \
       hipLaunchKernelGGL((layer_norm_kernel<D1, D2, W, O>), dim3(count), dim3(256), lds, s, residual, (const D1*)d1, n1,  \
                          (size_t)stride1, s1, (const D2*)d2, n2, (size_t)stride2, s2, row_scale, row_scale_stride, centred,       \
