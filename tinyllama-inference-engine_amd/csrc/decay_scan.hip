@@ -251,18 +251,13 @@ low_rank_decay_kernel(const float* __restrict__ low, int nsplit, size_t split_st
                       const W* __restrict__ bias, int kind, float tau, float* __restrict__ out, int tokens, int channels, int rank) {
   extern __shared__ float shared_low[];                // [TT][rank]
   const int t0 = blockIdx.x * TT;
-  // a channel's weights in pieces of eight where they fit, 64 asked for at once, the first channel's ahead of the low rows
-  // (4 tokens, 2048 channels of rank 64 in bfloat16: an element a load 7.6 us; with the low rows' parts asked for together 5.7)
+  // a channel's weights in pieces of eight where they fit, the first channel's first ahead of the low rows.  (A whole row of 64 asked for at once
+  // is slower, by its registers, 94 to 120, and by the code: 4 tokens, 2048 channels of rank 64 in bfloat16 4.9 us, of rank 128 7.3; so 4.5
+  // and 6.4; an element a load 5.2 and 6.8; 64 tokens, rank 64 9.2, 7.5 and 7.7; 2048 tokens 34.3, 26.0 and 38.0)
   const bool wide = rank % 8 == 0 && reinterpret_cast<uintptr_t>(weight) % (8 * sizeof(W)) == 0;
-  constexpr int kAhead = 8;
-  float rows[kAhead][8];
-  auto ask = [&](const W* row, int r0) {
-#pragma unroll
-    for (int p = 0; p < kAhead; ++p)
-      if (r0 + 8 * p < rank) load8(row + r0 + 8 * p, rows[p]);
-  };
+  float piece[8];
   const int first = blockIdx.y * blockDim.x + threadIdx.x;
-  if (wide && first < channels) ask(weight + static_cast<size_t>(first) * rank, 0);
+  if (wide && first < channels) load8(weight + static_cast<size_t>(first) * rank, piece);
   const int count = min(TT, tokens - t0);
   if (TT == 1 && nsplit > 4 && rank * 4 <= static_cast<int>(blockDim.x)) {
     // many parts of one token's few values (64 values in 32 parts): a thread a value and chain of `sum_splits`, its parts asked for
@@ -307,16 +302,12 @@ low_rank_decay_kernel(const float* __restrict__ low, int nsplit, size_t split_st
     for (int b = 0; b < TT; ++b) z[b] = start;
     const W* row = weight + static_cast<size_t>(c) * rank;
     if (wide) {
-      for (int r0 = 0; r0 < rank; r0 += 8 * kAhead) {
-        if (c != first || r0 > 0) ask(row, r0);
+      for (int r0 = 0; r0 < rank; r0 += 8) {
+        if (c != first || r0 > 0) load8(row + r0, piece);
 #pragma unroll
-        for (int p = 0; p < kAhead; ++p) {
-          if (r0 + 8 * p >= rank) break;
+        for (int j = 0; j < 8; ++j)
 #pragma unroll
-          for (int j = 0; j < 8; ++j)
-#pragma unroll
-            for (int b = 0; b < TT; ++b) z[b] += rows[p][j] * shared_low[b * rank + r0 + 8 * p + j];
-        }
+          for (int b = 0; b < TT; ++b) z[b] += piece[j] * shared_low[b * rank + r0 + j];
       }
     } else {
       for (int r = 0; r < rank; ++r) {
