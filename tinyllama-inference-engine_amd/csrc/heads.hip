@@ -15,7 +15,7 @@
 
 namespace tlie {
 
-template <typename D, typename W, typename A>
+template <typename D, typename W, typename A, bool PARTS>
 __global__ void __launch_bounds__(256)
 head_combine_kernel(const float* __restrict__ a, int heads, int dv, int pair_group, int parts, float lambda, float eps,
                     const W* __restrict__ weight, float mult, const D* __restrict__ gate, int gate_nsplit,
@@ -50,15 +50,22 @@ head_combine_kernel(const float* __restrict__ a, int heads, int dv, int pair_gro
   constexpr int kKept = 8;
   const bool fits = dv <= 64 * kKept;
   float kept[kKept];
-  // their gates' parts are asked for together, four parts of all dims at a time, each dim's added up as `sum_splits` does
-  // (4 rows of 4 heads of 512 dims, 8 parts: one dim after the other behind the norm 11.7 us, so 8.8)
+  // PARTS (split gates, heads of 129 to 512 dims): the gates' parts are asked for together, and with the result, four parts of all dims at
+  // a time, each dim's added up as `sum_splits` does (4 heads of 512 dims, 8 parts: 8 rows 11.3 us one dim after the other behind the norm,
+  // 6.2 so, 17 rows 15.7 and 6.9; 8 of 256: 6.4 and 5.1).  The form takes 138 registers in place of 54: a gate that comes whole, as prompts'
+  // do, has none of it (2048 rows of 8 heads of 256 floats 30.9 us with it, 19.7 without), nor have heads of one or two dims a lane, whose few
+  // loads it delays (16 heads of 80 in 8 parts, 8 rows: 4.7 with it, 4.1 without; of 128: 5.0 either way, 64 rows in 4 parts 4.8 and 4.9).
   float gates[kKept];
-  constexpr bool kTogether = sizeof(D) == sizeof(float);                  // (the products of this library leave their parts as floats)
-  if (fits && gate != nullptr && (!kTogether || gate_nsplit == 1 || dv <= 64)) {
+  if (PARTS) {
+#pragma unroll
+    for (int i = 0; i < kKept; ++i) kept[i] = fits && lane + 64 * i < dv ? value(lane + 64 * i) : 0.f;
+  }
+  if (!PARTS && fits && gate != nullptr) {
 #pragma unroll
     for (int k = 0; k < kKept; ++k)
       if (64 * k < dv) gates[k] = gate_value(min(lane + 64 * k, dv - 1));
-  } else if (kTogether && fits && gate != nullptr) {
+  } else if (PARTS && gate != nullptr) {
+    __builtin_assume(dv > 128);
     const D* from = gate + static_cast<size_t>(t) * gate_row + gate_col + h * dv;
     float chain[4][kKept] = {};
     int s = 0;
@@ -90,7 +97,7 @@ head_combine_kernel(const float* __restrict__ a, int heads, int dv, int pair_gro
 #pragma unroll
   for (int i = 0; i < kKept; ++i) {
     const int e = lane + 64 * i;
-    kept[i] = fits && e < dv ? value(e) : 0.f;
+    if (!PARTS) kept[i] = fits && e < dv ? value(e) : 0.f;
     if (gate_first && pair_group <= 0 && fits && e < dv) kept[i] *= gates[i];
     squares += kept[i] * kept[i];
   }
@@ -201,6 +208,7 @@ extern "C" int tlie_head_combine(const float* a, int tokens, int heads, int dv, 
                     (gate_nsplit <= 1 || gate_split_stride % 8 == 0) &&
                     ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(weight) | reinterpret_cast<uintptr_t>(gate) |
                       reinterpret_cast<uintptr_t>(out)) & 31) == 0;
+  const bool together = gate != nullptr && gate_nsplit > 1 && dv > 128 && dv <= 512;
 #define TLIE_CASE(GC, D, WC, W, AC, A)                                                                                   \
   if (gate_dtype == GC && weight_dtype == WC && out_dtype == AC) {                                                       \
     if (wide) {                                                                                                          \
@@ -209,9 +217,9 @@ extern "C" int tlie_head_combine(const float* a, int tokens, int heads, int dv, 
                          gate_col, gate_kind, gate_first, (A*)out);                                                                  \
       return launch_status();                                                                                            \
     }                                                                                                                    \
-    hipLaunchKernelGGL((head_combine_kernel<D, W, A>), grid, dim3(256), 0, s, a, heads, dv, pair_group, parts, lambda, eps,     \
-                       (const W*)weight, mult, (const D*)gate, gate_nsplit, (size_t)gate_split_stride, gate_row, gate_col, \
-                       gate_kind, gate_first, (A*)out);                                                                                          \
+    hipLaunchKernelGGL((together ? &head_combine_kernel<D, W, A, (sizeof(D) == sizeof(float))> : &head_combine_kernel<D, W, A, false>), grid, dim3(256), 0, s, \
+                       a, heads, dv, pair_group, parts, lambda, eps, (const W*)weight, mult, (const D*)gate, gate_nsplit, \
+                       (size_t)gate_split_stride, gate_row, gate_col, gate_kind, gate_first, (A*)out);                    \
     return launch_status();                                                                                              \
   }
   TLIE_CASE(kF32, float, kF32, float, kF32, float)
