@@ -329,6 +329,22 @@ def test_decays_from_a_low_rank_product(kind, tokens, channels, rank, dtype):
         assert float((torch.log(got.cpu().double()[mask]) - torch.log(want[mask])).abs().div(1.0 + torch.log(want[mask]).abs()).max()) < 1e-4
 
 
+@pytest.mark.parametrize("tokens,channels", [(63, 100), (512, 100), (513, 100), (64, 2048), (67, 2048), (256, 2040), (257, 2040)])
+@pytest.mark.parametrize("rank,dtype", [(5, torch.bfloat16), (16, torch.bfloat16), (72, torch.float32), (64, torch.bfloat16)])
+def test_decays_by_tiles_of_tokens_are_those_of_single_tokens(tokens, channels, rank, dtype):
+    """On both sides of the lines between the kernel's forms, ranks in eights and others, a last tile that is not full: the bits of
+    calls of a token each, and 64 bits (z up to some 20, of which 1e-6 are lost, exponentiated)."""
+    from tlie_amd import ops
+    generator = torch.Generator(device=DEVICE).manual_seed(tokens + rank)
+    low = torch.randn(tokens, rank, generator=generator, device=DEVICE)
+    weight, bias = (torch.randn(*shape, generator=generator, device=DEVICE).to(dtype) for shape in ((channels, rank), (channels,)))
+    got = ops.low_rank_decay(low, weight, bias, "sigmoid_root", tau=7.0)
+    for token in (0, 1, 7, 8, tokens // 2, tokens - 2, tokens - 1):
+        assert torch.equal(got[token:token + 1], ops.low_rank_decay(low[token:token + 1].contiguous(), weight, bias, "sigmoid_root", tau=7.0)), token
+    want = torch.sigmoid(low.double() @ weight.double().T + bias.double()) ** (1.0 / 7.0)
+    assert float((got.double() - want).abs().max()) < 2e-5
+
+
 def _scan_case(kind, heads, dim, vdim, plan, nsplit, dtype, generator):
     """q, k, v of two sequences, decays of the kind asked for, and the plain walk's results."""
     lengths, steps = plan

@@ -241,23 +241,26 @@ decay_carry_kernel(float* __restrict__ parts, float* __restrict__ state, const i
 
 // out[t, c] = decay(z), z = bias[c] + sum_r weight[c, r] * f(low[t, r]); f the identity or tanh.
 // kind 0: sigmoid(z)^(1 / tau), formed as exp(logsigmoid(z) / tau); kind 1: exp(-exp(z)).  Float throughout.
-// A workgroup takes TT tokens (their low rows lie in LDS) and a thread a channel for all of them, so that a channel's
-// weights are read once for the tile; a step of few tokens takes tiles of one, for the workgroups' number.
-constexpr int kDecayTokens = 8, kDecayTiledFrom = 64;
+// A workgroup takes TT tokens (their low rows lie in LDS) and a thread a channel for all of them, so that a channel's weights are read
+// once for the tile.  Tiles of one token while they come to two workgroups a unit, of four up to eight times that many, of eight beyond:
+// what few workgroups wait for is one token's chain (2048 channels of rank 64, tiles of 1, 4 and 8 in bfloat16: 64 tokens 5.5, 5.7 and 8.2 us,
+// 96 6.5, 5.5 and 7.7, 256 13.5, 7.5 and 8.3, 384 17.4, 9.4 and 9.1; in floats 7.3, 5.6 and 7.7, 9.3, 5.4 and 7.3, 19.1, 8.0 and 7.8, 26.1,
+// 10.2 and 8.9).  An element a load the line lies at 64 tokens (rank 60: 64 tokens 8.2 and, in tiles of eight, 6.9).
+// WIDE (a rank in eights, weights at multiples of their size): a channel's weights in pieces of eight, the first channel's first ahead of
+// the low rows, which come in fours.  (A whole row of 64 asked for at once is slower, by its registers, 94 to 120, and by the code: 4 tokens,
+// 2048 channels of rank 64 in bfloat16 4.5 us, of rank 128 6.5; so 4.1 and 5.5; an element a load 4.6 and 5.9; 100 tokens in tiles of eight, rank 64
+// 9.5, 7.9 and 7.8; 2048 tokens 34.7, 27.9 and 38.4)
+constexpr int kDecayTiledFrom = 64, kDecayWorkgroups = 512;
 
-template <typename W, int TT>
+template <typename W, int TT, bool WIDE>
 __global__ void __launch_bounds__(256)
 low_rank_decay_kernel(const float* __restrict__ low, int nsplit, size_t split_stride, int inner_tanh, const W* __restrict__ weight,
                       const W* __restrict__ bias, int kind, float tau, float* __restrict__ out, int tokens, int channels, int rank) {
-  extern __shared__ float shared_low[];                // [TT][rank]
+  extern __shared__ __attribute__((aligned(16))) float shared_low[];       // [TT][rank]
   const int t0 = blockIdx.x * TT;
-  // a channel's weights in pieces of eight where they fit, the first channel's first ahead of the low rows.  (A whole row of 64 asked for at once
-  // is slower, by its registers, 94 to 120, and by the code: 4 tokens, 2048 channels of rank 64 in bfloat16 4.9 us, of rank 128 7.3; so 4.5
-  // and 6.4; an element a load 5.2 and 6.8; 64 tokens, rank 64 9.2, 7.5 and 7.7; 2048 tokens 34.3, 26.0 and 38.0)
-  const bool wide = rank % 8 == 0 && reinterpret_cast<uintptr_t>(weight) % (8 * sizeof(W)) == 0;
   float piece[8];
   const int first = blockIdx.y * blockDim.x + threadIdx.x;
-  if (wide && first < channels) load8(weight + static_cast<size_t>(first) * rank, piece);
+  if (WIDE && first < channels) load8(weight + static_cast<size_t>(first) * rank, piece);
   const int count = min(TT, tokens - t0);
   if (TT == 1 && nsplit > 4 && rank * 4 <= static_cast<int>(blockDim.x)) {
     // many parts of one token's few values (64 values in 32 parts): a thread a value and chain of `sum_splits`, its parts asked for
@@ -301,13 +304,19 @@ low_rank_decay_kernel(const float* __restrict__ low, int nsplit, size_t split_st
 #pragma unroll
     for (int b = 0; b < TT; ++b) z[b] = start;
     const W* row = weight + static_cast<size_t>(c) * rank;
-    if (wide) {
+    if (WIDE) {
       for (int r0 = 0; r0 < rank; r0 += 8) {
         if (c != first || r0 > 0) load8(row + r0, piece);
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
+        for (int h = 0; h < 8; h += 4) {
+          float4 lows[TT];
 #pragma unroll
-          for (int b = 0; b < TT; ++b) z[b] += piece[j] * shared_low[b * rank + r0 + j];
+          for (int b = 0; b < TT; ++b) lows[b] = *reinterpret_cast<const float4*>(shared_low + b * rank + r0 + h);
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int b = 0; b < TT; ++b) z[b] += piece[h + j] * (&lows[b].x)[j];
+        }
       }
     } else {
       for (int r = 0; r < rank; ++r) {
@@ -431,20 +440,29 @@ extern "C" int tlie_low_rank_decay(const float* low, int nsplit, long long split
   if (tokens <= 0 || channels <= 0 || rank <= 0 || rank > 1024 || nsplit < 1 || kind < 0 || kind > 1 || (kind == 0 && !(tau > 0.f))) return kBadArgument;
   int across = (channels + 255) / 256;
   if (across > 64) across = 64;
-  const int tile = tokens >= kDecayTiledFrom ? kDecayTokens : 1;
+  const bool wide = rank % 8 == 0 && reinterpret_cast<uintptr_t>(weight) % (w_dtype == kF32 ? 32 : 16) == 0;
+  const long long single = static_cast<long long>(tokens) * across;
+  const int tile = wide ? (single <= kDecayWorkgroups ? 1 : single <= 4 * kDecayWorkgroups ? 4 : 8) : (tokens >= kDecayTiledFrom ? 8 : 1);
   const dim3 grid((tokens + tile - 1) / tile, across);
   const size_t lds = static_cast<size_t>(tile) * rank * sizeof(float);
   hipStream_t s = (hipStream_t)stream;
-#define TLIE_LAUNCH(W, TT)                                                                                             \
-  hipLaunchKernelGGL((low_rank_decay_kernel<W, TT>), grid, dim3(256), lds, s, low, nsplit, (size_t)split_stride, inner_tanh, (const W*)weight, \
+#define TLIE_LAUNCH(W, TT, WIDE)                                                                                       \
+  hipLaunchKernelGGL((low_rank_decay_kernel<W, TT, WIDE>), grid, dim3(256), lds, s, low, nsplit, (size_t)split_stride, inner_tanh, (const W*)weight, \
                      (const W*)bias, kind, tau, out, tokens, channels, rank)
+#define TLIE_TILES(W)                                                                                                  \
+  if (!wide && tile == 1) TLIE_LAUNCH(W, 1, false);                                                                    \
+  else if (!wide) TLIE_LAUNCH(W, 8, false);                                                                            \
+  else if (tile == 1) TLIE_LAUNCH(W, 1, true);                                                                         \
+  else if (tile == 4) TLIE_LAUNCH(W, 4, true);                                                                         \
+  else TLIE_LAUNCH(W, 8, true);
   if (w_dtype == kF32) {
-    if (tile == 1) TLIE_LAUNCH(float, 1);
-    else TLIE_LAUNCH(float, kDecayTokens);
+    TLIE_TILES(float)
   } else if (w_dtype == kBF16) {
-    if (tile == 1) TLIE_LAUNCH(bf16, 1);
-    else TLIE_LAUNCH(bf16, kDecayTokens);
-  } else return kBadArgument;
+    TLIE_TILES(bf16)
+  } else {
+    return kBadArgument;
+  }
+#undef TLIE_TILES
 #undef TLIE_LAUNCH
   return launch_status();
 }
