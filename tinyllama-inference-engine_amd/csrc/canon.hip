@@ -602,7 +602,7 @@ extern "C" int tlie_xielu(const void* in, int in_dtype, int nsplit, long long sp
 #define TLIE_CASE(IC, D, NC, W, OC, O)                                                                                   \
   if (in_dtype == IC && n_dtype == NC && out_dtype == OC) {                                                              \
     if (wide)                                                                                                            \
-      hipLaunchKernelGGL(TLIE_PARTS_FORM(nsplit, D, xielu_wide_kernel, D, W, O), dim3((unsigned)((blocks + 7) / 8)), dim3(256), 0, s, (const D*)in,  \
+      hipLaunchKernelGGL(TLIE_PARTS_FORM(nsplit, xielu_wide_kernel, D, W, O), dim3((unsigned)((blocks + 7) / 8)), dim3(256), 0, s, (const D*)in,  \
                          nsplit, (size_t)split_stride, (const W*)numbers, (O*)out, (size_t)count);                        \
     else                                                                                                                 \
       hipLaunchKernelGGL((xielu_kernel<D, W, O>), dim3((unsigned)blocks), dim3(256), 0, s, (const D*)in, nsplit,          \

@@ -212,8 +212,8 @@ __device__ __forceinline__ void load8_splits(const D* __restrict__ part, int nsp
   }
 }
 
-// Of a kernel's two forms, the one for this product (one of 16 bits takes no registers for parts: it has one form).
-#define TLIE_PARTS_FORM(nsplit, D, KERNEL, ...) ((nsplit) == 1 ? &KERNEL<__VA_ARGS__, (sizeof(D) < sizeof(float))> : &KERNEL<__VA_ARGS__, true>)
+// Of a kernel's two forms, the one for this product.
+#define TLIE_PARTS_FORM(nsplit, KERNEL, ...) ((nsplit) == 1 ? &KERNEL<__VA_ARGS__, false> : &KERNEL<__VA_ARGS__, true>)
 
 // The sum of squares of four, or eight, neighbouring columns of the 32-bit path's norms: one order for every kernel that forms it.
 __device__ __forceinline__ float squares_of4(float a, float b, float c, float d) { return fmaf(a, a, b * b) + fmaf(c, c, d * d); }

@@ -381,7 +381,7 @@ static int launch_add_rmsnorm(float* residual, const void* delta, int nsplit, si
   if ((hidden & 7) == 0 && aligned && wide_lds <= 160 * 1024 && (nsplit == 1 || (split_stride * sizeof(D)) % 32 == 0)) {
     const int chunks = hidden / 8;
     const int wide = chunks >= 1024 ? 1024 : (chunks + 63) / 64 * 64;
-    hipLaunchKernelGGL(TLIE_PARTS_FORM(nsplit, D, add_rmsnorm_wide_kernel, D, W, O), dim3(num_rows), dim3(wide), wide_lds, stream, residual,
+    hipLaunchKernelGGL(TLIE_PARTS_FORM(nsplit, add_rmsnorm_wide_kernel, D, W, O), dim3(num_rows), dim3(wide), wide_lds, stream, residual,
                        (const D*)delta, nsplit, split_stride, (const W*)weight, eps, (O*)out, rows, hidden);
     return launch_status();
   }
@@ -433,7 +433,7 @@ extern "C" int tlie_norm_add_rmsnorm(float* residual, const void* delta, int del
 #define TLIE_CASE(DC, D, WC, W, OC, O)                                                                              \
   if (delta_dtype == DC && weight_dtype == WC && out_dtype == OC) {                                                 \
     if (wide) {                                                                                                     \
-      hipLaunchKernelGGL(TLIE_PARTS_FORM(nsplit, D, norm_add_rmsnorm_wide_kernel, D, W, O), dim3(num_rows), dim3(wide_threads), \
+      hipLaunchKernelGGL(TLIE_PARTS_FORM(nsplit, norm_add_rmsnorm_wide_kernel, D, W, O), dim3(num_rows), dim3(wide_threads), \
                          lds, s, residual, (const D*)delta, nsplit, (size_t)split_stride, (const W*)post_weight, post_eps,            \
                          (const W*)weight, eps, (O*)out, rows, hidden);                                              \
       return launch_status();                                                                                       \

@@ -212,7 +212,7 @@ extern "C" int tlie_head_combine(const float* a, int tokens, int heads, int dv, 
 #define TLIE_CASE(GC, D, WC, W, AC, A)                                                                                   \
   if (gate_dtype == GC && weight_dtype == WC && out_dtype == AC) {                                                       \
     if (wide) {                                                                                                          \
-      hipLaunchKernelGGL(TLIE_PARTS_FORM(gate_nsplit, D, head_combine_wide_kernel, D, W, A), dim3(tokens, heads), dim3(256), 0, s, a, heads, dv, eps,    \
+      hipLaunchKernelGGL(TLIE_PARTS_FORM(gate_nsplit, head_combine_wide_kernel, D, W, A), dim3(tokens, heads), dim3(256), 0, s, a, heads, dv, eps,    \
                          (const W*)weight, mult, (const D*)gate, gate_nsplit, (size_t)gate_split_stride, gate_row,       \
                          gate_col, gate_kind, gate_first, (A*)out);                                                                  \
       return launch_status();                                                                                            \
