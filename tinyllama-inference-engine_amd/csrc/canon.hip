@@ -405,18 +405,14 @@ token_shift_kernel(const A* __restrict__ x, const W* __restrict__ mu, float* __r
   read(x + static_cast<size_t>(t) * width + c, now);
   if (held != nullptr) read(held + c, before);
   else read(x + static_cast<size_t>(t - 1) * width + c, before);
-  for (int m0 = 0; m0 < mixes; m0 += 4) {              // (four mixes' numbers asked for together)
-    float blend[4][V];
+  // (one after the other: four mixes' numbers asked for together gain nothing at any number of mixes, 8 rows of 2048 and 5 mixes 3.6 us and 3.7,
+  // and one mix of 2048 tokens takes 6.4 us in place of 5.7)
+  for (int m = 0; m < mixes; ++m) {
+    float blend[V], result[V];
+    read(mu + static_cast<size_t>(m) * width + c, blend);
 #pragma unroll
-    for (int u = 0; u < 4; ++u) read(mu + static_cast<size_t>(min(m0 + u, mixes - 1)) * width + c, blend[u]);
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      if (m0 + u >= mixes) break;
-      float result[V];
-#pragma unroll
-      for (int e = 0; e < V; ++e) result[e] = now[e] + (before[e] - now[e]) * blend[u][e];
-      write(out + (static_cast<size_t>(m0 + u) * tokens + t) * width + c, result);
-    }
+    for (int e = 0; e < V; ++e) result[e] = now[e] + (before[e] - now[e]) * blend[e];
+    write(out + (static_cast<size_t>(m) * tokens + t) * width + c, result);
   }
   if (held != nullptr) {
     float kept[V];
