@@ -215,3 +215,13 @@ def test_plain_depth_average_of_a_model_whose_last_weight_is_one(tmp_path):
     # the same model with a weight on the embedding's output differs from the first layer on
     config, weights = rewrite(folder, lambda w: w["l0.dwa"].__setitem__(0, 0.5))
     assert float((plain.forward(config, weights, tokens)[1][0] - after[0]).abs().max()) > 1e-3
+
+
+def test_norms_of_wide_rows_leave_the_convolution_to_its_own_kernel():
+    """The line lies where one workgroup a row stops being the faster form."""
+    from types import SimpleNamespace
+    from tlie_amd import ops
+    for width, together in ((2048, True), (4608, True), (4616, False), (8192, False)):
+        norm = ops.NormParams(torch.zeros(width), None, 1e-5, True)
+        ctx = SimpleNamespace(max_new=1, num_seqs=2, num_tokens=2, token_slot=torch.zeros(2, dtype=torch.int32))
+        assert (ops.conv_after(torch.zeros(width, 4), torch.zeros(2, 3, width), ctx, norm, torch.float32) is not None) == together, width

@@ -896,13 +896,21 @@ class Convolved:
     rows: torch.Tensor
 
 
+CONV_AFTER_MAX = 4608          # the widest row whose norm applies the convolution behind it
+
+
 def conv_after(taps: torch.Tensor, state: torch.Tensor, ctx, norm: "NormParams", out_dtype: torch.dtype) -> "ConvAfter | None":
     """What `layer_norm` needs to apply `input_conv` to its own result, where its kernel can: every sequence of the step brings one
     token (the convolution of several reads rows that other workgroups norm), four taps, and taps, norm and result of one type in
-    rows that 16-byte loads fit; else None."""
+    rows that 16-byte loads fit; else None.  None too for rows wider than CONV_AFTER_MAX: the norm has one workgroup a row, the
+    convolution by itself one for every 1024 columns (norm and convolution apart and in one, products in parts and depth mix, us: 8 rows of
+    2048 8.2 and 6.5, of 4096 10.4 and 9.4, of 4608 12.0 and 11.3, of 5120 12.2 and 11.7, of 6144 12.7 and 12.3, of 8192 15.1 and 15.7; whole
+    products 7.2 and 6.0, 8.7 and 8.2, 9.9 and 9.7, 10.0 and 10.0, 10.3 and 10.7, 12.5 and 12.8; the same order at 1 to 64 rows, at 128 a
+    little further up)."""
     tensors = [norm.weight, taps, state] + ([norm.bias] if norm.bias is not None else [])
-    if (ctx.max_new != 1 or ctx.num_seqs != ctx.num_tokens or taps.shape[1] != 4 or taps.shape[0] % 8 != 0 or state.stride(0) % 4 != 0
-            or taps.dtype != norm.weight.dtype or taps.dtype != out_dtype or any(tensor.data_ptr() % 16 != 0 for tensor in tensors)):
+    if (ctx.max_new != 1 or ctx.num_seqs != ctx.num_tokens or taps.shape[1] != 4 or taps.shape[0] % 8 != 0 or taps.shape[0] > CONV_AFTER_MAX
+            or state.stride(0) % 4 != 0 or taps.dtype != norm.weight.dtype or taps.dtype != out_dtype
+            or any(tensor.data_ptr() % 16 != 0 for tensor in tensors)):
         return None
     return ConvAfter(taps, state, ctx.token_slot)
 
