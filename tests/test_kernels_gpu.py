@@ -232,6 +232,27 @@ def test_kernels_add_up_parts_of_sixteen_bits_too(monkeypatch, nsplit):
             assert torch.equal(one, other), (heads, dv, first)
 
 
+@pytest.mark.parametrize("dv", [1, 63, 64, 65, 128, 129, 192, 512, 513])
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_heads_norm_and_gate_at_the_edges_of_their_forms(dv, dtype):
+    """Heads of one, two and up to eight dims a lane and of more than are kept; gates whole and in parts, before the norm and behind
+    it; against 64 bits on the values that the kernel reads."""
+    from tlie_amd import ops
+    torch.manual_seed(dv)
+    tokens, heads = 3, 5
+    a, weight = torch.randn(tokens, heads * dv, device=DEV), torch.randn(heads * dv, device=DEV).to(DT[dtype])
+    for nsplit in (1, 3, 8):
+        gate = torch.randn(nsplit, tokens, heads * dv, device=DEV)
+        gate = gate.to(DT[dtype]) if nsplit == 1 else gate
+        z = torch.nn.functional.silu(gate.double().sum(0)).view(tokens, heads, dv)
+        o = a.double().view(tokens, heads, dv)
+        for first in (False, True):
+            x = o * z if first else o
+            want = x / torch.sqrt((x * x).mean(-1, keepdim=True) + 1e-5) * weight.double().view(heads, dv) * (1.0 if first else z)
+            got = ops.head_combine(a, heads, dv, 1e-5, DT[dtype], weight=weight, gate=ops.Product(gate, nsplit), gate_kind="silu", gate_first=first)
+            assert rel_err(got.view(tokens, heads, dv), want) < (2e-6 if dtype == "float32" else 2.0 ** -8), (nsplit, first)
+
+
 @pytest.mark.parametrize("rows, n, k, whole", [(24, 12288, 4096, False), (64, 4096, 11008, False), (64, 2304, 14336, False), (24, 9000, 4096, True),
                                                (17, 2048, 1536, True), (20, 11264, 2048, False), (33, 4096, 14336, False)])
 def test_gemm_ring_is_as_exact_as_the_product_it_stands_in_for(rows, n, k, whole):

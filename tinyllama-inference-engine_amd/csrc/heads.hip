@@ -15,7 +15,7 @@
 
 namespace tlie {
 
-template <typename D, typename W, typename A, bool PARTS>
+template <typename D, typename W, typename A, bool PARTS, int KEPT>
 __global__ void __launch_bounds__(256)
 head_combine_kernel(const float* __restrict__ a, int heads, int dv, int pair_group, int parts, float lambda, float eps,
                     const W* __restrict__ weight, float mult, const D* __restrict__ gate, int gate_nsplit,
@@ -46,8 +46,10 @@ head_combine_kernel(const float* __restrict__ a, int heads, int dv, int pair_gro
     if (gate != nullptr && !gate_first) v *= gate_of;
     out[static_cast<size_t>(t) * heads * dv + c] = from_float<A>(v);
   };
-  // a lane's dims (lane, lane + 64, ...) are read once and kept, up to 512 dims a head; beyond, read again
-  constexpr int kKept = 8;
+  // a lane's dims (lane, lane + 64, ...) are read once and kept, up to 512 dims a head; beyond, read again.  Heads of at most 64, or 128, dims
+  // have forms of KEPT 1 and 2: a wave does so little that the questions whether there is a next dim count (2048 rows of 32 heads of 64 dims
+  // in bfloat16 27.7 us with room for eight, 23.4 with one, of 16 of 128 20.8 and 19.0)
+  constexpr int kKept = KEPT;
   const bool fits = dv <= 64 * kKept;
   float kept[kKept];
   // PARTS (split gates, heads of 129 to 512 dims): the gates' parts are asked for together, and with the result, four parts of all dims at
@@ -208,7 +210,7 @@ extern "C" int tlie_head_combine(const float* a, int tokens, int heads, int dv, 
                     (gate_nsplit <= 1 || gate_split_stride % 8 == 0) &&
                     ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(weight) | reinterpret_cast<uintptr_t>(gate) |
                       reinterpret_cast<uintptr_t>(out)) & 31) == 0;
-  const bool together = gate != nullptr && gate_nsplit > 1 && dv > 128 && dv <= 512;
+  const bool together = gate != nullptr && gate_nsplit > 1 && dv <= 512;
 #define TLIE_CASE(GC, D, WC, W, AC, A)                                                                                   \
   if (gate_dtype == GC && weight_dtype == WC && out_dtype == AC) {                                                       \
     if (wide) {                                                                                                          \
@@ -217,7 +219,8 @@ extern "C" int tlie_head_combine(const float* a, int tokens, int heads, int dv, 
                          gate_col, gate_kind, gate_first, (A*)out);                                                                  \
       return launch_status();                                                                                            \
     }                                                                                                                    \
-    hipLaunchKernelGGL((together ? &head_combine_kernel<D, W, A, (sizeof(D) == sizeof(float))> : &head_combine_kernel<D, W, A, false>), grid, dim3(256), 0, s, \
+    hipLaunchKernelGGL((dv <= 64 ? &head_combine_kernel<D, W, A, false, 1> : dv <= 128 ? &head_combine_kernel<D, W, A, false, 2> :  \
+                        together ? &head_combine_kernel<D, W, A, (sizeof(D) == sizeof(float)), 8> : &head_combine_kernel<D, W, A, false, 8>), grid, dim3(256), 0, s, \
                        a, heads, dv, pair_group, parts, lambda, eps, (const W*)weight, mult, (const D*)gate, gate_nsplit, \
                        (size_t)gate_split_stride, gate_row, gate_col, gate_kind, gate_first, (A*)out);                    \
     return launch_status();                                                                                              \
