@@ -88,10 +88,10 @@ class DecoderModel:
         dict) the named tensors of the reference's ModelTrace are left there as float32 copies:
         "embedding", per run i "layer{i}.input_norm", ".attention_output", ".post_attention_norm",
         ".mlp_output", ".output", then "final_norm" and "logits" at the wanted rows
-        (src/model.cpp:98-231).  A bfloat16 step of at most 16 tokens folds the norms into its
-        products when it serves; with a trace it does not, so that every name is left, unless
-        `ctx.trace_serving_route` asks for the serving route, which leaves the names that exist
-        as tensors there."""
+        (src/model.cpp:98-231).  A step of at most 16 tokens folds the norms into its products when it
+        serves (in bfloat16, and in 32 bits with the same bits as unfolded); with a trace it does
+        not, so that every name is left, unless `ctx.trace_serving_route` asks for the serving route,
+        which in bfloat16 leaves the names that exist as tensors there."""
         runs = self.spec.runs
         trace = getattr(ctx, "trace", None)
         if runs[0].depth_mix is not None:
