@@ -192,7 +192,7 @@ __device__ __forceinline__ float sum_splits(const D* __restrict__ first, int nsp
 // Eight neighbouring elements summed over the parts of a split product, in the order of their index.  The parts are asked for eight at a
 // time: one after the other, each waits for the one before, and a kernel of few rows is little else than that chain (the norm after a
 // product of 64 rows in 8 parts, 2048 columns, 5.2 us one by one, 4.7 so).  They take 64 registers, with which half as many waves fit a
-// compute unit: PARTS false for a product that comes whole, as those of many rows do (2048 x 2048 floats normed 14.7 us with them, 12.0 without).
+// compute unit: PARTS false for a product that comes whole, as those of many rows do (2048 x 2048 floats normed 14.3 us with them, 12.6 without).
 template <bool PARTS, typename D>
 __device__ __forceinline__ void load8_splits(const D* __restrict__ part, int nsplit, size_t stride, float (&d)[8]) {
   load8(part, d);
